@@ -2933,35 +2933,23 @@ __global__ void __launch_bounds__(256) k_mc_triangles(const QsMol *__restrict__ 
 
 /* ------------------------------------------------------------------------------------------ */
 /* closest atom per vertex (computeClosestAtom Kernels.cu:547-604)                              */
-/* closest atom of vertex v (position p) of molecule M, relative to its first atom (-1: none) */
-__device__ __forceinline__ int closest_one(const QsMol &M, float px, float py, float pz, const uint32_t *__restrict__ cstart_all,
-                                           const float4 *__restrict__ sx, const int *__restrict__ perm, int sorted_ids)
+/* The reference visits the 27 clamped cells x-major, z fastest, and keeps the first atom whose
+   rounded distance is strictly below the best so far.  The three z cells of an (x, y) column are
+   consecutive cells, so their atoms are one contiguous range in that same order; a cell the clamp
+   visits twice cannot improve on its first visit. */
+
+/* The walk as the reference's, with a root for every atom whose squared sum is below the best
+   one's (sqrtf is monotone: no other can win): for the vertices closest_one cannot decide. */
+__device__ __noinline__ int closest_walk(const float4 *__restrict__ sx, const uint32_t *__restrict__ cstart, int gn, int cx, int cy,
+                                         int z0, int z1, float px, float py, float pz)
 {
-    const QsGrid G = M.G;
-    const uint32_t *__restrict__ cstart = cstart_all + M.cell_off;
-    int cx = cell_of(px, G.ox, G.dxn), cy = cell_of(py, G.oy, G.dxn), cz = cell_of(pz, G.oz, G.dxn);
-    const int gn = G.gn;
-    /* The reference visits the 27 clamped cells x-major, z fastest, and keeps the first atom whose
-       rounded distance is strictly below the best so far.  The three z cells of an (x, y) column
-       are consecutive cells, so their atoms are one contiguous range in that same order; a cell
-       the clamp visits twice cannot improve on its first visit.  sqrtf is monotonic, so an atom
-       can only win if its squared sum is below the best one's; the root is taken only then. */
-    const int z0 = iclamp(cz - 1, 0, gn - 1), z1 = iclamp(cz + 1, 0, gn - 1);
     int best = -1;
     float min_d = 999999.0f, min_s = INFINITY;
-    /* the nine columns' ranges are loaded before any is walked */
-    int lo9[9], hi9[9];
-#pragma unroll
     for (int k = 0; k < 9; k++) {
         const int ix = iclamp(cx + k / 3 - 1, 0, gn - 1), iy = iclamp(cy + k % 3 - 1, 0, gn - 1);
         const int h = (gn * gn * ix) + (gn * iy);
-        lo9[k] = (int)cstart[h + z0];
-        hi9[k] = (int)cstart[h + z1 + 1];
-    }
-#pragma unroll
-    for (int k = 0; k < 9; k++) {
-        const int lo = lo9[k], hi = hi9[k];
-        for (int id = lo; id < hi; id++) {
+        const int hi = (int)cstart[h + z1 + 1];
+        for (int id = (int)cstart[h + z0]; id < hi; id++) {
             const float4 at = sx[id];
             const float sq = dist3_sq(at.x, at.y, at.z, px, py, pz);
             if (sq < min_s) {
@@ -2974,6 +2962,50 @@ __device__ __forceinline__ int closest_one(const QsMol &M, float px, float py, f
             }
         }
     }
+    return best;
+}
+
+/* closest atom of vertex v (position p) of molecule M, relative to its first atom (-1: none).
+   Bound by VALU issue and by lanes idling in the column loops.  A loop that roots every improving
+   candidate pays for the root on almost every iteration, as some lane of the wave improves on
+   most; so the loop keeps the smallest squared sum, its atom and the second smallest sum, with no
+   branch.  Rounded roots of two sums can only be equal when the sums agree to 2^-22, so unless the
+   two smallest agree to 1e-6 the atom of the smallest one is the reference's; else the vertex is
+   walked again with the roots (50,000-atom 0.2 A mesh 0.192 -> 0.183 ms, 256 molecules at 0.5 A
+   0.955 -> 0.910 ms). */
+__device__ __forceinline__ int closest_one(const QsMol &M, float px, float py, float pz, const uint32_t *__restrict__ cstart_all,
+                                           const float4 *__restrict__ sx, const int *__restrict__ perm, int sorted_ids)
+{
+    const QsGrid G = M.G;
+    const uint32_t *__restrict__ cstart = cstart_all + M.cell_off;
+    int cx = cell_of(px, G.ox, G.dxn), cy = cell_of(py, G.oy, G.dxn), cz = cell_of(pz, G.oz, G.dxn);
+    const int gn = G.gn;
+    const int z0 = iclamp(cz - 1, 0, gn - 1), z1 = iclamp(cz + 1, 0, gn - 1);
+    int best = -1;
+    float min_s = INFINITY, next_s = INFINITY;
+    /* the nine columns' ranges are loaded before any is walked */
+    int lo9[9], hi9[9];
+#pragma unroll
+    for (int k = 0; k < 9; k++) {
+        const int ix = iclamp(cx + k / 3 - 1, 0, gn - 1), iy = iclamp(cy + k % 3 - 1, 0, gn - 1);
+        const int h = (gn * gn * ix) + (gn * iy);
+        /* (a column that the clamp repeats is walked once: its atoms would tie with themselves) */
+        const bool again = (k / 3 && ix == iclamp(cx + k / 3 - 2, 0, gn - 1)) || (k % 3 && iy == iclamp(cy + k % 3 - 2, 0, gn - 1));
+        lo9[k] = (int)cstart[h + z0];
+        hi9[k] = again ? 0 : (int)cstart[h + z1 + 1];
+    }
+#pragma unroll
+    for (int k = 0; k < 9; k++) {
+        const int lo = lo9[k], hi = hi9[k];
+        for (int id = lo; id < hi; id++) {
+            const float4 at = sx[id];
+            const float sq = dist3_sq(at.x, at.y, at.z, px, py, pz);
+            next_s = __builtin_amdgcn_fmed3f(sq, min_s, next_s); /* second smallest: min_s <= next_s */
+            best = (sq < min_s) ? id : best;
+            min_s = fminf(sq, min_s);
+        }
+    }
+    if (!(next_s > min_s * 1.000001f) && best >= 0) best = closest_walk(sx, cstart, gn, cx, cy, z0, z1, px, py, pz);
     /* atom indices are returned relative to the molecule's first atom */
     return (best < 0) ? -1 : ((sorted_ids ? best : perm[best]) - (int)M.atom_off);
 }
@@ -3095,10 +3127,8 @@ __device__ __forceinline__ void smooth_sum(const SmoothView &S, uint32_t v, int 
             for (int t = 0; t < nt4[k]; t++) {
                 const int *tt = tri + 3 * (size_t)(tb4[k] + t);
                 const uint32_t a = (uint32_t)tt[0], b = (uint32_t)tt[1], c = (uint32_t)tt[2];
-                if (a == v) push_pair(src, b, c, sx, sy, sz);
-                else if (b == v) push_pair(src, a, c, sx, sy, sz);
-                else if (c == v) push_pair(src, a, b, sx, sy, sz);
-                else continue;
+                if (a != v && b != v && c != v) continue;
+                push_pair(src, a == v ? b : a, c == v ? b : c, sx, sy, sz);
                 cnt += 2;
             }
         }

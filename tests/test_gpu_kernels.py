@@ -1,0 +1,30 @@
+"""Kernels at the sizes and inputs where their rules change, against the CPU oracle (bit for bit)."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _same(a, b):
+    return (a[0].shape == b[0].shape and a[1].shape == b[1].shape and np.array_equal(a[1], b[1])
+            and np.array_equal(a[0].view(np.uint32), b[0].view(np.uint32)) and np.array_equal(a[2], b[2]))
+
+
+def _closest_case(qs, kind):
+    pos, rad = qs.synth_ball(61, 400)
+    if kind == "every atom twice":  # equal distances at every vertex: the first in (cell, index) order wins
+        return np.repeat(pos, 2, axis=0), np.repeat(rad, 2)
+    if kind == "far from the origin":  # coordinates in steps of 2^-9 A: many sums and roots agree
+        return pos + np.float32(20000.0), rad
+    if kind == "two atoms":  # a grid of a few cells, every column next to a clamped one
+        return np.array([[0, 0, 0], [3, 0, 0]], np.float32), np.array([1.7, 1.7], np.float32)
+    ax = np.arange(-2, 3, dtype=np.float32) * np.float32(2.5)  # mirror planes on grid planes
+    return np.stack(np.meshgrid(ax, ax, ax, indexing="ij"), -1).reshape(-1, 3), np.full(125, 1.6, np.float32)
+
+
+@pytest.mark.parametrize("kind", ["every atom twice", "far from the origin", "two atoms", "mirror planes"])
+@pytest.mark.parametrize("reso", [0.25, 0.5])
+def test_closest_atom_ties_and_clamps(qs, orc, kind, reso):
+    pos, rad = _closest_case(qs, kind)
+    print("case closest atom: %s reso=%.2f" % (kind, reso), flush=True)
+    assert _same(qs.compute_ses(pos, rad, reso, 0), orc.compute_ses(pos, rad, reso, 0))
