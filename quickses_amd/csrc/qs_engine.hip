@@ -232,7 +232,7 @@ int Engine::reserve(uint64_t vox, uint64_t atoms, uint64_t cells, uint64_t verts
     cells += 1;
     verts += 1;
     for (DevBuf *b : {&outm, &shellm, &negm, &zerom}) QS_TRY(ensure(*b, nw * 8));
-    for (DevBuf *b : {&wcnt, &vbw, &tbw, &alist, &avb, &atb}) QS_TRY(ensure(*b, nw * 4));
+    for (DevBuf *b : {&wcnt, &vbw, &tbw, &alist, &avb, &acb}) QS_TRY(ensure(*b, nw * 4));
     QS_TRY(ensure(s4, nw * 32));
     QS_TRY(ensure(ntb, nw * 24));
     QS_TRY(ensure(field, vox * 4));
@@ -545,9 +545,9 @@ int Engine::mesh_stage(size_t at_mc, uint32_t nb_mc, size_t at_wpre, StageTimer 
     QS_TRY(ensure(tbw, nw * 4));
     QS_TRY(ensure(alist, nw * 4));
     QS_TRY(ensure(avb, nw * 4));
-    QS_TRY(ensure(atb, nw * 4));
+    QS_TRY(ensure(acb, nw * 4));
     QS_TRY(ensure(ntb, nw * 24));
-    QS_TRY(ensure(totals, 16));
+    QS_TRY(ensure(totals, 20));
     /* Vertex and triangle pools.  The totals stay on the device: the emission, closest-atom,
        smoothing and filter kernels read them there and run as persistent blocks over the pools,
        so nothing waits for the host until the run's results are read back at its end, which is
@@ -564,7 +564,7 @@ int Engine::mesh_stage(size_t at_mc, uint32_t nb_mc, size_t at_wpre, StageTimer 
         qs_launch_mc_count(batch(at_mc, 0, nmol), nb_mc, as<uint64_t>(negm), as<uint64_t>(zerom), as<uint64_t>(s4),
                            as<uint32_t>(wcnt), as<uint64_t>(ntb), stream);
     if (scan_nw) {
-        QS_TRY(ensure(scan_tmp, 3 * qs_scan_tiles(scan_nw) * sizeof(uint32_t)));
+        QS_TRY(ensure(scan_tmp, 4 * qs_scan_tiles(scan_nw) * sizeof(uint32_t)));
         QsBlockStarts bs;
         bs.vstart = as<uint32_t>(vstart);
         bs.nv = pool_v / 256 + 1;
@@ -574,10 +574,10 @@ int Engine::mesh_stage(size_t at_mc, uint32_t nb_mc, size_t at_wpre, StageTimer 
         bs.nzero = pool_t / 256 + 1;
         qs_launch_mc_scans(as<uint32_t>(wcnt) + scan_w0, scan_nw, as<uint32_t>(scan_tmp),
                            as<uint32_t>(vbw) + scan_w0, as<uint32_t>(tbw) + scan_w0, as<uint32_t>(alist), as<uint32_t>(avb),
-                           as<uint32_t>(atb), as<uint32_t>(totals), (uint32_t)scan_w0, stream, bs);
+                           as<uint32_t>(acb), as<uint32_t>(totals), (uint32_t)scan_w0, stream, bs);
         QS_HIP(hipGetLastError());
     } else {
-        QS_HIP(hipMemsetAsync(totals.p, 0, 16, stream));
+        QS_HIP(hipMemsetAsync(totals.p, 0, 20, stream));
     }
     tm.mark("mc_count");
     /* per-molecule first vertex and triangle (the scans at each molecule's first word, from the
@@ -606,9 +606,9 @@ int Engine::mesh_stage(size_t at_mc, uint32_t nb_mc, size_t at_wpre, StageTimer 
     const bool fork_vertices = overlap && nmol == 1;
     qs_launch_mc_emit(as<QsMol>(d_mols), wpre, wcoarse, as<uint32_t>(alist), nact_max, as<uint32_t>(avb), as<uint32_t>(vstart),
                       pool_v, as<uint64_t>(s4), as<float>(field), field_sparse ? as<uint32_t>(spre) : nullptr, as<uint64_t>(outm),
-                      field_sparse ? as<uint64_t>(shellm) : nullptr, as<float>(vert), as<uint64_t>(vkey), as<uint32_t>(atb),
-                      as<uint32_t>(tstart), pool_t, as<uint64_t>(negm), as<uint64_t>(zerom), as<uint32_t>(vbw),
-                      as<uint64_t>(ntb), as<int>(tri), 0u, as<uint32_t>(deg_blk), as<uint32_t>(totals) + 3, counts, stream,
+                      field_sparse ? as<uint64_t>(shellm) : nullptr, as<float>(vert), as<uint64_t>(vkey), as<uint32_t>(acb),
+                      as<uint32_t>(tstart), pool_t, pool_t, as<uint64_t>(negm), as<uint32_t>(wcnt), as<uint32_t>(vbw),
+                      as<uint32_t>(tbw), as<uint64_t>(ntb), as<int>(tri), 0u, as<uint32_t>(deg_blk), as<uint32_t>(totals) + 3, counts, stream,
                       fork_vertices ? side : stream, ev_emit, ev_vert, scan_nw != 0);
     QS_HIP(hipGetLastError());
     vert_pending = fork_vertices;
@@ -719,28 +719,28 @@ int Engine::slab_mesh(size_t at_mc, uint32_t nb_mc, size_t at_wpre, uint64_t own
 {
     const uint64_t nw = std::max<uint64_t>(nw_total, 1);
     QS_TRY(ensure(s4, nw * 32));
-    for (DevBuf *b : {&wcnt, &vbw, &tbw, &alist, &avb, &atb}) QS_TRY(ensure(*b, nw * 4));
+    for (DevBuf *b : {&wcnt, &vbw, &tbw, &alist, &avb, &acb}) QS_TRY(ensure(*b, nw * 4));
     QS_TRY(ensure(ntb, nw * 24));
-    QS_TRY(ensure(totals, 16));
+    QS_TRY(ensure(totals, 20));
     if (nb_mc)
         qs_launch_mc_count(batch(at_mc, 0, 1), nb_mc, as<uint64_t>(negm), as<uint64_t>(zerom), as<uint64_t>(s4),
                            as<uint32_t>(wcnt), as<uint64_t>(ntb), stream);
-    QS_TRY(ensure(scan_tmp, 3 * qs_scan_tiles(std::max<uint64_t>(scan_nw, 1)) * sizeof(uint32_t)));
+    QS_TRY(ensure(scan_tmp, 4 * qs_scan_tiles(std::max<uint64_t>(scan_nw, 1)) * sizeof(uint32_t)));
     qs_launch_mc_scans(as<uint32_t>(wcnt) + scan_w0, scan_nw, as<uint32_t>(scan_tmp),
                        as<uint32_t>(vbw) + scan_w0, as<uint32_t>(tbw) + scan_w0, as<uint32_t>(alist), as<uint32_t>(avb),
-                       as<uint32_t>(atb), as<uint32_t>(totals), (uint32_t)scan_w0, stream);
+                       as<uint32_t>(acb), as<uint32_t>(totals), (uint32_t)scan_w0, stream);
     QS_HIP(hipGetLastError());
-    uint32_t hb[4] = {0, 0, 0, 0};
+    uint32_t hb[6] = {0, 0, 0, 0, 0, 0};
     uint32_t *hs = (uint32_t *)stage(sizeof(hb));
     uint32_t *hd = hs ? hs : hb;
-    QS_HIP(hipMemcpyAsync(hd, totals.p, 12, hipMemcpyDeviceToHost, stream));
+    QS_HIP(hipMemcpyAsync(hd, totals.p, 20, hipMemcpyDeviceToHost, stream));
     if (owned_word != ~0ull)
-        QS_HIP(hipMemcpyAsync(hd + 3, as<uint32_t>(vbw) + owned_word, 4, hipMemcpyDeviceToHost, stream));
+        QS_HIP(hipMemcpyAsync(hd + 5, as<uint32_t>(vbw) + owned_word, 4, hipMemcpyDeviceToHost, stream));
     QS_HIP(hipStreamSynchronize(stream));
     if (hs) memcpy(hb, hs, sizeof(hb));
     n_tri = hb[0];
     const uint32_t nact = hb[2];
-    n_owned = (owned_word != ~0ull) ? hb[3] : hb[1];
+    n_owned = (owned_word != ~0ull) ? hb[5] : hb[1];
     if ((uint64_t)vbase + n_owned >= (1ull << 31) || 3 * ((uint64_t)tbase + n_tri) >= (1ull << 31))
         return set_error(4, "mesh too large");
     QS_TRY(grow_keep(vert, ((size_t)vbase + n_owned + 1) * 12, (size_t)vbase * 12, stream));
@@ -753,8 +753,8 @@ int Engine::slab_mesh(size_t at_mc, uint32_t nb_mc, size_t at_wpre, uint64_t own
     const uint32_t *wcoarse = as<uint32_t>(d_meta) + at_wpre + 4;
     qs_launch_mc_emit(as<QsMol>(d_mols), wpre, wcoarse, as<uint32_t>(alist), nact, as<uint32_t>(avb), as<uint32_t>(vstart),
                       n_owned, as<uint64_t>(s4), as<float>(field), as<uint32_t>(spre), as<uint64_t>(outm), as<uint64_t>(shellm),
-                      as<float>(vert) + 3 * (size_t)vbase, as<uint64_t>(vkey), as<uint32_t>(atb), as<uint32_t>(tstart), n_tri,
-                      as<uint64_t>(negm), as<uint64_t>(zerom), as<uint32_t>(vbw), as<uint64_t>(ntb),
+                      as<float>(vert) + 3 * (size_t)vbase, as<uint64_t>(vkey), as<uint32_t>(acb), as<uint32_t>(tstart), hb[4], n_tri,
+                      as<uint64_t>(negm), as<uint32_t>(wcnt), as<uint32_t>(vbw), as<uint32_t>(tbw), as<uint64_t>(ntb),
                       as<int>(tri) + 3 * (size_t)tbase, vbase, as<uint32_t>(deg_blk), as<uint32_t>(totals) + 3, nullptr, stream);
     QS_HIP(hipGetLastError());
     return 0;

@@ -82,30 +82,31 @@ void qs_launch_labels_to_masks(const uint8_t *labels, int g, int W, uint64_t *ou
 uint32_t qs_mc_count_blocks(const QsMol &M);
 /* per row word: slot masks (words with vertices only), vertex and triangle counts, triangle-count
    bit planes (words with triangles only) */
-/* cnt: per row word its vertex count | triangle count << 16 */
+/* cnt: per row word its vertex, triangle and cube counts, packed */
 void qs_launch_mc_count(QsBatch B, uint32_t nblocks, const uint64_t *N, const uint64_t *Zm, uint64_t *S4, uint32_t *cnt,
                         uint64_t *NT, hipStream_t s);
-/* one thread per vertex / per triangle over the active words (list, with their first vertex ids
-   avb and first triangle ids atb), after one launch that gives vstart / tstart each 256-item
-   block's first active word (nv / 256 + 1 and ntri / 256 + 1 entries) and clears deg_blk, unless
-   starts_ready says that the word scans did (QsBlockStarts).  The
-   field F holds the shell voxels' values only, at their shell ranks (spre), the others come from
-   the outside / shell masks (shellm == nullptr: F holds every voxel in grid order, spre is
-   unused).  Triangle corners are vertex ids plus vbase; degenerate triangles are counted per
-   256-triangle block (deg_blk) and in total.  The block starts and the triangle kernel run on s;
+/* one thread per vertex / per polygonised cube over the active words (list, with their first
+   vertex ids avb and first cubes acb), after one launch that gives vstart / tstart each 256-item
+   block's first active word (nv / 256 + 1 and ncube / 256 + 1 entries) and clears deg_blk (ntri /
+   256 + 1 entries), unless starts_ready says that the word scans did (QsBlockStarts).  ncube: the
+   cubes, or a bound on them.  The field F holds the shell voxels' values only, at their shell ranks
+   (spre), the others come from the outside / shell masks (shellm == nullptr: F holds every voxel in
+   grid order, spre is unused).  cnt: the words' packed counts; tbw: their first triangles.  Triangle
+   corners are vertex ids plus vbase; degenerate triangles are counted per 256-triangle block
+   (deg_blk) and in total.  The block starts and the triangle kernel run on s;
    the vertex kernel on s_vert: when that is another stream it waits there for the block starts
    (event ev_fork), and ev_vert is recorded on s_vert after it. */
 void qs_launch_mc_emit(const QsMol *mols, const uint64_t *wpre, const uint32_t *wcoarse, const uint32_t *list, uint32_t nact,
                        const uint32_t *avb, uint32_t *vstart, uint32_t nv, const uint64_t *S4, const float *F,
                        const uint32_t *spre, const uint64_t *outm, const uint64_t *shellm, float *vert, uint64_t *vkey,
-                       const uint32_t *atb, uint32_t *tstart, uint32_t ntri, const uint64_t *N, const uint64_t *Zm,
-                       const uint32_t *vbw, const uint64_t *NT, int *tri, uint32_t vbase, uint32_t *deg_blk,
+                       const uint32_t *acb, uint32_t *tstart, uint32_t ncube, uint32_t ntri, const uint64_t *N, const uint32_t *cnt,
+                       const uint32_t *vbw, const uint32_t *tbw, const uint64_t *NT, int *tri, uint32_t vbase, uint32_t *deg_blk,
                        uint32_t *deg_total, const uint32_t *d_counts, hipStream_t s, hipStream_t s_vert = nullptr,
                        hipEvent_t ev_fork = nullptr, hipEvent_t ev_vert = nullptr, bool starts_ready = false);
 
 /* Launches whose item counts live on the device take them from the d_* pointers (when given),
    the host counts being the pools the launch covers: marching-cubes totals are counts[0]
-   triangles, counts[1] vertices, counts[2] active words. */
+   triangles, counts[1] vertices, counts[2] active words, counts[4] cubes. */
 
 /* per-molecule first vertex (vpre, u32) and first triangle (tpre, u64) from the word scans at each
    molecule's first word (wpre[m]; at or past the nw scanned words for none), nmol + 1 entries
@@ -175,7 +176,7 @@ void qs_launch_tile_scan(const uint32_t *in, uint32_t *out, uint64_t n, const ui
                          hipStream_t s, const uint32_t *self_sums = nullptr);
 void qs_launch_copy(const void *src, void *dst, uint64_t bytes, hipStream_t s);
 /* The emission launches' block starts, written by the word scans when the pools are known
-   before them: vstart / tstart hold the first active word of each 256-vertex / 256-triangle block
+   before them: vstart / tstart hold the first active word of each 256-vertex / 256-cube block
    (nv / nt entries), and the nzero counters at zero (the triangle kernel's degenerate counts) are
    cleared.  A null vstart writes none of them (qs_launch_mc_emit then computes them). */
 struct QsBlockStarts {
@@ -188,11 +189,11 @@ struct QsBlockStarts {
 };
 
 /* marching-cubes word scans over the packed counts of qs_launch_mc_count: vbw, tbw, the
-   active-word list and totals {triangles, vertices, active words}; sums holds
-   3 * qs_scan_tiles(nw) entries; list entries are list_base + the word's index in cnt; and the
+   active-word list with its words' first vertices and cubes (avb, acb), and totals {triangles,
+   vertices, active words, 0, cubes}; sums holds 4 * qs_scan_tiles(nw) entries; list entries are list_base + the word's index in cnt; and the
    block starts of bs */
 void qs_launch_mc_scans(const uint32_t *cnt, uint64_t nw, uint32_t *sums, uint32_t *vbw,
-                        uint32_t *tbw, uint32_t *list, uint32_t *avb, uint32_t *atb, uint32_t *totals, uint32_t list_base,
+                        uint32_t *tbw, uint32_t *list, uint32_t *avb, uint32_t *acb, uint32_t *totals, uint32_t list_base,
                         hipStream_t s, QsBlockStarts bs = QsBlockStarts{});
 void qs_launch_gather_u32(const uint32_t *src, const uint64_t *idx, int n, uint32_t *out, hipStream_t s);
 

@@ -46,6 +46,15 @@ constexpr uint32_t edge_axis_bits()
 constexpr uint32_t kEdgeLX = edge_low_bits(0), kEdgeLY = edge_low_bits(1), kEdgeLZ = edge_low_bits(2);
 constexpr uint32_t kEdgeAX = edge_axis_bits();
 static_assert(kEdgeLX == 0x622u && kEdgeLY == 0xC44u && kEdgeLZ == 0xF0u && kEdgeAX == 0xAA4444u, "edge tables");
+/* the same, five bits per edge: low corner's z offset, x offset, y offset, axis (two bits) */
+constexpr uint64_t edge_packed()
+{
+    uint64_t m = 0;
+    for (int e = 0; e < 12; e++)
+        m |= (uint64_t)(kEdgeLow[e][2] | kEdgeLow[e][0] << 1 | kEdgeLow[e][1] << 2 | kEdgeAxis[e] << 3) << (5 * e);
+    return m;
+}
+constexpr uint64_t kEdgePacked = edge_packed();
 
 /* ------------------------------------------------------------------------------------------ */
 /* small helpers                                                                                */
@@ -342,37 +351,48 @@ __global__ void __launch_bounds__(SCAN_NT) k_shell_scan(const uint64_t *__restri
     }
 }
 
-/* Marching-cubes word scans in one pass: per row word its vertex count, triangle count and
-   "active" flag (either nonzero) are scanned together.  Plane 0 = triangles, 1 = vertices,
-   2 = active words; tile sums are stored plane-major (3 x ntiles). */
-__global__ void __launch_bounds__(SCAN_NT) k_mc_reduce3(const uint32_t *__restrict__ cnt, uint64_t n, uint32_t *__restrict__ sums,
+/* a row word's counts, packed by k_mc_count: vertices (at most 4 x 64), triangles (at most 5 x 64)
+   and polygonised cubes (at most 64) */
+__device__ __forceinline__ uint32_t word_counts(uint32_t nv, uint32_t nt, uint32_t nc) { return nv | nt << 9 | nc << 18; }
+__device__ __forceinline__ uint32_t word_verts(uint32_t c) { return c & 511u; }
+__device__ __forceinline__ uint32_t word_tris(uint32_t c) { return (c >> 9) & 511u; }
+__device__ __forceinline__ uint32_t word_cubes(uint32_t c) { return c >> 18; }
+
+/* Marching-cubes word scans in one pass: per row word its vertex, triangle and cube counts and
+   "active" flag (any nonzero) are scanned together.  Plane 0 = triangles, 1 = vertices, 2 = active
+   words, 3 = cubes; tile sums are stored plane-major (4 x ntiles). */
+__global__ void __launch_bounds__(SCAN_NT) k_mc_reduce4(const uint32_t *__restrict__ cnt, uint64_t n, uint32_t *__restrict__ sums,
                                                         uint64_t ntiles)
 {
     __shared__ uint32_t lds[SCAN_NT / 64 + 1];
     const uint64_t base = (uint64_t)blockIdx.x * SCAN_TILE;
-    uint32_t sv = 0, st = 0, sa = 0;
+    uint32_t sv = 0, st = 0, sa = 0, sc = 0;
 #pragma unroll
     for (int k = 0; k < SCAN_IPT; k++) {
         const uint64_t i = base + (uint64_t)k * SCAN_NT + threadIdx.x;
         if (i < n) {
-            const uint32_t c = cnt[i], v = c & 0xFFFFu, t = c >> 16;
-            sv += v;
-            st += t;
-            sa += (v | t) ? 1u : 0u;
+            const uint32_t c = cnt[i];
+            sv += word_verts(c);
+            st += word_tris(c);
+            sc += word_cubes(c);
+            sa += c ? 1u : 0u;
         }
     }
     const uint32_t tt = block_sum<SCAN_NT>(st, lds);
     const uint32_t tv = block_sum<SCAN_NT>(sv, lds);
     const uint32_t ta = block_sum<SCAN_NT>(sa, lds);
+    const uint32_t tc = block_sum<SCAN_NT>(sc, lds);
     if (threadIdx.x == 0) {
         sums[blockIdx.x] = tt;
         sums[ntiles + blockIdx.x] = tv;
         sums[2 * ntiles + blockIdx.x] = ta;
+        sums[3 * ntiles + blockIdx.x] = tc;
     }
 }
 
-/* block p: exclusive scan of plane p of the tile sums in place, total to totals[p]; the slot
-   after the plane totals (the degenerate-triangle count, accumulated later) starts at zero */
+/* block p: exclusive scan of plane p of the tile sums in place, total to totals[p], plane 3's to
+   totals[4]: totals[3] (the degenerate-triangle count, accumulated later), or the slot after a
+   single plane's total, starts at zero */
 __global__ void __launch_bounds__(SCAN_NT) k_scan_planes(uint32_t *__restrict__ sums, uint64_t ntiles,
                                                          uint32_t *__restrict__ totals)
 {
@@ -396,8 +416,8 @@ __global__ void __launch_bounds__(SCAN_NT) k_scan_planes(uint32_t *__restrict__ 
         }
         carry += tot;
     }
-    if (threadIdx.x == 0) totals[blockIdx.x] = carry;
-    if (blockIdx.x == 0 && threadIdx.x == 0) totals[gridDim.x] = 0u;
+    if (threadIdx.x == 0) totals[blockIdx.x + (blockIdx.x >= 3u ? 1u : 0u)] = carry;
+    if (blockIdx.x == 0 && threadIdx.x == 0) totals[min(gridDim.x, 3u)] = 0u;
 }
 
 /* An active word with items [first, first + count) is where every 256-item block whose first
@@ -410,38 +430,38 @@ __device__ __forceinline__ void mark_block_starts(uint32_t *__restrict__ start, 
 }
 
 /* per word: first vertex (vbw) and first triangle (tbw); active words listed in order; with
-   bs.vstart, the first active word of every 256-vertex and 256-triangle block, and the triangle
+   bs.vstart, the first active word of every 256-vertex and 256-cube block, and the triangle
    blocks' counters cleared */
-__global__ void __launch_bounds__(SCAN_NT) k_mc_scan3(const uint32_t *__restrict__ cnt, uint64_t n, const uint32_t *__restrict__ sums, uint64_t ntiles,
+__global__ void __launch_bounds__(SCAN_NT) k_mc_scan4(const uint32_t *__restrict__ cnt, uint64_t n, const uint32_t *__restrict__ sums, uint64_t ntiles,
                                                       uint32_t *__restrict__ vbw, uint32_t *__restrict__ tbw,
                                                       uint32_t *__restrict__ list, uint32_t *__restrict__ avb,
-                                                      uint32_t *__restrict__ atb, uint32_t list_base, int self,
+                                                      uint32_t *__restrict__ acb, uint32_t list_base, int self,
                                                       uint32_t *__restrict__ totals, QsBlockStarts bs)
 {
     if (bs.zero)
         for (uint32_t i = blockIdx.x * SCAN_NT + threadIdx.x; i < bs.nzero; i += gridDim.x * SCAN_NT) bs.zero[i] = 0u;
     /* (self: sums holds the raw tile sums of at most QS_SCAN_SELF_TILES tiles, each tile adds up
-       the ones before it, and the last tile writes totals = {triangles, vertices, active, 0}) */
+       the ones before it, and the last tile writes totals = {triangles, vertices, active, 0, cubes}) */
     /* wave w of the block takes words [w * 512, (w + 1) * 512) of the tile, 64 consecutive words
        per load (as k_shell_scan); the three scans run per group of 64 in order, carried across
        groups, and each group's active words are listed in order by ballot */
-    __shared__ uint32_t wsum[3][SCAN_NT / 64];
+    __shared__ uint32_t wsum[4][SCAN_NT / 64];
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
     const uint64_t base = (uint64_t)blockIdx.x * SCAN_TILE + (uint64_t)wid * (64 * SCAN_IPT) + lane;
     const uint64_t below = (1ull << lane) - 1ull;
-    uint32_t v[SCAN_IPT], t[SCAN_IPT], pv[SCAN_IPT], pt[SCAN_IPT], pa[SCAN_IPT];
-    uint64_t am[SCAN_IPT];
+    uint32_t cw[SCAN_IPT], pv[SCAN_IPT], pt[SCAN_IPT], pc[SCAN_IPT], pa[SCAN_IPT];
 #pragma unroll
     for (int k = 0; k < SCAN_IPT; k++) {
         const uint64_t i = base + 64 * k;
-        const uint32_t c = (i < n) ? cnt[i] : 0u;
-        v[k] = c & 0xFFFFu;
-        t[k] = c >> 16;
+        cw[k] = (i < n) ? cnt[i] : 0u;
     }
-    uint32_t rv = 0, rt = 0, ra = 0; /* the wave's earlier groups */
+    uint32_t rv = 0, rt = 0, rc = 0, ra = 0; /* the wave's earlier groups */
 #pragma unroll
     for (int k = 0; k < SCAN_IPT; k++) {
-        uint32_t xv = v[k], xt = t[k];
+        /* triangles and cubes of a group of 64 words are scanned in one register (at most 64 x 320
+           and 64 x 64) */
+        uint32_t xv = word_verts(cw[k]), xt = word_tris(cw[k]) | word_cubes(cw[k]) << 16;
+        const uint32_t own = xt;
 #pragma unroll
         for (int d = 1; d < 64; d <<= 1) {
             const uint32_t yv = __shfl_up(xv, d, 64), yt = __shfl_up(xt, d, 64);
@@ -450,46 +470,55 @@ __global__ void __launch_bounds__(SCAN_NT) k_mc_scan3(const uint32_t *__restrict
                 xt += yt;
             }
         }
-        am[k] = __ballot((v[k] | t[k]) != 0u);
-        pv[k] = rv + xv - v[k];
-        pt[k] = rt + xt - t[k];
-        pa[k] = ra + (uint32_t)__popcll(am[k] & below);
+        const uint64_t am = __ballot(cw[k] != 0u);
+        pv[k] = rv + xv - word_verts(cw[k]);
+        pt[k] = rt + ((xt - own) & 0xFFFFu);
+        pc[k] = rc + ((xt - own) >> 16);
+        pa[k] = ra + (uint32_t)__popcll(am & below);
         rv += __shfl(xv, 63, 64);
-        rt += __shfl(xt, 63, 64);
-        ra += (uint32_t)__popcll(am[k]);
+        const uint32_t last = __shfl(xt, 63, 64);
+        rt += last & 0xFFFFu;
+        rc += last >> 16;
+        ra += (uint32_t)__popcll(am);
     }
     if (lane == 0) {
         wsum[0][wid] = rv;
         wsum[1][wid] = rt;
         wsum[2][wid] = ra;
+        wsum[3][wid] = rc;
     }
     __syncthreads();
-    uint32_t ov, ot, oa;
+    uint32_t ov, ot, oa, oc;
     if (self) {
         ot = wave_sum_below(sums, blockIdx.x);
         ov = wave_sum_below(sums + ntiles, blockIdx.x);
         oa = wave_sum_below(sums + 2 * ntiles, blockIdx.x);
+        oc = wave_sum_below(sums + 3 * ntiles, blockIdx.x);
         if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) {
-            uint32_t tv = ov, tt = ot, ta = oa;
+            uint32_t tv = ov, tt = ot, ta = oa, tc = oc;
             for (int w = 0; w < SCAN_NT / 64; w++) {
                 tv += wsum[0][w];
                 tt += wsum[1][w];
                 ta += wsum[2][w];
+                tc += wsum[3][w];
             }
             totals[0] = tt;
             totals[1] = tv;
             totals[2] = ta;
             totals[3] = 0u;
+            totals[4] = tc;
         }
     } else {
         ov = sums[ntiles + blockIdx.x];
         ot = sums[blockIdx.x];
         oa = sums[2 * ntiles + blockIdx.x];
+        oc = sums[3 * ntiles + blockIdx.x];
     }
     for (int w = 0; w < wid; w++) {
         ov += wsum[0][w];
         ot += wsum[1][w];
         oa += wsum[2][w];
+        oc += wsum[3][w];
     }
 #pragma unroll
     for (int k = 0; k < SCAN_IPT; k++) {
@@ -497,14 +526,14 @@ __global__ void __launch_bounds__(SCAN_NT) k_mc_scan3(const uint32_t *__restrict
         if (i < n) {
             vbw[i] = ov + pv[k];
             tbw[i] = ot + pt[k];
-            if ((am[k] >> lane) & 1ull) {
+            if (cw[k]) {
                 const uint32_t r = oa + pa[k];
                 avb[r] = ov + pv[k];
-                atb[r] = ot + pt[k];
+                acb[r] = oc + pc[k];
                 list[r] = list_base + (uint32_t)i;
                 if (bs.vstart) {
-                    mark_block_starts(bs.vstart, bs.nv, ov + pv[k], v[k], r);
-                    mark_block_starts(bs.tstart, bs.nt, ot + pt[k], t[k], r);
+                    mark_block_starts(bs.vstart, bs.nv, ov + pv[k], word_verts(cw[k]), r);
+                    mark_block_starts(bs.tstart, bs.nt, oc + pc[k], word_cubes(cw[k]), r);
                 }
             }
         }
@@ -603,49 +632,51 @@ __global__ void __launch_bounds__(SCAN1_NT) k_shell_scan1(const uint64_t *__rest
     }
 }
 
-/* marching-cubes word scans (as k_mc_reduce3, k_scan_planes, k_mc_scan3): totals = {triangles,
-   vertices, active words, 0} */
+/* marching-cubes word scans (as k_mc_reduce4, k_scan_planes, k_mc_scan4): totals = {triangles,
+   vertices, active words, 0, cubes} */
 __global__ void __launch_bounds__(SCAN1_NT) k_mc_scan1(const uint32_t *__restrict__ cnt, uint64_t n, uint32_t *__restrict__ vbw, uint32_t *__restrict__ tbw,
                                                        uint32_t *__restrict__ list, uint32_t *__restrict__ avb,
-                                                       uint32_t *__restrict__ atb, uint32_t list_base,
+                                                       uint32_t *__restrict__ acb, uint32_t list_base,
                                                        uint32_t *__restrict__ totals, QsBlockStarts bs)
 {
-    __shared__ uint32_t wsum[3][SCAN1_W];
+    __shared__ uint32_t wsum[4][SCAN1_W];
     if (bs.zero)
         for (uint32_t i = threadIdx.x; i < bs.nzero; i += SCAN1_NT) bs.zero[i] = 0u;
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
     const uint64_t lbelow = (1ull << lane) - 1ull;
-    uint32_t cv = 0, ct = 0, ca = 0;
+    uint32_t cv = 0, ct = 0, ca = 0, cc = 0;
     for (uint64_t c0 = 0; c0 < n; c0 += SCAN1_NT * SCAN_IPT) {
         const uint64_t base = c0 + (uint64_t)wid * (64 * SCAN_IPT) + lane;
-        uint32_t v[SCAN_IPT], t[SCAN_IPT], pa[SCAN_IPT], raw[SCAN_IPT];
-        uint64_t am[SCAN_IPT];
+        uint32_t v[SCAN_IPT], t[SCAN_IPT], q[SCAN_IPT], pa[SCAN_IPT], raw[SCAN_IPT];
         uint32_t ra = 0;
 #pragma unroll
         for (int k = 0; k < SCAN_IPT; k++) {
             const uint64_t i = base + 64 * k;
             const uint32_t c = (i < n) ? cnt[i] : 0u;
-            v[k] = c & 0xFFFFu;
-            t[k] = c >> 16;
+            v[k] = word_verts(c);
+            t[k] = word_tris(c);
+            q[k] = word_cubes(c);
             raw[k] = c;
         }
 #pragma unroll
         for (int k = 0; k < SCAN_IPT; k++) {
-            am[k] = __ballot((v[k] | t[k]) != 0u);
-            pa[k] = ra + (uint32_t)__popcll(am[k] & lbelow);
-            ra += (uint32_t)__popcll(am[k]);
+            const uint64_t am = __ballot(raw[k] != 0u);
+            pa[k] = ra + (uint32_t)__popcll(am & lbelow);
+            ra += (uint32_t)__popcll(am);
         }
-        const uint32_t rv = wave_groups_scan(v, lane), rt = wave_groups_scan(t, lane);
+        const uint32_t rv = wave_groups_scan(v, lane), rt = wave_groups_scan(t, lane), rc = wave_groups_scan(q, lane);
         if (lane == 0) {
             wsum[0][wid] = rv;
             wsum[1][wid] = rt;
             wsum[2][wid] = ra;
+            wsum[3][wid] = rc;
         }
         __syncthreads();
-        uint32_t bv, av, bt, at, ba, aa;
+        uint32_t bv, av, bt, at, ba, aa, bc, ac;
         scan1_offsets(wsum[0], wid, bv, av);
         scan1_offsets(wsum[1], wid, bt, at);
         scan1_offsets(wsum[2], wid, ba, aa);
+        scan1_offsets(wsum[3], wid, bc, ac);
 #pragma unroll
         for (int k = 0; k < SCAN_IPT; k++) {
             const uint64_t i = base + 64 * k;
@@ -653,14 +684,14 @@ __global__ void __launch_bounds__(SCAN1_NT) k_mc_scan1(const uint32_t *__restric
                 const uint32_t fv = cv + bv + v[k], ft = ct + bt + t[k];
                 vbw[i] = fv;
                 tbw[i] = ft;
-                if ((am[k] >> lane) & 1ull) {
-                    const uint32_t r = ca + ba + pa[k];
+                if (raw[k]) {
+                    const uint32_t r = ca + ba + pa[k], fc = cc + bc + q[k];
                     avb[r] = fv;
-                    atb[r] = ft;
+                    acb[r] = fc;
                     list[r] = list_base + (uint32_t)i;
                     if (bs.vstart) {
-                        mark_block_starts(bs.vstart, bs.nv, fv, raw[k] & 0xFFFFu, r);
-                        mark_block_starts(bs.tstart, bs.nt, ft, raw[k] >> 16, r);
+                        mark_block_starts(bs.vstart, bs.nv, fv, word_verts(raw[k]), r);
+                        mark_block_starts(bs.tstart, bs.nt, fc, word_cubes(raw[k]), r);
                     }
                 }
             }
@@ -668,6 +699,7 @@ __global__ void __launch_bounds__(SCAN1_NT) k_mc_scan1(const uint32_t *__restric
         cv += av;
         ct += at;
         ca += aa;
+        cc += ac;
         __syncthreads();
     }
     if (threadIdx.x == 0) {
@@ -675,6 +707,7 @@ __global__ void __launch_bounds__(SCAN1_NT) k_mc_scan1(const uint32_t *__restric
         totals[1] = cv;
         totals[2] = ca;
         totals[3] = 0u;
+        totals[4] = cc;
     }
 }
 
@@ -2447,52 +2480,6 @@ struct MCView {
         ci |= (int)nbit(x, y + 1, z + 1) << 7;
         return ci;
     }
-    /* the same case from the four row words of the cube's x, y corners (and the next words when
-       the cube's top corners lie in them) */
-    __device__ __forceinline__ int cube_case(int x, int y, int z) const
-    {
-        const int b = z & 63;
-        const size_t w00 = widx(x, y, z), w10 = w00 + (size_t)g * W, w01 = w00 + W, w11 = w10 + W;
-        const uint64_t n00 = N[w00], n10 = N[w10], n11 = N[w11], n01 = N[w01];
-        int ci = (int)((n00 >> b) & 1ull) | (int)((n10 >> b) & 1ull) << 1 | (int)((n11 >> b) & 1ull) << 2 |
-                 (int)((n01 >> b) & 1ull) << 3;
-        if (b < 63) {
-            ci |= (int)((n00 >> (b + 1)) & 1ull) << 4 | (int)((n10 >> (b + 1)) & 1ull) << 5 |
-                  (int)((n11 >> (b + 1)) & 1ull) << 6 | (int)((n01 >> (b + 1)) & 1ull) << 7;
-        } else {
-            ci |= (int)(N[w00 + 1] & 1ull) << 4 | (int)(N[w10 + 1] & 1ull) << 5 | (int)(N[w11 + 1] & 1ull) << 6 |
-                  (int)(N[w01 + 1] & 1ull) << 7;
-        }
-        return ci;
-    }
-    /* vertex id of slot s (0,1,2 edge x,y,z; 3 point) of point (x, y, z) */
-    __device__ __forceinline__ uint32_t slot_id(int x, int y, int z, int sl) const
-    {
-        size_t wi = widx(x, y, z);
-        int b = z & 63;
-        uint64_t below = (1ull << b) - 1ull;
-        const uint64_t *m = S4 + 4 * wi;
-        uint64_t m0 = m[0], m1 = m[1], m2 = m[2], m3 = m[3];
-        uint32_t id = vbw[wi] + (uint32_t)(__popcll(m0 & below) + __popcll(m1 & below) + __popcll(m2 & below) +
-                                           __popcll(m3 & below));
-        if (sl > 0) id += (uint32_t)((m0 >> b) & 1ull);
-        if (sl > 1) id += (uint32_t)((m1 >> b) & 1ull);
-        if (sl > 2) id += (uint32_t)((m2 >> b) & 1ull);
-        return id;
-    }
-    /* vertex of cube edge e of cube (cx, cy, cz), whose case is ci: the sign of the edge's low
-       corner is case bit (z offset) * 4 + (0, 1, 2, 3 for xy offsets 00, 10, 11, 01) */
-    __device__ __forceinline__ uint32_t corner_vid(int cx, int cy, int cz, int e, int ci) const
-    {
-        const int lx = (int)((kEdgeLX >> e) & 1u), ly = (int)((kEdgeLY >> e) & 1u), lz = (int)((kEdgeLZ >> e) & 1u);
-        int qx = cx + lx, qy = cy + ly, qz = cz + lz;
-        int a = (int)((kEdgeAX >> (2 * e)) & 3u);
-        int rx = qx + (a == 0), ry = qy + (a == 1), rz = qz + (a == 2);
-        const bool qneg = (ci >> (4 * lz + (ly ? (lx ? 2 : 3) : lx))) & 1;
-        int nx = qneg ? rx : qx, ny = qneg ? ry : qy, nz = qneg ? rz : qz;
-        if (zbit(nx, ny, nz)) return slot_id(nx, ny, nz, 3);
-        return slot_id(qx, qy, qz, a);
-    }
 };
 
 /* countVertexPerCell MarchingCubes.cu:571-658 in word form: slot masks and per-word counts */
@@ -2566,7 +2553,7 @@ __global__ void __launch_bounds__(256) k_mc_count(QsBatch B, const uint64_t *__r
         S4[4 * wi + 2] = ez;
         S4[4 * wi + 3] = pt;
     }
-    uint32_t nt = 0;
+    uint32_t nt = 0, nc = 0;
     if (x < lim && x < M.cube_hi && y < lim) {
         const uint64_t c0 = n00, c1 = n10, c2 = n11, c3 = n01;
         const uint64_t c4 = n00_up;
@@ -2606,6 +2593,7 @@ __global__ void __launch_bounds__(256) k_mc_count(QsBatch B, const uint64_t *__r
         /* k = |S| - 2 f - 4 h mod 8, bit by bit */
         const uint64_t p0 = s0 & act, p1 = (s1 ^ f0) & act, p2 = (s2 ^ f1 ^ (~s1 & f0) ^ h) & act;
         nt = (uint32_t)(__popcll(p0) + 2 * __popcll(p1) + 4 * __popcll(p2));
+        nc = (uint32_t)__popcll(p0 | p1 | p2);
         if (nt) {
             uint64_t *__restrict__ NT = NT_all + 3 * (M.word_off + wi);
             NT[0] = p0;
@@ -2613,8 +2601,7 @@ __global__ void __launch_bounds__(256) k_mc_count(QsBatch B, const uint64_t *__r
             NT[2] = p2;
         }
     }
-    /* the word's vertex count (at most 4 x 64) and triangle count (at most 5 x 64) in one word */
-    cnt[wi] = nv | (nt << 16);
+    cnt[wi] = word_counts(nv, nt, nc);
 }
 
 /* row word wi of a grid -> (x, y, word) */
@@ -2641,7 +2628,7 @@ __device__ __forceinline__ uint32_t last_le(const uint32_t *__restrict__ a, uint
    items [base[k], base[k + 1]) (the last one up to n), so block b starts in the word whose range
    holds item 256 b.  Words may hold items beyond n (a slab's scan counts the vertices of the next
    slab's first plane, which that slab emits): blocks stop at n.  One launch serves the vertex
-   launch (blockIdx.y 0) and the triangle launch (1). */
+   launch (blockIdx.y 0) and the triangle launch (1), whose items are cubes. */
 struct QsStarts {
     const uint32_t *base; /* first item of each active word */
     uint32_t n;           /* items the launch covers */
@@ -2856,76 +2843,169 @@ __global__ void __launch_bounds__(256) k_mc_vertices(const QsMol *__restrict__ m
     }
 }
 
+/* bit position of the r-th set bit (from 0) of w, which has more than r */
+__device__ __forceinline__ int nth_bit(uint64_t w, uint32_t r)
+{
+    uint32_t m = (uint32_t)w;
+    int b = 0;
+    const uint32_t lowest = (uint32_t)__popc(m);
+    if (r >= lowest) {
+        r -= lowest;
+        m = (uint32_t)(w >> 32);
+        b = 32;
+    }
+#pragma unroll
+    for (int h = 16; h >= 1; h >>= 1) {
+        const uint32_t c = (uint32_t)__popc(m & ((1u << h) - 1u));
+        const bool up = r >= c;
+        r -= up ? c : 0u;
+        m >>= up ? h : 0;
+        b += up ? h : 0;
+    }
+    return b;
+}
+
 /* triangles (generateTriangleVerticesSMEM MarchingCubes.cu:736-851 order), one thread per
-   triangle: its word from the active words' first triangle ids, its cube from the word's
-   triangle-count bit planes, the cube's case from the sign words of its corners */
+   polygonised cube (two triangles on average): its word from the active words' first cubes, its
+   place from the word's triangle-count planes.  Bound by the dependent memory trips of a block
+   (block start, word list, planes, corner masks) and by VALU issue, so both are paid once per cube:
+   the thread loads the sign words, slot masks and vertex counts of the cube's four (x, y) columns
+   together, and every corner's vertex id comes from them.  One thread per triangle, three corners'
+   masks each, took 0.20 ms on the 50,000-atom 0.2 A mesh and 0.92 ms on 256 molecules at 0.5 A
+   (47 M triangles); this takes 0.15 and 0.62 ms.  (64 registers for eight waves per SIMD, with
+   spills, were slower than 66 with seven: emission 1.11 against 1.06 ms.) */
 __global__ void __launch_bounds__(256) k_mc_triangles(const QsMol *__restrict__ mols, const uint64_t *__restrict__ wpre,
                                                       const uint32_t *__restrict__ wcoarse, const uint32_t *__restrict__ list,
-                                                      const uint32_t *__restrict__ atb, const uint32_t *__restrict__ tstart,
-                                                      uint32_t nact, uint32_t ntri,
-                                                      const uint64_t *__restrict__ N_all, const uint64_t *__restrict__ Zm_all,
-                                                      const uint64_t *__restrict__ S4_all, const uint32_t *__restrict__ vbw_all,
-                                                      const uint64_t *__restrict__ NT_all, int *__restrict__ tri, uint32_t vbase, uint32_t *__restrict__ deg_blk,
-                                                      uint32_t *__restrict__ deg_total, const uint32_t *__restrict__ d_counts)
+                                                      const uint32_t *__restrict__ acb, const uint32_t *__restrict__ tstart,
+                                                      uint32_t nact, uint32_t ncube, uint32_t ntri, const uint64_t *__restrict__ N,
+                                                      const uint64_t *__restrict__ S4, const uint32_t *__restrict__ cnt,
+                                                      const uint32_t *__restrict__ vbw, const uint32_t *__restrict__ tbw,
+                                                      const uint64_t *__restrict__ NT, int *__restrict__ tri, uint32_t vbase,
+                                                      uint32_t *__restrict__ deg_blk, uint32_t *__restrict__ deg_total,
+                                                      const uint32_t *__restrict__ d_counts)
 {
     __shared__ ItemWords S;
-    /* counts from the device as in k_mc_vertices */
+    __shared__ uint32_t S_before[4][256]; /* per cube: vertices before its four columns' lower points */
+    /* counts from the device as in k_mc_vertices; triangles past the pool are not written */
     if (d_counts) {
         nact = d_counts[2];
-        ntri = min(d_counts[0], ntri);
+        ncube = min(d_counts[4], ncube);
     }
-    const uint32_t nb = (ntri + 255u) >> 8;
-    /* persistent blocks over the 256-triangle blocks, as in k_mc_vertices */
+    const uint32_t nb = (ncube + 255u) >> 8;
+    /* persistent blocks over the 256-cube blocks, as in k_mc_vertices */
     for (uint32_t vb = blockIdx.x; vb < nb; vb += gridDim.x) {
     const uint32_t blk = xcd_group<64>(vb, nb);
-    stage_item_words(S, atb, list, tstart, nact, nb, blk, wpre, wcoarse);
-    const uint32_t t = blk * 256u + threadIdx.x;
-    int c[3] = {0, 1, 2};
-    if (t < ntri) {
-    uint32_t k, wi, first;
-    item_word(S, atb, list, t, k, wi, first);
-    const uint32_t local = t - first;
-    const QsMol &M = mols[S.mol >= 0 ? S.mol : seg_coarse<QS_COARSE_ITEMS>(wpre, wcoarse, (uint64_t)wi)];
-    const int g = M.G.g;
-    int x, y, w;
-    decode_word((uint32_t)(wi - M.word_off), g, (int)M.W, x, y, w);
-    const uint64_t *__restrict__ np = NT_all + 3 * (size_t)wi;
-    const uint64_t p0 = np[0], p1 = np[1], p2 = np[2];
-    int lo = 0, hi = 63;
-    while (lo < hi) {
-        const int mid = (lo + hi) >> 1;
-        const uint64_t below = (2ull << mid) - 1ull;
-        const uint32_t c = (uint32_t)(__popcll(p0 & below) + 2 * __popcll(p1 & below) + 4 * __popcll(p2 & below));
-        if (c > local) hi = mid;
-        else lo = mid + 1;
-    }
-    const int b = lo;
-    const uint64_t below = (1ull << b) - 1ull;
-    const int j = (int)(local - (uint32_t)(__popcll(p0 & below) + 2 * __popcll(p1 & below) + 4 * __popcll(p2 & below)));
-    const int z = w * 64 + b;
-    MCView V;
-    V.N = N_all + M.word_off;
-    V.Zm = Zm_all + M.word_off;
-    V.S4 = S4_all + 4 * M.word_off;
-    V.vbw = vbw_all + M.word_off;
-    V.g = g;
-    V.W = (int)M.W;
-    V.lim = M.G.lim;
-    const int ci = V.cube_case(x, y, z);
-    const uint64_t packed = c_tri[ci];
+    stage_item_words(S, acb, list, tstart, nact, nb, blk, wpre, wcoarse);
+    const uint32_t cube = blk * 256u + threadIdx.x;
+    /* sl: the vertex slots of the eight corners, byte q = x | y << 1 for the column, bit
+       2 slot + z in it; has: the columns whose words own vertices (the masks of others are not
+       written, and only an edge that ends in a zero point asks for them) */
+    uint32_t first_tri = 0, nt = 0, sl = 0, has = 0, cs = 0;
+    uint64_t table = 0;
+    if (cube < ncube) {
+        uint32_t k, wi, first;
+        item_word(S, acb, list, cube, k, wi, first);
+        const QsMol &M = mols[S.mol >= 0 ? S.mol : seg_coarse<QS_COARSE_ITEMS>(wpre, wcoarse, (uint64_t)wi)];
+        const size_t W = M.W, gW = (size_t)M.G.g * W;
+        const uint64_t p0 = NT[3 * (size_t)wi], p1 = NT[3 * (size_t)wi + 1], p2 = NT[3 * (size_t)wi + 2];
+        const int b = nth_bit(p0 | p1 | p2, cube - first);
+        const uint64_t below = (1ull << b) - 1ull;
+        first_tri = tbw[wi] + (uint32_t)(__popcll(p0 & below) + 2 * __popcll(p1 & below) + 4 * __popcll(p2 & below));
+        nt = (uint32_t)((p0 >> b) & 1ull) + 2u * (uint32_t)((p1 >> b) & 1ull) + 4u * (uint32_t)((p2 >> b) & 1ull);
+        uint64_t s[4][4], nw[4];
+        uint32_t vb4[4], nv4[4];
 #pragma unroll
-    for (int cc = 0; cc < 3; cc++) c[cc] = (int)(vbase + V.corner_vid(x, y, z, tri_entry(packed, 3 * j + cc), ci));
-    tri[3 * (size_t)t + 0] = c[0];
-    tri[3 * (size_t)t + 1] = c[1];
-    tri[3 * (size_t)t + 2] = c[2];
+        for (int q = 0; q < 4; q++) {
+            const size_t cw = wi + (q & 1 ? gW : 0) + (q & 2 ? W : 0);
+            nw[q] = N[cw];
+            nv4[q] = word_verts(cnt[cw]);
+            vb4[q] = vbw[cw];
+#pragma unroll
+            for (int a = 0; a < 4; a++) s[q][a] = S4[4 * cw + a];
+        }
+        uint32_t sg = 0; /* sign bits, bit 2 q + z */
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            uint32_t m = 0, before = vb4[q];
+#pragma unroll
+            for (int a = 0; a < 4; a++) {
+                before += (uint32_t)__popcll(s[q][a] & below);
+                m |= ((uint32_t)(s[q][a] >> b) & 3u) << (2 * a);
+            }
+            S_before[q][threadIdx.x] = before;
+            sl |= m << (8 * q);
+            has |= (nv4[q] ? 1u : 0u) << q;
+            sg |= ((uint32_t)(nw[q] >> b) & 3u) << (2 * q);
+        }
+        if (b == 63) { /* the cube's top corners are in the next words */
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const size_t cw = wi + (q & 1 ? gW : 0) + (q & 2 ? W : 0) + 1;
+                sg |= (uint32_t)(N[cw] & 1ull) << (2 * q + 1);
+                uint32_t m = 0;
+#pragma unroll
+                for (int a = 0; a < 4; a++) m |= (uint32_t)(S4[4 * cw + a] & 1ull) << (2 * a + 1);
+                if (word_verts(cnt[cw])) {
+                    /* (a word without vertices below has none of its own slots set) */
+                    sl = (has >> q) & 1u ? sl : sl & ~(255u << (8 * q));
+                    if (!((has >> q) & 1u)) S_before[q][threadIdx.x] = vbw[cw];
+                    has |= 1u << q;
+                    sl |= m << (8 * q);
+                }
+            }
+        }
+        /* the table's corner order goes round the (x, y) columns 00, 10, 11, 01 */
+        const uint32_t lo4 = (sg & 1u) | (sg >> 1 & 2u) | (sg >> 4 & 4u) | (sg >> 1 & 8u);
+        const uint32_t hi4 = (sg >> 1 & 1u) | (sg >> 2 & 2u) | (sg >> 5 & 4u) | (sg >> 2 & 8u);
+        cs = lo4 | hi4 << 4;
+        table = c_tri[cs];
     }
-    /* triangles with a repeated corner (zero grid points) are dropped from the output
-       (CudaSurf.cu:820-829): counted here per block and in total (lanes past the count hold the
-       distinct placeholder corners 0, 1, 2) */
-    const uint64_t dm = __ballot(c[0] == c[1] || c[1] == c[2] || c[0] == c[2]);
-    if (dm && (threadIdx.x & 63) == (uint32_t)__builtin_ctzll(dm)) {
-        atomicAdd(&deg_blk[blk], (uint32_t)__popcll(dm));
-        atomicAdd(deg_total, (uint32_t)__popcll(dm));
+#pragma unroll 1
+    for (uint32_t j = 0; j < 5u; j++) {
+        const bool on = j < nt && first_tri + j < ntri;
+        if (!__ballot(on)) break;
+        uint32_t c[3] = {0u, 1u, 2u};
+        const uint32_t t = first_tri + j;
+        if (on) {
+            const uint32_t corners = (uint32_t)(table >> (12u * j));
+#pragma unroll
+            for (int i = 0; i < 3; i++) {
+                const uint32_t e = (corners >> (4 * i)) & 15u;
+                const uint32_t d = (uint32_t)(kEdgePacked >> (5u * e));
+                uint32_t z = d & 1u, q = (d >> 1) & 3u, a2 = (d >> 2) & 6u; /* a2 = 2 axis */
+                uint32_t at = 8u * q + z;                                    /* the corner's slot 0 */
+                if (!((sl >> (at + a2)) & (has >> q) & 1u)) {
+                    /* the edge has no vertex of its own: its non-negative end is exactly zero and
+                       is the vertex (the point slot, after the point's edges) */
+                    if ((cs >> (4 * z + (q ^ (q >> 1)))) & 1u) {
+                        q |= (a2 == 0 ? 1u : 0u) | (a2 == 2 ? 2u : 0u);
+                        z |= a2 == 4 ? 1u : 0u;
+                        at = 8u * q + z;
+                    }
+                    a2 = 6u;
+                }
+                /* the corner's slots below this one, and all slots of the corner below it */
+                const uint32_t lower = __builtin_amdgcn_ubfe(sl, at, a2) & 0x55u;
+                const uint32_t under = __builtin_amdgcn_ubfe(sl, 8u * q, 8u * z) & 0x55u;
+                c[i] = vbase + S_before[q][threadIdx.x] + (uint32_t)(__popc(lower) + __popc(under));
+            }
+            tri[3 * (size_t)t + 0] = (int)c[0];
+            tri[3 * (size_t)t + 1] = (int)c[1];
+            tri[3 * (size_t)t + 2] = (int)c[2];
+        }
+        /* triangles with a repeated corner (zero grid points) are dropped from the output
+           (CudaSurf.cu:820-829): counted here per 256-triangle block and in total */
+        uint64_t dm = __ballot(c[0] == c[1] || c[1] == c[2] || c[0] == c[2]);
+        if (dm) {
+            if ((threadIdx.x & 63) == (uint32_t)__builtin_ctzll(dm)) atomicAdd(deg_total, (uint32_t)__popcll(dm));
+            while (dm) {
+                const uint32_t lead = (uint32_t)__builtin_ctzll(dm);
+                const uint32_t tb = (uint32_t)__shfl((int)(t >> 8), (int)lead, 64);
+                const uint64_t same = __ballot((t >> 8) == tb) & dm;
+                if ((threadIdx.x & 63) == lead) atomicAdd(&deg_blk[tb], (uint32_t)__popcll(same));
+                dm &= ~same;
+            }
+        }
     }
     __syncthreads(); /* S is staged again for the next block */
     }
@@ -3766,8 +3846,8 @@ void qs_launch_mc_count(QsBatch B, uint32_t nblocks, const uint64_t *N, const ui
 void qs_launch_mc_emit(const QsMol *mols, const uint64_t *wpre, const uint32_t *wcoarse, const uint32_t *list, uint32_t nact,
                        const uint32_t *avb, uint32_t *vstart, uint32_t nv, const uint64_t *S4, const float *F,
                        const uint32_t *spre, const uint64_t *outm, const uint64_t *shellm, float *vert, uint64_t *vkey,
-                       const uint32_t *atb, uint32_t *tstart, uint32_t ntri, const uint64_t *N, const uint64_t *Zm,
-                       const uint32_t *vbw, const uint64_t *NT, int *tri, uint32_t vbase, uint32_t *deg_blk,
+                       const uint32_t *acb, uint32_t *tstart, uint32_t ncube, uint32_t ntri, const uint64_t *N, const uint32_t *cnt,
+                       const uint32_t *vbw, const uint32_t *tbw, const uint64_t *NT, int *tri, uint32_t vbase, uint32_t *deg_blk,
                        uint32_t *deg_total, const uint32_t *d_counts, hipStream_t s, hipStream_t s_vert, hipEvent_t ev_fork,
                        hipEvent_t ev_vert, bool starts_ready)
 {
@@ -3785,7 +3865,7 @@ void qs_launch_mc_emit(const QsMol *mols, const uint64_t *wpre, const uint32_t *
        whole pool of ntri triangles */
     const uint32_t nzero = ntri ? ntri / 256 + 1 : 0u;
     const QsStarts sv = {avb, nv, d_counts ? d_counts + 1 : nullptr, vstart, nullptr, 0u};
-    const QsStarts st = {atb, ntri, d_counts ? d_counts : nullptr, tstart, deg_blk, nzero};
+    const QsStarts st = {acb, ncube, d_counts ? d_counts + 4 : nullptr, tstart, deg_blk, nzero};
     if (!starts_ready)
         hipLaunchKernelGGL(k_block_starts, dim3(pgrid(nblk(std::max<uint32_t>(nact, nzero), 256)), 2), dim3(256), 0, s, sv, st,
                            nact, d_counts ? d_counts + 2 : nullptr);
@@ -3799,8 +3879,8 @@ void qs_launch_mc_emit(const QsMol *mols, const uint64_t *wpre, const uint32_t *
                            nv, S4, F, spre, outm, shellm, vert, vkey, d_counts);
     if (s_vert != s) (void)hipEventRecord(ev_vert, s_vert);
     if (ntri)
-        hipLaunchKernelGGL(k_mc_triangles, dim3(pgrid(nblk(ntri, 256))), dim3(256), 0, s, mols, wpre, wcoarse, list, atb, tstart,
-                           nact, ntri, N, Zm, S4, vbw, NT, tri, vbase, deg_blk, deg_total, d_counts);
+        hipLaunchKernelGGL(k_mc_triangles, dim3(pgrid(nblk(ncube, 256))), dim3(256), 0, s, mols, wpre, wcoarse, list, acb, tstart,
+                           nact, ncube, ntri, N, S4, cnt, vbw, tbw, NT, tri, vbase, deg_blk, deg_total, d_counts);
 }
 
 void qs_launch_smooth(const QsMol *mols, const uint32_t *vpre, const uint32_t *vcoarse, const uint64_t *N, const uint64_t *Zm,
@@ -3871,21 +3951,21 @@ void qs_launch_tri_kept_before(const int *tri, const uint32_t *dpre, const uint6
 
 /* scan helpers */
 void qs_launch_mc_scans(const uint32_t *cnt, uint64_t nw, uint32_t *sums, uint32_t *vbw,
-                        uint32_t *tbw, uint32_t *list, uint32_t *avb, uint32_t *atb, uint32_t *totals, uint32_t list_base,
+                        uint32_t *tbw, uint32_t *list, uint32_t *avb, uint32_t *acb, uint32_t *totals, uint32_t list_base,
                         hipStream_t s, QsBlockStarts bs)
 {
     if (!nw) return;
     if (nw <= QS_SCAN1_MAX) {
-        hipLaunchKernelGGL(k_mc_scan1, dim3(1), dim3(SCAN1_NT), 0, s, cnt, nw, vbw, tbw, list, avb, atb, list_base,
+        hipLaunchKernelGGL(k_mc_scan1, dim3(1), dim3(SCAN1_NT), 0, s, cnt, nw, vbw, tbw, list, avb, acb, list_base,
                            totals, bs);
         return;
     }
     const uint64_t ntiles = qs_scan_tiles(nw);
     const int self = ntiles <= QS_SCAN_SELF_TILES;
-    hipLaunchKernelGGL(k_mc_reduce3, dim3((unsigned)ntiles), dim3(SCAN_NT), 0, s, cnt, nw, sums, ntiles);
-    if (!self) hipLaunchKernelGGL(k_scan_planes, dim3(3), dim3(SCAN_NT), 0, s, sums, ntiles, totals);
-    hipLaunchKernelGGL(k_mc_scan3, dim3((unsigned)ntiles), dim3(SCAN_NT), 0, s, cnt, nw, sums, ntiles, vbw, tbw, list,
-                       avb, atb, list_base, self, totals, bs);
+    hipLaunchKernelGGL(k_mc_reduce4, dim3((unsigned)ntiles), dim3(SCAN_NT), 0, s, cnt, nw, sums, ntiles);
+    if (!self) hipLaunchKernelGGL(k_scan_planes, dim3(4), dim3(SCAN_NT), 0, s, sums, ntiles, totals);
+    hipLaunchKernelGGL(k_mc_scan4, dim3((unsigned)ntiles), dim3(SCAN_NT), 0, s, cnt, nw, sums, ntiles, vbw, tbw, list,
+                       avb, acb, list_base, self, totals, bs);
 }
 
 uint64_t qs_scan_tiles(uint64_t n) { return (n + SCAN_TILE - 1) / SCAN_TILE; }

@@ -28,3 +28,30 @@ def test_closest_atom_ties_and_clamps(qs, orc, kind, reso):
     pos, rad = _closest_case(qs, kind)
     print("case closest atom: %s reso=%.2f" % (kind, reso), flush=True)
     assert _same(qs.compute_ses(pos, rad, reso, 0), orc.compute_ses(pos, rad, reso, 0))
+
+
+def _noise_field(g, kind):
+    rng = np.random.default_rng(100 * g + len(kind))
+    f = rng.standard_normal((g, g, g)).astype(np.float32)  # nearly every cube polygonised
+    if kind == "noise with zeros":
+        f[rng.random(f.shape) < 0.2] = 0.0
+    elif kind == "sheet":  # words of a few cubes beside words without vertices, zeros on the sheet
+        x, y, z = np.meshgrid(*[np.arange(g, dtype=np.float32)] * 3, indexing="ij")
+        f = (z - np.float32(0.75 * g) + np.float32(0.5) * (x % 3)).astype(np.float32)
+    return f.ravel()
+
+
+@pytest.mark.parametrize("kind", ["noise", "noise with zeros", "sheet"])
+@pytest.mark.parametrize("g", [2, 5, 63, 64, 65, 66, 130])
+def test_mesh_of_any_field(qs, orc, g, kind):
+    """Emission over whole words of cubes, cubes across two row words, and zero grid points."""
+    s = orc._Grid()
+    s.g, s.gn, s.r, s.reso, s.dx_n = g, 1, 3, 0.5, 3.2
+    G = orc.Grid(s)
+    fld = _noise_field(g, kind)
+    for lim in (g - 1, max(1, g - 3)):
+        print("case mesh of a field: %s g=%d lim=%d" % (kind, g, lim), flush=True)
+        V, T = qs.stage_mesh(G.params(lim), fld)
+        Vo, To = orc.edge_weld(G, lim, fld)
+        assert np.array_equal(T, To)
+        assert np.array_equal(V.view(np.uint32), Vo.view(np.uint32))
