@@ -960,6 +960,23 @@ __device__ __forceinline__ void row_interval(const RowAtom &A, float ss, int zlo
     R = r;
 }
 
+/* The interval of row_interval from its closed form, zc -+ h in voxel units (h2 = ss - S, h = sqrt(h2)
+   / dx), without evaluating the predicate.  The predicate's roundings move a boundary by at most
+   u (A + g dx + 5/2 H + ss / 2H) / dx voxels and the closed form is off by at most u (4 g dx + 5 H) / dx
+   (u = 2^-24, A the largest |z| of the grid, H = sqrt(h2) <= (1 + ss) / 2), so an end that is farther
+   than eps = 2 u (A + 5 g dx + 4 + 8 ss) / dx from every grid point is decided by its side of it; the
+   bound takes H >= 1/8.  False: an end is nearer than that, or H is smaller (a few intervals in a
+   thousand). */
+__device__ __forceinline__ bool fast_interval(float h2, float zc, float inv_dx, float eps, int zlo, int zhi, int &L, int &R)
+{
+    const float h = __builtin_amdgcn_sqrtf(h2) * inv_dx;
+    const float lo = zc - h, hi = zc + h;
+    L = max((int)ceilf(lo), zlo);
+    R = min((int)floorf(hi), zhi);
+    const float d = fminf(fabsf(lo - rintf(lo)), fabsf(hi - rintf(hi)));
+    return d > eps && h2 > 0.015625f;
+}
+
 /* per atom in cell order, once: the atom (perm gives its input index) as float4 x, y, z, r, the
    exact float thresholds of its near (r + probe) and inside (r - dx) tests, and its neighbour-cell
    y and z (packed) */
@@ -1234,13 +1251,21 @@ __global__ void __launch_bounds__(256) k_pass1_rows(QsBatch B, const uint32_t *_
     }
 }
 
-/* OR bits [L, R] (absolute z) into a row's words in LDS */
-__device__ __forceinline__ void lds_or_range(uint64_t *row, int L, int R)
+/* OR bits [L, R] (absolute z) into a row's words in LDS (32-bit halves of the row words).  An
+   interval of at most 32 voxels takes one or two of them, from one 64-bit shift. */
+__device__ __forceinline__ void lds_or_range(uint32_t *row, int L, int R)
 {
-    for (int w = L >> 6; w <= (R >> 6); w++) {
-        const int z0 = w << 6;
-        atomicOr((unsigned long long *)&row[w], (unsigned long long)bit_range(max(L, z0) - z0, min(R, z0 + 63) - z0));
+    const int n = R - L;
+    uint32_t *w = row + (L >> 5);
+    if (n < 32) {
+        const uint64_t m = (uint64_t)(~0u >> (31 - n)) << (L & 31);
+        atomicOr(w, (uint32_t)m);
+        if (m >> 32) atomicOr(w + 1, (uint32_t)(m >> 32));
+        return;
     }
+    atomicOr(w, ~0u << (L & 31));
+    for (w++; w < row + (R >> 5); w++) atomicOr(w, ~0u);
+    atomicOr(w, ~0u >> (31 - (R & 31)));
 }
 
 /* Field pass 1 by scatter into LDS: one block per slab of up to P1S_MAXROWS consecutive y rows of
@@ -1249,16 +1274,22 @@ __device__ __forceinline__ void lds_or_range(uint64_t *row, int L, int R)
    z-intervals (the ones of k_pass1_rows) into the slab's two masks.  The z-intervals are clipped
    to the voxels whose z cell admits the atom, so each voxel sees exactly the atoms of its 27
    neighbour cells, as in probeIntersection (Kernels.cu:394-475); inside wins over near, which
-   makes the result independent of the order of the ORs. */
+   makes the result independent of the order of the ORs.
+   Bound by VALU issue over the (atom, row) pairs, 730 an atom at 0.2 A.  Three things keep a pair
+   short: its interval comes from the closed form (fast_interval), not from walking the predicate;
+   the inside intervals, which one pair in seven has at 0.5 A, are taken apart from the near ones,
+   so that the lanes without one do not wait; and an interval of 32 voxels is ORed with one 64-bit
+   shift.  50,000 atoms at 0.2 A 0.313 -> 0.185 ms, 256 molecules at 0.5 A 1.05 -> 0.60 ms, a million
+   atoms at 0.5 A 0.87 -> 0.49 ms. */
 #define P1S_MAXROWS 256   /* rows per slab block at most (row indexes in the queue are 8-bit) */
 #define P1S_DEFROWS 64    /* rows per slab block when no tuned count is set */
 #define P1S_MAXCOL 256
-/* a wave takes its queued atoms as (atom, row) items when K1 * (item rounds of 64) < K2 * (the
-   largest row count of one atom), i.e. when walking atoms would leave most lanes idle */
-#ifndef P1_FLAT_K1
-#define P1_FLAT_K1 3
-#define P1_FLAT_K2 2
-#endif
+/* a wave takes its queued atoms as (atom, row) items when twice the item rounds of 64 are fewer than
+   the largest row count of one atom, i.e. when walking atoms would leave most lanes idle (an item
+   costs the shuffles of its atom's values).  Pass 1 on the 50,000-atom 0.2 A mesh and on 256
+   molecules at 0.5 A: ratio 1 0.208 and 0.775 ms, 3/2 0.191 and 0.612, 2 0.185 and 0.600, 3 0.186
+   and 0.622. */
+#define P1_FLAT 2
 __global__ void __launch_bounds__(256) k_pass1_slab(QsBatch B, const uint32_t *__restrict__ cstart_all,
                                                     const float4 *__restrict__ sx, const float4 *__restrict__ aux,
                                                     uint64_t *__restrict__ outm_all, uint64_t *__restrict__ shellm_all,
@@ -1304,6 +1335,11 @@ __global__ void __launch_bounds__(256) k_pass1_slab(QsBatch B, const uint32_t *_
     for (int t = threadIdx.x; t < gn + 2; t += 256) yfirst[t] = zfirst[t] = g;
     __syncthreads();
     const float dx = G.dx, inv_dx = 1.0f / G.dx;
+    /* fast_interval's bound: eps0 + eps1 * ss (|oz| + g dx >= A) */
+    const float eps0 = 1.2e-7f * inv_dx * (fabsf(G.oz) + 6.0f * (float)g * dx + 4.0f), eps1 = 9.6e-7f * inv_dx;
+    /* margin of the rows an atom reaches, each of which is tested exactly: fast_interval's bound
+       along y, and the root of 4 u ss for a half-width near zero (sqrt(ss) = r + probe at most) */
+    const float ymargin = 1.2e-7f * inv_dx * (fabsf(G.oy) + 6.0f * (float)g * dx + 4.0f) + 1.0e-3f, ymargin_r = 6.0e-4f * inv_dx;
     for (int i = threadIdx.x; i < g; i += 256) {
         const int cy = min(cell_of(grid_pos(G.oy, i, dx), G.oy, G.dxn), gn + 1);
         const int cyp = i ? min(cell_of(grid_pos(G.oy, i - 1, dx), G.oy, G.dxn), gn + 1) : -1;
@@ -1349,38 +1385,22 @@ __global__ void __launch_bounds__(256) k_pass1_slab(QsBatch B, const uint32_t *_
     const int rows_hi = ylast - y0; /* rows 0..rows_hi of the slab are labelled */
     int *qid = q_id[wid], *qrows = q_rows[wid], *qz = q_z[wid];
 
-    /* One (atom, row) pair: the atom's exact near and inside z-intervals in the row, ORed into the
-       slab's masks (the ORs are order-independent). */
-    auto row_item = [&](int yr, float X, float sN, float sD, float zc, float az, float ay, int zr, int zb) {
-        const int zlo = zr & 0xFFFF, zhi = zr >> 16;
-        RowAtom A;
-        A.az = az;
-        A.dx = dx;
-        A.oz = G.oz;
-        const float ey = ay - grid_pos(G.oy, y0 + yr, dx);
-        const float Y = ey * ey;
-        A.S = X + Y;
-        if (!(A.S < sN)) return;
-        int L, Rr;
-        row_interval(A, sN, zlo, zhi, zb, zc, inv_dx, L, Rr);
-        if (L > Rr) return;
-        lds_or_range(nearw + (size_t)yr * W, L, Rr);
-        if (!(A.S < sD)) return;
-        row_interval(A, sD, L, Rr, zb, zc, inv_dx, L, Rr);
-        if (L <= Rr) lds_or_range(insw + (size_t)yr * W, L, Rr);
-    };
-    /* The wave's queued atoms, lane k < count holding atom k.  Each lane walks its own atom's rows
-       r0..r1, unless the row counts are so uneven that most lanes would idle: the atoms' rows are
-       then items pre_k .. pre_k + r1 - r0 that the lanes take 64 at a time, each with its atom's
-       values from the lane that holds it.  Called by the whole wave. */
+    /* The wave's queued atoms, lane k < count holding atom k: first their near intervals, then
+       their inside ones.  Each lane walks its own atom's rows, unless the row counts are so uneven
+       that most lanes would idle: the atoms' rows are then items pre_k .. pre_k + rows - 1 that the
+       lanes take 64 at a time, each with its atom's values from the lane that holds it.  An (atom,
+       row) pair gives the atom's exact z-interval in the row, ORed into the slab's mask (the ORs are
+       order-independent).  One loop body serves both ways and both masks: four copies of it took
+       32 KB of code.  Called by the whole wave. */
     auto process = [&](int count) {
-        int rr = 0, nrows = 0, zr = 0, zb = 0;
+        int rr = 0, zr = 0, nr[2] = {0, 0}, r0[2] = {0, 0};
         float X = 0.0f, sN = 0.0f, sD = 0.0f, zc = 0.0f, az = 0.0f, ay = 0.0f;
         if (lane < count) {
             const int id = qid[lane];
             rr = qrows[lane];
             zr = qz[lane];
-            nrows = (rr >> 8) - (rr & 0xFF) + 1;
+            r0[0] = rr & 0xFF;
+            nr[0] = (rr >> 8) - r0[0] + 1;
             const float4 a = sx[id], ax = aux[id];
             sN = ax.x;
             sD = ax.y;
@@ -1389,47 +1409,79 @@ __global__ void __launch_bounds__(256) k_pass1_slab(QsBatch B, const uint32_t *_
             zc = (a.z - G.oz) * inv_dx;
             az = a.z;
             ay = a.y;
-            const int zlo = zr & 0xFFFF, zhi = zr >> 16;
-            RowAtom A;
-            A.az = a.z;
-            A.dx = dx;
-            A.oz = G.oz;
-            zb = iclamp((int)floorf(zc), zlo, zhi);
-            if (zb + 1 <= zhi && A.Zf(zb + 1) < A.Zf(zb)) zb = zb + 1;
+            if (X < sD) {
+                const float h = __builtin_amdgcn_sqrtf(sD - X) * inv_dx, yc = (ay - G.oy) * inv_dx - (float)y0;
+                const float ym = ymargin + ymargin_r * (a.w + QS_PROBE);
+                r0[1] = max((int)ceilf(yc - h - ym), r0[0]);
+                nr[1] = max(min((int)floorf(yc + h + ym), rr >> 8) - r0[1] + 1, 0);
+            }
         }
-        int pre = nrows;
+#pragma unroll 1
+        for (int p = 0; p < 2; p++) {
+            const int n = p ? nr[1] : nr[0], first = p ? r0[1] : r0[0];
+            const float thr = p ? sD : sN;
+            uint32_t *const mask = (uint32_t *)(p ? insw : nearw);
+            int pre = n, most = n;
 #pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-            const int t = __shfl_up(pre, d, 64);
-            if (lane >= d) pre += t;
-        }
-        const int nitems = __shfl(pre, 63, 64);
-        pre -= nrows; /* exclusive */
-        int maxrows = nrows;
+            for (int d = 1; d < 64; d <<= 1) {
+                const int t = __shfl_up(pre, d, 64);
+                if (lane >= d) pre += t;
+            }
+            const int nitems = __shfl(pre, 63, 64);
+            pre -= n; /* exclusive */
 #pragma unroll
-        for (int d = 1; d < 64; d <<= 1) maxrows = max(maxrows, __shfl_xor(maxrows, d, 64));
-        if (P1_FLAT_K1 * ((nitems + 63) >> 6) >= P1_FLAT_K2 * maxrows) {
-            if (lane < count)
-                for (int yr = rr & 0xFF; yr <= (rr >> 8); yr++) row_item(yr, X, sN, sD, zc, az, ay, zr, zb);
-            return;
-        }
-        for (int base = 0; base < nitems; base += 64) {
-            const int j = base + lane;
-            /* the item's atom: the last lane whose first item is at or below j */
-            int o = 0;
+            for (int d = 1; d < 64; d <<= 1) most = max(most, __shfl_xor(most, d, 64));
+            const bool walk = P1_FLAT * ((nitems + 63) >> 6) >= most;
+            const int rounds = walk ? most : (nitems + 63) >> 6;
+#pragma unroll 1
+            for (int it = 0; it < rounds; it++) {
+                bool on = it < n;
+                int yr = first + it, iz = zr;
+                float iX = X, ithr = thr, izc = zc, iaz = az, iay = ay;
+                if (!walk) {
+                    const int j = it * 64 + lane;
+                    /* the item's atom: the last lane whose first item is at or below j */
+                    int o = 0;
 #pragma unroll
-            for (int step = 32; step >= 1; step >>= 1)
-                if (__shfl(pre, o + step, 64) <= j) o += step;
-            const float oX = __shfl(X, o, 64), osN = __shfl(sN, o, 64), osD = __shfl(sD, o, 64);
-            const float ozc = __shfl(zc, o, 64), oaz = __shfl(az, o, 64), oay = __shfl(ay, o, 64);
-            const int orr = __shfl(rr, o, 64), ozr = __shfl(zr, o, 64), ozb = __shfl(zb, o, 64), opre = __shfl(pre, o, 64);
-            if (j < nitems) row_item((orr & 0xFF) + (j - opre), oX, osN, osD, ozc, oaz, oay, ozr, ozb);
+                    for (int step = 32; step >= 1; step >>= 1)
+                        if (__shfl(pre, o + step, 64) <= j) o += step;
+                    iX = __shfl(X, o, 64);
+                    ithr = __shfl(thr, o, 64);
+                    izc = __shfl(zc, o, 64);
+                    iaz = __shfl(az, o, 64);
+                    iay = __shfl(ay, o, 64);
+                    iz = __shfl(zr, o, 64);
+                    yr = __shfl(first, o, 64) + j - __shfl(pre, o, 64);
+                    on = j < nitems;
+                }
+                if (!on) continue;
+                const float ey = iay - grid_pos(G.oy, y0 + yr, dx);
+                const float Y = ey * ey;
+                const float S = iX + Y;
+                if (!(S < ithr)) continue;
+                const int zlo = iz & 0xFFFF, zhi = iz >> 16;
+                int L, Rr;
+                if (!fast_interval(ithr - S, izc, inv_dx, eps0 + eps1 * ithr, zlo, zhi, L, Rr)) {
+                    RowAtom A;
+                    A.az = iaz;
+                    A.S = S;
+                    A.dx = dx;
+                    A.oz = G.oz;
+                    int zb = iclamp((int)floorf(izc), zlo, zhi);
+                    if (zb + 1 <= zhi && A.Zf(zb + 1) < A.Zf(zb)) zb = zb + 1;
+                    row_interval(A, ithr, zlo, zhi, zb, izc, inv_dx, L, Rr);
+                }
+                if (L <= Rr) lds_or_range(mask + (size_t)yr * (2 * W), L, Rr);
+            }
         }
     };
 
     int qn = 0;
     if (rows_hi >= 0) {
-        for (int base = wid * 64; base < total; base += 256) {
+        /* (one place calls process: its code is inlined once) */
+        bool more = true;
+        for (int base = wid * 64; more; base += 256) {
+            more = base < total;
             const int k = base + lane;
             bool keep = false;
             int id = 0, rows = 0, zr = 0;
@@ -1450,11 +1502,11 @@ __global__ void __launch_bounds__(256) k_pass1_slab(QsBatch B, const uint32_t *_
                     /* rows whose y cell admits the atom: cy >= acy - 1, and cy <= acy + 1 unless acy is the last cell */
                     int ylo = yfirst[max(acy - 1, 0)];
                     int yhi = (acy == gn - 1) ? g - 1 : yfirst[acy + 2] - 1;
-                    /* rows the atom can reach in y (a superset with a row of margin: the exact
-                       test is per row, so the hardware root serves) */
-                    const float h = __builtin_amdgcn_sqrtf(ax.x - X);
-                    ylo = max(ylo, (int)floorf((a.y - h - G.oy) * inv_dx) - 1);
-                    yhi = min(yhi, (int)ceilf((a.y + h - G.oy) * inv_dx) + 1);
+                    /* rows the atom can reach in y (a superset: the exact test is per row) */
+                    const float h = __builtin_amdgcn_sqrtf(ax.x - X) * inv_dx, yc = (a.y - G.oy) * inv_dx;
+                    const float ym = ymargin + ymargin_r * (a.w + QS_PROBE);
+                    ylo = max(ylo, (int)ceilf(yc - h - ym));
+                    yhi = min(yhi, (int)floorf(yc + h + ym));
                     const int r0 = max(ylo - y0, 0), r1 = min(yhi - y0, rows_hi);
                     /* voxels whose z cell admits the atom, labelled ones only (z <= g - 2) */
                     const int zlo = zfirst[max(acz - 1, 0)];
@@ -1473,9 +1525,13 @@ __global__ void __launch_bounds__(256) k_pass1_slab(QsBatch B, const uint32_t *_
             }
             qn += __popcll(km);
             wave_lds_sync();
-            if (qn >= 64) {
-                process(64);
+            if (qn >= 64 || (!more && qn > 0)) {
+                process(min(qn, 64));
                 wave_lds_sync();
+                if (qn <= 64) {
+                    qn = 0;
+                    continue;
+                }
                 const int rest = qn - 64;
                 int m0 = 0, m1 = 0, m2 = 0;
                 if (lane < rest) {
@@ -1493,7 +1549,6 @@ __global__ void __launch_bounds__(256) k_pass1_slab(QsBatch B, const uint32_t *_
                 qn = rest;
             }
         }
-        if (qn > 0) process(qn);
     }
     __syncthreads();
     for (int t = threadIdx.x; t < ny * W; t += 256) {
