@@ -30,6 +30,21 @@ struct QsNormFlags {
     uint64_t w[4];
 };
 
+/* Field pass 2: the shell voxels whose values a mesh can read, by their window minimum n of squared
+   integer norms.  A vertex reads the two ends of an edge whose signs differ, so a voxel is read only
+   if a neighbour one step away has the other sign (or is zero).  The distance to the nearest
+   outside voxel changes by at most one voxel per step: n <= lo is positive with only positive
+   neighbours, n >= hi is negative with only negative ones, and only lo < n < hi is evaluated and
+   stored; the signs of the others follow from n.  The window (r voxels along each axis) limits n to
+   offsets within it: a negative voxel next to a voxel whose nearest outside voxel lies r steps along
+   an axis may see it no longer.  That takes a non-negative value at norm r^2, so a probe of r whole
+   voxels (`edge`): then far voxels (n >= hi, or none in reach) with an outside voxel r + 1 steps away
+   along an axis are stored too.  `all`: every shell voxel is stored. */
+struct QsBand {
+    int lo, hi;
+    int edge, all;
+};
+
 /* One molecule of a batch: its grid and where its rows live in the concatenated arrays. */
 struct QsMol {
     QsGrid G;

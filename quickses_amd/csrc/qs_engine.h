@@ -109,6 +109,7 @@ struct OffsetTables {
     int r = -1;
     float dx = 0, cmax = 0, bound = 0;
     std::vector<int> offs, norm_start, enum_end;
+    QsBand band = {0, 255, 0, 1};
 };
 
 void build_offset_tables(int r, float dx, float coord_max, OffsetTables &T);
@@ -182,8 +183,13 @@ struct MolIn {
 struct P2Tables {
     int r;
     float dx, cmax;
-    DevBuf offs, norm, end;
+    DevBuf dev; /* offs, then norm_start, then enum_end; none when every norm is decided by flags */
+    size_t norm_at, end_at;
     QsNormFlags flags;
+    QsBand band;
+    const int *offs() const { return (const int *)dev.p; }
+    const int *norm() const { return dev.p ? (const int *)dev.p + norm_at : nullptr; }
+    const int *end() const { return dev.p ? (const int *)dev.p + end_at : nullptr; }
 };
 
 /* molecules sharing a field-pass-2 kernel (path, r) and candidate tables (dx, coordinate range) */
@@ -304,6 +310,11 @@ struct Engine {
     /* field holds the shell voxels' values only (field pass 2), densely in shell-rank order (spre);
        the others come from outm / shellm.  Else field holds every voxel in grid order. */
     bool field_sparse = false;
+    /* the stored shell values are those the mesh reads only (QsBand); complete_field evaluates the
+       rest.  normals_used: the last result's normals were asked for, so the next run stores every
+       value at once, as its normals would need them (the mesh is the same either way) */
+    bool field_band = false, normals_used = false;
+    const uint8_t *run_flags = nullptr; /* the run's tile marks, null when field pass 1 set none */
     /* the last run's atom ids are cell-sorted positions (option atom_ids_sorted at run time) */
     bool ids_sorted = false;
     /* row words the marching-cubes scans cover: [scan_w0, scan_w0 + scan_nw) */
@@ -348,9 +359,7 @@ struct Engine {
                           &tpre_d, &tflag, &spre, &stot, &field_dense})
             release(*b);
         for (P2Tables *t : tables) {
-            release(t->offs);
-            release(t->norm);
-            release(t->end);
+            release(t->dev);
             delete t;
         }
         tables.clear();
@@ -457,6 +466,8 @@ struct Engine {
     int run_batch(const float *d_pos, const float *d_rad, const std::vector<MolIn> &in, int smooth,
                   const std::vector<BBox> *host_bbox);
     int field_stage(uint32_t nb_p1, size_t at_p1, StageTimer &tm);
+    int run_pass2(bool all);
+    int complete_field();
     int fill_field(const void **dense);
     int mesh_stage(size_t at_mc, uint32_t nb_mc, size_t at_wpre, StageTimer &tm, bool with_atoms);
     int group_tables(P2Group &grp);

@@ -221,6 +221,22 @@ void build_offset_tables(int r, float dx, float coord_max, OffsetTables &T)
         while (hi + 1 <= nmax && std::sqrt((double)(hi + 1)) <= lim) hi++;
         T.enum_end[n] = T.norm_start[hi + 1];
     }
+    /* QsBand: klo, khi = the largest norms whose float distance is below the probe radius for
+       certain, and possibly not above it */
+    const double probe = (double)QS_PROBE, ddx = (double)dx;
+    int klo = -1, khi = -1;
+    for (int n = 0; n <= nmax; n++) {
+        const double d = ddx * std::sqrt((double)n);
+        if (d + delta < probe) klo = n;
+        if (d - delta <= probe) khi = n;
+    }
+    T.band = QsBand{0, 255, 0, 1};
+    if (klo >= 0 && khi <= r * r && nmax < 255) {
+        int lo = -1;
+        while (std::sqrt((double)(lo + 1)) + 1.0 <= std::sqrt((double)klo) + 1e-9) lo++;
+        const double far = std::sqrt((double)khi) + 1.0;
+        T.band = QsBand{lo, std::min((int)std::floor(far * far + 1e-9) + 1, 255), khi == r * r ? 1 : 0, 0};
+    }
 }
 
 
@@ -446,23 +462,29 @@ int Engine::build_meta(size_t &at_atoms, size_t &at_p1, size_t &at_mc, size_t &a
 int Engine::group_tables(P2Group &grp)
 {
     for (P2Tables *t : tables)
-        if (t->r == grp.r && t->dx == grp.dx && t->cmax == grp.cmax) {
+        if (t->r == grp.r && t->dx == grp.dx && t->cmax == grp.cmax && (grp.path == 0 || t->dev.p)) {
             grp.tab = t;
             return 0;
         }
     OffsetTables T;
     build_offset_tables(grp.r, grp.dx, grp.cmax, T);
-    P2Tables *t = new P2Tables{grp.r, grp.dx, grp.cmax, DevBuf{}, DevBuf{}, DevBuf{}, QsNormFlags{{0, 0, 0, 0}}};
-    for (int n = 0; n < 256 && n + 1 < (int)T.norm_start.size(); n++)
+    P2Tables *t = new P2Tables{grp.r, grp.dx, grp.cmax, DevBuf{}, T.offs.size(), T.offs.size() + T.norm_start.size(),
+                               QsNormFlags{{0, 0, 0, 0}}, T.band};
+    bool decided = grp.path == 0;
+    for (int n = 0; n < 256 && n + 1 < (int)T.norm_start.size(); n++) {
         if (T.enum_end[n] == T.norm_start[n + 1]) t->flags.w[n >> 6] |= 1ull << (n & 63);
+        else decided = false;
+    }
     tables.push_back(t);
-    QS_TRY(ensure(t->offs, T.offs.size() * 4));
-    QS_TRY(ensure(t->norm, T.norm_start.size() * 4));
-    QS_TRY(ensure(t->end, T.enum_end.size() * 4));
-    /* synchronous copies: T is freed on return */
-    QS_HIP(hipMemcpy(t->offs.p, T.offs.data(), T.offs.size() * 4, hipMemcpyHostToDevice));
-    QS_HIP(hipMemcpy(t->norm.p, T.norm_start.data(), T.norm_start.size() * 4, hipMemcpyHostToDevice));
-    QS_HIP(hipMemcpy(t->end.p, T.enum_end.data(), T.enum_end.size() * 4, hipMemcpyHostToDevice));
+    /* (the fixed-R kernel looks a norm up in the tables only when its flag is not set) */
+    if (!decided) {
+        std::vector<int> all(T.offs);
+        all.insert(all.end(), T.norm_start.begin(), T.norm_start.end());
+        all.insert(all.end(), T.enum_end.begin(), T.enum_end.end());
+        QS_TRY(ensure(t->dev, all.size() * 4));
+        /* a synchronous copy: its source is freed on return */
+        QS_HIP(hipMemcpy(t->dev.p, all.data(), all.size() * 4, hipMemcpyHostToDevice));
+    }
     grp.tab = t;
     return 0;
 }
@@ -505,17 +527,37 @@ int Engine::field_stage(uint32_t nb_p1, size_t at_p1, StageTimer &tm)
        (the shell voxels are at most the voxels, which the field is sized for) */
     qs_launch_shell_scan(as<uint64_t>(shellm), nw_total, as<uint32_t>(scan_tmp), as<uint32_t>(stot), as<uint32_t>(spre), stream);
     tm.mark("shell_scan");
-    for (auto &grp : groups) {
-        QS_TRY(group_tables(grp));
-        qs_launch_pass2(batch(grp.bpre_at, grp.mid_at, (int)grp.mols.size()), grp.nblocks, grp.r, grp.path, as<uint64_t>(outm),
-                        as<uint64_t>(shellm), as<uint32_t>(spre), as<float>(field), as<uint32_t>(negm), as<uint32_t>(zerom), as<int>(grp.tab->offs),
-                        as<int>(grp.tab->norm), as<int>(grp.tab->end), grp.tab->flags,
-                        (tf && grp.path == 0) ? tf + mols[grp.mols[0]].tile_off : nullptr, tmark, grp.xchunk, stream);
-        QS_HIP(hipGetLastError());
-    }
+    run_flags = tf;
+    QS_TRY(run_pass2(normals_used));
+    normals_used = false;
     field_sparse = true;
     tm.mark("pass2");
     return 0;
+}
+
+/* field pass 2 over every molecule: the values a mesh reads, or all */
+int Engine::run_pass2(bool all)
+{
+    field_band = false;
+    for (auto &grp : groups) {
+        QS_TRY(group_tables(grp));
+        QsBand band = grp.tab->band;
+        if (all) band = QsBand{0, 255, 0, 1};
+        if (grp.path == 0 && !band.all) field_band = true;
+        qs_launch_pass2(batch(grp.bpre_at, grp.mid_at, (int)grp.mols.size()), grp.nblocks, grp.r, grp.path, as<uint64_t>(outm),
+                        as<uint64_t>(shellm), as<uint32_t>(spre), as<float>(field), as<uint32_t>(negm), as<uint32_t>(zerom),
+                        grp.tab->offs(), grp.tab->norm(), grp.tab->end(), grp.tab->flags, band,
+                        (run_flags && grp.path == 0) ? run_flags + mols[grp.mols[0]].tile_off : nullptr, tmark, grp.xchunk, stream);
+        QS_HIP(hipGetLastError());
+    }
+    return 0;
+}
+
+/* the shell values that the last run left out (its masks, ranks and tile marks are still there; the
+   sign words are written again with the same bits) */
+int Engine::complete_field()
+{
+    return field_sparse && field_band ? run_pass2(true) : 0;
 }
 
 /* every voxel of every molecule's field in grid order (pass 2 stores the shell voxels only):
@@ -524,6 +566,7 @@ int Engine::fill_field(const void **dense)
 {
     *dense = field.p;
     if (!field_sparse) return 0;
+    QS_TRY(complete_field());
     QS_TRY(ensure(field_dense, std::max<uint64_t>(vox_total, 1) * 4));
     for (const QsMol &M : mols)
         qs_launch_field_expand(as<float>(field), as<uint32_t>(spre) + M.word_off, as<uint64_t>(outm) + M.word_off,
@@ -1733,6 +1776,8 @@ static int launch_normals(Engine &E, float *d_out)
 {
     if (!E.batch_valid) return set_error(3, "no mesh to take normals of");
     if (E.multi_slab) return set_error(3, "normals: the last mesh was built in x-slabs; its field is not kept");
+    QS_TRY(E.complete_field());
+    E.normals_used = true;
     const int nmol = (int)E.mols.size();
     const uint32_t *d_vpre = as<uint32_t>(E.d_off) + (nmol + 1);
     qs_launch_vertex_normals(as<QsMol>(E.d_mols), d_vpre, d_vpre + nmol + 1, as<uint64_t>(E.vkey), E.nv, as<float>(E.field),
@@ -1950,14 +1995,8 @@ int qs_stage_pass2(const float *fp, const int *ip, const uint8_t *labels, float 
     QS_TRY(ensure(E.scan_tmp, qs_scan_tiles(E.nw_total) * sizeof(uint32_t)));
     qs_launch_shell_scan(as<uint64_t>(E.shellm), E.nw_total, as<uint32_t>(E.scan_tmp), as<uint32_t>(E.stot), as<uint32_t>(E.spre),
                          E.stream);
-    for (auto &grp : E.groups) {
-        QS_TRY(E.group_tables(grp));
-        qs_launch_pass2(E.batch(grp.bpre_at, grp.mid_at, (int)grp.mols.size()), grp.nblocks, grp.r, grp.path,
-                        as<uint64_t>(E.outm), as<uint64_t>(E.shellm), as<uint32_t>(E.spre), as<float>(E.field), as<uint32_t>(E.negm),
-                        as<uint32_t>(E.zerom), as<int>(grp.tab->offs), as<int>(grp.tab->norm), as<int>(grp.tab->end),
-                        grp.tab->flags, nullptr, 0, grp.xchunk, E.stream);
-        QS_HIP(hipGetLastError());
-    }
+    E.run_flags = nullptr;
+    QS_TRY(E.run_pass2(true));
     E.field_sparse = true;
     const void *dense = nullptr;
     QS_TRY(E.fill_field(&dense));

@@ -235,6 +235,28 @@ __device__ __forceinline__ uint32_t wave_sum_below(const uint32_t *__restrict__ 
     return x;
 }
 
+/* bit position of the r-th set bit (from 0) of m, which has more than r */
+__device__ __forceinline__ int nth_bit32(uint32_t m, uint32_t r)
+{
+    int b = 0;
+#pragma unroll
+    for (int h = 16; h >= 1; h >>= 1) {
+        const uint32_t c = (uint32_t)__popc(m & ((1u << h) - 1u));
+        const bool up = r >= c;
+        r -= up ? c : 0u;
+        m >>= up ? h : 0;
+        b += up ? h : 0;
+    }
+    return b;
+}
+
+__device__ __forceinline__ int nth_bit(uint64_t w, uint32_t r)
+{
+    const uint32_t low = (uint32_t)__popc((uint32_t)w);
+    const bool up = r >= low;
+    return (up ? 32 : 0) + nth_bit32((uint32_t)(up ? w >> 32 : w), up ? r - low : r);
+}
+
 /* ------------------------------------------------------------------------------------------ */
 /* device-wide exclusive scan of uint32 (reduce tiles, scan tile sums, scan tiles)              */
 
@@ -1884,12 +1906,17 @@ __device__ __forceinline__ uint32_t zdist2(uint64_t m, int z)
    Kernels.cu:478-545), one 16 x 8 x 32 tile per block:
    - the tile's own shell and outside bits; a tile without a shell voxel writes its sign words only;
    - the outside rows of the tile and its R halo in LDS;
-   - the exact minimal squared norm n_min of every shell voxel by separable minima: z distances
-     from the row bits, y minima (with the masks of the attaining y offsets) for the listed
-     columns only, x minima two outputs per register;
+   - the voxels whose value the mesh can read (QsBand) and the signs of the others, by dilating the
+     outside bits 32 voxels at a time; a tile with none of them is done;
+   - for those, the exact minimal squared norm n_min by separable minima: z distances from the row
+     bits, y minima (with the masks of the attaining y offsets) for the columns they read, x minima;
    - the exact float distance of the minimisers, traced back through the masks (or enumerated
      from a norm-sorted table where another norm could tie), rooted once;
-   - the field of shell voxels (the others follow from the masks) and every voxel's sign bits. */
+   - the field of those voxels, and every voxel's sign bits.
+   Bound by VALU issue and, at R = 7, by LDS reads of the dilated rows.  Evaluating every shell
+   voxel with an outside voxel in reach (28 to 38 % of the shell; 8 to 15 % are read) by x minima and
+   trace took 0.592 ms on the 50,000-atom 0.2 A mesh (R 7), 0.610 on 200,000 atoms at 0.3 A (R 5) and
+   0.923 on 100 frames of 10,000 atoms at 0.5 A (R 3); this takes 0.468, 0.431 and 0.614. */
 
 /* entry it of a per-plane bit list: the plane lx with cpre[lx] <= it < cpre[lx + 1] (binary
    search) and the z of the (it - cpre[lx])-th set bit of cmask[lx] */
@@ -1921,31 +1948,39 @@ __global__ void __launch_bounds__(256) k_pass2_r(QsBatch B, const uint64_t *__re
                                                  float *__restrict__ field, uint32_t *__restrict__ negm_all,
                                                  uint32_t *__restrict__ zerom_all, const int *__restrict__ offs,
                                                  const int *__restrict__ norm_start, const int *__restrict__ enum_end,
-                                                 QsNormFlags nf, const uint8_t *__restrict__ tflag, uint8_t tmark, uint32_t xchunk)
+                                                 QsNormFlags nf, QsBand band, const uint8_t *__restrict__ tflag, uint8_t tmark,
+                                                 uint32_t xchunk)
 {
     constexpr int LX = P2R_TX + 2 * R, LY = P2_TY + 2 * R, LZ = P2_TZ + 2 * R;
     constexpr int INF = 255;
     static_assert(LZ <= 64 && 3 * R * R < INF, "window too wide for this kernel");
-    __shared__ uint64_t rows[LX * LY];
+    constexpr int NR = LX * LY;
+    __shared__ uint64_t rows[NR];
     /* ownout: the own rows' outside bits, read only by a tile without a shell voxel; after that
        test the array holds the own rows' shell ranks (sbase) instead */
     __shared__ uint32_t own[P2R_TX * P2_TY], ownout[P2R_TX * P2_TY];
     uint32_t *const sbase = ownout;
-    __shared__ uint32_t DYw[LX * P2_TY * P2_TZ / 4];
-    uint8_t *DY = (uint8_t *)DYw;
+    /* y offsets (bit b + R) attaining each DY value */
+    using BMask = typename std::conditional<(2 * R + 1 <= 8), uint8_t,
+                                            typename std::conditional<(2 * R + 1 <= 16), uint16_t, uint32_t>::type>::type;
+    /* first the rows' own 32 voxels dilated by 0 .. R along z (dil[c * NR + row]), then the y minima
+       (DY) and their masks (BM) */
+    constexpr int NDY = LX * P2_TY * P2_TZ;
+    __shared__ uint32_t pool[(R + 1) * NR * 4 > NDY * (1 + (int)sizeof(BMask)) ? (R + 1) * NR : NDY * (1 + (int)sizeof(BMask)) / 4];
+    uint32_t *const dil = pool;
+    uint8_t *const DY = (uint8_t *)pool;
+    BMask *const BM = (BMask *)(pool + NDY / 4);
     /* y-pass work list: per halo x plane lx, the z columns (bit z) that need y minima, and the
        exclusive prefix of their counts (cpre[LX] = total) */
     __shared__ uint32_t shx[P2R_TX], cmask[LX], cpre[LX + 1];
     /* norms whose minimisers are traced back (bit n), from nf */
     __shared__ uint32_t nfw[8];
-    /* y offsets (bit b + R) attaining each DY value */
-    using BMask = typename std::conditional<(2 * R + 1 <= 8), uint8_t,
-                                            typename std::conditional<(2 * R + 1 <= 16), uint16_t, uint32_t>::type>::type;
-    __shared__ BMask BM[LX * P2_TY * P2_TZ];
-    /* per wave, the voxels whose minimisers are still to be traced back (tx | row bit << 4 | z << 5),
-       and per own (x, y) row of the tile its sign and zero words */
-    __shared__ uint16_t tq[4][128];
-    __shared__ uint32_t sneg[P2R_TX * P2_TY], szero[P2R_TX * P2_TY];
+    /* half-lengths along z of the balls of norms below band.hi (0) and up to band.lo (1) at x and y
+       offsets |a|, |b| (255: none) */
+    __shared__ uint8_t zlen[2][R + 1][R + 1];
+    /* per own (x, y) row of the tile: the voxels whose minimisers are to be traced back, its sign
+       words and its zero words */
+    __shared__ uint32_t strace[P2R_TX * P2_TY], sneg[P2R_TX * P2_TY], szero[P2R_TX * P2_TY];
     uint32_t lb;
     /* each XCD takes xchunk consecutive tiles at a time (whole rows of z tiles: the y and z halos
        of a tile are then mostly read by tiles of the same XCD, from its L2) */
@@ -1983,6 +2018,15 @@ __global__ void __launch_bounds__(256) k_pass2_r(QsBatch B, const uint64_t *__re
                 m = row_bits(outm + ((size_t)gx * g + gy_) * W, W, tz0 - R, LZ);
             rows[row] = m;
             fl |= (m != 0ull);
+            /* bit z of d: an outside voxel within c of z (bit z + R of m is z) */
+            uint32_t d = __builtin_amdgcn_alignbit((uint32_t)(m >> 32), (uint32_t)m, R);
+            dil[row] = d;
+#pragma unroll
+            for (int c = 1; c <= R; c++) {
+                d |= __builtin_amdgcn_alignbit((uint32_t)(m >> 32), (uint32_t)m, R - c) |
+                     __builtin_amdgcn_alignbit((uint32_t)(m >> 32), (uint32_t)m, R + c);
+                dil[c * NR + row] = d;
+            }
         }
     };
     /* a tile marked by field pass 1 has a shell voxel: its halo rows are loaded together with its
@@ -1999,6 +2043,14 @@ __global__ void __launch_bounds__(256) k_pass2_r(QsBatch B, const uint64_t *__re
         const uint64_t w = t < 2 ? nf.w[0] : (t < 4 ? nf.w[1] : (t < 6 ? nf.w[2] : nf.w[3]));
         nfw[t] = (uint32_t)(w >> (32 * (t & 1)));
     }
+    if (threadIdx.x < 2 * (R + 1) * (R + 1)) {
+        const int set = threadIdx.x / ((R + 1) * (R + 1)), ab = threadIdx.x - set * (R + 1) * (R + 1);
+        const int a = ab / (R + 1), b = ab - a * (R + 1);
+        const int rem = (set ? band.lo : band.hi - 1) - a * a - b * b; /* c^2 <= rem */
+        int c = rem < 0 ? 255 : min((int)__builtin_amdgcn_sqrtf((float)rem + 0.5f), R);
+        if (band.all) c = set ? 255 : R; /* the whole window, and nothing */
+        zlen[set][a][b] = (uint8_t)c;
+    }
     int has_shell;
     uint32_t sb = 0u;
     {
@@ -2014,14 +2066,31 @@ __global__ void __launch_bounds__(256) k_pass2_r(QsBatch B, const uint64_t *__re
             m = (uint32_t)(wv >> (tz0 & 63));
             if (threadIdx.x < 128) sb = spre[wi] + (uint32_t)__popcll(wv & bits_below(tz0 & 63, 0));
         }
-        if (marked) load_rows();
-        if (threadIdx.x < 128) {
-            own[t] = m;
-            /* shell bits of each own x plane, over its P2_TY rows (consecutive lanes) */
-            uint32_t sx = m;
+        /* with band.edge: the row's outside words R + 1 steps away along x and y, and the ones next
+           to its own along z (a place outside the grid reads the row's own word and is masked), in
+           flight with the halo rows */
+        uint32_t ew[7] = {0u, 0u, 0u, 0u, 0u, 0u, 0u}, ek[7] = {0u, 0u, 0u, 0u, 0u, 0u, 0u};
+        if (band.edge && threadIdx.x < 128 && gx < x1 && gx < g && gy_ < g) {
+            const uint32_t *__restrict__ o32 = (const uint32_t *)outm + ((size_t)gx * g + gy_) * (2 * (size_t)W) + (tz0 >> 5);
+            const ptrdiff_t wy = 2 * (ptrdiff_t)W, wx = g * wy;
+            const bool k[7] = {true, tz0 > 0, (tz0 >> 5) + 1 < 2 * W, gx - (R + 1) >= M.p1_lo, gx + (R + 1) < M.p1_hi,
+                               gy_ - (R + 1) >= 0, gy_ + (R + 1) < g};
+            const ptrdiff_t at[7] = {0, -1, 1, -(R + 1) * wx, (R + 1) * wx, -(R + 1) * wy, (R + 1) * wy};
 #pragma unroll
-            for (int k = 1; k < P2_TY; k *= 2) sx |= (uint32_t)__shfl_xor((int)sx, k);
-            if (ty_ == 0) shx[tx] = sx;
+            for (int i = 0; i < 7; i++) {
+                ew[i] = o32[k[i] ? at[i] : 0];
+                ek[i] = k[i] ? ~0u : 0u;
+            }
+        }
+        if (marked) load_rows();
+#pragma unroll
+        for (int i = 0; i < 7; i++) ew[i] &= ek[i];
+        /* the row's voxels with an outside voxel R + 1 steps away along an axis */
+        const uint32_t far = (ew[0] << (R + 1) | ew[1] >> (31 - R)) | (ew[0] >> (R + 1) | ew[2] << (31 - R)) | ew[3] | ew[4] | ew[5] | ew[6];
+        if (threadIdx.x < 128) {
+            strace[t] = szero[t] = 0u;
+            sneg[t] = far;
+            own[t] = m;
         } else {
             ownout[t] = m;
         }
@@ -2054,16 +2123,6 @@ __global__ void __launch_bounds__(256) k_pass2_r(QsBatch B, const uint64_t *__re
     };
 
     if (!marked) load_rows();
-    /* every y minimum starts unreachable; only listed columns are computed */
-    for (int i = threadIdx.x; i < LX * P2_TY * P2_TZ / 4; i += 256) DYw[i] = 0x01010101u * INF;
-    /* a column (lx, z) is read by the x pass only for shell voxels of own planes lx - 2R .. lx */
-    uint32_t need = 0;
-    if (threadIdx.x < LX) {
-        const int lx = threadIdx.x;
-#pragma unroll
-        for (int tx = 0; tx < P2R_TX; tx++)
-            if (tx >= lx - 2 * R && tx <= lx) need |= shx[tx];
-    }
     if (!(marked ? has_shell : __syncthreads_or(fl))) {
         /* no outside voxel within reach: every voxel of the tile is -dx (a marked tile has passed
            no barrier since its shell ranks were written) */
@@ -2071,19 +2130,86 @@ __global__ void __launch_bounds__(256) k_pass2_r(QsBatch B, const uint64_t *__re
         for (int tx = 0; tx < P2R_TX; tx++) {
             int gx = tx0 + tx;
             if (gx >= x1 || gx >= g) break;
-            if (vyz && ((own[tx * P2_TY + ty] >> tz) & 1u)) field[fidx(tx, ty, tz)] = -dx;
+            if ((band.all || band.edge) && vyz && ((own[tx * P2_TY + ty] >> tz) & 1u)) field[fidx(tx, ty, tz)] = -dx;
             emit_sign_bits(negm, zerom, W, g, gx, gy, tz0, vyz, -dx);
         }
         return;
     }
 
-    /* the work list: columns needed by a shell voxel with an outside voxel within R of their z
+    /* Which voxels are near enough to the surface to be read (QsBand), and the signs of the others,
+       for 32 voxels of a row at a time: the outside bits dilated by the ball of norms below band.hi
+       (strace) and by the one up to band.lo (szero), each clipped to the window.  A ball is a disc of
+       (x, y) offsets with a z length each, so a row is the OR of the rows at those offsets, dilated
+       along z (dil).  A lane takes two rows, each wave some of the x offsets; offsets x = -a and a
+       have the same lengths, which the lanes hold per y offset.  (From the x minima of every shell voxel
+       instead, with the y minima of every column a shell voxel reads, this took more than half of
+       the kernel at 0.5 A.) */
+    const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    {
+        const int r0 = ((lane >> 2) + R) * LY + 2 * (lane & 3); /* + (y offset + R), + x offset * LY */
+#pragma unroll 1
+        for (int set = 0; set < 2; set++) {
+            uint32_t acc0 = 0u, acc1 = 0u;
+            /* wave w takes the x offsets w, 7 - w and 8 + w (discs of about the same total width) */
+#pragma unroll 1
+            for (int i = 0; i < 3; i++) {
+                const int a = i == 0 ? wid : (i == 1 ? 7 - wid : 8 + wid);
+                if (a > R) continue;
+                const int c = lane <= 2 * R ? (int)zlen[set][a][lane < R ? R - lane : lane - R] : 255;
+                const int at = c * NR + lane; /* per y offset + R = lane */
+                const uint64_t some = __ballot(c != 255); /* y offsets -nb .. nb, or none */
+                const int nb = (int)__popcll(some) >> 1;
+                if (!some) continue;
+                const uint32_t *const pu = dil + r0 + a * LY, *const pv = dil + r0 - a * LY;
+#pragma unroll 4
+                for (int b = R - nb; b <= R + nb; b++) {
+                    const int o = __builtin_amdgcn_readlane(at, b);
+                    acc0 |= pu[o] | pv[o];
+                    acc1 |= pu[o + 1] | pv[o + 1];
+                }
+            }
+            uint32_t *const acc = set ? szero : strace;
+            const int t = (lane >> 2) * P2_TY + 2 * (lane & 3);
+            if (acc0) atomicOr(&acc[t], acc0);
+            if (acc1) atomicOr(&acc[t + 1], acc1);
+        }
+    }
+    __syncthreads();
+    bool any = false;
+    if (threadIdx.x < 128) {
+        const int t = threadIdx.x, tx = t / P2_TY, ty_ = t - tx * P2_TY;
+        const bool in = tx0 + tx < x1 && tx0 + tx < g && ty0 + ty_ < g;
+        const uint32_t valid = !in ? 0u : (tz0 + P2_TZ <= g ? ~0u : (1u << (g - tz0)) - 1u);
+        const uint32_t hi = strace[t], lo = szero[t], far = sneg[t], sh = own[t] & valid, o = dil[(tx + R) * LY + ty_ + R];
+        const uint32_t tr = sh & ((hi & ~lo) | (far & ~hi));
+        /* negative: inside, and shell beyond the band (a traced voxel's bits follow from its value) */
+        strace[t] = tr;
+        sneg[t] = valid & ~o & ~(sh & lo) & ~tr;
+        szero[t] = 0u;
+        any = tr != 0u;
+        if (band.all) /* shell voxels without an outside voxel in the window: -dx */
+            for (uint32_t w = sh & ~hi; w; w &= w - 1u) field[fidx(tx, ty_, __builtin_ctz(w))] = -dx;
+        /* the traced voxels of each own x plane, over its P2_TY rows (consecutive lanes) */
+        uint32_t sx = tr;
+#pragma unroll
+        for (int k = 1; k < P2_TY; k *= 2) sx |= (uint32_t)__shfl_xor((int)sx, k);
+        if (ty_ == 0) shx[tx] = sx;
+    }
+    if (__syncthreads_or(any)) {
+    /* every y minimum starts unreachable; only listed columns are computed */
+    for (int i = threadIdx.x; i < NDY / 4; i += 256) pool[i] = 0x01010101u * INF;
+    /* the work list: columns needed by a traced voxel with an outside voxel within R of their z
        in some row (else every minimum is INF, as filled) */
     static_assert(LX <= 64, "one lane per halo x plane");
     if (threadIdx.x < 64) {
         const int lx = threadIdx.x;
         uint32_t c = 0;
         if (lx < LX) {
+            /* a column (lx, z) is read by the x taps of traced voxels of own planes lx - 2R .. lx */
+            uint32_t need = 0;
+#pragma unroll
+            for (int tx = 0; tx < P2R_TX; tx++)
+                if (tx >= lx - 2 * R && tx <= lx) need |= shx[tx];
             uint64_t o = 0;
 #pragma unroll
             for (int ly = 0; ly < LY; ly++) o |= rows[lx * LY + ly];
@@ -2182,20 +2308,11 @@ __global__ void __launch_bounds__(256) k_pass2_r(QsBatch B, const uint64_t *__re
     }
     __syncthreads();
 
-    /* x, one (ty, tz) column per thread, in two phases.  Phase 1: each voxel's minimal squared
-       norm over its x window; a voxel with nothing to trace back gets its field value and sign
-       bits at once, the others join the wave's queue.  Phase 2: the wave's 64 lanes take queued
-       voxels 64 at a time (so lanes whose own voxels need nothing do not idle), find the x
-       offsets attaining the minimum again, trace the minimisers back through the y masks and
-       take the exact float distance.  The sign and zero words gather in LDS and are stored once
-       per row at the end. */
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    uint16_t *__restrict__ queue = tq[wid];
-    int qn = 0;
-    auto trace_items = [&](int count) {
-        if (lane >= count) return;
-        const uint32_t it = queue[lane];
-        const int tx = (int)(it & 15u), ty_ = 2 * wid + (int)((it >> 4) & 1u), tz_ = (int)(it >> 5);
+    /* the block's marked voxels, 64 at a time per wave in row order: the x minimum and the offsets
+       attaining it, the minimisers traced back through the y masks, and their exact float distance.
+       (Traced as soon as a wave had queued 64, from inside an unrolled loop over the x minima, the
+       kernel had 16 copies of the trace, 60 KB of code.) */
+    auto trace_voxel = [&](int tx, int ty_, int tz_) {
         const int gx = tx0 + tx, gy_ = ty0 + ty_, gz_ = tz0 + tz_;
         /* the x offsets (bit a + R) attaining the minimal norm */
         int nmin = INF;
@@ -2244,7 +2361,9 @@ __global__ void __launch_bounds__(256) k_pass2_r(QsBatch B, const uint64_t *__re
         /* the smallest squared distance, rooted once at the end: sqrtf rounds correctly and is
            monotone, so the root of the minimum is the minimum of the roots */
         float min_sq = __builtin_inff();
-        if ((nfw[nmin >> 5] >> (nmin & 31)) & 1u) {
+        if (nmin >= INF) {
+            /* no outside voxel in the window: -dx */
+        } else if ((nfw[nmin >> 5] >> (nmin & 31)) & 1u) {
             /* trace the minimisers back through the separable passes: the x offsets, then their y
                offsets from the recorded masks */
             while (amask) {
@@ -2284,92 +2403,37 @@ __global__ void __launch_bounds__(256) k_pass2_r(QsBatch B, const uint64_t *__re
         if (res < 0.0f) atomicOr(&sneg[tx * P2_TY + ty_], 1u << tz_);
         if (res == 0.0f) atomicOr(&szero[tx * P2_TY + ty_], 1u << tz_);
     };
-    /* voxel tx of the thread's column, whose minimal norm is nmin (INF: no outside voxel within
-       the window): settled now, or queued */
-    auto handle = [&](int tx, int nmin) {
-        const bool out = (rows[(tx + R) * LY + (ty + R)] >> (tz + R)) & 1ull;
-        const bool shell = (own[tx * P2_TY + ty] >> tz) & 1u; /* never outside */
-        const bool traced = vyz && shell && nmin < INF;
-        /* outside: the probe radius; inside, or shell without an outside voxel in reach: -dx */
-        if (vyz && shell && !traced) field[fidx(tx, ty, tz)] = -dx;
-        const uint64_t nb = __ballot(vyz && !traced && !out);
-        if ((lane & 31) == 0) {
-            sneg[tx * P2_TY + ty] = (uint32_t)(lane ? (nb >> 32) : nb);
-            szero[tx * P2_TY + ty] = 0u;
+    {
+        /* lane l's rows are 2 l and 2 l + 1 */
+        const uint32_t m0 = strace[2 * lane], m1 = strace[2 * lane + 1];
+        const uint32_t n0 = (uint32_t)__popc(m0), nn = n0 + (uint32_t)__popc(m1);
+        uint32_t pre = nn;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const uint32_t t = (uint32_t)__shfl_up((int)pre, d, 64);
+            if (lane >= d) pre += t;
         }
-        const uint64_t tm = __ballot(traced);
-        if (traced) queue[qn + __popcll(tm & ((1ull << lane) - 1ull))] = (uint16_t)(tx | ((lane >> 5) << 4) | (tz << 5));
-        qn += __popcll(tm);
-        if (qn >= 64) {
-            wave_lds_sync();
-            trace_items(64);
-            wave_lds_sync();
-            const int rest = qn - 64;
-            const uint16_t mv = (lane < rest) ? queue[64 + lane] : (uint16_t)0;
-            wave_lds_sync();
-            if (lane < rest) queue[lane] = mv;
-            wave_lds_sync();
-            qn = rest;
-        }
-    };
-
-    if constexpr (2 * R + 1 <= 16) {
-        /* two x outputs per 32-bit register: the minimum over the 2R+1 taps (16-bit lanes) */
-        typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
-        u16x2 U[LX - 1];
-        {
-            uint32_t u[LX];
+        const uint32_t total = (uint32_t)__shfl((int)pre, 63, 64);
+        pre -= nn; /* exclusive */
+#pragma unroll 1
+        for (uint32_t base = 64u * (uint32_t)wid; base < total; base += 256u) {
+            const uint32_t j = base + (uint32_t)lane;
+            /* the item's pair of rows: the last lane whose first item is at or below j */
+            int o = 0;
 #pragma unroll
-            for (int lx = 0; lx < LX; lx++) u[lx] = DY[(lx * P2_TY + ty) * P2_TZ + tz];
-#pragma unroll
-            for (int k = 0; k < LX - 1; k++) U[k] = __builtin_bit_cast(u16x2, u[k] | (u[k + 1] << 16));
-        }
-        static_assert(P2R_TX % 2 == 0, "x outputs in pairs");
-#pragma unroll
-        for (int tx = 0; tx < P2R_TX; tx += 2) {
-            const int gx = tx0 + tx;
-            if (gx >= x1 || gx >= g) break;
-            const bool two = gx + 1 < x1 && gx + 1 < g;
-            const uint32_t sh = ((own[tx * P2_TY + ty] >> tz) & 1u) | (two ? ((own[(tx + 1) * P2_TY + ty] >> tz) & 1u) << 1 : 0u);
-            uint32_t nm = (uint32_t)INF * 0x10001u;
-            if (vyz && sh) {
-                constexpr int NT = 2 * R + 1;
-                u16x2 t[NT];
-#pragma unroll
-                for (int a = 0; a < NT; a++) {
-                    const uint16_t c = (uint16_t)((a - R) * (a - R));
-                    t[a] = U[tx + a] + (u16x2){c, c};
-                }
-#pragma unroll
-                for (int s2 = 1; s2 < NT; s2 *= 2)
-#pragma unroll
-                    for (int a = 0; a + s2 < NT; a += 2 * s2) t[a] = __builtin_elementwise_min(t[a], t[a + s2]);
-                nm = __builtin_bit_cast(uint32_t, __builtin_elementwise_min(t[0], (u16x2){(uint16_t)INF, (uint16_t)INF}));
-            }
-            handle(tx, (int)(nm & 0xFFFFu));
-            if (two) handle(tx + 1, (int)(nm >> 16));
-        }
-    } else {
-        int u[LX];
-#pragma unroll
-        for (int lx = 0; lx < LX; lx++) u[lx] = DY[(lx * P2_TY + ty) * P2_TZ + tz];
-#pragma unroll
-        for (int tx = 0; tx < P2R_TX; tx++) {
-            const int gx = tx0 + tx;
-            if (gx >= x1 || gx >= g) break;
-            int nmin = INF;
-            if (vyz && ((own[tx * P2_TY + ty] >> tz) & 1u)) {
-#pragma unroll
-                for (int a = 0; a <= 2 * R; a++) nmin = min(nmin, u[tx + a] + (a - R) * (a - R));
-            }
-            handle(tx, nmin);
+            for (int step = 32; step >= 1; step >>= 1)
+                if ((uint32_t)__shfl((int)pre, o + step, 64) <= j) o += step;
+            uint32_t r = j - (uint32_t)__shfl((int)pre, o, 64);
+            const uint32_t on0 = (uint32_t)__shfl((int)n0, o, 64);
+            const uint32_t om0 = (uint32_t)__shfl((int)m0, o, 64), om1 = (uint32_t)__shfl((int)m1, o, 64);
+            const bool second = r >= on0;
+            r -= second ? on0 : 0u;
+            const int row = 2 * o + (second ? 1 : 0);
+            if (j < total) trace_voxel(row / P2_TY, row % P2_TY, nth_bit32(second ? om1 : om0, r));
         }
     }
-    if (qn > 0) {
-        wave_lds_sync();
-        trace_items(qn);
+    __syncthreads();
     }
-    wave_lds_sync();
     /* the wave's sign and zero words: lane = x (0-15) | row bit << 4 | zero word << 5 */
     {
         const int tx = lane & 15, ty_ = 2 * wid + ((lane >> 4) & 1);
@@ -2896,28 +2960,6 @@ __global__ void __launch_bounds__(256) k_mc_vertices(const QsMol *__restrict__ m
     }
     __syncthreads(); /* S is staged again for the next block */
     }
-}
-
-/* bit position of the r-th set bit (from 0) of w, which has more than r */
-__device__ __forceinline__ int nth_bit(uint64_t w, uint32_t r)
-{
-    uint32_t m = (uint32_t)w;
-    int b = 0;
-    const uint32_t lowest = (uint32_t)__popc(m);
-    if (r >= lowest) {
-        r -= lowest;
-        m = (uint32_t)(w >> 32);
-        b = 32;
-    }
-#pragma unroll
-    for (int h = 16; h >= 1; h >>= 1) {
-        const uint32_t c = (uint32_t)__popc(m & ((1u << h) - 1u));
-        const bool up = r >= c;
-        r -= up ? c : 0u;
-        m >>= up ? h : 0;
-        b += up ? h : 0;
-    }
-    return b;
 }
 
 /* triangles (generateTriangleVerticesSMEM MarchingCubes.cu:736-851 order), one thread per
@@ -3835,14 +3877,14 @@ uint32_t qs_pass2_blocks(const QsMol &M, int path)
 /* one launch for a group of molecules sharing r (and so the path) */
 void qs_launch_pass2(QsBatch B, uint32_t nblocks, int r, int path, const uint64_t *outm, const uint64_t *shellm,
                      const uint32_t *spre, float *field, uint32_t *negm, uint32_t *zerom, const int *offs, const int *norm_start, const int *enum_end,
-                     QsNormFlags nf, const uint8_t *tflag, uint8_t tmark, uint32_t xchunk, hipStream_t s)
+                     QsNormFlags nf, QsBand band, const uint8_t *tflag, uint8_t tmark, uint32_t xchunk, hipStream_t s)
 {
     if (path == 0) {
         xchunk = std::max(xchunk, 1u);
 #define QS_P2R(RR)                                                                                                    \
     case RR:                                                                                                          \
         hipLaunchKernelGGL(k_pass2_r<RR>, dim3(nblocks), dim3(256), 0, s, B, outm, shellm, spre, field, negm, zerom, \
-                           offs, norm_start, enum_end, nf, tflag, tmark, xchunk);                                            \
+                           offs, norm_start, enum_end, nf, band, tflag, tmark, xchunk);                                            \
         return;
         switch (r) {
             QS_P2R(1)

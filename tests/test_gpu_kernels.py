@@ -55,3 +55,25 @@ def test_mesh_of_any_field(qs, orc, g, kind):
         Vo, To = orc.edge_weld(G, lim, fld)
         assert np.array_equal(T, To)
         assert np.array_equal(V.view(np.uint32), Vo.view(np.uint32))
+
+
+@pytest.mark.parametrize("reso,n", [(0.16, 60), (0.2, 300), (0.28, 300), (0.35, 400), (0.5, 800), (0.7, 800), (1.0, 1500), (1.4, 1500),
+                                    (1.6, 1500)])
+@pytest.mark.parametrize("offset", [0.0, 30000.0])
+def test_field_values_left_out_and_completed(qs, orc, reso, n, offset):
+    """A mesh whose field pass stored only the values it reads equals the oracle's, the field asked
+    for afterwards is whole, and the mesh after a normals call (which stores every value) is the same."""
+    pos, rad = qs.synth_ball(78, n)
+    pos = pos + np.float32(offset)
+    print("case field left out: reso=%.2f offset=%g" % (reso, offset), flush=True)
+    ref = orc.compute_ses(pos, rad, reso, 1)
+    first = qs.compute_ses(pos, rad, reso, 1)
+    assert _same(first, ref)
+    g = qs.last_grid()["g"]
+    whole = qs.fetch("field", np.float32, g ** 3)
+    assert np.array_equal(whole.view(np.uint32), orc.field(pos, rad, reso)[6].view(np.uint32))
+    a = qs.compute_ses(pos, rad, reso, 1)
+    normals = qs.vertex_normals(len(a[0]))
+    b = qs.compute_ses(pos, rad, reso, 1)
+    assert np.array_equal(qs.vertex_normals(len(b[0])).view(np.uint32), normals.view(np.uint32))
+    assert _same(a, ref) and _same(b, ref)
