@@ -652,7 +652,7 @@ int Engine::mesh_stage(size_t at_mc, uint32_t nb_mc, size_t at_wpre, StageTimer 
                       field_sparse ? as<uint64_t>(shellm) : nullptr, as<float>(vert), as<uint64_t>(vkey), as<uint32_t>(acb),
                       as<uint32_t>(tstart), pool_t, pool_t, as<uint64_t>(negm), as<uint32_t>(wcnt), as<uint32_t>(vbw),
                       as<uint32_t>(tbw), as<uint64_t>(ntb), as<int>(tri), 0u, as<uint32_t>(deg_blk), as<uint32_t>(totals) + 3, counts, stream,
-                      fork_vertices ? side : stream, ev_emit, ev_vert, scan_nw != 0);
+                      fork_vertices ? side : stream, ev_emit, ev_vert, scan_nw != 0, expect_v);
     QS_HIP(hipGetLastError());
     vert_pending = fork_vertices;
     tm.mark("mc_emit");
@@ -665,7 +665,7 @@ int Engine::mesh_stage(size_t at_mc, uint32_t nb_mc, size_t at_wpre, StageTimer 
         }
         ids_sorted = g_opt.atom_ids_sorted != 0;
         qs_launch_closest_atom(as<QsMol>(d_mols), d_vpre, d_vpre + nmol + 1, as<uint32_t>(start), as<float4>(sx), as<int>(perm),
-                               as<float>(vert), pool_v, ids_sorted ? 1 : 0, as<int>(atom), counts + 1, cs);
+                               as<float>(vert), pool_v, ids_sorted ? 1 : 0, as<int>(atom), counts + 1, expect_v, cs);
         QS_HIP(hipGetLastError());
         if (overlap) {
             QS_HIP(hipEventRecord(ev_side, side));
@@ -677,17 +677,27 @@ int Engine::mesh_stage(size_t at_mc, uint32_t nb_mc, size_t at_wpre, StageTimer 
 }
 
 /* Vertex and triangle pools of a run: about 8 A^2 of surface per atom (measured 2-6 A^2 on the
-   benchmark molecules, cavities included), at least what earlier runs needed (cap_v, cap_t) */
+   benchmark molecules, cavities included), at least what earlier runs needed (cap_v, cap_t).
+   expect_v: the vertices (and about the cubes) that launches over the pools have blocks for, 15 %
+   above the area of a packed ball of the molecule's atoms; blocks past the pool's contents leave at
+   once, but 240,000 of them took 60 us on 256 molecules at 0.5 A (4.91 -> 4.77 ms of stages with the
+   compaction's), and blocks loop where a mesh has more. */
 void Engine::plan_pools()
 {
     uint64_t ev = 4096;
+    double expect = 256.0;
     for (const QsMol &M : mols)
-        if (M.G.g) ev += 256 + (uint64_t)(8.0 * M.n_atoms / ((double)M.G.dx * M.G.dx));
+        if (M.G.g) {
+            const double per = (double)M.n_atoms / ((double)M.G.dx * M.G.dx);
+            ev += 256 + (uint64_t)(8.0 * per);
+            expect += 256.0 + per * (2.76 + 55.0 / std::cbrt((double)M.n_atoms));
+        }
     ev = std::min<uint64_t>(ev, 4 * vox_total + 4096);
     ev = std::max<uint64_t>(ev, cap_v);
     uint64_t et = std::max<uint64_t>(2 * ev + 4096, cap_t);
     pool_v = (uint32_t)std::min<uint64_t>(ev, (1ull << 31) - 1);
     pool_t = (uint32_t)std::min<uint64_t>(et, (1ull << 31) / 3 - 1);
+    expect_v = mols.empty() || !n_atoms_total ? pool_v : (uint32_t)std::min(expect, (double)pool_v);
 }
 
 /* after a run's results are read: did its pools hold the mesh?  If not, they grow to fit */
@@ -884,7 +894,7 @@ int Engine::run_slabs(int planes, int smooth, StageTimer &tm)
     }
     ids_sorted = g_opt.atom_ids_sorted != 0;
     qs_launch_closest_atom(as<QsMol>(d_mols), d_vpre, d_vpre + 2, as<uint32_t>(start), as<float4>(sx), as<int>(perm),
-                           as<float>(vert), nv, ids_sorted ? 1 : 0, as<int>(atom), nullptr, cs);
+                           as<float>(vert), nv, ids_sorted ? 1 : 0, as<int>(atom), nullptr, nv, cs);
     QS_HIP(hipGetLastError());
     if (overlap) {
         QS_HIP(hipEventRecord(ev_side, side));
@@ -1040,7 +1050,7 @@ int Engine::run_batch(const float *d_pos, const float *d_rad, const std::vector<
         for (int it = 0; it < smooth; it++) {
             qs_launch_smooth(as<QsMol>(d_mols), d_vpre, d_vpre + nmol + 1, as<uint64_t>(negm), as<uint64_t>(zerom), as<uint64_t>(s4),
                              as<uint32_t>(vbw), as<uint64_t>(vkey), pool_v, as<uint64_t>(ntb), as<uint32_t>(tbw), as<int>(tri),
-                             src, dst, as<uint32_t>(totals) + 1, stream);
+                             src, dst, as<uint32_t>(totals) + 1, expect_v, stream);
             src = dst;
             dst = (dst == as<float>(vert2)) ? as<float>(vert3) : as<float>(vert2);
         }

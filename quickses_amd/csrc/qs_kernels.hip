@@ -3732,6 +3732,10 @@ static inline unsigned pgrid(uint64_t nb)
     return nb <= g_persist_blocks ? (unsigned)std::max<uint64_t>(nb, 1) : g_persist_blocks;
 }
 
+/* blocks of the triangle compaction at most: it streams, or leaves at once where nothing is dropped,
+   which 335,000 blocks over the pool of 256 molecules at 0.5 A took 70 us for */
+constexpr unsigned COMPACT_BLOCKS = 4096;
+
 /* partial boxes per molecule: about 8 atoms per thread of the largest molecule, 1 to BB_PMAX */
 int qs_bbox_parts(uint32_t max_atoms)
 {
@@ -3946,7 +3950,7 @@ void qs_launch_mc_emit(const QsMol *mols, const uint64_t *wpre, const uint32_t *
                        const uint32_t *acb, uint32_t *tstart, uint32_t ncube, uint32_t ntri, const uint64_t *N, const uint32_t *cnt,
                        const uint32_t *vbw, const uint32_t *tbw, const uint64_t *NT, int *tri, uint32_t vbase, uint32_t *deg_blk,
                        uint32_t *deg_total, const uint32_t *d_counts, hipStream_t s, hipStream_t s_vert, hipEvent_t ev_fork,
-                       hipEvent_t ev_vert, bool starts_ready)
+                       hipEvent_t ev_vert, bool starts_ready, uint32_t expect)
 {
     if (!s_vert) s_vert = s;
     if (!nact || (!nv && !ntri)) {
@@ -3972,21 +3976,21 @@ void qs_launch_mc_emit(const QsMol *mols, const uint64_t *wpre, const uint32_t *
         (void)hipStreamWaitEvent(s_vert, ev_fork, 0);
     }
     if (nv)
-        hipLaunchKernelGGL(k_mc_vertices, dim3(pgrid(nblk(nv, 256))), dim3(256), 0, s_vert, mols, wpre, wcoarse, list, avb, vstart, nact,
+        hipLaunchKernelGGL(k_mc_vertices, dim3(pgrid(nblk(std::min(nv, expect), 256))), dim3(256), 0, s_vert, mols, wpre, wcoarse, list, avb, vstart, nact,
                            nv, S4, F, spre, outm, shellm, vert, vkey, d_counts);
     if (s_vert != s) (void)hipEventRecord(ev_vert, s_vert);
     if (ntri)
-        hipLaunchKernelGGL(k_mc_triangles, dim3(pgrid(nblk(ncube, 256))), dim3(256), 0, s, mols, wpre, wcoarse, list, acb, tstart,
+        hipLaunchKernelGGL(k_mc_triangles, dim3(pgrid(nblk(std::min(ncube, expect), 256))), dim3(256), 0, s, mols, wpre, wcoarse, list, acb, tstart,
                            nact, ncube, ntri, N, S4, cnt, vbw, tbw, NT, tri, vbase, deg_blk, deg_total, d_counts);
 }
 
 void qs_launch_smooth(const QsMol *mols, const uint32_t *vpre, const uint32_t *vcoarse, const uint64_t *N, const uint64_t *Zm,
                       const uint64_t *S4, const uint32_t *vbw, const uint64_t *vkey, uint32_t nv,
                       const uint64_t *NT, const uint32_t *tbw, const int *tri, const float *src, float *dst,
-                      const uint32_t *d_nv, hipStream_t s)
+                      const uint32_t *d_nv, uint32_t expect, hipStream_t s)
 {
     if (!nv) return;
-    hipLaunchKernelGGL(k_smooth, dim3(pgrid(nblk(nv, 256))), dim3(256), 0, s, mols, vpre, vcoarse, N, Zm, S4, vbw, vkey, nv,
+    hipLaunchKernelGGL(k_smooth, dim3(pgrid(nblk(std::min(nv, expect), 256))), dim3(256), 0, s, mols, vpre, vcoarse, N, Zm, S4, vbw, vkey, nv,
                        NT, tbw, tri, src, dst, d_nv);
 }
 
@@ -4010,10 +4014,10 @@ void qs_launch_vertex_colors(const QsMol *mols, const uint32_t *vpre, const uint
 void qs_launch_closest_atom(const QsMol *mols, const uint32_t *vpre, const uint32_t *vcoarse, const uint32_t *cstart,
                             const float4 *sx,
                             const int *perm, const float *vert, uint32_t nv, int sorted_ids, int *out, const uint32_t *d_nv,
-                            hipStream_t s)
+                            uint32_t expect, hipStream_t s)
 {
     if (!nv) return;
-    hipLaunchKernelGGL(k_closest_atom, dim3(pgrid(nblk(nv, 256))), dim3(256), 0, s, mols, vpre, vcoarse, cstart, sx, perm, vert,
+    hipLaunchKernelGGL(k_closest_atom, dim3(pgrid(nblk(std::min(nv, expect), 256))), dim3(256), 0, s, mols, vpre, vcoarse, cstart, sx, perm, vert,
                        nv, sorted_ids, out, d_nv);
 }
 
@@ -4036,7 +4040,7 @@ void qs_launch_tri_compact(const int *tri, uint32_t nt, const uint32_t *dpre, co
                            const uint32_t *d_nt, hipStream_t s)
 {
     if (!nt) return;
-    hipLaunchKernelGGL(k_tri_compact, dim3(pgrid(nblk(nt, 256))), dim3(256), 0, s, tri, nt, dpre, ndeg, out, d_nt);
+    hipLaunchKernelGGL(k_tri_compact, dim3(std::min(nblk(nt, 256), COMPACT_BLOCKS)), dim3(256), 0, s, tri, nt, dpre, ndeg, out, d_nt);
 }
 
 void qs_launch_tri_kept_before(const int *tri, const uint32_t *dpre, const uint64_t *idx, int n, uint32_t tcap, uint32_t *out,

@@ -77,3 +77,15 @@ def test_field_values_left_out_and_completed(qs, orc, reso, n, offset):
     b = qs.compute_ses(pos, rad, reso, 1)
     assert np.array_equal(qs.vertex_normals(len(b[0])).view(np.uint32), normals.view(np.uint32))
     assert _same(a, ref) and _same(b, ref)
+
+
+@pytest.mark.parametrize("n", [3, 6])
+def test_mesh_beyond_the_expected_size(qs, orc, n):
+    """Separate spheres have several times the surface that a launch expects of so many atoms: the
+    pools are grown and the launches' blocks take more than one block of items."""
+    ax = np.arange(n, dtype=np.float32) * np.float32(7.0)
+    pos = np.stack(np.meshgrid(ax, ax, ax, indexing="ij"), -1).reshape(-1, 3)
+    rad = np.full(len(pos), 1.7, np.float32)
+    print("case separate spheres n=%d" % len(rad), flush=True)
+    for _ in range(2):  # with the pools of the start, then with grown ones
+        assert _same(qs.compute_ses(pos, rad, 0.5, 1), orc.compute_ses(pos, rad, 0.5, 1))
