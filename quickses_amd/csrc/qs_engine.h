@@ -225,7 +225,6 @@ struct Engine {
     DevBuf inc_cnt, inc_start, inc_ent; /* per-vertex triangle incidences (smoothing of slab meshes) */
     DevBuf tpre_d;                      /* per-molecule first triangle (u64, nmol + 1), on the device */
     DevBuf tflag;                       /* field-pass-2 tiles holding a shell voxel (u8 per tile) */
-    DevBuf spre, stot;                  /* shell rank of each row word (u32), shell total (2 x u32) */
     DevBuf field_dense;                 /* the whole field in grid order, expanded on request */
     std::vector<P2Group> groups;
     std::vector<P2Tables *> tables;
@@ -307,8 +306,8 @@ struct Engine {
     uint32_t nv = 0, nt_all = 0, nt = 0, n_active = 0;
     size_t p1_lds = 0; /* dynamic LDS of the field pass 1 launch (largest molecule of the batch) */
     bool batch_valid = false; /* result arrays, vert_off / tri_off and their device copies belong to run_batch */
-    /* field holds the shell voxels' values only (field pass 2), densely in shell-rank order (spre);
-       the others come from outm / shellm.  Else field holds every voxel in grid order. */
+    /* field holds shell voxels' values only (field pass 2), the others come from outm / shellm; else
+       it holds every voxel.  In grid order either way. */
     bool field_sparse = false;
     /* the stored shell values are those the mesh reads only (QsBand); complete_field evaluates the
        rest.  normals_used: the last result's normals were asked for, so the next run stores every
@@ -341,7 +340,7 @@ struct Engine {
                           &perm, &cse, &sx, &aux, &labels, &outm, &shellm, &field, &negm, &zerom, &s4, &wcnt,
                           &vbw, &tbw, &alist, &ntb, &avb, &acb, &vstart, &tstart, &normals, &colors_in, &totals, &bounds, &rback, &vert, &vert2, &vert3, &vkey,
                           &tri, &tri_out, &atom, &deg_blk, &keeppos, &tri_loc, &scan_tmp, &inc_cnt, &inc_start, &inc_ent,
-                          &tpre_d, &tflag, &spre, &stot, &field_dense})
+                          &tpre_d, &tflag, &field_dense})
             *b = DevBuf{};
         for (P2Tables *t : tables) delete t;
         tables.clear();
@@ -356,7 +355,7 @@ struct Engine {
                           &perm, &cse, &sx, &aux, &labels, &outm, &shellm, &field, &negm, &zerom, &s4, &wcnt,
                           &vbw, &tbw, &alist, &ntb, &avb, &acb, &vstart, &tstart, &normals, &colors_in, &totals, &bounds, &rback, &vert, &vert2, &vert3, &vkey,
                           &tri, &tri_out, &atom, &deg_blk, &keeppos, &tri_loc, &scan_tmp, &inc_cnt, &inc_start, &inc_ent,
-                          &tpre_d, &tflag, &spre, &stot, &field_dense})
+                          &tpre_d, &tflag, &field_dense})
             release(*b);
         for (P2Tables *t : tables) {
             release(t->dev);

@@ -252,8 +252,6 @@ int Engine::reserve(uint64_t vox, uint64_t atoms, uint64_t cells, uint64_t verts
     QS_TRY(ensure(s4, nw * 32));
     QS_TRY(ensure(ntb, nw * 24));
     QS_TRY(ensure(field, vox * 4));
-    QS_TRY(ensure(spre, nw * 4));
-    QS_TRY(ensure(stot, 8));
     QS_TRY(ensure(in_pos, atoms * 12));
     for (DevBuf *b : {&in_rad, &perm}) QS_TRY(ensure(*b, atoms * 4));
     QS_TRY(ensure(key, atoms * 8));
@@ -498,9 +496,6 @@ int Engine::field_stage(uint32_t nb_p1, size_t at_p1, StageTimer &tm)
     QS_TRY(ensure(field, std::max<uint64_t>(vox_total, 1) * 4));
     QS_TRY(ensure(negm, std::max<uint64_t>(nw_total, 1) * 8));
     QS_TRY(ensure(zerom, std::max<uint64_t>(nw_total, 1) * 8));
-    QS_TRY(ensure(spre, std::max<uint64_t>(nw_total, 1) * 4));
-    QS_TRY(ensure(stot, 8));
-    QS_TRY(ensure(scan_tmp, qs_scan_tiles(std::max<uint64_t>(nw_total, 1)) * sizeof(uint32_t)));
     /* the slab kernel of field pass 1 writes every voxel's default sign words and marks the
        pass-2 tiles that hold a shell voxel; pass 2 then runs on the marked tiles only */
     const int p1mode = qs_pass1_mode(g_opt.pass1_direct != 0, g_opt.pass1_rows != 0);
@@ -523,10 +518,6 @@ int Engine::field_stage(uint32_t nb_p1, size_t at_p1, StageTimer &tm)
         QS_HIP(hipGetLastError());
     }
     tm.mark("pass1");
-    /* every row word's shell rank: pass 2 stores the shell voxels' values densely in that order
-       (the shell voxels are at most the voxels, which the field is sized for) */
-    qs_launch_shell_scan(as<uint64_t>(shellm), nw_total, as<uint32_t>(scan_tmp), as<uint32_t>(stot), as<uint32_t>(spre), stream);
-    tm.mark("shell_scan");
     run_flags = tf;
     QS_TRY(run_pass2(normals_used));
     normals_used = false;
@@ -545,7 +536,7 @@ int Engine::run_pass2(bool all)
         if (all) band = QsBand{0, 255, 0, 1};
         if (grp.path == 0 && !band.all) field_band = true;
         qs_launch_pass2(batch(grp.bpre_at, grp.mid_at, (int)grp.mols.size()), grp.nblocks, grp.r, grp.path, as<uint64_t>(outm),
-                        as<uint64_t>(shellm), as<uint32_t>(spre), as<float>(field), as<uint32_t>(negm), as<uint32_t>(zerom),
+                        as<uint64_t>(shellm), as<float>(field), as<uint32_t>(negm), as<uint32_t>(zerom),
                         grp.tab->offs(), grp.tab->norm(), grp.tab->end(), grp.tab->flags, band,
                         (run_flags && grp.path == 0) ? run_flags + mols[grp.mols[0]].tile_off : nullptr, tmark, grp.xchunk, stream);
         QS_HIP(hipGetLastError());
@@ -553,14 +544,14 @@ int Engine::run_pass2(bool all)
     return 0;
 }
 
-/* the shell values that the last run left out (its masks, ranks and tile marks are still there; the
+/* the shell values that the last run left out (its masks and tile marks are still there; the
    sign words are written again with the same bits) */
 int Engine::complete_field()
 {
     return field_sparse && field_band ? run_pass2(true) : 0;
 }
 
-/* every voxel of every molecule's field in grid order (pass 2 stores the shell voxels only):
+/* every voxel of every molecule's field (pass 2 stores the shell voxels only):
    *dense receives the device array, molecule m at its voxel offset */
 int Engine::fill_field(const void **dense)
 {
@@ -569,9 +560,8 @@ int Engine::fill_field(const void **dense)
     QS_TRY(complete_field());
     QS_TRY(ensure(field_dense, std::max<uint64_t>(vox_total, 1) * 4));
     for (const QsMol &M : mols)
-        qs_launch_field_expand(as<float>(field), as<uint32_t>(spre) + M.word_off, as<uint64_t>(outm) + M.word_off,
-                               as<uint64_t>(shellm) + M.word_off, as<float>(field_dense) + M.vox_off, M.G.g, (int)M.W,
-                               M.G.dx, stream);
+        qs_launch_field_expand(as<float>(field) + M.vox_off, as<uint64_t>(outm) + M.word_off, as<uint64_t>(shellm) + M.word_off,
+                               as<float>(field_dense) + M.vox_off, M.G.g, (int)M.W, M.G.dx, stream);
     QS_HIP(hipGetLastError());
     *dense = field_dense.p;
     return 0;
@@ -648,7 +638,7 @@ int Engine::mesh_stage(size_t at_mc, uint32_t nb_mc, size_t at_wpre, StageTimer 
     const bool overlap = with_atoms && !tm.on;
     const bool fork_vertices = overlap && nmol == 1;
     qs_launch_mc_emit(as<QsMol>(d_mols), wpre, wcoarse, as<uint32_t>(alist), nact_max, as<uint32_t>(avb), as<uint32_t>(vstart),
-                      pool_v, as<uint64_t>(s4), as<float>(field), field_sparse ? as<uint32_t>(spre) : nullptr, as<uint64_t>(outm),
+                      pool_v, as<uint64_t>(s4), as<float>(field), as<uint64_t>(outm),
                       field_sparse ? as<uint64_t>(shellm) : nullptr, as<float>(vert), as<uint64_t>(vkey), as<uint32_t>(acb),
                       as<uint32_t>(tstart), pool_t, pool_t, as<uint64_t>(negm), as<uint32_t>(wcnt), as<uint32_t>(vbw),
                       as<uint32_t>(tbw), as<uint64_t>(ntb), as<int>(tri), 0u, as<uint32_t>(deg_blk), as<uint32_t>(totals) + 3, counts, stream,
@@ -805,7 +795,7 @@ int Engine::slab_mesh(size_t at_mc, uint32_t nb_mc, size_t at_wpre, uint64_t own
     const uint64_t *wpre = (const uint64_t *)(as<uint32_t>(d_meta) + at_wpre);
     const uint32_t *wcoarse = as<uint32_t>(d_meta) + at_wpre + 4;
     qs_launch_mc_emit(as<QsMol>(d_mols), wpre, wcoarse, as<uint32_t>(alist), nact, as<uint32_t>(avb), as<uint32_t>(vstart),
-                      n_owned, as<uint64_t>(s4), as<float>(field), as<uint32_t>(spre), as<uint64_t>(outm), as<uint64_t>(shellm),
+                      n_owned, as<uint64_t>(s4), as<float>(field), as<uint64_t>(outm), as<uint64_t>(shellm),
                       as<float>(vert) + 3 * (size_t)vbase, as<uint64_t>(vkey), as<uint32_t>(acb), as<uint32_t>(tstart), hb[4], n_tri,
                       as<uint64_t>(negm), as<uint32_t>(wcnt), as<uint32_t>(vbw), as<uint32_t>(tbw), as<uint64_t>(ntb),
                       as<int>(tri) + 3 * (size_t)tbase, vbase, as<uint32_t>(deg_blk), as<uint32_t>(totals) + 3, nullptr, stream);
@@ -1791,7 +1781,7 @@ static int launch_normals(Engine &E, float *d_out)
     const int nmol = (int)E.mols.size();
     const uint32_t *d_vpre = as<uint32_t>(E.d_off) + (nmol + 1);
     qs_launch_vertex_normals(as<QsMol>(E.d_mols), d_vpre, d_vpre + nmol + 1, as<uint64_t>(E.vkey), E.nv, as<float>(E.field),
-                             E.field_sparse ? as<uint32_t>(E.spre) : nullptr, as<uint64_t>(E.outm),
+                             as<uint64_t>(E.outm),
                              E.field_sparse ? as<uint64_t>(E.shellm) : nullptr, d_out, E.stream);
     QS_HIP(hipGetLastError());
     return 0;
@@ -2000,11 +1990,6 @@ int qs_stage_pass2(const float *fp, const int *ip, const uint8_t *labels, float 
     QS_TRY(ensure(E.field, V * 4));
     QS_TRY(ensure(E.negm, E.nw_total * 8));
     QS_TRY(ensure(E.zerom, E.nw_total * 8));
-    QS_TRY(ensure(E.spre, E.nw_total * 4));
-    QS_TRY(ensure(E.stot, 8));
-    QS_TRY(ensure(E.scan_tmp, qs_scan_tiles(E.nw_total) * sizeof(uint32_t)));
-    qs_launch_shell_scan(as<uint64_t>(E.shellm), E.nw_total, as<uint32_t>(E.scan_tmp), as<uint32_t>(E.stot), as<uint32_t>(E.spre),
-                         E.stream);
     E.run_flags = nullptr;
     QS_TRY(E.run_pass2(true));
     E.field_sparse = true;

@@ -51,28 +51,23 @@ size_t qs_pass2_lds_bytes(int r);
 int qs_pass2_path(int r, bool direct);
 /* blocks of one molecule's launch over its planes [p2_lo, p2_hi) */
 uint32_t qs_pass2_blocks(const QsMol &M, int path);
-/* the shell voxels' values go to field at their shell ranks (spre, from qs_launch_shell_scan), on
-   path 0 those of band only (the others' places keep what they held);
+/* the shell voxels' values go to field in grid order, on path 0 those of band only (the others'
+   places, and those of voxels outside the shell, keep what they held);
    tflag (path 0 only, may be NULL): the marks of the launch's tiles in its block order (from the
    group's first molecule's tile_off on); tiles field pass 1 did not mark with tmark are skipped; xchunk
    (path 0): consecutive tiles each XCD takes in turn */
 void qs_launch_pass2(QsBatch B, uint32_t nblocks, int r, int path, const uint64_t *outm, const uint64_t *shellm,
-                     const uint32_t *spre, float *field, uint32_t *negm, uint32_t *zerom, const int *offs, const int *norm_start, const int *enum_end,
+                     float *field, uint32_t *negm, uint32_t *zerom, const int *offs, const int *norm_start, const int *enum_end,
                      QsNormFlags nf, QsBand band, const uint8_t *tflag, uint8_t tmark, uint32_t xchunk, hipStream_t s);
 /* pass-2 tiles of the fixed-R kernel of one molecule (its tile-flag count) */
 uint32_t qs_pass2_tiles(const QsMol &M);
 /* z tiles per (x, y) tile row of the fixed-R pass-2 kernel */
 uint32_t qs_pass2_ztiles(const QsMol &M);
 
-/* shell ranks (spre, one per word) of the words [0, nw) of shellm: the place of each word's first
-   shell voxel in the stored field (sums: qs_scan_tiles(nw) scratch entries; totals: 2 entries,
-   the total shell voxels first) */
-void qs_launch_shell_scan(const uint64_t *shellm, uint64_t nw, uint32_t *sums, uint32_t *totals, uint32_t *spre, hipStream_t s);
-/* field pass 2 stores the shell voxels' values only, in shell-rank order: one molecule's whole
-   field in grid order (out), from them and its outside / shell masks (spre, outm, shellm at the
-   molecule's first word; F the stored values of the whole launch) */
-void qs_launch_field_expand(const float *F, const uint32_t *spre, const uint64_t *outm, const uint64_t *shellm, float *out, int g,
-                            int W, float dx, hipStream_t s);
+/* one molecule's whole field in grid order (out), from the stored shell values and its outside and
+   shell masks */
+void qs_launch_field_expand(const float *F, const uint64_t *outm, const uint64_t *shellm, float *out, int g, int W, float dx,
+                            hipStream_t s);
 
 /* stage-wise helpers (one molecule) */
 void qs_launch_field_signs(const float *F, int g, int W, uint32_t *negm, uint32_t *zerom, hipStream_t s);
@@ -90,16 +85,15 @@ void qs_launch_mc_count(QsBatch B, uint32_t nblocks, const uint64_t *N, const ui
    vertex ids avb and first cubes acb), after one launch that gives vstart / tstart each 256-item
    block's first active word (nv / 256 + 1 and ncube / 256 + 1 entries) and clears deg_blk (ntri /
    256 + 1 entries), unless starts_ready says that the word scans did (QsBlockStarts).  ncube: the
-   cubes, or a bound on them.  The field F holds the shell voxels' values only, at their shell ranks
-   (spre), the others come from the outside / shell masks (shellm == nullptr: F holds every voxel in
-   grid order, spre is unused).  cnt: the words' packed counts; tbw: their first triangles.  Triangle
-   corners are vertex ids plus vbase; degenerate triangles are counted per 256-triangle block
+   cubes, or a bound on them.  The field F (grid order) holds shell voxels' values only, the others
+   come from the outside / shell masks (shellm == nullptr: F holds every voxel).  cnt: the words'
+   packed counts; tbw: their first triangles.  Triangle corners are vertex ids plus vbase; degenerate triangles are counted per 256-triangle block
    (deg_blk) and in total.  The block starts and the triangle kernel run on s;
    the vertex kernel on s_vert: when that is another stream it waits there for the block starts
    (event ev_fork), and ev_vert is recorded on s_vert after it. */
 void qs_launch_mc_emit(const QsMol *mols, const uint64_t *wpre, const uint32_t *wcoarse, const uint32_t *list, uint32_t nact,
                        const uint32_t *avb, uint32_t *vstart, uint32_t nv, const uint64_t *S4, const float *F,
-                       const uint32_t *spre, const uint64_t *outm, const uint64_t *shellm, float *vert, uint64_t *vkey,
+                       const uint64_t *outm, const uint64_t *shellm, float *vert, uint64_t *vkey,
                        const uint32_t *acb, uint32_t *tstart, uint32_t ncube, uint32_t ntri, const uint64_t *N, const uint32_t *cnt,
                        const uint32_t *vbw, const uint32_t *tbw, const uint64_t *NT, int *tri, uint32_t vbase, uint32_t *deg_blk,
                        uint32_t *deg_total, const uint32_t *d_counts, hipStream_t s, hipStream_t s_vert = nullptr,
@@ -142,7 +136,7 @@ void qs_launch_deg_count(const int *tri, uint32_t nt, uint32_t *deg_blk, uint32_
 /* unit field gradient at each vertex's marching-cubes position, 3 floats per vertex (field as for
    the vertex kernel) */
 void qs_launch_vertex_normals(const QsMol *mols, const uint32_t *vpre, const uint32_t *vcoarse, const uint64_t *vkey, uint32_t nv,
-                              const float *F, const uint32_t *spre, const uint64_t *outm, const uint64_t *shellm, float *out,
+                              const float *F, const uint64_t *outm, const uint64_t *shellm, float *out,
                               hipStream_t s);
 /* colour of each vertex's closest atom from a per-atom RGBA table (batch atom layout); perm maps
    cell-sorted atom ids to input indices (nullptr: the ids are input indices) */
@@ -167,8 +161,8 @@ uint32_t qs_persistent_blocks(void);
 /* device-wide exclusive scan pieces */
 uint64_t qs_scan_tiles(uint64_t n);
 /* inputs of at most this many entries are scanned by one block in one launch (the generic scan,
-   the shell ranks and the marching-cubes word scans; one block's memory throughput makes more
-   entries slower than several blocks); inputs of at most QS_SCAN_SELF_TILES tiles of 2,048 are
+   and the marching-cubes word scans; one block's memory throughput makes more entries slower than
+   several blocks); inputs of at most QS_SCAN_SELF_TILES tiles of 2,048 are
    scanned in two launches, each tile adding up the sums of the tiles before it itself */
 #define QS_SCAN1_MAX 8192u
 #define QS_SCAN_SELF_TILES 64u

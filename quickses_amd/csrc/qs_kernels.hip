@@ -308,71 +308,6 @@ __global__ void __launch_bounds__(SCAN_NT) k_tile_scan(const uint32_t *in, uint3
     if (total && blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) *total = off + tot;
 }
 
-/* Shell ranks: spre[i] = shell voxels (set bits of shellm) in words [0, i).  Field pass 2 stores
-   the shell voxels' values only, densely in that order: voxel bit b of word i at
-   spre[i] + popcount(shellm[i] below b). */
-__global__ void __launch_bounds__(SCAN_NT) k_shell_reduce(const uint64_t *__restrict__ shellm, uint64_t n,
-                                                          uint32_t *__restrict__ sums)
-{
-    __shared__ uint32_t lds[SCAN_NT / 64 + 1];
-    const uint64_t base = (uint64_t)blockIdx.x * SCAN_TILE;
-    uint32_t s = 0;
-#pragma unroll
-    for (int k = 0; k < SCAN_IPT; k++) {
-        const uint64_t i = base + (uint64_t)k * SCAN_NT + threadIdx.x;
-        if (i < n) s += (uint32_t)__popcll(shellm[i]);
-    }
-    const uint32_t t = block_sum<SCAN_NT>(s, lds);
-    if (threadIdx.x == 0) sums[blockIdx.x] = t;
-}
-
-/* (self: offsets holds the raw tile sums of at most QS_SCAN_SELF_TILES tiles, each tile adds up
-   the ones before it, and the last tile writes totals = {shell voxels, 0}) */
-__global__ void __launch_bounds__(SCAN_NT) k_shell_scan(const uint64_t *__restrict__ shellm, uint64_t n,
-                                                        const uint32_t *__restrict__ offsets, uint32_t *__restrict__ spre,
-                                                        int self, uint32_t *__restrict__ totals)
-{
-    /* wave w of the block takes words [w * 512, (w + 1) * 512) of the tile, 64 consecutive words
-       per load, and scans them in order: lane prefixes per group of 64, carried across groups */
-    __shared__ uint32_t wsum[SCAN_NT / 64];
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    const uint64_t base = (uint64_t)blockIdx.x * SCAN_TILE + (uint64_t)wid * (64 * SCAN_IPT) + lane;
-    uint32_t v[SCAN_IPT];
-#pragma unroll
-    for (int k = 0; k < SCAN_IPT; k++) {
-        const uint64_t i = base + 64 * k;
-        v[k] = (i < n) ? (uint32_t)__popcll(shellm[i]) : 0u;
-    }
-    uint32_t run = 0; /* words of the wave's earlier groups */
-#pragma unroll
-    for (int k = 0; k < SCAN_IPT; k++) {
-        uint32_t x = v[k];
-#pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-            const uint32_t y = __shfl_up(x, d, 64);
-            if (lane >= d) x += y;
-        }
-        const uint32_t tot = __shfl(x, 63, 64);
-        v[k] = run + x - v[k]; /* exclusive prefix inside the wave's range */
-        run += tot;
-    }
-    if (lane == 0) wsum[wid] = run;
-    __syncthreads();
-    uint32_t off = self ? wave_sum_below(offsets, blockIdx.x) : offsets[blockIdx.x];
-    if (self && blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) {
-        uint32_t t = off;
-        for (int w = 0; w < SCAN_NT / 64; w++) t += wsum[w];
-        totals[0] = t;
-        totals[1] = 0u;
-    }
-    for (int w = 0; w < wid; w++) off += wsum[w];
-#pragma unroll
-    for (int k = 0; k < SCAN_IPT; k++) {
-        const uint64_t i = base + 64 * k;
-        if (i < n) spre[i] = off + v[k];
-    }
-}
-
 /* a row word's counts, packed by k_mc_count: vertices (at most 4 x 64), triangles (at most 5 x 64)
    and polygonised cubes (at most 64) */
 __device__ __forceinline__ uint32_t word_counts(uint32_t nv, uint32_t nt, uint32_t nc) { return nv | nt << 9 | nc << 18; }
@@ -413,8 +348,7 @@ __global__ void __launch_bounds__(SCAN_NT) k_mc_reduce4(const uint32_t *__restri
 }
 
 /* block p: exclusive scan of plane p of the tile sums in place, total to totals[p], plane 3's to
-   totals[4]: totals[3] (the degenerate-triangle count, accumulated later), or the slot after a
-   single plane's total, starts at zero */
+   totals[4]: totals[3] (the degenerate-triangle count, accumulated later) starts at zero */
 __global__ void __launch_bounds__(SCAN_NT) k_scan_planes(uint32_t *__restrict__ sums, uint64_t ntiles,
                                                          uint32_t *__restrict__ totals)
 {
@@ -439,7 +373,7 @@ __global__ void __launch_bounds__(SCAN_NT) k_scan_planes(uint32_t *__restrict__ 
         carry += tot;
     }
     if (threadIdx.x == 0) totals[blockIdx.x + (blockIdx.x >= 3u ? 1u : 0u)] = carry;
-    if (blockIdx.x == 0 && threadIdx.x == 0) totals[min(gridDim.x, 3u)] = 0u;
+    if (blockIdx.x == 0 && threadIdx.x == 0) totals[3] = 0u;
 }
 
 /* An active word with items [first, first + count) is where every 256-item block whose first
@@ -465,8 +399,7 @@ __global__ void __launch_bounds__(SCAN_NT) k_mc_scan4(const uint32_t *__restrict
     /* (self: sums holds the raw tile sums of at most QS_SCAN_SELF_TILES tiles, each tile adds up
        the ones before it, and the last tile writes totals = {triangles, vertices, active, 0, cubes}) */
     /* wave w of the block takes words [w * 512, (w + 1) * 512) of the tile, 64 consecutive words
-       per load (as k_shell_scan); the three scans run per group of 64 in order, carried across
-       groups, and each group's active words are listed in order by ballot */
+       per load; the scans run per group of 64 in order, carried across groups, and each group's active words are listed in order by ballot */
     __shared__ uint32_t wsum[4][SCAN_NT / 64];
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
     const uint64_t base = (uint64_t)blockIdx.x * SCAN_TILE + (uint64_t)wid * (64 * SCAN_IPT) + lane;
@@ -623,35 +556,6 @@ __global__ void __launch_bounds__(SCAN1_NT) k_scan1(const uint32_t *in, uint32_t
         __syncthreads(); /* wsum is written again for the next chunk */
     }
     if (total && threadIdx.x == 0) *total = carry;
-}
-
-/* shell ranks (as k_shell_reduce, k_scan_planes, k_shell_scan): totals = {shell voxels, 0} */
-__global__ void __launch_bounds__(SCAN1_NT) k_shell_scan1(const uint64_t *__restrict__ shellm, uint64_t n,
-                                                          uint32_t *__restrict__ totals, uint32_t *__restrict__ spre)
-{
-    __shared__ uint32_t wsum[SCAN1_W];
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    uint32_t carry = 0;
-    for (uint64_t c0 = 0; c0 < n; c0 += SCAN1_NT * SCAN_IPT) {
-        const uint64_t base = c0 + (uint64_t)wid * (64 * SCAN_IPT) + lane;
-        uint32_t v[SCAN_IPT];
-#pragma unroll
-        for (int k = 0; k < SCAN_IPT; k++) v[k] = (base + 64 * k < n) ? (uint32_t)__popcll(shellm[base + 64 * k]) : 0u;
-        const uint32_t run = wave_groups_scan(v, lane);
-        if (lane == 0) wsum[wid] = run;
-        __syncthreads();
-        uint32_t below, all;
-        scan1_offsets(wsum, wid, below, all);
-#pragma unroll
-        for (int k = 0; k < SCAN_IPT; k++)
-            if (base + 64 * k < n) spre[base + 64 * k] = carry + below + v[k];
-        carry += all;
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) {
-        totals[0] = carry;
-        totals[1] = 0u;
-    }
 }
 
 /* marching-cubes word scans (as k_mc_reduce4, k_scan_planes, k_mc_scan4): totals = {triangles,
@@ -1710,15 +1614,14 @@ __device__ __forceinline__ void emit_sign_bits(uint32_t *__restrict__ negm, uint
 
 template <typename DT>
 __global__ void __launch_bounds__(256) k_pass2_tile(QsBatch B, const uint64_t *__restrict__ outm_all,
-                                                    const uint64_t *__restrict__ shellm_all, const uint32_t *__restrict__ spre_all,
-                                                    float *__restrict__ field,
+                                                    const uint64_t *__restrict__ shellm_all,
+                                                    float *__restrict__ field_all,
                                                     uint32_t *__restrict__ negm_all, uint32_t *__restrict__ zerom_all,
                                                     const int *__restrict__ offs, const int *__restrict__ norm_start,
                                                     const int *__restrict__ enum_end)
 {
     extern __shared__ __align__(16) uint8_t smem[];
     __shared__ int s_flags;
-    __shared__ uint32_t sbase[P2_TX * P2_TY]; /* shell rank of each own row's first tile voxel */
     constexpr int INF = (sizeof(DT) == 1) ? 0xFF : 0xFFFF;
     uint32_t lb;
     const QsMol &M = B.mols[batch_mol(B, blockIdx.x, lb)];
@@ -1726,7 +1629,7 @@ __global__ void __launch_bounds__(256) k_pass2_tile(QsBatch B, const uint64_t *_
     const int r = G.r, g = G.g, W = (int)M.W;
     const uint64_t *__restrict__ outm = outm_all + M.word_off;
     const uint64_t *__restrict__ shellm = shellm_all + M.word_off;
-    const uint32_t *__restrict__ spre = spre_all + M.word_off;
+    float *__restrict__ field = field_all + M.vox_off;
     uint32_t *__restrict__ negm = negm_all + 2 * M.word_off;
     uint32_t *__restrict__ zerom = zerom_all + 2 * M.word_off;
     const int x0 = M.p2_lo, x1 = M.p2_hi;
@@ -1759,11 +1662,7 @@ __global__ void __launch_bounds__(256) k_pass2_tile(QsBatch B, const uint64_t *_
         uint32_t m = 0u;
         if (gx < x1 && gx < g && gy < g) m = (uint32_t)row_bits(shellm + ((size_t)gx * g + gy) * W, W, tz0, P2_TZ);
         own[t] = m;
-        if (m) {
-            fl |= 1;
-            const size_t wi = ((size_t)gx * g + gy) * W + (tz0 >> 6);
-            sbase[t] = spre[wi] + (uint32_t)__popcll(shellm[wi] & bits_below(tz0 & 63, 0));
-        }
+        if (m) fl |= 1;
     }
     if (fl) atomicOr(&s_flags, fl);
     __syncthreads();
@@ -1781,7 +1680,7 @@ __global__ void __launch_bounds__(256) k_pass2_tile(QsBatch B, const uint64_t *_
             bool out = (rows[(size_t)(tx + r) * LY + (ty + r)] >> (tz + r)) & 1ull;
             float res = out ? QS_PROBE : -dx;
             const uint32_t om = own[tx * P2_TY + ty];
-            if (vyz && ((om >> tz) & 1u)) field[sbase[tx * P2_TY + ty] + (uint32_t)__popc(om & ((1u << tz) - 1u))] = res;
+            if (vyz && ((om >> tz) & 1u)) field[((size_t)gx * g + gy) * g + gz] = res;
             emit_sign_bits(negm, zerom, W, g, gx, gy, tz0, vyz, res);
         }
         return;
@@ -1880,7 +1779,7 @@ __global__ void __launch_bounds__(256) k_pass2_tile(QsBatch B, const uint64_t *_
             }
         }
         if (vyz && shell)
-            field[sbase[tx * P2_TY + ty] + (uint32_t)__popc(own[tx * P2_TY + ty] & ((1u << tz) - 1u))] = res;
+            field[((size_t)gx * g + gy) * g + gz] = res;
         emit_sign_bits(negm, zerom, W, g, gx, gy, tz0, vyz, res);
     }
 }
@@ -1912,7 +1811,7 @@ __device__ __forceinline__ uint32_t zdist2(uint64_t m, int z)
      bits, y minima (with the masks of the attaining y offsets) for the columns they read, x minima;
    - the exact float distance of the minimisers, traced back through the masks (or enumerated
      from a norm-sorted table where another norm could tie), rooted once;
-   - the field of those voxels, and every voxel's sign bits.
+   - the field of those voxels at their grid places, and every voxel's sign bits.
    Bound by VALU issue and, at R = 7, by LDS reads of the dilated rows.  Evaluating every shell
    voxel with an outside voxel in reach (28 to 38 % of the shell; 8 to 15 % are read) by x minima and
    trace took 0.592 ms on the 50,000-atom 0.2 A mesh (R 7), 0.610 on 200,000 atoms at 0.3 A (R 5) and
@@ -1944,8 +1843,7 @@ __device__ __forceinline__ void list_column(const uint32_t *cpre, const uint32_t
 
 template <int R>
 __global__ void __launch_bounds__(256) k_pass2_r(QsBatch B, const uint64_t *__restrict__ outm_all,
-                                                 const uint64_t *__restrict__ shellm_all, const uint32_t *__restrict__ spre_all,
-                                                 float *__restrict__ field, uint32_t *__restrict__ negm_all,
+                                                 const uint64_t *__restrict__ shellm_all, float *__restrict__ field_all, uint32_t *__restrict__ negm_all,
                                                  uint32_t *__restrict__ zerom_all, const int *__restrict__ offs,
                                                  const int *__restrict__ norm_start, const int *__restrict__ enum_end,
                                                  QsNormFlags nf, QsBand band, const uint8_t *__restrict__ tflag, uint8_t tmark,
@@ -1956,10 +1854,8 @@ __global__ void __launch_bounds__(256) k_pass2_r(QsBatch B, const uint64_t *__re
     static_assert(LZ <= 64 && 3 * R * R < INF, "window too wide for this kernel");
     constexpr int NR = LX * LY;
     __shared__ uint64_t rows[NR];
-    /* ownout: the own rows' outside bits, read only by a tile without a shell voxel; after that
-       test the array holds the own rows' shell ranks (sbase) instead */
+    /* ownout: the own rows' outside bits, read only by a tile without a shell voxel */
     __shared__ uint32_t own[P2R_TX * P2_TY], ownout[P2R_TX * P2_TY];
-    uint32_t *const sbase = ownout;
     /* y offsets (bit b + R) attaining each DY value */
     using BMask = typename std::conditional<(2 * R + 1 <= 8), uint8_t,
                                             typename std::conditional<(2 * R + 1 <= 16), uint16_t, uint32_t>::type>::type;
@@ -1993,7 +1889,7 @@ __global__ void __launch_bounds__(256) k_pass2_r(QsBatch B, const uint64_t *__re
     const int g = G.g, W = (int)M.W;
     const uint64_t *__restrict__ outm = outm_all + M.word_off;
     const uint64_t *__restrict__ shellm = shellm_all + M.word_off;
-    const uint32_t *__restrict__ spre = spre_all + M.word_off;
+    float *__restrict__ field = field_all + M.vox_off;
     uint32_t *__restrict__ negm = negm_all + 2 * M.word_off;
     uint32_t *__restrict__ zerom = zerom_all + 2 * M.word_off;
     const int x1 = M.p2_hi;
@@ -2052,19 +1948,14 @@ __global__ void __launch_bounds__(256) k_pass2_r(QsBatch B, const uint64_t *__re
         zlen[set][a][b] = (uint8_t)c;
     }
     int has_shell;
-    uint32_t sb = 0u;
     {
         const int t = threadIdx.x & 127, tx = t / P2_TY, ty_ = t - tx * P2_TY;
         const int gx = tx0 + tx, gy_ = ty0 + ty_;
         const uint64_t *__restrict__ src = threadIdx.x < 128 ? shellm : outm;
         uint32_t m = 0u;
         if (gx < x1 && gx < g && gy_ < g) {
-            /* the tile's 32 z of the row are one half of a row word (tz0 is a multiple of 32); the
-               shell threads also take the row's shell rank there, loaded alongside */
-            const size_t wi = ((size_t)gx * g + gy_) * W + (tz0 >> 6);
-            const uint64_t wv = src[wi];
-            m = (uint32_t)(wv >> (tz0 & 63));
-            if (threadIdx.x < 128) sb = spre[wi] + (uint32_t)__popcll(wv & bits_below(tz0 & 63, 0));
+            /* the tile's 32 z of the row are one half of a row word (tz0 is a multiple of 32) */
+            m = (uint32_t)(src[((size_t)gx * g + gy_) * W + (tz0 >> 6)] >> (tz0 & 63));
         }
         /* with band.edge: the row's outside words R + 1 steps away along x and y, and the ones next
            to its own along z (a place outside the grid reads the row's own word and is masked), in
@@ -2113,20 +2004,12 @@ __global__ void __launch_bounds__(256) k_pass2_r(QsBatch B, const uint64_t *__re
         }
         return;
     }
-    /* shell rank of each own row's first tile voxel: the row's shell voxels are stored from there
-       (ownout was last read before the barrier above) */
-    if (threadIdx.x < 128) sbase[threadIdx.x] = sb;
-    /* index of own voxel (tx, ty, tz) in the stored shell field */
-    auto fidx = [&](int tx, int ty_, int tz_) {
-        const int t = tx * P2_TY + ty_;
-        return sbase[t] + (uint32_t)__popc(own[t] & ((1u << tz_) - 1u));
-    };
+    /* index of own voxel (tx, ty, tz) in the field */
+    auto fidx = [&](int tx, int ty_, int tz_) { return ((size_t)(tx0 + tx) * g + (ty0 + ty_)) * g + (tz0 + tz_); };
 
     if (!marked) load_rows();
     if (!(marked ? has_shell : __syncthreads_or(fl))) {
-        /* no outside voxel within reach: every voxel of the tile is -dx (a marked tile has passed
-           no barrier since its shell ranks were written) */
-        if (marked) __syncthreads();
+        /* no outside voxel within reach: every voxel of the tile is -dx */
         for (int tx = 0; tx < P2R_TX; tx++) {
             int gx = tx0 + tx;
             if (gx >= x1 || gx >= g) break;
@@ -2454,7 +2337,7 @@ __device__ __forceinline__ bool mask_bit(const uint64_t *__restrict__ m, int g, 
 /* direct (2r+1)^3 window, one thread per voxel: any r; also a cross-check of the tile kernel */
 __global__ void __launch_bounds__(256) k_pass2_direct(QsBatch B, const uint64_t *__restrict__ outm_all,
                                                       const uint64_t *__restrict__ shellm_all,
-                                                      const uint32_t *__restrict__ spre_all, float *__restrict__ field,
+                                                      float *__restrict__ field_all,
                                                       uint32_t *__restrict__ negm_all, uint32_t *__restrict__ zerom_all)
 {
     uint32_t lb;
@@ -2463,7 +2346,7 @@ __global__ void __launch_bounds__(256) k_pass2_direct(QsBatch B, const uint64_t 
     const int g = G.g, r = G.r, W = (int)M.W;
     const uint64_t *__restrict__ outm = outm_all + M.word_off;
     const uint64_t *__restrict__ shellm = shellm_all + M.word_off;
-    const uint32_t *__restrict__ spre = spre_all + M.word_off;
+    float *__restrict__ field = field_all + M.vox_off;
     uint32_t *__restrict__ negm = negm_all + 2 * M.word_off;
     uint32_t *__restrict__ zerom = zerom_all + 2 * M.word_off;
     const uint32_t nbx = (g + 63) / 64, nby = (g + 3) / 4;
@@ -2498,10 +2381,7 @@ __global__ void __launch_bounds__(256) k_pass2_direct(QsBatch B, const uint64_t 
         }
         res = (min_dist < 999.0f) ? (QS_PROBE - min_dist) : -dx;
     }
-    if (shell) {
-        const size_t wi = ((size_t)x * g + y) * W + (z >> 6);
-        field[spre[wi] + (uint32_t)__popcll(shellm[wi] & bits_below(z & 63, 0))] = res;
-    }
+    if (shell) field[((size_t)x * g + y) * g + z] = res;
     uint64_t n = __ballot(valid && res < 0.0f), zr = __ballot(valid && res == 0.0f);
     if ((threadIdx.x & 63) == 0) {
         size_t w32 = ((size_t)x * g + y) * (2 * (size_t)W) + 2 * (size_t)bidx;
@@ -2827,47 +2707,42 @@ __device__ __forceinline__ void item_word(const ItemWords &S, const uint32_t *__
     }
 }
 
-/* Field value of voxel z of grid row `row` (= x * g + y).  Field pass 2 stores the shell voxels'
-   values only, densely in shell-rank order (F[spre[word] + shell voxels of the word below z]);
-   every other voxel is the probe radius outside and -dx inside, read from the outside and shell
-   masks (W words per row).  shellm == nullptr: F holds every voxel, in grid order. */
-__device__ __forceinline__ float field_at(const float *__restrict__ F, const uint32_t *__restrict__ spre,
-                                          const uint64_t *__restrict__ outm, const uint64_t *__restrict__ shellm, size_t row,
-                                          int g, int W, int z, float dx)
+/* Field value of voxel z of grid row `row` (= x * g + y).  Field pass 2 stores shell voxels only, at
+   their grid places; every other voxel is the probe radius outside and -dx inside, read from the
+   outside and shell masks (W words per row), which are loaded together with the place.  shellm ==
+   nullptr: F holds every voxel. */
+__device__ __forceinline__ float field_at(const float *__restrict__ F, const uint64_t *__restrict__ outm,
+                                          const uint64_t *__restrict__ shellm, size_t row, int g, int W, int z, float dx)
 {
-    if (!shellm) return F[row * g + z];
+    const float f = F[row * g + z];
+    if (!shellm) return f;
     const size_t wi = row * W + (z >> 6);
     const uint64_t sh = shellm[wi], ou = outm[wi];
-    const uint32_t base = spre[wi];
     const int b = z & 63;
-    if ((sh >> b) & 1ull) return F[base + (uint32_t)__popcll(sh & ((1ull << b) - 1ull))];
-    return ((ou >> b) & 1ull) ? QS_PROBE : -dx;
+    return ((sh >> b) & 1ull) ? f : (((ou >> b) & 1ull) ? QS_PROBE : -dx);
 }
 
-/* every voxel of one molecule's field in grid order (out) from the stored shell values (F, global
-   shell ranks spre) and the masks, one thread per mask word */
-__global__ void __launch_bounds__(256) k_field_expand(const float *__restrict__ F, const uint32_t *__restrict__ spre,
-                                                      const uint64_t *__restrict__ outm, const uint64_t *__restrict__ shellm,
-                                                      float *__restrict__ out, int g, int W, float dx)
+/* every voxel of one molecule's field in grid order (out) from the stored shell values (F) and the
+   masks: a wave per mask word, a lane per voxel */
+__global__ void __launch_bounds__(256) k_field_expand(const float *__restrict__ F, const uint64_t *__restrict__ outm,
+                                                      const uint64_t *__restrict__ shellm, float *__restrict__ out, int g, int W,
+                                                      float dx)
 {
-    const size_t wi = (size_t)blockIdx.x * 256 + threadIdx.x;
+    const size_t wi = (size_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     if (wi >= (size_t)g * g * W) return;
     const size_t row = wi / W;
-    const int z0 = (int)(wi - row * W) * 64;
-    const uint64_t o = outm[wi], sh = shellm[wi];
-    uint32_t k = spre[wi];
-    for (int b = 0; b < 64 && z0 + b < g; b++) {
-        if ((sh >> b) & 1ull) out[row * g + z0 + b] = F[k++];
-        else out[row * g + z0 + b] = ((o >> b) & 1ull) ? QS_PROBE : -dx;
-    }
+    const int b = threadIdx.x & 63, z = (int)(wi - row * W) * 64 + b;
+    if (z >= g) return;
+    const bool sh = (shellm[wi] >> b) & 1ull, o = (outm[wi] >> b) & 1ull;
+    out[row * g + z] = sh ? F[row * g + z] : (o ? QS_PROBE : -dx);
 }
 
-void qs_launch_field_expand(const float *F, const uint32_t *spre, const uint64_t *outm, const uint64_t *shellm, float *out, int g,
-                            int W, float dx, hipStream_t s)
+void qs_launch_field_expand(const float *F, const uint64_t *outm, const uint64_t *shellm, float *out, int g, int W, float dx,
+                            hipStream_t s)
 {
     const size_t n = (size_t)g * g * W;
     if (!n) return;
-    k_field_expand<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(F, spre, outm, shellm, out, g, W, dx);
+    k_field_expand<<<(unsigned)((n + 3) / 4), 256, 0, s>>>(F, outm, shellm, out, g, W, dx);
 }
 
 /* vertices (vertexInterp/lerp MarchingCubes.cu:715-734, edge oriented low->high), one thread per
@@ -2877,8 +2752,7 @@ __global__ void __launch_bounds__(256) k_mc_vertices(const QsMol *__restrict__ m
                                                      const uint32_t *__restrict__ wcoarse, const uint32_t *__restrict__ list,
                                                      const uint32_t *__restrict__ avb, const uint32_t *__restrict__ vstart,
                                                      uint32_t nact, uint32_t nv, const uint64_t *__restrict__ S4_all,
-                                                     const float *__restrict__ F_all, const uint32_t *__restrict__ spre_all,
-                                                     const uint64_t *__restrict__ outm_all,
+                                                     const float *__restrict__ F_all, const uint64_t *__restrict__ outm_all,
                                                      const uint64_t *__restrict__ shellm_all, float *__restrict__ vert,
                                                      uint64_t *__restrict__ vkey, const uint32_t *__restrict__ d_counts)
 {
@@ -2933,16 +2807,13 @@ __global__ void __launch_bounds__(256) k_mc_vertices(const QsMol *__restrict__ m
     const float A[3] = {grid_pos(G.ox, x, dx), grid_pos(G.oy, y, dx), grid_pos(G.oz, z, dx)};
     float P[3] = {A[0], A[1], A[2]};
     if (sl < 3) {
-        /* stored shell values are addressed by global shell rank; a full field by the molecule's
-           voxel offset */
-        const float *__restrict__ F = shellm_all ? F_all : F_all + M.vox_off;
-        const uint32_t *__restrict__ sp = shellm_all ? spre_all + M.word_off : nullptr;
+        const float *__restrict__ F = F_all + M.vox_off;
         const uint64_t *__restrict__ om = outm_all + M.word_off;
         const uint64_t *__restrict__ sm = shellm_all ? shellm_all + M.word_off : nullptr;
         const size_t row = (size_t)x * g + y;
         const int W = (int)M.W;
-        const float f0 = field_at(F, sp, om, sm, row, g, W, z, dx);
-        const float f1 = field_at(F, sp, om, sm, row + (sl == 0 ? (size_t)g : (sl == 1 ? 1 : 0)), g, W, z + (sl == 2), dx);
+        const float f0 = field_at(F, om, sm, row, g, W, z, dx);
+        const float f1 = field_at(F, om, sm, row + (sl == 0 ? (size_t)g : (sl == 1 ? 1 : 0)), g, W, z + (sl == 2), dx);
         float B[3] = {A[0], A[1], A[2]};
         B[sl] = A[sl] + dx;
         const float t = (0.0f - f0) / (f1 - f0);
@@ -3493,11 +3364,10 @@ __global__ void __launch_bounds__(256) k_smooth_incid(const uint32_t *__restrict
 /* one molecule's field, addressed by grid row (x * g + y) and z */
 struct FieldView {
     const float *F;
-    const uint32_t *spre;
     const uint64_t *outm, *shellm;
     int g, W;
     float dx;
-    __device__ __forceinline__ float at(size_t row, int z) const { return field_at(F, spre, outm, shellm, row, g, W, z, dx); }
+    __device__ __forceinline__ float at(size_t row, int z) const { return field_at(F, outm, shellm, row, g, W, z, dx); }
 };
 
 /* derivative along axis a (0 x, 1 y, 2 z) at grid point (row, z), whose coordinate on that axis is i */
@@ -3513,7 +3383,7 @@ __device__ __forceinline__ float grad_axis(const FieldView &F, size_t row, int z
 __global__ void __launch_bounds__(256) k_vertex_normals(const QsMol *__restrict__ mols, const uint32_t *__restrict__ vpre,
                                                         const uint32_t *__restrict__ vcoarse, const uint64_t *__restrict__ vkey,
                                                         uint32_t nv, const float *__restrict__ F_all,
-                                                        const uint32_t *__restrict__ spre_all, const uint64_t *__restrict__ outm_all,
+                                                        const uint64_t *__restrict__ outm_all,
                                                         const uint64_t *__restrict__ shellm_all, float *__restrict__ out)
 {
     const uint32_t v = blockIdx.x * blockDim.x + threadIdx.x;
@@ -3521,7 +3391,7 @@ __global__ void __launch_bounds__(256) k_vertex_normals(const QsMol *__restrict_
     const QsMol &M = mols[seg_of_wave(vpre, vcoarse, v)];
     const int g = M.G.g;
     const float dx = M.G.dx;
-    const FieldView F{shellm_all ? F_all : F_all + M.vox_off, shellm_all ? spre_all + M.word_off : nullptr, outm_all + M.word_off,
+    const FieldView F{F_all + M.vox_off, outm_all + M.word_off,
                       shellm_all ? shellm_all + M.word_off : nullptr, g, (int)M.W, dx};
     const uint64_t key = vkey[v];
     const int sl = (int)(key & 3ull);
@@ -3880,14 +3750,14 @@ uint32_t qs_pass2_blocks(const QsMol &M, int path)
 
 /* one launch for a group of molecules sharing r (and so the path) */
 void qs_launch_pass2(QsBatch B, uint32_t nblocks, int r, int path, const uint64_t *outm, const uint64_t *shellm,
-                     const uint32_t *spre, float *field, uint32_t *negm, uint32_t *zerom, const int *offs, const int *norm_start, const int *enum_end,
+                     float *field, uint32_t *negm, uint32_t *zerom, const int *offs, const int *norm_start, const int *enum_end,
                      QsNormFlags nf, QsBand band, const uint8_t *tflag, uint8_t tmark, uint32_t xchunk, hipStream_t s)
 {
     if (path == 0) {
         xchunk = std::max(xchunk, 1u);
 #define QS_P2R(RR)                                                                                                    \
     case RR:                                                                                                          \
-        hipLaunchKernelGGL(k_pass2_r<RR>, dim3(nblocks), dim3(256), 0, s, B, outm, shellm, spre, field, negm, zerom, \
+        hipLaunchKernelGGL(k_pass2_r<RR>, dim3(nblocks), dim3(256), 0, s, B, outm, shellm, field, negm, zerom, \
                            offs, norm_start, enum_end, nf, band, tflag, tmark, xchunk);                                            \
         return;
         switch (r) {
@@ -3906,25 +3776,11 @@ void qs_launch_pass2(QsBatch B, uint32_t nblocks, int r, int path, const uint64_
 #undef QS_P2R
     }
     if (path <= 1) {
-        hipLaunchKernelGGL(k_pass2_tile<uint16_t>, dim3(nblocks), dim3(256), qs_pass2_lds_bytes(r), s, B, outm, shellm, spre,
+        hipLaunchKernelGGL(k_pass2_tile<uint16_t>, dim3(nblocks), dim3(256), qs_pass2_lds_bytes(r), s, B, outm, shellm,
                            field, negm, zerom, offs, norm_start, enum_end);
         return;
     }
-    hipLaunchKernelGGL(k_pass2_direct, dim3(nblocks), dim3(256), 0, s, B, outm, shellm, spre, field, negm, zerom);
-}
-
-void qs_launch_shell_scan(const uint64_t *shellm, uint64_t nw, uint32_t *sums, uint32_t *totals, uint32_t *spre, hipStream_t s)
-{
-    if (!nw) return;
-    if (nw <= QS_SCAN1_MAX) {
-        hipLaunchKernelGGL(k_shell_scan1, dim3(1), dim3(SCAN1_NT), 0, s, shellm, nw, totals, spre);
-        return;
-    }
-    const uint64_t ntiles = qs_scan_tiles(nw);
-    const int self = ntiles <= QS_SCAN_SELF_TILES;
-    hipLaunchKernelGGL(k_shell_reduce, dim3((unsigned)ntiles), dim3(SCAN_NT), 0, s, shellm, nw, sums);
-    if (!self) hipLaunchKernelGGL(k_scan_planes, dim3(1), dim3(SCAN_NT), 0, s, sums, ntiles, totals);
-    hipLaunchKernelGGL(k_shell_scan, dim3((unsigned)ntiles), dim3(SCAN_NT), 0, s, shellm, nw, sums, spre, self, totals);
+    hipLaunchKernelGGL(k_pass2_direct, dim3(nblocks), dim3(256), 0, s, B, outm, shellm, field, negm, zerom);
 }
 
 void qs_launch_labels_to_masks(const uint8_t *labels, int g, int W, uint64_t *outm, uint64_t *shellm, hipStream_t s)
@@ -3946,7 +3802,7 @@ void qs_launch_mc_count(QsBatch B, uint32_t nblocks, const uint64_t *N, const ui
 
 void qs_launch_mc_emit(const QsMol *mols, const uint64_t *wpre, const uint32_t *wcoarse, const uint32_t *list, uint32_t nact,
                        const uint32_t *avb, uint32_t *vstart, uint32_t nv, const uint64_t *S4, const float *F,
-                       const uint32_t *spre, const uint64_t *outm, const uint64_t *shellm, float *vert, uint64_t *vkey,
+                       const uint64_t *outm, const uint64_t *shellm, float *vert, uint64_t *vkey,
                        const uint32_t *acb, uint32_t *tstart, uint32_t ncube, uint32_t ntri, const uint64_t *N, const uint32_t *cnt,
                        const uint32_t *vbw, const uint32_t *tbw, const uint64_t *NT, int *tri, uint32_t vbase, uint32_t *deg_blk,
                        uint32_t *deg_total, const uint32_t *d_counts, hipStream_t s, hipStream_t s_vert, hipEvent_t ev_fork,
@@ -3977,7 +3833,7 @@ void qs_launch_mc_emit(const QsMol *mols, const uint64_t *wpre, const uint32_t *
     }
     if (nv)
         hipLaunchKernelGGL(k_mc_vertices, dim3(pgrid(nblk(std::min(nv, expect), 256))), dim3(256), 0, s_vert, mols, wpre, wcoarse, list, avb, vstart, nact,
-                           nv, S4, F, spre, outm, shellm, vert, vkey, d_counts);
+                           nv, S4, F, outm, shellm, vert, vkey, d_counts);
     if (s_vert != s) (void)hipEventRecord(ev_vert, s_vert);
     if (ntri)
         hipLaunchKernelGGL(k_mc_triangles, dim3(pgrid(nblk(std::min(ncube, expect), 256))), dim3(256), 0, s, mols, wpre, wcoarse, list, acb, tstart,
@@ -3995,11 +3851,11 @@ void qs_launch_smooth(const QsMol *mols, const uint32_t *vpre, const uint32_t *v
 }
 
 void qs_launch_vertex_normals(const QsMol *mols, const uint32_t *vpre, const uint32_t *vcoarse, const uint64_t *vkey, uint32_t nv,
-                              const float *F, const uint32_t *spre, const uint64_t *outm, const uint64_t *shellm, float *out,
+                              const float *F, const uint64_t *outm, const uint64_t *shellm, float *out,
                               hipStream_t s)
 {
     if (!nv) return;
-    hipLaunchKernelGGL(k_vertex_normals, dim3(nblk(nv, 256)), dim3(256), 0, s, mols, vpre, vcoarse, vkey, nv, F, spre, outm, shellm,
+    hipLaunchKernelGGL(k_vertex_normals, dim3(nblk(nv, 256)), dim3(256), 0, s, mols, vpre, vcoarse, vkey, nv, F, outm, shellm,
                        out);
 }
 
