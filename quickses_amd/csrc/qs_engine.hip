@@ -257,7 +257,7 @@ int Engine::reserve(uint64_t vox, uint64_t atoms, uint64_t cells, uint64_t verts
     QS_TRY(ensure(key, atoms * 8));
     for (DevBuf *b : {&sx, &aux}) QS_TRY(ensure(*b, atoms * 16));
     QS_TRY(ensure(count, (cells + 1) * 4));
-    QS_TRY(ensure(start, (cells + 1) * 4));
+    QS_TRY(ensure(start, (cells + 1) * 4 + 16));
     QS_TRY(ensure(cse, cells * 8));
     for (DevBuf *b : {&vert, &vert2, &vert3}) QS_TRY(ensure(*b, verts * 12));
     QS_TRY(ensure(vkey, verts * 8));
@@ -995,7 +995,7 @@ int Engine::run_batch(const float *d_pos, const float *d_rad, const std::vector<
     /* per atom its cell and rank within the cell; per cell its atom count (cleared by a fill) */
     QS_TRY(ensure(key, (size_t)std::max<uint32_t>(n, 1) * 8));
     QS_TRY(ensure(count, ncell * 4));
-    QS_TRY(ensure(start, (ncell + 1) * 4));
+    QS_TRY(ensure(start, (ncell + 1) * 4 + 16)); /* (padding: column_starts) */
     QS_TRY(ensure(perm, (size_t)std::max<uint32_t>(n, 1) * 4));
     QS_TRY(ensure(cse, ncell * 8));
     QS_TRY(ensure(sx, (size_t)std::max<uint32_t>(n, 1) * 16));

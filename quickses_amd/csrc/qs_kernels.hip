@@ -2989,8 +2989,9 @@ __global__ void __launch_bounds__(256) k_mc_triangles(const QsMol *__restrict__ 
 /* The walk as the reference's, with a root for every atom whose squared sum is below the best
    one's (sqrtf is monotone: no other can win): for the vertices closest_one cannot decide. */
 __device__ __noinline__ int closest_walk(const float4 *__restrict__ sx, const uint32_t *__restrict__ cstart, int gn, int cx, int cy,
-                                         int z0, int z1, float px, float py, float pz)
+                                         int cz, float px, float py, float pz)
 {
+    const int z0 = iclamp(cz - 1, 0, gn - 1), z1 = iclamp(cz + 1, 0, gn - 1);
     int best = -1;
     float min_d = 999999.0f, min_s = INFINITY;
     for (int k = 0; k < 9; k++) {
@@ -3013,47 +3014,130 @@ __device__ __noinline__ int closest_walk(const float4 *__restrict__ sx, const ui
     return best;
 }
 
+/* One axis of a vertex's 3 x 3 x 3 cells: its own cell o, and the squared distance that an atom of
+   the cell below (o - 1) or above (o + 1) is away at least (infinite where the clamp leaves none).
+   A cell's atoms lie beyond its boundary up to the rounding of cell_of, which margin covers. */
+struct AxisCells {
+    int o;
+    float dn2, up2;
+    __device__ __forceinline__ bool near_dn() const { return dn2 < up2; }
+    __device__ __forceinline__ int nr() const { return near_dn() ? o - 1 : o + 1; }
+    __device__ __forceinline__ int fr() const { return near_dn() ? o + 1 : o - 1; }
+    __device__ __forceinline__ float nr2() const { return fminf(dn2, up2); }
+    __device__ __forceinline__ float fr2() const { return fmaxf(dn2, up2); }
+};
+__device__ __forceinline__ AxisCells axis_cells(float p, float org, float dxn, int gn, float margin)
+{
+    AxisCells A;
+    const int c = cell_of(p, org, dxn);
+    const float f = p - org;
+    A.o = iclamp(c, 0, gn - 1);
+    const float dn = fmaxf(f - (float)A.o * dxn - margin, 0.0f), up = fmaxf((float)(A.o + 1) * dxn - f - margin, 0.0f);
+    A.dn2 = iclamp(c - 1, 0, gn - 1) == A.o ? INFINITY : dn * dn;
+    A.up2 = iclamp(c + 1, 0, gn - 1) == A.o ? INFINITY : up * up;
+    return A;
+}
+
+/* A column's three z cells around z cell o as places in the cell-sorted atoms: below [a, b), own
+   [b, c), above [c, d), read in one load (past the column's ends they hold its neighbours' places,
+   past the last cell the padding of the array: callers use those of cells that exist only) */
+struct ColumnStarts {
+    int a, b, c, d;
+};
+__device__ __forceinline__ ColumnStarts column_starts(const uint32_t *__restrict__ cstart, int h, int o)
+{
+    struct __attribute__((packed, aligned(4))) U4 {
+        int x, y, z, w;
+    };
+    const U4 e = *(const U4 *)(cstart + (h + max(o - 1, 0)));
+    ColumnStarts C;
+    C.a = e.x;
+    C.b = o ? e.y : e.x;
+    C.c = o ? e.z : e.y;
+    C.d = o ? e.w : e.z;
+    return C;
+}
+
 /* closest atom of vertex v (position p) of molecule M, relative to its first atom (-1: none).
-   Bound by VALU issue and by lanes idling in the column loops.  A loop that roots every improving
-   candidate pays for the root on almost every iteration, as some lane of the wave improves on
-   most; so the loop keeps the smallest squared sum, its atom and the second smallest sum, with no
-   branch.  Rounded roots of two sums can only be equal when the sums agree to 2^-22, so unless the
-   two smallest agree to 1e-6 the atom of the smallest one is the reference's; else the vertex is
-   walked again with the roots (50,000-atom 0.2 A mesh 0.192 -> 0.183 ms, 256 molecules at 0.5 A
-   0.955 -> 0.910 ms). */
+   Bound by the L1's lookups: a lane's gather of an atom or of a column's places takes one each,
+   nearly independent of its width.  So the eight cells of the vertex's octant (its own and the nearer
+   neighbour on each axis) come first, and of the other 19 only those are visited whose boundary is
+   not further than the best atom so far: 9 atoms per vertex instead of 24, 33 iterations per wave
+   instead of 47 (most vertices need none of the 19, as the closest atom is about 1.9 A away and the
+   far cells at least 1.6); and a column's places are one load.  All 27 cells, two loads per column,
+   took 0.185 ms on the 50,000-atom 0.2 A mesh and 0.907 ms on 256 molecules at 0.5 A; this takes
+   0.126 and 0.716 (0.134 and 0.756 with two loads per column; the far columns walked from a mask of
+   those to visit, their places loaded when it is their turn, 0.143 and 0.777).
+   A loop that roots every improving candidate pays for the root on almost every iteration, so the
+   loop keeps the smallest squared sum, its atom and the second smallest sum, with no branch.
+   Rounded roots of two sums can only be equal when the sums agree to 2^-22, so unless the two
+   smallest agree to 1e-6 the atom of the smallest one is the reference's, whatever the order of the
+   visit (a cell is left out only if its atoms' sums are 1e-4 above); else the vertex is walked
+   again in the reference's order with the roots. */
 __device__ __forceinline__ int closest_one(const QsMol &M, float px, float py, float pz, const uint32_t *__restrict__ cstart_all,
                                            const float4 *__restrict__ sx, const int *__restrict__ perm, int sorted_ids)
 {
     const QsGrid G = M.G;
     const uint32_t *__restrict__ cstart = cstart_all + M.cell_off;
-    int cx = cell_of(px, G.ox, G.dxn), cy = cell_of(py, G.oy, G.dxn), cz = cell_of(pz, G.oz, G.dxn);
     const int gn = G.gn;
-    const int z0 = iclamp(cz - 1, 0, gn - 1), z1 = iclamp(cz + 1, 0, gn - 1);
+    const float margin = (float)(gn + 1) * G.dxn * 1e-6f; /* 8 roundings at the grid's extent */
+    const AxisCells X = axis_cells(px, G.ox, G.dxn, gn, margin), Y = axis_cells(py, G.oy, G.dxn, gn, margin),
+                    Z = axis_cells(pz, G.oz, G.dxn, gn, margin);
     int best = -1;
     float min_s = INFINITY, next_s = INFINITY;
-    /* the nine columns' ranges are loaded before any is walked */
-    int lo9[9], hi9[9];
-#pragma unroll
-    for (int k = 0; k < 9; k++) {
-        const int ix = iclamp(cx + k / 3 - 1, 0, gn - 1), iy = iclamp(cy + k % 3 - 1, 0, gn - 1);
-        const int h = (gn * gn * ix) + (gn * iy);
-        /* (a column that the clamp repeats is walked once: its atoms would tie with themselves) */
-        const bool again = (k / 3 && ix == iclamp(cx + k / 3 - 2, 0, gn - 1)) || (k % 3 && iy == iclamp(cy + k % 3 - 2, 0, gn - 1));
-        lo9[k] = (int)cstart[h + z0];
-        hi9[k] = again ? 0 : (int)cstart[h + z1 + 1];
-    }
-#pragma unroll
-    for (int k = 0; k < 9; k++) {
-        const int lo = lo9[k], hi = hi9[k];
+    const auto walk = [&](int lo, int hi) {
         for (int id = lo; id < hi; id++) {
             const float4 at = sx[id];
             const float sq = dist3_sq(at.x, at.y, at.z, px, py, pz);
             next_s = __builtin_amdgcn_fmed3f(sq, min_s, next_s); /* second smallest: min_s <= next_s */
             best = (sq < min_s) ? id : best;
-            min_s = fminf(sq, min_s);
+            min_s = (sq < min_s) ? sq : min_s;
         }
+    };
+    const auto column = [&](int ix, int iy) { return (gn * gn * ix) + (gn * iy); };
+    const bool zdn = Z.near_dn();
+    const float xn2 = X.nr2(), xf2 = X.fr2(), yn2 = Y.nr2(), yf2 = Y.fr2(), zf2 = Z.fr2();
+    const bool xn = xn2 < INFINITY, yn = yn2 < INFINITY, zn = Z.nr2() < INFINITY;
+    const int xnr = xn ? X.nr() : X.o, ynr = yn ? Y.nr() : Y.o;
+    /* the octant's four columns: own and near z cell; the far z cell's range is kept for later */
+    int flo[4], fhi[4];
+    {
+        int lo[4], hi[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const ColumnStarts C = column_starts(cstart, column(k & 1 ? xnr : X.o, k & 2 ? ynr : Y.o), Z.o);
+            const bool is = (!(k & 1) || xn) && (!(k & 2) || yn);
+            lo[k] = zn && zdn ? C.a : C.b;
+            hi[k] = is ? (zn && !zdn ? C.d : C.c) : 0;
+            flo[k] = zdn ? C.c : C.a;
+            fhi[k] = zdn ? C.d : C.b;
+        }
+#pragma unroll
+        for (int k = 0; k < 4; k++) walk(lo[k], hi[k]);
     }
-    if (!(next_s > min_s * 1.000001f) && best >= 0) best = closest_walk(sx, cstart, gn, cx, cy, z0, z1, px, py, pz);
+    {
+        /* the far cells in reach */
+        const float lim = fminf(min_s * 1.0001f, 3.0e38f);
+        const float near2[4] = {0.0f, xn2, yn2, xn2 + yn2};
+        const float far2[5] = {xf2, xf2 + yn2, yf2, xn2 + yf2, xf2 + yf2};
+        const int ix[5] = {X.fr(), X.fr(), X.o, xnr, X.fr()}, iy[5] = {Y.o, ynr, Y.fr(), Y.fr(), Y.fr()};
+        int lo[5], hi[5];
+#pragma unroll
+        for (int k = 0; k < 5; k++) {
+            lo[k] = hi[k] = 0;
+            if (far2[k] <= lim) {
+                const ColumnStarts C = column_starts(cstart, column(ix[k], iy[k]), Z.o);
+                lo[k] = far2[k] + Z.dn2 <= lim ? C.a : C.b;
+                hi[k] = far2[k] + Z.up2 <= lim ? C.d : C.c;
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < 4; k++) walk(flo[k], near2[k] + zf2 <= lim ? fhi[k] : 0);
+#pragma unroll
+        for (int k = 0; k < 5; k++) walk(lo[k], hi[k]);
+    }
+    if (!(next_s > min_s * 1.000001f) && best >= 0)
+        best = closest_walk(sx, cstart, gn, cell_of(px, G.ox, G.dxn), cell_of(py, G.oy, G.dxn), cell_of(pz, G.oz, G.dxn), px, py, pz);
     /* atom indices are returned relative to the molecule's first atom */
     return (best < 0) ? -1 : ((sorted_ids ? best : perm[best]) - (int)M.atom_off);
 }

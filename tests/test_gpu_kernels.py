@@ -30,6 +30,28 @@ def test_closest_atom_ties_and_clamps(qs, orc, kind, reso):
     assert _same(qs.compute_ses(pos, rad, reso, 0), orc.compute_ses(pos, rad, reso, 0))
 
 
+def _far_cells_case(qs, kind):
+    rng = np.random.default_rng(11)
+    if kind == "two large atoms":  # 7 A from their vertices: past the octant's cells on every side
+        return np.array([[0, 0, 0], [3, 0, 0]], np.float32), np.full(2, 7.0, np.float32)
+    if kind == "mixed radii":  # large empty cells beside crowded ones
+        return (rng.random((60, 3)) * 40).astype(np.float32), np.where(rng.random(60) < 0.1, 6.0, 0.9).astype(np.float32)
+    n, step = 9, np.float32(3.25)  # every atom on a cell boundary (cell size 3.25), 1000 A off the origin
+    ax = np.arange(n, dtype=np.float32) * step + np.float32(1000.0)
+    pos = np.stack(np.meshgrid(ax, ax, ax, indexing="ij"), -1).reshape(-1, 3)
+    return pos[rng.random(len(pos)) < 0.4], np.full(n ** 3, 1.85, np.float32)
+
+
+@pytest.mark.parametrize("kind", ["two large atoms", "mixed radii", "cell boundaries"])
+@pytest.mark.parametrize("reso", [0.3, 0.5])
+def test_closest_atom_beyond_the_octant(qs, orc, kind, reso):
+    """The closest atom in a cell of the far side, in none, and on the boundary of two."""
+    pos, rad = _far_cells_case(qs, kind)
+    rad = rad[:len(pos)]
+    print("case far cells: %s reso=%.2f" % (kind, reso), flush=True)
+    assert _same(qs.compute_ses(pos, rad, reso, 0), orc.compute_ses(pos, rad, reso, 0))
+
+
 def _noise_field(g, kind):
     rng = np.random.default_rng(100 * g + len(kind))
     f = rng.standard_normal((g, g, g)).astype(np.float32)  # nearly every cube polygonised
