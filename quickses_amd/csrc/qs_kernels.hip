@@ -3029,7 +3029,9 @@ struct AxisCells {
 __device__ __forceinline__ AxisCells axis_cells(float p, float org, float dxn, int gn, float margin)
 {
     AxisCells A;
-    const int c = cell_of(p, org, dxn);
+    /* (clamped to one cell off the grid, where the reference's three clamped cells are the same as
+       further off: the neighbours' indexes hold for any p) */
+    const int c = iclamp(cell_of(p, org, dxn), -1, gn);
     const float f = p - org;
     A.o = iclamp(c, 0, gn - 1);
     const float dn = fmaxf(f - (float)A.o * dxn - margin, 0.0f), up = fmaxf((float)(A.o + 1) * dxn - f - margin, 0.0f);
