@@ -71,6 +71,13 @@ __device__ __forceinline__ float grid_pos(float o, int i, float dx)
 /* spaceToGrid Kernels.cu:119-123: truncation of (p - o) / dx */
 __device__ __forceinline__ int cell_of(float p, float o, float dx) { return (int)((p - o) / dx); }
 
+/* one axis' term of dist3_sq */
+__device__ __forceinline__ float sq_dist(float a, float b)
+{
+    const float e = a - b;
+    return e * e;
+}
+
 /* fast_distance Kernels.cu:149-155, left to right, IEEE sqrt */
 /* the squared sum under dist3's root, with dist3's roundings */
 __device__ __forceinline__ float dist3_sq(float ax, float ay, float az, float bx, float by, float bz)
@@ -2247,26 +2254,34 @@ __global__ void __launch_bounds__(256) k_pass2_r(QsBatch B, const uint64_t *__re
         if (nmin >= INF) {
             /* no outside voxel in the window: -dx */
         } else if ((nfw[nmin >> 5] >> (nmin & 31)) & 1u) {
-            /* trace the minimisers back through the separable passes: the x offsets, then their y
-               offsets from the recorded masks */
-            while (amask) {
-                const int a = __builtin_ctz(amask) - R;
-                amask &= amask - 1u;
-                const int dy = nmin - a * a;
-                uint32_t bmask = BM[((tx + R + a) * P2_TY + ty_) * P2_TZ + tz_];
-                while (bmask) {
-                    const int b = __builtin_ctz(bmask) - R;
-                    bmask &= bmask - 1u;
-                    /* dz = c^2 exactly, c <= R: the hardware root is within an ulp of c */
-                    const int dz = dy - b * b;
-                    const int c = (int)(__builtin_amdgcn_sqrtf((float)dz) + 0.5f);
-                    const uint64_t m = rows[(tx + R + a) * LY + (ty_ + R + b)];
-                    const float qx = grid_pos(G.ox, gx + a, dx), qy = grid_pos(G.oy, gy_ + b, dx);
-                    if ((m >> (tz_ + R + c)) & 1ull)
-                        min_sq = fminf(dist3_sq(qx, qy, grid_pos(G.oz, gz_ + c, dx), vx, vy, vz), min_sq);
-                    if (c && ((m >> (tz_ + R - c)) & 1ull))
-                        min_sq = fminf(dist3_sq(qx, qy, grid_pos(G.oz, gz_ - c, dx), vx, vy, vz), min_sq);
+            /* trace the minimisers back through the separable passes: the x offsets, their y offsets
+               from the recorded masks, and the nearest outside voxels of those rows along z (one
+               loop over the (x, y) offsets, as the lanes' numbers of x and of y offsets differ: an
+               outer and an inner one, with a root for the z offset and 64-bit shifts of the row for
+               its two ends, took 0.611 instead of 0.581 ms on 100 frames of 10,000 atoms at 0.5 A
+               and 0.869 instead of 0.825 on 256 molecules) */
+            int at = 0;             /* own voxel (tx + R + a, ty_) as the row of DY and BM */
+            uint32_t bmask = 0;
+            float ex2 = 0.0f;
+            while (amask | bmask) {
+                if (!bmask) {
+                    const int a = __builtin_ctz(amask);
+                    amask &= amask - 1u;
+                    at = tx + a;
+                    bmask = BM[(at * P2_TY + ty_) * P2_TZ + tz_];
+                    ex2 = sq_dist(grid_pos(G.ox, gx + a - R, dx), vx);
                 }
+                const int b = __builtin_ctz(bmask);
+                bmask &= bmask - 1u;
+                const uint64_t m = rows[at * LY + ty_ + b];
+                const uint32_t w = __builtin_amdgcn_alignbit((uint32_t)(m >> 32), (uint32_t)m, (uint32_t)tz_);
+                const int up = __builtin_ctz((w >> R) | 0x80000000u), dn = __builtin_clz((w << (31 - R)) | 1u);
+                const int c = min(up, dn);
+                const float exy = ex2 + sq_dist(grid_pos(G.oy, gy_ + b - R, dx), vy);
+                const float su = exy + sq_dist(grid_pos(G.oz, gz_ + c, dx), vz);
+                const float sd = exy + sq_dist(grid_pos(G.oz, gz_ - c, dx), vz);
+                min_sq = fminf(min_sq, up <= dn ? su : sd);
+                min_sq = fminf(min_sq, dn <= up ? sd : su);
             }
         } else {
 #pragma unroll 1
