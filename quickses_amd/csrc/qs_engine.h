@@ -206,9 +206,8 @@ struct P2Group {
 struct Engine {
     int device = -1;
     hipStream_t stream = nullptr, side = nullptr;
-    hipEvent_t ev_emit = nullptr, ev_side = nullptr, ev_vert = nullptr;
+    hipEvent_t ev_emit = nullptr, ev_side = nullptr;
     bool side_pending = false; /* closest-atom work on `side` not yet joined into `stream` */
-    bool vert_pending = false; /* the vertex kernel on `side` not yet joined into `stream` */
 
     DevBuf in_pos, in_rad, d_off, bb_part, bb_out, d_mols, d_meta;
     DevBuf key /* cell and rank within the cell per atom */, count, start, perm, cse, sx, aux;
@@ -229,8 +228,7 @@ struct Engine {
     std::vector<P2Group> groups;
     std::vector<P2Tables *> tables;
     /* host staging of uploads that kernels read later in the same call */
-    std::vector<uint32_t> h_meta, h_vpre;
-    std::vector<uint64_t> h_bidx; /* first triangle of each molecule, staged for the filter */
+    std::vector<uint32_t> h_meta;
     /* pinned staging for a run's small uploads (molecule records, prefixes, indices): copies from
        it are queued at once, where the runtime stages pageable sources on the host first */
     void *up = nullptr;
@@ -373,8 +371,7 @@ struct Engine {
         side = nullptr;
         if (ev_emit) (void)hipEventDestroy(ev_emit);
         if (ev_side) (void)hipEventDestroy(ev_side);
-        if (ev_vert) (void)hipEventDestroy(ev_vert);
-        ev_emit = ev_side = ev_vert = nullptr;
+        ev_emit = ev_side = nullptr;
         device = -1;
         batch_valid = false;
     }
@@ -391,7 +388,6 @@ struct Engine {
         QS_HIP(hipStreamCreateWithFlags(&side, hipStreamNonBlocking));
         QS_HIP(hipEventCreateWithFlags(&ev_emit, hipEventDisableTiming));
         QS_HIP(hipEventCreateWithFlags(&ev_side, hipEventDisableTiming));
-        QS_HIP(hipEventCreateWithFlags(&ev_vert, hipEventDisableTiming));
         return 0;
     }
 
@@ -451,13 +447,16 @@ struct Engine {
         QsBatch B;
         B.mols = (const QsMol *)d_mols.p;
         B.bpre = (const uint32_t *)d_meta.p + bpre_at;
-        B.coarse = B.bpre + n + 1; /* the coarse index follows each prefix */
+        /* the coarse index follows each prefix; one molecule needs neither */
+        B.coarse = mols.size() > 1 ? B.bpre + n + 1 : nullptr;
         B.mid = mid_at ? (const int *)((const uint32_t *)d_meta.p + mid_at) : nullptr;
         B.n = n;
         return B;
     }
 
     int setup(const std::vector<MolIn> &in, const std::vector<BBox> &bb);
+    int upload_mols();
+    int fork_side();
     int build_meta(size_t &at_atoms, size_t &at_p1, size_t &at_mc, size_t &at_wpre,
                    uint32_t &nb_atoms, uint32_t &nb_p1, uint32_t &nb_mc);
     /* allocate the workspace for batches up to these totals in one go */

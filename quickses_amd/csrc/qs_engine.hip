@@ -267,7 +267,7 @@ int Engine::reserve(uint64_t vox, uint64_t atoms, uint64_t cells, uint64_t verts
     const size_t m = (size_t)nmol + 1;
     QS_TRY(ensure(d_off, m * 8 + 64));
     QS_TRY(ensure(bb_out, m * 8 * sizeof(float)));
-    QS_TRY(ensure(bb_part, qs_bbox_part_floats((int)m, qs_bbox_parts((uint32_t)std::min<uint64_t>(atoms, UINT32_MAX))) *
+    QS_TRY(ensure(bb_part, qs_bbox_part_floats((int)m, qs_bbox_parts((uint32_t)std::min<uint64_t>(atoms, UINT32_MAX), nmol + 1)) *
                                sizeof(float)));
     QS_TRY(ensure(bounds, m * 8));
     QS_TRY(ensure(rback, (4 + 2 * m) * 4));
@@ -353,7 +353,8 @@ int Engine::build_meta(size_t &at_atoms, size_t &at_p1, size_t &at_mc, size_t &a
     const int nmol = (int)mols.size();
     std::vector<uint32_t> &meta = h_meta;
     meta.assign(1, 0u); /* index 0 is never a prefix start (mid_at == 0 means none) */
-    /* each block prefix (nmol + 1 entries) is followed by its coarse index */
+    /* each block prefix (nmol + 1 entries) is followed by its coarse index (but for one molecule:
+       its launches read neither, see Engine::batch) */
     auto prefix = [&](auto blocks_of, uint32_t &total) {
         size_t at = meta.size();
         uint64_t acc = 0;
@@ -364,7 +365,7 @@ int Engine::build_meta(size_t &at_atoms, size_t &at_p1, size_t &at_mc, size_t &a
         meta.push_back((uint32_t)acc);
         total = (uint32_t)acc;
         std::vector<uint32_t> pre(meta.begin() + at, meta.end());
-        append_coarse(meta, pre.data(), nmol, acc, QS_COARSE_BLOCKS);
+        if (nmol > 1) append_coarse(meta, pre.data(), nmol, acc, QS_COARSE_BLOCKS);
         return at;
     };
     at_atoms = prefix([](const QsMol &M) { return (uint64_t)((M.n_atoms + 255) / 256); }, nb_atoms);
@@ -401,7 +402,7 @@ int Engine::build_meta(size_t &at_atoms, size_t &at_p1, size_t &at_mc, size_t &a
         meta.push_back((uint32_t)w);
         meta.push_back((uint32_t)(w >> 32));
     }
-    append_coarse(meta, wp.data(), nmol, nw_total, QS_COARSE_ITEMS);
+    if (nmol > 1) append_coarse(meta, wp.data(), nmol, nw_total, QS_COARSE_ITEMS);
     /* field pass 2 groups: same kernel path, r, dx and coordinate range */
     groups.resize(0);
     std::vector<P2Group> gs;
@@ -448,12 +449,25 @@ int Engine::build_meta(size_t &at_atoms, size_t &at_p1, size_t &at_mc, size_t &a
         meta.push_back((uint32_t)acc);
         grp.nblocks = (uint32_t)acc;
         std::vector<uint32_t> pre(meta.begin() + grp.bpre_at, meta.end());
-        append_coarse(meta, pre.data(), (int)grp.mols.size(), acc, QS_COARSE_BLOCKS);
+        if (nmol > 1) append_coarse(meta, pre.data(), (int)grp.mols.size(), acc, QS_COARSE_BLOCKS);
         grp.mid_at = meta.size();
         for (int m : grp.mols) meta.push_back((uint32_t)m);
     }
     groups.swap(gs);
     return 0;
+}
+
+/* the molecules' records and the block prefixes to the device.  One molecule needs no prefixes (see
+   batch), and its record goes in a launch's arguments: a copy takes two to three times as long */
+int Engine::upload_mols()
+{
+    if (mols.size() == 1) {
+        qs_launch_put_mol(mols[0], as<QsMol>(d_mols), stream);
+        QS_HIP(hipGetLastError());
+        return 0;
+    }
+    QS_TRY(upload(d_mols.p, mols.data(), mols.size() * sizeof(QsMol)));
+    return upload(d_meta.p, h_meta.data(), h_meta.size() * 4);
 }
 
 /* candidate tables of field pass 2 for one group (built once per (r, dx, coordinate range)) */
@@ -567,6 +581,16 @@ int Engine::fill_field(const void **dense)
     return 0;
 }
 
+/* the side stream follows the main stream up to here (the caller records ev_side on it, and the run
+   joins it before its results are read) */
+int Engine::fork_side()
+{
+    QS_HIP(hipEventRecord(ev_emit, stream));
+    QS_HIP(hipStreamWaitEvent(side, ev_emit, 0));
+    side_pending = true;
+    return 0;
+}
+
 /* marching cubes over every molecule (sign masks must be ready) */
 int Engine::mesh_stage(size_t at_mc, uint32_t nb_mc, size_t at_wpre, StageTimer &tm, bool with_atoms)
 {
@@ -616,51 +640,48 @@ int Engine::mesh_stage(size_t at_mc, uint32_t nb_mc, size_t at_wpre, StageTimer 
     /* per-molecule first vertex and triangle (the scans at each molecule's first word, from the
        word prefix) and the vertex coarse index, computed on the device */
     const uint64_t *wpre = (const uint64_t *)(as<uint32_t>(d_meta) + at_wpre);
-    const uint32_t *wcoarse = as<uint32_t>(d_meta) + at_wpre + 2 * ((size_t)nmol + 1);
+    const uint32_t *wcoarse = nmol > 1 ? as<uint32_t>(d_meta) + at_wpre + 2 * ((size_t)nmol + 1) : nullptr;
     QS_TRY(ensure(bounds, ((size_t)nmol + 1) * 8));
     QS_TRY(ensure(tpre_d, ((size_t)nmol + 1) * 8));
     const uint32_t ncoarse = (pool_v >> QS_COARSE_ITEMS) + 2;
     QS_TRY(ensure(d_off, ((size_t)nmol + 1) * 8 + (size_t)ncoarse * 4 + 64));
     uint32_t *d_vpre = as<uint32_t>(d_off) + (nmol + 1);
-    qs_launch_mesh_bases(as<uint32_t>(vbw), as<uint32_t>(tbw), wpre, nw_total, nmol, as<uint32_t>(totals), d_vpre,
-                         as<uint64_t>(tpre_d), d_vpre + nmol + 1, ncoarse, stream);
+    if (nmol > 1) /* (the filter writes one molecule's) */
+        qs_launch_mesh_bases(as<uint32_t>(vbw), as<uint32_t>(tbw), wpre, nw_total, nmol, as<uint32_t>(totals), d_vpre,
+                             as<uint64_t>(tpre_d), d_vpre + nmol + 1, ncoarse, stream);
     QS_TRY(ensure(vert, (size_t)pool_v * 12));
     QS_TRY(ensure(vkey, (size_t)pool_v * 8));
     QS_TRY(ensure(tri, (size_t)pool_t * 12));
     /* every scanned word may be active */
     const uint32_t nact_max = (uint32_t)std::max<uint64_t>(scan_nw, 1);
     const uint32_t *counts = as<uint32_t>(totals);
-    /* Without stage timing the closest-atom pass (which reads only the unsmoothed vertices) runs
-       on the side stream beside the smoothing passes, and is joined before the filter (ev_side).
-       For one molecule the vertex kernel runs there too, before it, beside the triangle kernel
-       (the smoothing passes wait for the vertices, ev_vert): the 50,000-atom 0.2 A mesh 1.972 ->
-       1.956 ms, while a batch of 256 molecules was 0.4 % slower that way. */
-    const bool overlap = with_atoms && !tm.on;
-    const bool fork_vertices = overlap && nmol == 1;
+    /* The closest atoms in the vertex kernel save a launch and the vertices' way through memory, which
+       is 11 us of 45 on 10,007 atoms at 0.4 A; but that kernel has fewer waves in flight, and on
+       256 molecules at 0.5 A (24 M vertices) both passes together took 1.84 ms in one kernel and 1.72
+       in two, on 1M atoms at 0.5 A 0.783 and 0.772, on 200,000 at 0.3 A (4.5 M) 0.510 and 0.511. */
+    const bool fused = expect_v <= (1u << 20);
+    QsClosest near{};
+    if (with_atoms) {
+        QS_TRY(ensure(atom, (size_t)pool_v * 4));
+        ids_sorted = g_opt.atom_ids_sorted != 0;
+        near = QsClosest{as<uint32_t>(start), as<float4>(sx), as<int>(perm), ids_sorted ? 1 : 0, as<int>(atom)};
+    }
     qs_launch_mc_emit(as<QsMol>(d_mols), wpre, wcoarse, as<uint32_t>(alist), nact_max, as<uint32_t>(avb), as<uint32_t>(vstart),
                       pool_v, as<uint64_t>(s4), as<float>(field), as<uint64_t>(outm),
                       field_sparse ? as<uint64_t>(shellm) : nullptr, as<float>(vert), as<uint64_t>(vkey), as<uint32_t>(acb),
                       as<uint32_t>(tstart), pool_t, pool_t, as<uint64_t>(negm), as<uint32_t>(wcnt), as<uint32_t>(vbw),
-                      as<uint32_t>(tbw), as<uint64_t>(ntb), as<int>(tri), 0u, as<uint32_t>(deg_blk), as<uint32_t>(totals) + 3, counts, stream,
-                      fork_vertices ? side : stream, ev_emit, ev_vert, scan_nw != 0, expect_v);
+                      as<uint32_t>(tbw), as<uint64_t>(ntb), as<int>(tri), 0u, as<uint32_t>(deg_blk), as<uint32_t>(totals) + 3, counts,
+                      stream, with_atoms && fused ? &near : nullptr, scan_nw != 0, expect_v);
     QS_HIP(hipGetLastError());
-    vert_pending = fork_vertices;
     tm.mark("mc_emit");
-    if (with_atoms) {
-        QS_TRY(ensure(atom, (size_t)pool_v * 4));
-        hipStream_t cs = overlap ? side : stream;
-        if (overlap && !fork_vertices) {
-            QS_HIP(hipEventRecord(ev_emit, stream));
-            QS_HIP(hipStreamWaitEvent(side, ev_emit, 0));
-        }
-        ids_sorted = g_opt.atom_ids_sorted != 0;
-        qs_launch_closest_atom(as<QsMol>(d_mols), d_vpre, d_vpre + nmol + 1, as<uint32_t>(start), as<float4>(sx), as<int>(perm),
-                               as<float>(vert), pool_v, ids_sorted ? 1 : 0, as<int>(atom), counts + 1, expect_v, cs);
+    if (with_atoms && !fused) {
+        /* (beside the smoothing passes, which read the same vertices, unless stages are timed: 4.79
+           instead of 4.85 ms for the 256 molecules) */
+        if (!tm.on) QS_TRY(fork_side());
+        qs_launch_closest_atom(as<QsMol>(d_mols), d_vpre, nmol > 1 ? d_vpre + nmol + 1 : nullptr, near, as<float>(vert), pool_v,
+                               counts + 1, expect_v, side_pending ? side : stream);
         QS_HIP(hipGetLastError());
-        if (overlap) {
-            QS_HIP(hipEventRecord(ev_side, side));
-            side_pending = true;
-        }
+        if (side_pending) QS_HIP(hipEventRecord(ev_side, side));
         tm.mark("closest_atom");
     }
     return 0;
@@ -793,7 +814,7 @@ int Engine::slab_mesh(size_t at_mc, uint32_t nb_mc, size_t at_wpre, uint64_t own
     QS_TRY(ensure(tstart, ((size_t)n_tri / 256 + 1) * 4));
     QS_TRY(ensure(deg_blk, ((size_t)n_tri / 256 + 1) * 4));
     const uint64_t *wpre = (const uint64_t *)(as<uint32_t>(d_meta) + at_wpre);
-    const uint32_t *wcoarse = as<uint32_t>(d_meta) + at_wpre + 4;
+    const uint32_t *wcoarse = nullptr;
     qs_launch_mc_emit(as<QsMol>(d_mols), wpre, wcoarse, as<uint32_t>(alist), nact, as<uint32_t>(avb), as<uint32_t>(vstart),
                       n_owned, as<uint64_t>(s4), as<float>(field), as<uint64_t>(outm), as<uint64_t>(shellm),
                       as<float>(vert) + 3 * (size_t)vbase, as<uint64_t>(vkey), as<uint32_t>(acb), as<uint32_t>(tstart), hb[4], n_tri,
@@ -843,8 +864,7 @@ int Engine::run_slabs(int planes, int smooth, StageTimer &tm)
         uint32_t nb_atoms, nb_p1, nb_mc;
         QS_TRY(build_meta(at_atoms, at_p1, at_mc, at_wpre, nb_atoms, nb_p1, nb_mc));
         QS_TRY(ensure(d_meta, h_meta.size() * 4));
-        QS_TRY(upload(d_mols.p, mols.data(), sizeof(QsMol)));
-        QS_TRY(upload(d_meta.p, h_meta.data(), h_meta.size() * 4));
+        QS_TRY(upload_mols());
         QS_TRY(field_stage(nb_p1, at_p1, none));
         uint32_t n_owned = 0, n_tri = 0;
         QS_TRY(slab_mesh(at_mc, nb_mc, at_wpre, owned_word, (uint32_t)vbase, (uint32_t)tbase, n_owned, n_tri));
@@ -861,35 +881,19 @@ int Engine::run_slabs(int planes, int smooth, StageTimer &tm)
     M.n_tri = nt_all;
     vert_off.assign(2, 0);
     vert_off[1] = nv;
-    QS_TRY(upload(d_mols.p, mols.data(), sizeof(QsMol)));
-    std::vector<uint32_t> &vpre = h_vpre;
-    vpre.assign({0u, nv});
-    {
-        std::vector<uint32_t> vc;
-        append_coarse(vc, vpre.data(), 1, nv, QS_COARSE_ITEMS);
-        vpre.insert(vpre.end(), vc.begin(), vc.end());
-    }
-    QS_TRY(ensure(d_off, 2 * 4 + vpre.size() * 4 + 64));
-    uint32_t *d_vpre = as<uint32_t>(d_off) + 2;
-    QS_TRY(upload(d_vpre, vpre.data(), vpre.size() * 4));
+    QS_TRY(upload_mols());
+    QS_TRY(ensure(d_off, 4 * 4 + 64));
 
     /* closest atom per unsmoothed vertex, beside the smoothing passes unless stages are timed */
     /* (vert and tri already hold the whole mesh: grow_keep sized them) */
     QS_TRY(ensure(atom, (size_t)std::max<uint32_t>(nv, 1) * 4));
-    const bool overlap = !tm.on;
-    hipStream_t cs = overlap ? side : stream;
-    if (overlap) {
-        QS_HIP(hipEventRecord(ev_emit, stream));
-        QS_HIP(hipStreamWaitEvent(side, ev_emit, 0));
-    }
+    if (!tm.on) QS_TRY(fork_side());
     ids_sorted = g_opt.atom_ids_sorted != 0;
-    qs_launch_closest_atom(as<QsMol>(d_mols), d_vpre, d_vpre + 2, as<uint32_t>(start), as<float4>(sx), as<int>(perm),
-                           as<float>(vert), nv, ids_sorted ? 1 : 0, as<int>(atom), nullptr, nv, cs);
+    const QsClosest near{as<uint32_t>(start), as<float4>(sx), as<int>(perm), ids_sorted ? 1 : 0, as<int>(atom)};
+    qs_launch_closest_atom(as<QsMol>(d_mols), nullptr, nullptr, near, as<float>(vert), nv, nullptr, nv,
+                           side_pending ? side : stream);
     QS_HIP(hipGetLastError());
-    if (overlap) {
-        QS_HIP(hipEventRecord(ev_side, side));
-        side_pending = true;
-    }
+    if (side_pending) QS_HIP(hipEventRecord(ev_side, side));
     tm.mark("closest_atom");
 
     /* Laplacian passes (Jacobi) over the triangle array's incidences */
@@ -927,6 +931,10 @@ int Engine::run_batch(const float *d_pos, const float *d_rad, const std::vector<
     /* (inputs queued through the staging by upload_begin stay) */
     if (!inputs_staged) QS_TRY(upload_reset());
     inputs_staged = false;
+    if (side_pending) { /* a run that stopped before it joined its side stream */
+        QS_HIP(hipStreamSynchronize(side));
+        side_pending = false;
+    }
     batch_valid = false;
     nv = nt = nt_all = n_active = 0;
     res_vert = nullptr;
@@ -958,15 +966,17 @@ int Engine::run_batch(const float *d_pos, const float *d_rad, const std::vector<
         QS_TRY(ensure(bb_out, (size_t)nmol * 8 * sizeof(float)));
         uint32_t max_n = 0;
         for (int m = 0; m < nmol; m++) max_n = std::max(max_n, in[m].n);
-        const int parts = qs_bbox_parts(max_n);
+        const int parts = qs_bbox_parts(max_n, nmol);
         QS_TRY(ensure(bb_part, qs_bbox_part_floats(nmol, parts) * sizeof(float)));
         /* (one molecule's atom range goes in the launch's arguments) */
         if (nmol > 1) QS_TRY(upload(d_off.p, off.data(), (nmol + 1) * 4));
-        qs_launch_bbox(d_pos, d_rad, nmol > 1 ? as<uint32_t>(d_off) : nullptr, off[0], off[1], nmol, parts, as<float>(bb_part),
-                       as<float>(bb_out), stream);
+        /* the boxes go straight to the pinned staging: a copy would be another 8 us */
         std::vector<float> h((size_t)nmol * 8);
         float *hs = (float *)stage(h.size() * 4);
-        QS_HIP(hipMemcpyAsync(hs ? (void *)hs : (void *)h.data(), bb_out.p, h.size() * 4, hipMemcpyDeviceToHost, stream));
+        qs_launch_bbox(d_pos, d_rad, nmol > 1 ? as<uint32_t>(d_off) : nullptr, off[0], off[1], nmol, parts, as<float>(bb_part),
+                       hs ? hs : as<float>(bb_out), stream);
+        QS_HIP(hipGetLastError());
+        if (!hs) QS_HIP(hipMemcpyAsync(h.data(), bb_out.p, h.size() * 4, hipMemcpyDeviceToHost, stream));
         QS_HIP(hipStreamSynchronize(stream));
         if (hs) memcpy(h.data(), hs, h.size() * 4);
         for (int m = 0; m < nmol; m++) {
@@ -986,8 +996,7 @@ int Engine::run_batch(const float *d_pos, const float *d_rad, const std::vector<
     QS_TRY(build_meta(at_atoms, at_p1, at_mc, at_wpre, nb_atoms, nb_p1, nb_mc));
     QS_TRY(ensure(d_mols, mols.size() * sizeof(QsMol)));
     QS_TRY(ensure(d_meta, h_meta.size() * 4));
-    QS_TRY(upload(d_mols.p, mols.data(), mols.size() * sizeof(QsMol)));
-    QS_TRY(upload(d_meta.p, h_meta.data(), h_meta.size() * 4));
+    QS_TRY(upload_mols());
 
     /* ---- atoms into cells (CudaSurf.cu:594-622), global over the batch ---- */
     const uint32_t n = n_atoms_total;
@@ -1033,12 +1042,8 @@ int Engine::run_batch(const float *d_pos, const float *d_rad, const std::vector<
         if (smooth > 1) QS_TRY(ensure(vert3, (size_t)pool_v * 12));
         const float *src = as<float>(vert);
         float *dst = as<float>(vert2);
-        if (vert_pending) {
-            QS_HIP(hipStreamWaitEvent(stream, ev_vert, 0));
-            vert_pending = false;
-        }
         for (int it = 0; it < smooth; it++) {
-            qs_launch_smooth(as<QsMol>(d_mols), d_vpre, d_vpre + nmol + 1, as<uint64_t>(negm), as<uint64_t>(zerom), as<uint64_t>(s4),
+            qs_launch_smooth(as<QsMol>(d_mols), d_vpre, nmol > 1 ? d_vpre + nmol + 1 : nullptr, as<uint64_t>(negm), as<uint64_t>(zerom), as<uint64_t>(s4),
                              as<uint32_t>(vbw), as<uint64_t>(vkey), pool_v, as<uint64_t>(ntb), as<uint32_t>(tbw), as<int>(tri),
                              src, dst, as<uint32_t>(totals) + 1, expect_v, stream);
             src = dst;
@@ -1050,14 +1055,10 @@ int Engine::run_batch(const float *d_pos, const float *d_rad, const std::vector<
     }
     }
 
-    /* the closest-atom pass (after the vertex kernel on the same stream) joins the main stream */
+    /* a closest-atom pass on the side stream joins the main stream */
     if (side_pending) {
         QS_HIP(hipStreamWaitEvent(stream, ev_side, 0));
         side_pending = false;
-    }
-    if (vert_pending) {
-        QS_HIP(hipStreamWaitEvent(stream, ev_vert, 0));
-        vert_pending = false;
     }
 
     /* ---- degenerate filter (CudaSurf.cu:820-829), per-molecule kept counts ---- */
@@ -1075,26 +1076,31 @@ int Engine::run_batch(const float *d_pos, const float *d_rad, const std::vector<
         QS_HIP(hipMemsetAsync(as<uint32_t>(totals) + 3, 0, 4, stream));
         qs_launch_deg_count(as<int>(tri), nt_all, as<uint32_t>(deg_blk), as<uint32_t>(totals) + 3, stream);
         QS_HIP(hipGetLastError());
-        /* the molecule's first triangle and the end, for the kept counts */
-        h_bidx.assign({0ull, (uint64_t)nt_all});
-        QS_TRY(ensure(tpre_d, 2 * 8));
-        QS_TRY(upload(tpre_d.p, h_bidx.data(), 2 * 8));
     }
     QS_TRY(ensure(keeppos, (nblk_t + 1) * 4));
     QS_TRY(ensure(tri_out, (size_t)std::max<uint32_t>(tcap, 1) * 12));
-    QS_TRY(scan(as<uint32_t>(deg_blk), as<uint32_t>(keeppos), nblk_t, as<uint32_t>(keeppos) + nblk_t));
-    qs_launch_tri_compact(as<int>(tri), tcap, as<uint32_t>(keeppos), as<uint32_t>(totals) + 3, as<int>(tri_out),
-                          multi_slab ? nullptr : as<uint32_t>(totals), stream);
     QS_TRY(ensure(bounds, ((size_t)nmol + 1) * 8));
-    /* the run's one read-back, gathered by the last kernel: totals, per-molecule first vertices
-       and kept-triangle offsets */
+    /* the run's one read-back, gathered by the last kernel (straight into the pinned staging): totals,
+       per-molecule first vertices and kept-triangle offsets */
     std::vector<uint32_t> hb(4 + 2 * ((size_t)nmol + 1));
     QS_TRY(ensure(rback, hb.size() * 4));
-    qs_launch_tri_kept_before(as<int>(tri), as<uint32_t>(keeppos), as<uint64_t>(tpre_d), nmol + 1, tcap, as<uint32_t>(bounds),
-                              as<uint32_t>(totals), as<uint32_t>(d_off) + (nmol + 1), as<uint32_t>(rback), stream);
     uint32_t *fs = (uint32_t *)stage(hb.size() * 4);
-    uint32_t *fd = fs ? fs : hb.data();
-    QS_HIP(hipMemcpyAsync(fd, rback.p, hb.size() * 4, hipMemcpyDeviceToHost, stream));
+    uint32_t *rb = fs ? fs : as<uint32_t>(rback);
+    uint32_t *vpre = as<uint32_t>(d_off) + (nmol + 1);
+    /* a block of the compaction adds up the counts of up to TRI_SELF_BLOCKS blocks itself */
+    const bool self = nmol == 1 && nblk_t <= TRI_SELF_BLOCKS;
+    if (!self) QS_TRY(scan(as<uint32_t>(deg_blk), as<uint32_t>(keeppos), nblk_t, as<uint32_t>(keeppos) + nblk_t));
+    const uint32_t *dpre = self ? as<uint32_t>(deg_blk) : as<uint32_t>(keeppos);
+    if (nmol == 1) {
+        qs_launch_tri_compact_one(as<int>(tri), tcap, dpre, self, as<uint32_t>(totals), as<int>(tri_out),
+                                  multi_slab ? nullptr : as<uint32_t>(totals), nv, vpre, as<uint32_t>(bounds), rb, stream);
+    } else {
+        qs_launch_tri_compact(as<int>(tri), tcap, dpre, as<uint32_t>(totals), as<int>(tri_out), as<uint32_t>(totals), stream);
+        qs_launch_tri_kept_before(as<int>(tri), dpre, as<uint64_t>(tpre_d), nmol + 1, tcap, as<uint32_t>(bounds),
+                                  as<uint32_t>(totals), vpre, rb, stream);
+    }
+    QS_HIP(hipGetLastError());
+    if (!fs) QS_HIP(hipMemcpyAsync(hb.data(), rb, hb.size() * 4, hipMemcpyDeviceToHost, stream));
     QS_HIP(hipStreamSynchronize(stream));
     if (fs) memcpy(hb.data(), fs, hb.size() * 4);
     tm.mark("filter");
@@ -1780,7 +1786,7 @@ static int launch_normals(Engine &E, float *d_out)
     E.normals_used = true;
     const int nmol = (int)E.mols.size();
     const uint32_t *d_vpre = as<uint32_t>(E.d_off) + (nmol + 1);
-    qs_launch_vertex_normals(as<QsMol>(E.d_mols), d_vpre, d_vpre + nmol + 1, as<uint64_t>(E.vkey), E.nv, as<float>(E.field),
+    qs_launch_vertex_normals(as<QsMol>(E.d_mols), d_vpre, nmol > 1 ? d_vpre + nmol + 1 : nullptr, as<uint64_t>(E.vkey), E.nv, as<float>(E.field),
                              as<uint64_t>(E.outm),
                              E.field_sparse ? as<uint64_t>(E.shellm) : nullptr, d_out, E.stream);
     QS_HIP(hipGetLastError());
@@ -1838,7 +1844,7 @@ int qs_vertex_colors(const float *atom_rgba, unsigned int natoms, float *out, un
     QS_HIP(hipMemcpyAsync(E.colors_in.p, atom_rgba, (size_t)natoms * 16, hipMemcpyHostToDevice, E.stream));
     const int nmol = (int)E.mols.size();
     const uint32_t *d_vpre = as<uint32_t>(E.d_off) + (nmol + 1);
-    qs_launch_vertex_colors(as<QsMol>(E.d_mols), d_vpre, d_vpre + nmol + 1, E.res_atom, E.ids_sorted ? as<int>(E.perm) : nullptr,
+    qs_launch_vertex_colors(as<QsMol>(E.d_mols), d_vpre, nmol > 1 ? d_vpre + nmol + 1 : nullptr, E.res_atom, E.ids_sorted ? as<int>(E.perm) : nullptr,
                             E.nv, as<float4>(E.colors_in), as<float4>(E.normals), E.stream);
     QS_HIP(hipGetLastError());
     QS_HIP(hipMemcpyAsync(out, E.normals.p, (size_t)E.nv * 16, hipMemcpyDeviceToHost, E.stream));

@@ -10,8 +10,12 @@
 #include "qs_common.h"
 
 /* atoms into cells */
-/* bounding boxes: `parts` partial boxes per molecule (qs_bbox_parts of the largest atom count) */
-int qs_bbox_parts(uint32_t max_atoms);
+/* one molecule's record to the device, in the launch's arguments */
+void qs_launch_put_mol(const QsMol &m, QsMol *dst, hipStream_t s);
+
+/* bounding boxes: `parts` partial boxes per molecule (qs_bbox_parts of the largest atom count); out
+   may be pinned host memory */
+int qs_bbox_parts(uint32_t max_atoms, int nmol);
 size_t qs_bbox_part_floats(int nmol, int parts);
 /* off: per-molecule atom offsets (nmol + 1); or nullptr for one molecule of atoms [o0, o1) */
 void qs_launch_bbox(const float *pos, const float *rad, const uint32_t *off, uint32_t o0, uint32_t o1, int nmol, int parts,
@@ -87,23 +91,29 @@ void qs_launch_mc_count(QsBatch B, uint32_t nblocks, const uint64_t *N, const ui
    256 + 1 entries), unless starts_ready says that the word scans did (QsBlockStarts).  ncube: the
    cubes, or a bound on them.  The field F (grid order) holds shell voxels' values only, the others
    come from the outside / shell masks (shellm == nullptr: F holds every voxel).  cnt: the words'
-   packed counts; tbw: their first triangles.  Triangle corners are vertex ids plus vbase; degenerate triangles are counted per 256-triangle block
-   (deg_blk) and in total.  The block starts and the triangle kernel run on s;
-   the vertex kernel on s_vert: when that is another stream it waits there for the block starts
-   (event ev_fork), and ev_vert is recorded on s_vert after it. */
+   packed counts; tbw: their first triangles.  Triangle corners are vertex ids plus vbase; degenerate
+   triangles are counted per 256-triangle block (deg_blk) and in total.  atoms (may be NULL): the
+   vertices' closest atoms are written in the same pass.  Here and below wcoarse / vcoarse ==
+   nullptr: one molecule (the prefixes are not read). */
+struct QsClosest {
+    const uint32_t *cstart; /* the molecules' cell starts, with padding for column_starts */
+    const float4 *sx;
+    const int *perm;
+    int sorted_ids;
+    int *atom;
+};
 void qs_launch_mc_emit(const QsMol *mols, const uint64_t *wpre, const uint32_t *wcoarse, const uint32_t *list, uint32_t nact,
                        const uint32_t *avb, uint32_t *vstart, uint32_t nv, const uint64_t *S4, const float *F,
                        const uint64_t *outm, const uint64_t *shellm, float *vert, uint64_t *vkey,
                        const uint32_t *acb, uint32_t *tstart, uint32_t ncube, uint32_t ntri, const uint64_t *N, const uint32_t *cnt,
                        const uint32_t *vbw, const uint32_t *tbw, const uint64_t *NT, int *tri, uint32_t vbase, uint32_t *deg_blk,
-                       uint32_t *deg_total, const uint32_t *d_counts, hipStream_t s, hipStream_t s_vert = nullptr,
-                       hipEvent_t ev_fork = nullptr, hipEvent_t ev_vert = nullptr, bool starts_ready = false,
-                       uint32_t expect = ~0u);
+                       uint32_t *deg_total, const uint32_t *d_counts, hipStream_t s, const QsClosest *atoms = nullptr,
+                       bool starts_ready = false, uint32_t expect = ~0u);
 
 /* Launches whose item counts live on the device take them from the d_* pointers (when given),
    the host counts being the pools the launch covers: marching-cubes totals are counts[0]
-   triangles, counts[1] vertices, counts[2] active words, counts[4] cubes.    expect: items to launch blocks for
-   (at most the host count's); if there are more, the blocks loop. */
+   triangles, counts[1] vertices, counts[2] active words, counts[4] cubes.  expect: items to launch
+   blocks for (at most the host count's); if there are more, the blocks loop. */
 
 /* per-molecule first vertex (vpre, u32) and first triangle (tpre, u64) from the word scans at each
    molecule's first word (wpre[m]; at or past the nw scanned words for none), nmol + 1 entries
@@ -112,10 +122,8 @@ void qs_launch_mesh_bases(const uint32_t *vbw, const uint32_t *tbw, const uint64
                           const uint32_t *counts, uint32_t *vpre, uint64_t *tpre, uint32_t *vcoarse, uint32_t ncoarse, hipStream_t s);
 
 /* per-vertex stages */
-void qs_launch_closest_atom(const QsMol *mols, const uint32_t *vpre, const uint32_t *vcoarse, const uint32_t *cstart,
-                            const float4 *sx,
-                            const int *perm, const float *vert, uint32_t nv, int sorted_ids, int *out, const uint32_t *d_nv,
-                            uint32_t expect, hipStream_t s);
+void qs_launch_closest_atom(const QsMol *mols, const uint32_t *vpre, const uint32_t *vcoarse, const QsClosest &A,
+                            const float *vert, uint32_t nv, const uint32_t *d_nv, uint32_t expect, hipStream_t s);
 void qs_launch_smooth(const QsMol *mols, const uint32_t *vpre, const uint32_t *vcoarse, const uint64_t *N, const uint64_t *Zm,
                       const uint64_t *S4, const uint32_t *vbw, const uint64_t *vkey, uint32_t nv,
                       const uint64_t *NT, const uint32_t *tbw, const int *tri, const float *src, float *dst,
@@ -143,12 +151,20 @@ void qs_launch_vertex_normals(const QsMol *mols, const uint32_t *vpre, const uin
 void qs_launch_vertex_colors(const QsMol *mols, const uint32_t *vpre, const uint32_t *vcoarse, const int *atom,
                              const int *perm, uint32_t nv, const float4 *table, float4 *out, hipStream_t s);
 /* degenerate-triangle filter: dpre = exclusive prefix of the per-256-triangle-block degenerate
-   counts that the triangle kernel leaves, ndeg their total (device); with ndeg == 0 the compaction
+   counts that the triangle kernel leaves, totals[3] their total (device); if that is 0 the compaction
    writes nothing */
-void qs_launch_tri_compact(const int *tri, uint32_t nt, const uint32_t *dpre, const uint32_t *ndeg, int *out,
+void qs_launch_tri_compact(const int *tri, uint32_t nt, const uint32_t *dpre, const uint32_t *totals, int *out,
                            const uint32_t *d_nt, hipStream_t s);
+/* the same for one molecule, with the run's read-back {totals[0..3], vpre[0..1], kept[0..1]} in rb
+   (device or pinned host memory) and its last two pairs in vpre and kept, so that no other launch
+   follows.  self: dpre is the per-block counts themselves, at most TRI_SELF_BLOCKS of them; nv, nt:
+   the mesh's counts if d_nt is nullptr */
+#define TRI_SELF_BLOCKS 2048u
+void qs_launch_tri_compact_one(const int *tri, uint32_t nt, const uint32_t *dpre, bool self, const uint32_t *totals, int *out,
+                               const uint32_t *d_nt, uint32_t nv, uint32_t *vpre, uint32_t *kept, uint32_t *rb, hipStream_t s);
 /* kept triangles before each of n boundaries (idx, triangle ids) into out; with rb also the run's
-   read-back gathered in one array: {totals[0..3], vpre[0..n), out[0..n)} */
+   read-back gathered in one array (device or pinned host memory): {totals[0..3], vpre[0..n),
+   out[0..n)} */
 void qs_launch_tri_kept_before(const int *tri, const uint32_t *dpre, const uint64_t *idx, int n, uint32_t tcap, uint32_t *out,
                                const uint32_t *totals, const uint32_t *vpre, uint32_t *rb, hipStream_t s);
 void qs_launch_tri_localize(const int *tri, uint32_t nt, const uint32_t *tpre, const uint32_t *vpre, int nmol, int *out,

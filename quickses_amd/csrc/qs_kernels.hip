@@ -167,6 +167,10 @@ __device__ __forceinline__ uint32_t xcd_group_rt(uint32_t b, uint32_t nb, uint32
 /* molecule of block b of a batched launch, and the block's index inside the molecule */
 __device__ __forceinline__ int batch_mol(const QsBatch &B, uint32_t b, uint32_t &local)
 {
+    if (!B.coarse) { /* one molecule: mols[0] */
+        local = b;
+        return 0;
+    }
     const int j = seg_coarse<QS_COARSE_BLOCKS>(B.bpre, B.coarse, b);
     local = b - B.bpre[j];
     return B.mid ? B.mid[j] : j;
@@ -185,9 +189,11 @@ __device__ __forceinline__ int seg_of(const uint32_t *__restrict__ pre, int n, u
 }
 
 /* segment of v for a wavefront whose items usually share one: the first active lane's segment
-   is found with scalar loads, the others fall back to their own lookup */
+   is found with scalar loads, the others fall back to their own lookup (coarse == nullptr: one
+   segment) */
 __device__ __forceinline__ int seg_of_wave(const uint32_t *__restrict__ pre, const uint32_t *__restrict__ coarse, uint32_t v)
 {
+    if (!coarse) return 0;
     const uint32_t v0 = __builtin_amdgcn_readfirstlane(v);
     const int m0 = __builtin_amdgcn_readfirstlane(seg_coarse<QS_COARSE_ITEMS>(pre, coarse, v0));
     if (v >= pre[m0] && v < pre[m0 + 1]) return m0;
@@ -658,48 +664,68 @@ __device__ __forceinline__ void bb_combine(float *v, const float *w)
     v[7] += w[7];
 }
 
-/* block (p, m) of P partial boxes per molecule: atoms off[m] + p*BB_NT + k*P*BB_NT + t of molecule m
-   -> part[m][p] (off == nullptr: one molecule, atoms [o0, o1)) */
-__global__ void __launch_bounds__(BB_NT) k_bbox_part(const float *__restrict__ pos, const float *__restrict__ rad,
-                                                     const uint32_t *__restrict__ off, uint32_t o0, uint32_t o1,
-                                                     float *__restrict__ part)
+/* the wave's lanes combined (minima, maxima and a sum of small integer counts: the same box in any
+   order) */
+__device__ __forceinline__ void bb_wave(float *v)
 {
-    const uint32_t P = gridDim.x;
-    __shared__ float s[BB_NV][BB_NT];
-    const int m = blockIdx.y, p = blockIdx.x;
-    float v[BB_NV] = {100000.0f, 100000.0f, 100000.0f, -100000.0f, -100000.0f, -100000.0f, 0.0f, 0.0f};
-    const uint32_t beg = off ? off[m] : o0, end = off ? off[m + 1] : o1;
-    for (uint32_t i = beg + p * BB_NT + threadIdx.x; i < end; i += P * BB_NT) {
-        for (int c = 0; c < 3; c++) {
-            float q = pos[3 * (size_t)i + c];
-            v[c] = fminf(v[c], q);
-            v[3 + c] = fmaxf(v[3 + c], q);
-            if (!isfinite(q)) v[7] += 1.0f;
-        }
-        float ra = rad[i];
-        v[6] = fmaxf(v[6], ra);
-        if (!isfinite(ra)) v[7] += 1.0f;
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) {
+        float w[BB_NV];
+#pragma unroll
+        for (int c = 0; c < BB_NV; c++) w[c] = __shfl_xor(v[c], d, 64);
+        bb_combine(v, w);
     }
-    for (int c = 0; c < BB_NV; c++) s[c][threadIdx.x] = v[c];
-    __syncthreads();
-    for (int st = BB_NT / 2; st > 0; st >>= 1) {
-        if ((int)threadIdx.x < st) {
-            float w[BB_NV];
-            for (int c = 0; c < BB_NV; c++) {
-                v[c] = s[c][threadIdx.x];
-                w[c] = s[c][threadIdx.x + st];
-            }
-            bb_combine(v, w);
-            for (int c = 0; c < BB_NV; c++) s[c][threadIdx.x] = v[c];
-        }
-        __syncthreads();
-    }
-    if (threadIdx.x < BB_NV) part[((size_t)m * P + p) * BB_NV + threadIdx.x] = s[threadIdx.x][0];
 }
 
-/* one wavefront per molecule: combine its P partial boxes, lane k taking partials k, k + 64, ...,
-   then across the lanes (minima, maxima and a sum of small integer counts: the same box in any
-   order) */
+/* block (p, m) of P partial boxes per molecule: atoms off[m] + p*NT + k*P*NT + t of molecule m ->
+   part[m][p] (off == nullptr: one molecule, atoms [o0, o1)).  Bound by the latency of its loads:
+   four atoms per thread are in flight. */
+template <int NT>
+__global__ void __launch_bounds__(NT) k_bbox_part(const float *__restrict__ pos, const float *__restrict__ rad,
+                                                  const uint32_t *__restrict__ off, uint32_t o0, uint32_t o1,
+                                                  float *__restrict__ part)
+{
+    const uint32_t P = gridDim.x;
+    __shared__ float s[NT / 64][BB_NV];
+    const int m = blockIdx.y, p = blockIdx.x, lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    float v[BB_NV] = {100000.0f, 100000.0f, 100000.0f, -100000.0f, -100000.0f, -100000.0f, 0.0f, 0.0f};
+    const uint32_t beg = off ? off[m] : o0, end = off ? off[m + 1] : o1;
+    for (uint32_t i0 = beg + p * NT + threadIdx.x; i0 < end; i0 += 4 * P * NT) {
+        float q[4][4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            /* (past the end the thread's first atom again; 32-bit wrap-around included) */
+            const uint32_t j = i0 + k * P * NT, i = (j < end && j >= i0) ? j : i0;
+#pragma unroll
+            for (int c = 0; c < 3; c++) q[k][c] = pos[3 * (size_t)i + c];
+            q[k][3] = rad[i];
+        }
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+#pragma unroll
+            for (int c = 0; c < 3; c++) {
+                v[c] = fminf(v[c], q[k][c]);
+                v[3 + c] = fmaxf(v[3 + c], q[k][c]);
+                if (!isfinite(q[k][c])) v[7] += 1.0f;
+            }
+            v[6] = fmaxf(v[6], q[k][3]);
+            if (!isfinite(q[k][3])) v[7] += 1.0f;
+        }
+        if (i0 + 4 * P * NT < i0) break; /* (the index would wrap around) */
+    }
+    bb_wave(v);
+    if (lane == 0)
+        for (int c = 0; c < BB_NV; c++) s[wid][c] = v[c];
+    __syncthreads();
+    if (threadIdx.x < BB_NV) {
+        const int c = threadIdx.x;
+        float r = s[0][c];
+        for (int w = 1; w < NT / 64; w++) r = c < 3 ? fminf(r, s[w][c]) : (c < 7 ? fmaxf(r, s[w][c]) : r + s[w][c]);
+        part[((size_t)m * P + p) * BB_NV + c] = r;
+    }
+}
+
+/* one wavefront per molecule: combine its P partial boxes, lane k taking partials k, k + 64, ... */
 __global__ void __launch_bounds__(64) k_bbox_final(const float *__restrict__ part, int P, float *__restrict__ out)
 {
     const int m = blockIdx.x, lane = threadIdx.x;
@@ -710,13 +736,7 @@ __global__ void __launch_bounds__(64) k_bbox_final(const float *__restrict__ par
         for (int c = 0; c < BB_NV; c++) w[c] = part[((size_t)m * P + p) * BB_NV + c];
         bb_combine(v, w);
     }
-#pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) {
-        float w[BB_NV];
-#pragma unroll
-        for (int c = 0; c < BB_NV; c++) w[c] = __shfl_xor(v[c], d, 64);
-        bb_combine(v, w);
-    }
+    bb_wave(v);
     if (lane < BB_NV) {
         float r = v[0];
 #pragma unroll
@@ -2688,9 +2708,12 @@ __device__ __forceinline__ void stage_item_words(ItemWords &S, const uint32_t *_
     if (threadIdx.x == 0) {
         S.k0 = k0;
         S.nk = nk;
-        const int m0 = seg_coarse<QS_COARSE_ITEMS>(wpre, wcoarse, (uint64_t)list[k0]);
-        const int m1 = seg_coarse<QS_COARSE_ITEMS>(wpre, wcoarse, (uint64_t)list[k1]);
-        S.mol = (m0 == m1) ? m0 : -1;
+        S.mol = 0;
+        if (wcoarse) { /* (nullptr: one molecule) */
+            const int m0 = seg_coarse<QS_COARSE_ITEMS>(wpre, wcoarse, (uint64_t)list[k0]);
+            const int m1 = seg_coarse<QS_COARSE_ITEMS>(wpre, wcoarse, (uint64_t)list[k1]);
+            S.mol = (m0 == m1) ? m0 : -1;
+        }
     }
     if (nk <= 257u)
         for (uint32_t t = threadIdx.x; t < nk; t += 256) {
@@ -2758,240 +2781,6 @@ void qs_launch_field_expand(const float *F, const uint64_t *outm, const uint64_t
     const size_t n = (size_t)g * g * W;
     if (!n) return;
     k_field_expand<<<(unsigned)((n + 3) / 4), 256, 0, s>>>(F, outm, shellm, out, g, W, dx);
-}
-
-/* vertices (vertexInterp/lerp MarchingCubes.cu:715-734, edge oriented low->high), one thread per
-   vertex: its word from the active words' first vertex ids, its point and slot from the word's
-   four slot masks (vertex ids run over the word's points in z order, slots x, y, z, point) */
-__global__ void __launch_bounds__(256) k_mc_vertices(const QsMol *__restrict__ mols, const uint64_t *__restrict__ wpre,
-                                                     const uint32_t *__restrict__ wcoarse, const uint32_t *__restrict__ list,
-                                                     const uint32_t *__restrict__ avb, const uint32_t *__restrict__ vstart,
-                                                     uint32_t nact, uint32_t nv, const uint64_t *__restrict__ S4_all,
-                                                     const float *__restrict__ F_all, const uint64_t *__restrict__ outm_all,
-                                                     const uint64_t *__restrict__ shellm_all, float *__restrict__ vert,
-                                                     uint64_t *__restrict__ vkey, const uint32_t *__restrict__ d_counts)
-{
-    __shared__ ItemWords S;
-    /* with d_counts (triangles, vertices, active words) the counts come from the device, the
-       launch covering the pool of nv vertices: blocks past the count leave at once */
-    if (d_counts) {
-        nact = d_counts[2];
-        nv = min(d_counts[1], nv);
-    }
-    const uint32_t nb = (nv + 255u) >> 8;
-    /* persistent blocks over the 256-vertex blocks; the grid is a multiple of 8, so block vb runs
-       on XCD vb % 8 and the renumbering keeps neighbouring rows' words on one L2 */
-    for (uint32_t vb = blockIdx.x; vb < nb; vb += gridDim.x) {
-    const uint32_t blk = xcd_group<64>(vb, nb);
-    stage_item_words(S, avb, list, vstart, nact, nb, blk, wpre, wcoarse);
-    const uint32_t v = blk * 256u + threadIdx.x;
-    if (v < nv) {
-    uint32_t k, wi, first;
-    item_word(S, avb, list, v, k, wi, first);
-    const uint32_t local = v - first;
-    const QsMol &M = mols[S.mol >= 0 ? S.mol : seg_coarse<QS_COARSE_ITEMS>(wpre, wcoarse, (uint64_t)wi)];
-    const QsGrid G = M.G;
-    const int g = G.g;
-    int x, y, w;
-    decode_word((uint32_t)(wi - M.word_off), g, (int)M.W, x, y, w);
-    const uint64_t *__restrict__ m = S4_all + 4 * (size_t)wi;
-    const uint64_t m0 = m[0], m1 = m[1], m2 = m[2], m3 = m[3];
-    /* the point: smallest b whose slots below b + 1 exceed local */
-    int lo = 0, hi = 63;
-    while (lo < hi) {
-        const int mid = (lo + hi) >> 1;
-        const uint64_t below = (2ull << mid) - 1ull;
-        const uint32_t c = (uint32_t)(__popcll(m0 & below) + __popcll(m1 & below) + __popcll(m2 & below) + __popcll(m3 & below));
-        if (c > local) hi = mid;
-        else lo = mid + 1;
-    }
-    const int b = lo;
-    const uint64_t below = (1ull << b) - 1ull;
-    uint32_t r = local - (uint32_t)(__popcll(m0 & below) + __popcll(m1 & below) + __popcll(m2 & below) + __popcll(m3 & below));
-    const uint32_t bits = (uint32_t)((m0 >> b) & 1ull) | (uint32_t)((m1 >> b) & 1ull) << 1 |
-                          (uint32_t)((m2 >> b) & 1ull) << 2 | (uint32_t)((m3 >> b) & 1ull) << 3;
-    uint32_t bb = bits;
-    while (r) {
-        bb &= bb - 1u;
-        r--;
-    }
-    const int sl = bb ? __builtin_ctz(bb) : 3;
-    const int z = w * 64 + b;
-    const float dx = G.dx;
-    const size_t pidx = ((size_t)x * g + y) * g + z;
-    const float A[3] = {grid_pos(G.ox, x, dx), grid_pos(G.oy, y, dx), grid_pos(G.oz, z, dx)};
-    float P[3] = {A[0], A[1], A[2]};
-    if (sl < 3) {
-        const float *__restrict__ F = F_all + M.vox_off;
-        const uint64_t *__restrict__ om = outm_all + M.word_off;
-        const uint64_t *__restrict__ sm = shellm_all ? shellm_all + M.word_off : nullptr;
-        const size_t row = (size_t)x * g + y;
-        const int W = (int)M.W;
-        const float f0 = field_at(F, om, sm, row, g, W, z, dx);
-        const float f1 = field_at(F, om, sm, row + (sl == 0 ? (size_t)g : (sl == 1 ? 1 : 0)), g, W, z + (sl == 2), dx);
-        float B[3] = {A[0], A[1], A[2]};
-        B[sl] = A[sl] + dx;
-        const float t = (0.0f - f0) / (f1 - f0);
-#pragma unroll
-        for (int c3 = 0; c3 < 3; c3++) {
-            float dd = B[c3] - A[c3];
-            float s = t * dd;
-            P[c3] = A[c3] + s;
-        }
-    }
-    vert[3 * (size_t)v + 0] = P[0];
-    vert[3 * (size_t)v + 1] = P[1];
-    vert[3 * (size_t)v + 2] = P[2];
-    vkey[v] = ((uint64_t)pidx << 2) | (uint64_t)sl;
-    }
-    __syncthreads(); /* S is staged again for the next block */
-    }
-}
-
-/* triangles (generateTriangleVerticesSMEM MarchingCubes.cu:736-851 order), one thread per
-   polygonised cube (two triangles on average): its word from the active words' first cubes, its
-   place from the word's triangle-count planes.  Bound by the dependent memory trips of a block
-   (block start, word list, planes, corner masks) and by VALU issue, so both are paid once per cube:
-   the thread loads the sign words, slot masks and vertex counts of the cube's four (x, y) columns
-   together, and every corner's vertex id comes from them.  One thread per triangle, three corners'
-   masks each, took 0.20 ms on the 50,000-atom 0.2 A mesh and 0.92 ms on 256 molecules at 0.5 A
-   (47 M triangles); this takes 0.15 and 0.62 ms.  (64 registers for eight waves per SIMD, with
-   spills, were slower than 66 with seven: emission 1.11 against 1.06 ms.) */
-__global__ void __launch_bounds__(256) k_mc_triangles(const QsMol *__restrict__ mols, const uint64_t *__restrict__ wpre,
-                                                      const uint32_t *__restrict__ wcoarse, const uint32_t *__restrict__ list,
-                                                      const uint32_t *__restrict__ acb, const uint32_t *__restrict__ tstart,
-                                                      uint32_t nact, uint32_t ncube, uint32_t ntri, const uint64_t *__restrict__ N,
-                                                      const uint64_t *__restrict__ S4, const uint32_t *__restrict__ cnt,
-                                                      const uint32_t *__restrict__ vbw, const uint32_t *__restrict__ tbw,
-                                                      const uint64_t *__restrict__ NT, int *__restrict__ tri, uint32_t vbase,
-                                                      uint32_t *__restrict__ deg_blk, uint32_t *__restrict__ deg_total,
-                                                      const uint32_t *__restrict__ d_counts)
-{
-    __shared__ ItemWords S;
-    __shared__ uint32_t S_before[4][256]; /* per cube: vertices before its four columns' lower points */
-    /* counts from the device as in k_mc_vertices; triangles past the pool are not written */
-    if (d_counts) {
-        nact = d_counts[2];
-        ncube = min(d_counts[4], ncube);
-    }
-    const uint32_t nb = (ncube + 255u) >> 8;
-    /* persistent blocks over the 256-cube blocks, as in k_mc_vertices */
-    for (uint32_t vb = blockIdx.x; vb < nb; vb += gridDim.x) {
-    const uint32_t blk = xcd_group<64>(vb, nb);
-    stage_item_words(S, acb, list, tstart, nact, nb, blk, wpre, wcoarse);
-    const uint32_t cube = blk * 256u + threadIdx.x;
-    /* sl: the vertex slots of the eight corners, byte q = x | y << 1 for the column, bit
-       2 slot + z in it; has: the columns whose words own vertices (the masks of others are not
-       written, and only an edge that ends in a zero point asks for them) */
-    uint32_t first_tri = 0, nt = 0, sl = 0, has = 0, cs = 0;
-    uint64_t table = 0;
-    if (cube < ncube) {
-        uint32_t k, wi, first;
-        item_word(S, acb, list, cube, k, wi, first);
-        const QsMol &M = mols[S.mol >= 0 ? S.mol : seg_coarse<QS_COARSE_ITEMS>(wpre, wcoarse, (uint64_t)wi)];
-        const size_t W = M.W, gW = (size_t)M.G.g * W;
-        const uint64_t p0 = NT[3 * (size_t)wi], p1 = NT[3 * (size_t)wi + 1], p2 = NT[3 * (size_t)wi + 2];
-        const int b = nth_bit(p0 | p1 | p2, cube - first);
-        const uint64_t below = (1ull << b) - 1ull;
-        first_tri = tbw[wi] + (uint32_t)(__popcll(p0 & below) + 2 * __popcll(p1 & below) + 4 * __popcll(p2 & below));
-        nt = (uint32_t)((p0 >> b) & 1ull) + 2u * (uint32_t)((p1 >> b) & 1ull) + 4u * (uint32_t)((p2 >> b) & 1ull);
-        uint64_t s[4][4], nw[4];
-        uint32_t vb4[4], nv4[4];
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-            const size_t cw = wi + (q & 1 ? gW : 0) + (q & 2 ? W : 0);
-            nw[q] = N[cw];
-            nv4[q] = word_verts(cnt[cw]);
-            vb4[q] = vbw[cw];
-#pragma unroll
-            for (int a = 0; a < 4; a++) s[q][a] = S4[4 * cw + a];
-        }
-        uint32_t sg = 0; /* sign bits, bit 2 q + z */
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-            uint32_t m = 0, before = vb4[q];
-#pragma unroll
-            for (int a = 0; a < 4; a++) {
-                before += (uint32_t)__popcll(s[q][a] & below);
-                m |= ((uint32_t)(s[q][a] >> b) & 3u) << (2 * a);
-            }
-            S_before[q][threadIdx.x] = before;
-            sl |= m << (8 * q);
-            has |= (nv4[q] ? 1u : 0u) << q;
-            sg |= ((uint32_t)(nw[q] >> b) & 3u) << (2 * q);
-        }
-        if (b == 63) { /* the cube's top corners are in the next words */
-#pragma unroll
-            for (int q = 0; q < 4; q++) {
-                const size_t cw = wi + (q & 1 ? gW : 0) + (q & 2 ? W : 0) + 1;
-                sg |= (uint32_t)(N[cw] & 1ull) << (2 * q + 1);
-                uint32_t m = 0;
-#pragma unroll
-                for (int a = 0; a < 4; a++) m |= (uint32_t)(S4[4 * cw + a] & 1ull) << (2 * a + 1);
-                if (word_verts(cnt[cw])) {
-                    /* (a word without vertices below has none of its own slots set) */
-                    sl = (has >> q) & 1u ? sl : sl & ~(255u << (8 * q));
-                    if (!((has >> q) & 1u)) S_before[q][threadIdx.x] = vbw[cw];
-                    has |= 1u << q;
-                    sl |= m << (8 * q);
-                }
-            }
-        }
-        /* the table's corner order goes round the (x, y) columns 00, 10, 11, 01 */
-        const uint32_t lo4 = (sg & 1u) | (sg >> 1 & 2u) | (sg >> 4 & 4u) | (sg >> 1 & 8u);
-        const uint32_t hi4 = (sg >> 1 & 1u) | (sg >> 2 & 2u) | (sg >> 5 & 4u) | (sg >> 2 & 8u);
-        cs = lo4 | hi4 << 4;
-        table = c_tri[cs];
-    }
-#pragma unroll 1
-    for (uint32_t j = 0; j < 5u; j++) {
-        const bool on = j < nt && first_tri + j < ntri;
-        if (!__ballot(on)) break;
-        uint32_t c[3] = {0u, 1u, 2u};
-        const uint32_t t = first_tri + j;
-        if (on) {
-            const uint32_t corners = (uint32_t)(table >> (12u * j));
-#pragma unroll
-            for (int i = 0; i < 3; i++) {
-                const uint32_t e = (corners >> (4 * i)) & 15u;
-                const uint32_t d = (uint32_t)(kEdgePacked >> (5u * e));
-                uint32_t z = d & 1u, q = (d >> 1) & 3u, a2 = (d >> 2) & 6u; /* a2 = 2 axis */
-                uint32_t at = 8u * q + z;                                    /* the corner's slot 0 */
-                if (!((sl >> (at + a2)) & (has >> q) & 1u)) {
-                    /* the edge has no vertex of its own: its non-negative end is exactly zero and
-                       is the vertex (the point slot, after the point's edges) */
-                    if ((cs >> (4 * z + (q ^ (q >> 1)))) & 1u) {
-                        q |= (a2 == 0 ? 1u : 0u) | (a2 == 2 ? 2u : 0u);
-                        z |= a2 == 4 ? 1u : 0u;
-                        at = 8u * q + z;
-                    }
-                    a2 = 6u;
-                }
-                /* the corner's slots below this one, and all slots of the corner below it */
-                const uint32_t lower = __builtin_amdgcn_ubfe(sl, at, a2) & 0x55u;
-                const uint32_t under = __builtin_amdgcn_ubfe(sl, 8u * q, 8u * z) & 0x55u;
-                c[i] = vbase + S_before[q][threadIdx.x] + (uint32_t)(__popc(lower) + __popc(under));
-            }
-            tri[3 * (size_t)t + 0] = (int)c[0];
-            tri[3 * (size_t)t + 1] = (int)c[1];
-            tri[3 * (size_t)t + 2] = (int)c[2];
-        }
-        /* triangles with a repeated corner (zero grid points) are dropped from the output
-           (CudaSurf.cu:820-829): counted here per 256-triangle block and in total */
-        uint64_t dm = __ballot(c[0] == c[1] || c[1] == c[2] || c[0] == c[2]);
-        if (dm) {
-            if ((threadIdx.x & 63) == (uint32_t)__builtin_ctzll(dm)) atomicAdd(deg_total, (uint32_t)__popcll(dm));
-            while (dm) {
-                const uint32_t lead = (uint32_t)__builtin_ctzll(dm);
-                const uint32_t tb = (uint32_t)__shfl((int)(t >> 8), (int)lead, 64);
-                const uint64_t same = __ballot((t >> 8) == tb) & dm;
-                if ((threadIdx.x & 63) == lead) atomicAdd(&deg_blk[tb], (uint32_t)__popcll(same));
-                dm &= ~same;
-            }
-        }
-    }
-    __syncthreads(); /* S is staged again for the next block */
-    }
 }
 
 /* ------------------------------------------------------------------------------------------ */
@@ -3160,10 +2949,8 @@ __device__ __forceinline__ int closest_one(const QsMol &M, float px, float py, f
 }
 
 __global__ void __launch_bounds__(256) k_closest_atom(const QsMol *__restrict__ mols, const uint32_t *__restrict__ vpre,
-                                                      const uint32_t *__restrict__ vcoarse, const uint32_t *__restrict__ cstart_all,
-                                                      const float4 *__restrict__ sx, const int *__restrict__ perm,
-                                                      const float *__restrict__ vert, uint32_t nv, int sorted_ids,
-                                                      int *__restrict__ out, const uint32_t *__restrict__ d_nv)
+                                                      const uint32_t *__restrict__ vcoarse, const float *__restrict__ vert,
+                                                      uint32_t nv, const uint32_t *__restrict__ d_nv, QsClosest A)
 {
     if (d_nv) nv = min(*d_nv, nv); /* the device count within the launch's pool */
     const uint32_t nb = (nv + 255u) >> 8;
@@ -3172,8 +2959,246 @@ __global__ void __launch_bounds__(256) k_closest_atom(const QsMol *__restrict__ 
         const uint32_t v = xcd_group<64>(vb, nb) * 256u + threadIdx.x;
         if (v >= nv) continue;
         const QsMol &M = mols[seg_of_wave(vpre, vcoarse, v)];
-        out[v] = closest_one(M, vert[3 * (size_t)v], vert[3 * (size_t)v + 1], vert[3 * (size_t)v + 2], cstart_all, sx, perm,
-                             sorted_ids);
+        A.atom[v] = closest_one(M, vert[3 * (size_t)v], vert[3 * (size_t)v + 1], vert[3 * (size_t)v + 2], A.cstart, A.sx, A.perm,
+                                A.sorted_ids);
+    }
+}
+
+/* ------------------------------------------------------------------------------------------ */
+/* vertices (vertexInterp/lerp MarchingCubes.cu:715-734, edge oriented low->high), one thread per
+   vertex: its word from the active words' first vertex ids, its point and slot from the word's
+   four slot masks (vertex ids run over the word's points in z order, slots x, y, z, point).
+   ATOMS: the vertex's closest atom in the same pass (A). */
+template <bool ATOMS>
+__global__ void __launch_bounds__(256) k_mc_vertices(const QsMol *__restrict__ mols, const uint64_t *__restrict__ wpre,
+                                                     const uint32_t *__restrict__ wcoarse, const uint32_t *__restrict__ list,
+                                                     const uint32_t *__restrict__ avb, const uint32_t *__restrict__ vstart,
+                                                     uint32_t nact, uint32_t nv, const uint64_t *__restrict__ S4_all,
+                                                     const float *__restrict__ F_all, const uint64_t *__restrict__ outm_all,
+                                                     const uint64_t *__restrict__ shellm_all, float *__restrict__ vert,
+                                                     uint64_t *__restrict__ vkey, const uint32_t *__restrict__ d_counts, QsClosest A)
+{
+    __shared__ ItemWords S;
+    /* with d_counts (triangles, vertices, active words) the counts come from the device, the
+       launch covering the pool of nv vertices: blocks past the count leave at once */
+    if (d_counts) {
+        nact = d_counts[2];
+        nv = min(d_counts[1], nv);
+    }
+    const uint32_t nb = (nv + 255u) >> 8;
+    /* persistent blocks over the 256-vertex blocks; the grid is a multiple of 8, so block vb runs
+       on XCD vb % 8 and the renumbering keeps neighbouring rows' words on one L2 */
+    for (uint32_t vb = blockIdx.x; vb < nb; vb += gridDim.x) {
+    const uint32_t blk = xcd_group<64>(vb, nb);
+    stage_item_words(S, avb, list, vstart, nact, nb, blk, wpre, wcoarse);
+    const uint32_t v = blk * 256u + threadIdx.x;
+    if (v < nv) {
+    uint32_t k, wi, first;
+    item_word(S, avb, list, v, k, wi, first);
+    const uint32_t local = v - first;
+    const QsMol &M = mols[S.mol >= 0 ? S.mol : seg_coarse<QS_COARSE_ITEMS>(wpre, wcoarse, (uint64_t)wi)];
+    const QsGrid G = M.G;
+    const int g = G.g;
+    int x, y, w;
+    decode_word((uint32_t)(wi - M.word_off), g, (int)M.W, x, y, w);
+    const uint64_t *__restrict__ m = S4_all + 4 * (size_t)wi;
+    const uint64_t m0 = m[0], m1 = m[1], m2 = m[2], m3 = m[3];
+    /* the point: smallest b whose slots below b + 1 exceed local */
+    int lo = 0, hi = 63;
+    while (lo < hi) {
+        const int mid = (lo + hi) >> 1;
+        const uint64_t below = (2ull << mid) - 1ull;
+        const uint32_t c = (uint32_t)(__popcll(m0 & below) + __popcll(m1 & below) + __popcll(m2 & below) + __popcll(m3 & below));
+        if (c > local) hi = mid;
+        else lo = mid + 1;
+    }
+    const int b = lo;
+    const uint64_t below = (1ull << b) - 1ull;
+    uint32_t r = local - (uint32_t)(__popcll(m0 & below) + __popcll(m1 & below) + __popcll(m2 & below) + __popcll(m3 & below));
+    const uint32_t bits = (uint32_t)((m0 >> b) & 1ull) | (uint32_t)((m1 >> b) & 1ull) << 1 |
+                          (uint32_t)((m2 >> b) & 1ull) << 2 | (uint32_t)((m3 >> b) & 1ull) << 3;
+    uint32_t bb = bits;
+    while (r) {
+        bb &= bb - 1u;
+        r--;
+    }
+    const int sl = bb ? __builtin_ctz(bb) : 3;
+    const int z = w * 64 + b;
+    const float dx = G.dx;
+    const size_t pidx = ((size_t)x * g + y) * g + z;
+    const float C[3] = {grid_pos(G.ox, x, dx), grid_pos(G.oy, y, dx), grid_pos(G.oz, z, dx)};
+    float P[3] = {C[0], C[1], C[2]};
+    if (sl < 3) {
+        const float *__restrict__ F = F_all + M.vox_off;
+        const uint64_t *__restrict__ om = outm_all + M.word_off;
+        const uint64_t *__restrict__ sm = shellm_all ? shellm_all + M.word_off : nullptr;
+        const size_t row = (size_t)x * g + y;
+        const int W = (int)M.W;
+        const float f0 = field_at(F, om, sm, row, g, W, z, dx);
+        const float f1 = field_at(F, om, sm, row + (sl == 0 ? (size_t)g : (sl == 1 ? 1 : 0)), g, W, z + (sl == 2), dx);
+        float B[3] = {C[0], C[1], C[2]};
+        B[sl] = C[sl] + dx;
+        const float t = (0.0f - f0) / (f1 - f0);
+#pragma unroll
+        for (int c3 = 0; c3 < 3; c3++) {
+            float dd = B[c3] - C[c3];
+            float s = t * dd;
+            P[c3] = C[c3] + s;
+        }
+    }
+    vert[3 * (size_t)v + 0] = P[0];
+    vert[3 * (size_t)v + 1] = P[1];
+    vert[3 * (size_t)v + 2] = P[2];
+    vkey[v] = ((uint64_t)pidx << 2) | (uint64_t)sl;
+    if constexpr (ATOMS) A.atom[v] = closest_one(M, P[0], P[1], P[2], A.cstart, A.sx, A.perm, A.sorted_ids);
+    }
+    __syncthreads(); /* S is staged again for the next block */
+    }
+}
+
+/* triangles (generateTriangleVerticesSMEM MarchingCubes.cu:736-851 order), one thread per
+   polygonised cube (two triangles on average): its word from the active words' first cubes, its
+   place from the word's triangle-count planes.  Bound by the dependent memory trips of a block
+   (block start, word list, planes, corner masks) and by VALU issue, so both are paid once per cube:
+   the thread loads the sign words, slot masks and vertex counts of the cube's four (x, y) columns
+   together, and every corner's vertex id comes from them.  One thread per triangle, three corners'
+   masks each, took 0.20 ms on the 50,000-atom 0.2 A mesh and 0.92 ms on 256 molecules at 0.5 A
+   (47 M triangles); this takes 0.15 and 0.62 ms.  (64 registers for eight waves per SIMD, with
+   spills, were slower than 66 with seven: emission 1.11 against 1.06 ms.) */
+__global__ void __launch_bounds__(256) k_mc_triangles(const QsMol *__restrict__ mols, const uint64_t *__restrict__ wpre,
+                                                      const uint32_t *__restrict__ wcoarse, const uint32_t *__restrict__ list,
+                                                      const uint32_t *__restrict__ acb, const uint32_t *__restrict__ tstart,
+                                                      uint32_t nact, uint32_t ncube, uint32_t ntri, const uint64_t *__restrict__ N,
+                                                      const uint64_t *__restrict__ S4, const uint32_t *__restrict__ cnt,
+                                                      const uint32_t *__restrict__ vbw, const uint32_t *__restrict__ tbw,
+                                                      const uint64_t *__restrict__ NT, int *__restrict__ tri, uint32_t vbase,
+                                                      uint32_t *__restrict__ deg_blk, uint32_t *__restrict__ deg_total,
+                                                      const uint32_t *__restrict__ d_counts)
+{
+    __shared__ ItemWords S;
+    __shared__ uint32_t S_before[4][256]; /* per cube: vertices before its four columns' lower points */
+    /* counts from the device as in k_mc_vertices; triangles past the pool are not written */
+    if (d_counts) {
+        nact = d_counts[2];
+        ncube = min(d_counts[4], ncube);
+    }
+    const uint32_t nb = (ncube + 255u) >> 8;
+    /* persistent blocks over the 256-cube blocks, as in k_mc_vertices */
+    for (uint32_t vb = blockIdx.x; vb < nb; vb += gridDim.x) {
+    const uint32_t blk = xcd_group<64>(vb, nb);
+    stage_item_words(S, acb, list, tstart, nact, nb, blk, wpre, wcoarse);
+    const uint32_t cube = blk * 256u + threadIdx.x;
+    /* sl: the vertex slots of the eight corners, byte q = x | y << 1 for the column, bit
+       2 slot + z in it; has: the columns whose words own vertices (the masks of others are not
+       written, and only an edge that ends in a zero point asks for them) */
+    uint32_t first_tri = 0, nt = 0, sl = 0, has = 0, cs = 0;
+    uint64_t table = 0;
+    if (cube < ncube) {
+        uint32_t k, wi, first;
+        item_word(S, acb, list, cube, k, wi, first);
+        const QsMol &M = mols[S.mol >= 0 ? S.mol : seg_coarse<QS_COARSE_ITEMS>(wpre, wcoarse, (uint64_t)wi)];
+        const size_t W = M.W, gW = (size_t)M.G.g * W;
+        const uint64_t p0 = NT[3 * (size_t)wi], p1 = NT[3 * (size_t)wi + 1], p2 = NT[3 * (size_t)wi + 2];
+        const int b = nth_bit(p0 | p1 | p2, cube - first);
+        const uint64_t below = (1ull << b) - 1ull;
+        first_tri = tbw[wi] + (uint32_t)(__popcll(p0 & below) + 2 * __popcll(p1 & below) + 4 * __popcll(p2 & below));
+        nt = (uint32_t)((p0 >> b) & 1ull) + 2u * (uint32_t)((p1 >> b) & 1ull) + 4u * (uint32_t)((p2 >> b) & 1ull);
+        uint64_t s[4][4], nw[4];
+        uint32_t vb4[4], nv4[4];
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const size_t cw = wi + (q & 1 ? gW : 0) + (q & 2 ? W : 0);
+            nw[q] = N[cw];
+            nv4[q] = word_verts(cnt[cw]);
+            vb4[q] = vbw[cw];
+#pragma unroll
+            for (int a = 0; a < 4; a++) s[q][a] = S4[4 * cw + a];
+        }
+        uint32_t sg = 0; /* sign bits, bit 2 q + z */
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            uint32_t m = 0, before = vb4[q];
+#pragma unroll
+            for (int a = 0; a < 4; a++) {
+                before += (uint32_t)__popcll(s[q][a] & below);
+                m |= ((uint32_t)(s[q][a] >> b) & 3u) << (2 * a);
+            }
+            S_before[q][threadIdx.x] = before;
+            sl |= m << (8 * q);
+            has |= (nv4[q] ? 1u : 0u) << q;
+            sg |= ((uint32_t)(nw[q] >> b) & 3u) << (2 * q);
+        }
+        if (b == 63) { /* the cube's top corners are in the next words */
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const size_t cw = wi + (q & 1 ? gW : 0) + (q & 2 ? W : 0) + 1;
+                sg |= (uint32_t)(N[cw] & 1ull) << (2 * q + 1);
+                uint32_t m = 0;
+#pragma unroll
+                for (int a = 0; a < 4; a++) m |= (uint32_t)(S4[4 * cw + a] & 1ull) << (2 * a + 1);
+                if (word_verts(cnt[cw])) {
+                    /* (a word without vertices below has none of its own slots set) */
+                    sl = (has >> q) & 1u ? sl : sl & ~(255u << (8 * q));
+                    if (!((has >> q) & 1u)) S_before[q][threadIdx.x] = vbw[cw];
+                    has |= 1u << q;
+                    sl |= m << (8 * q);
+                }
+            }
+        }
+        /* the table's corner order goes round the (x, y) columns 00, 10, 11, 01 */
+        const uint32_t lo4 = (sg & 1u) | (sg >> 1 & 2u) | (sg >> 4 & 4u) | (sg >> 1 & 8u);
+        const uint32_t hi4 = (sg >> 1 & 1u) | (sg >> 2 & 2u) | (sg >> 5 & 4u) | (sg >> 2 & 8u);
+        cs = lo4 | hi4 << 4;
+        table = c_tri[cs];
+    }
+#pragma unroll 1
+    for (uint32_t j = 0; j < 5u; j++) {
+        const bool on = j < nt && first_tri + j < ntri;
+        if (!__ballot(on)) break;
+        uint32_t c[3] = {0u, 1u, 2u};
+        const uint32_t t = first_tri + j;
+        if (on) {
+            const uint32_t corners = (uint32_t)(table >> (12u * j));
+#pragma unroll
+            for (int i = 0; i < 3; i++) {
+                const uint32_t e = (corners >> (4 * i)) & 15u;
+                const uint32_t d = (uint32_t)(kEdgePacked >> (5u * e));
+                uint32_t z = d & 1u, q = (d >> 1) & 3u, a2 = (d >> 2) & 6u; /* a2 = 2 axis */
+                uint32_t at = 8u * q + z;                                    /* the corner's slot 0 */
+                if (!((sl >> (at + a2)) & (has >> q) & 1u)) {
+                    /* the edge has no vertex of its own: its non-negative end is exactly zero and
+                       is the vertex (the point slot, after the point's edges) */
+                    if ((cs >> (4 * z + (q ^ (q >> 1)))) & 1u) {
+                        q |= (a2 == 0 ? 1u : 0u) | (a2 == 2 ? 2u : 0u);
+                        z |= a2 == 4 ? 1u : 0u;
+                        at = 8u * q + z;
+                    }
+                    a2 = 6u;
+                }
+                /* the corner's slots below this one, and all slots of the corner below it */
+                const uint32_t lower = __builtin_amdgcn_ubfe(sl, at, a2) & 0x55u;
+                const uint32_t under = __builtin_amdgcn_ubfe(sl, 8u * q, 8u * z) & 0x55u;
+                c[i] = vbase + S_before[q][threadIdx.x] + (uint32_t)(__popc(lower) + __popc(under));
+            }
+            tri[3 * (size_t)t + 0] = (int)c[0];
+            tri[3 * (size_t)t + 1] = (int)c[1];
+            tri[3 * (size_t)t + 2] = (int)c[2];
+        }
+        /* triangles with a repeated corner (zero grid points) are dropped from the output
+           (CudaSurf.cu:820-829): counted here per 256-triangle block and in total */
+        uint64_t dm = __ballot(c[0] == c[1] || c[1] == c[2] || c[0] == c[2]);
+        if (dm) {
+            if ((threadIdx.x & 63) == (uint32_t)__builtin_ctzll(dm)) atomicAdd(deg_total, (uint32_t)__popcll(dm));
+            while (dm) {
+                const uint32_t lead = (uint32_t)__builtin_ctzll(dm);
+                const uint32_t tb = (uint32_t)__shfl((int)(t >> 8), (int)lead, 64);
+                const uint64_t same = __ballot((t >> 8) == tb) & dm;
+                if ((threadIdx.x & 63) == lead) atomicAdd(&deg_blk[tb], (uint32_t)__popcll(same));
+                dm &= ~same;
+            }
+        }
+    }
+    __syncthreads(); /* S is staged again for the next block */
     }
 }
 
@@ -3612,12 +3637,27 @@ __global__ void __launch_bounds__(256) k_deg_count(const int *__restrict__ tri, 
     }
 }
 
+/* ONE: one molecule.  Its read-back {totals[0..3], first vertices (0, nv), kept triangles before its
+   first and last (0, nt - *ndeg)} and the last two pairs (vpre, kept) are written here too.
+   self: dpre holds the per-block counts themselves (at most TRI_SELF_BLOCKS of them) and each block
+   adds up those before it, which only happens when there is something to drop. */
+template <bool ONE>
 __global__ void __launch_bounds__(256) k_tri_compact(const int *__restrict__ tri, uint32_t nt,
-                                                     const uint32_t *__restrict__ dpre, const uint32_t *__restrict__ ndeg,
-                                                     int *__restrict__ out, const uint32_t *__restrict__ d_nt)
+                                                     const uint32_t *__restrict__ dpre, const uint32_t *__restrict__ totals,
+                                                     int *__restrict__ out, const uint32_t *__restrict__ d_nt, int self, uint32_t nv,
+                                                     uint32_t *__restrict__ vpre, uint32_t *__restrict__ kept,
+                                                     uint32_t *__restrict__ rb)
 {
-    __shared__ uint32_t wkeep[4];
-    if (*ndeg == 0) return; /* nothing to drop: the caller keeps the input array */
+    __shared__ uint32_t wkeep[4], lds[256 / 64 + 1];
+    const uint32_t ndeg = totals[3];
+    if (ONE && blockIdx.x == 0 && threadIdx.x < 8) {
+        const uint32_t t = threadIdx.x, all_t = d_nt ? *d_nt : nt, all_v = d_nt ? totals[1] : nv;
+        const uint32_t end = t == 5 ? all_v : (t == 7 ? all_t - ndeg : 0u);
+        rb[t] = t < 4 ? totals[t] : end;
+        if (t >= 6) kept[t - 6] = end;
+        else if (t >= 4) vpre[t - 4] = end;
+    }
+    if (ndeg == 0) return; /* nothing to drop: the caller keeps the input array */
     if (d_nt) nt = min(*d_nt, nt); /* the device count within the launch's pool */
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
     /* persistent blocks over the 256-triangle blocks */
@@ -3627,7 +3667,15 @@ __global__ void __launch_bounds__(256) k_tri_compact(const int *__restrict__ tri
         const uint64_t km = __ballot(keep);
         if (lane == 0) wkeep[wid] = (uint32_t)__popcll(km);
         __syncthreads();
-        uint32_t o = b * 256u - dpre[b] + (uint32_t)__popcll(km & ((1ull << lane) - 1ull));
+        uint32_t before;
+        if (ONE && self) {
+            uint32_t x = 0;
+            for (uint32_t k = threadIdx.x; k < b; k += 256u) x += dpre[k];
+            before = block_sum<256>(x, lds);
+        } else {
+            before = dpre[b];
+        }
+        uint32_t o = b * 256u - before + (uint32_t)__popcll(km & ((1ull << lane) - 1ull));
         for (int k = 0; k < wid; k++) o += wkeep[k];
         if (keep) {
             out[3 * (size_t)o] = tri[3 * (size_t)t];
@@ -3664,6 +3712,12 @@ __global__ void __launch_bounds__(256) k_tri_kept_before(const int *__restrict__
         out[i] = t - dpre[b] - d;
         if (rb) rb[4 + n + i] = t - dpre[b] - d;
     }
+}
+
+/* one molecule's record, from the launch's arguments */
+__global__ void __launch_bounds__(64) k_put_mol(QsMol m, QsMol *__restrict__ dst)
+{
+    if (threadIdx.x == 0) *dst = m;
 }
 
 /* plain device copy (16-byte vectors, grid-stride): the reference point for traffic counters */
@@ -3708,8 +3762,10 @@ static inline unsigned pgrid(uint64_t nb)
 constexpr unsigned COMPACT_BLOCKS = 4096;
 
 /* partial boxes per molecule: about 8 atoms per thread of the largest molecule, 1 to BB_PMAX */
-int qs_bbox_parts(uint32_t max_atoms)
+/* (a single molecule of up to 8,192 atoms is one block of 1,024 threads and one launch) */
+int qs_bbox_parts(uint32_t max_atoms, int nmol)
 {
+    if (nmol == 1 && max_atoms <= 8192u) return 1;
     const uint32_t p = (max_atoms + 8 * BB_NT - 1) / (8 * BB_NT);
     return (int)std::min<uint32_t>(std::max<uint32_t>(p, 1u), BB_PMAX);
 }
@@ -3720,11 +3776,12 @@ void qs_launch_bbox(const float *pos, const float *rad, const uint32_t *off, uin
                     float *part, float *out, hipStream_t s)
 {
     /* one partial box per molecule is its box (part[m][0] and out[m] are at the same offset) */
-    if (parts == 1) {
-        hipLaunchKernelGGL(k_bbox_part, dim3(1, nmol), dim3(BB_NT), 0, s, pos, rad, off, o0, o1, out);
+    if (parts == 1 && nmol == 1) {
+        hipLaunchKernelGGL(k_bbox_part<1024>, dim3(1, 1), dim3(1024), 0, s, pos, rad, off, o0, o1, out);
         return;
     }
-    hipLaunchKernelGGL(k_bbox_part, dim3(parts, nmol), dim3(BB_NT), 0, s, pos, rad, off, o0, o1, part);
+    hipLaunchKernelGGL(k_bbox_part<BB_NT>, dim3(parts, nmol), dim3(BB_NT), 0, s, pos, rad, off, o0, o1, parts == 1 ? out : part);
+    if (parts == 1) return;
     hipLaunchKernelGGL(k_bbox_final, dim3(nmol), dim3(64), 0, s, part, parts, out);
 }
 
@@ -3906,19 +3963,10 @@ void qs_launch_mc_emit(const QsMol *mols, const uint64_t *wpre, const uint32_t *
                        const uint64_t *outm, const uint64_t *shellm, float *vert, uint64_t *vkey,
                        const uint32_t *acb, uint32_t *tstart, uint32_t ncube, uint32_t ntri, const uint64_t *N, const uint32_t *cnt,
                        const uint32_t *vbw, const uint32_t *tbw, const uint64_t *NT, int *tri, uint32_t vbase, uint32_t *deg_blk,
-                       uint32_t *deg_total, const uint32_t *d_counts, hipStream_t s, hipStream_t s_vert, hipEvent_t ev_fork,
-                       hipEvent_t ev_vert, bool starts_ready, uint32_t expect)
+                       uint32_t *deg_total, const uint32_t *d_counts, hipStream_t s, const QsClosest *atoms, bool starts_ready,
+                       uint32_t expect)
 {
-    if (!s_vert) s_vert = s;
-    if (!nact || (!nv && !ntri)) {
-        /* nothing to emit: s_vert still follows s up to here */
-        if (s_vert != s) {
-            (void)hipEventRecord(ev_fork, s);
-            (void)hipStreamWaitEvent(s_vert, ev_fork, 0);
-            (void)hipEventRecord(ev_vert, s_vert);
-        }
-        return;
-    }
+    if (!nact || (!nv && !ntri)) return;
     /* the per-block degenerate counts start at zero (the triangle kernel adds to them), over the
        whole pool of ntri triangles */
     const uint32_t nzero = ntri ? ntri / 256 + 1 : 0u;
@@ -3927,15 +3975,15 @@ void qs_launch_mc_emit(const QsMol *mols, const uint64_t *wpre, const uint32_t *
     if (!starts_ready)
         hipLaunchKernelGGL(k_block_starts, dim3(pgrid(nblk(std::max<uint32_t>(nact, nzero), 256)), 2), dim3(256), 0, s, sv, st,
                            nact, d_counts ? d_counts + 2 : nullptr);
-    /* the vertex kernel on s_vert (after the block starts), beside the triangle kernel on s */
-    if (s_vert != s) {
-        (void)hipEventRecord(ev_fork, s);
-        (void)hipStreamWaitEvent(s_vert, ev_fork, 0);
+    if (nv) {
+        const dim3 grid(pgrid(nblk(std::min(nv, expect), 256)));
+        if (atoms)
+            hipLaunchKernelGGL(k_mc_vertices<true>, grid, dim3(256), 0, s, mols, wpre, wcoarse, list, avb, vstart, nact, nv, S4, F,
+                               outm, shellm, vert, vkey, d_counts, *atoms);
+        else
+            hipLaunchKernelGGL(k_mc_vertices<false>, grid, dim3(256), 0, s, mols, wpre, wcoarse, list, avb, vstart, nact, nv, S4, F,
+                               outm, shellm, vert, vkey, d_counts, QsClosest{});
     }
-    if (nv)
-        hipLaunchKernelGGL(k_mc_vertices, dim3(pgrid(nblk(std::min(nv, expect), 256))), dim3(256), 0, s_vert, mols, wpre, wcoarse, list, avb, vstart, nact,
-                           nv, S4, F, outm, shellm, vert, vkey, d_counts);
-    if (s_vert != s) (void)hipEventRecord(ev_vert, s_vert);
     if (ntri)
         hipLaunchKernelGGL(k_mc_triangles, dim3(pgrid(nblk(std::min(ncube, expect), 256))), dim3(256), 0, s, mols, wpre, wcoarse, list, acb, tstart,
                            nact, ncube, ntri, N, S4, cnt, vbw, tbw, NT, tri, vbase, deg_blk, deg_total, d_counts);
@@ -3968,15 +4016,15 @@ void qs_launch_vertex_colors(const QsMol *mols, const uint32_t *vpre, const uint
                        out);
 }
 
-void qs_launch_closest_atom(const QsMol *mols, const uint32_t *vpre, const uint32_t *vcoarse, const uint32_t *cstart,
-                            const float4 *sx,
-                            const int *perm, const float *vert, uint32_t nv, int sorted_ids, int *out, const uint32_t *d_nv,
-                            uint32_t expect, hipStream_t s)
+void qs_launch_closest_atom(const QsMol *mols, const uint32_t *vpre, const uint32_t *vcoarse, const QsClosest &A,
+                            const float *vert, uint32_t nv, const uint32_t *d_nv, uint32_t expect, hipStream_t s)
 {
     if (!nv) return;
-    hipLaunchKernelGGL(k_closest_atom, dim3(pgrid(nblk(std::min(nv, expect), 256))), dim3(256), 0, s, mols, vpre, vcoarse, cstart, sx, perm, vert,
-                       nv, sorted_ids, out, d_nv);
+    hipLaunchKernelGGL(k_closest_atom, dim3(pgrid(nblk(std::min(nv, expect), 256))), dim3(256), 0, s, mols, vpre, vcoarse, vert, nv,
+                       d_nv, A);
 }
+
+void qs_launch_put_mol(const QsMol &m, QsMol *dst, hipStream_t s) { hipLaunchKernelGGL(k_put_mol, dim3(1), dim3(64), 0, s, m, dst); }
 
 void qs_launch_copy(const void *src, void *dst, uint64_t bytes, hipStream_t s)
 {
@@ -3993,11 +4041,19 @@ void qs_launch_tri_localize(const int *tri, uint32_t nt, const uint32_t *tpre, c
     hipLaunchKernelGGL(k_tri_localize, dim3(nblk(nt, 256)), dim3(256), 0, s, tri, nt, tpre, vpre, nmol, out);
 }
 
-void qs_launch_tri_compact(const int *tri, uint32_t nt, const uint32_t *dpre, const uint32_t *ndeg, int *out,
+void qs_launch_tri_compact(const int *tri, uint32_t nt, const uint32_t *dpre, const uint32_t *totals, int *out,
                            const uint32_t *d_nt, hipStream_t s)
 {
     if (!nt) return;
-    hipLaunchKernelGGL(k_tri_compact, dim3(std::min(nblk(nt, 256), COMPACT_BLOCKS)), dim3(256), 0, s, tri, nt, dpre, ndeg, out, d_nt);
+    hipLaunchKernelGGL(k_tri_compact<false>, dim3(std::min(nblk(nt, 256), COMPACT_BLOCKS)), dim3(256), 0, s, tri, nt, dpre, totals,
+                       out, d_nt, 0, 0u, (uint32_t *)nullptr, (uint32_t *)nullptr, (uint32_t *)nullptr);
+}
+
+void qs_launch_tri_compact_one(const int *tri, uint32_t nt, const uint32_t *dpre, bool self, const uint32_t *totals, int *out,
+                               const uint32_t *d_nt, uint32_t nv, uint32_t *vpre, uint32_t *kept, uint32_t *rb, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_tri_compact<true>, dim3(std::max(1u, std::min(nblk(nt, 256), COMPACT_BLOCKS))), dim3(256), 0, s, tri, nt,
+                       dpre, totals, out, d_nt, self ? 1 : 0, nv, vpre, kept, rb);
 }
 
 void qs_launch_tri_kept_before(const int *tri, const uint32_t *dpre, const uint64_t *idx, int n, uint32_t tcap, uint32_t *out,

@@ -111,3 +111,26 @@ def test_mesh_beyond_the_expected_size(qs, orc, n):
     print("case separate spheres n=%d" % len(rad), flush=True)
     for _ in range(2):  # with the pools of the start, then with grown ones
         assert _same(qs.compute_ses(pos, rad, 0.5, 1), orc.compute_ses(pos, rad, 0.5, 1))
+
+
+@pytest.mark.parametrize("n", [1278, 1279])
+def test_dropped_triangles_with_and_without_the_count_scan(qs, orc, n):
+    """Degenerate triangles dropped (a probe of seven whole voxels gives zero grid points) from pools
+    of 2,047 and 2,049 blocks: up to 2,048 each block adds up the counts before it itself."""
+    pos, rad = qs.synth_ball(5, n)
+    print("case dropped triangles: n=%d" % n, flush=True)
+    assert _same(qs.compute_ses(pos, rad, 0.2, 1), orc.compute_ses(pos, rad, 0.2, 1))
+
+
+@pytest.mark.parametrize("n", [5, 1025, 4097, 8191, 8192, 8193])
+def test_bounding_box_on_the_device(qs, n):
+    """The box found by one block (up to 8,192 atoms) or several is the host's: the same mesh."""
+    from quickses_amd import hipmem
+
+    pos, rad = qs.synth_ball(17, n)
+    pos[n // 2] += np.float32(9.0)  # one atom alone sets three faces
+    dp, dr = hipmem.DeviceArray(pos), hipmem.DeviceArray(rad)
+    print("case device box: n=%d" % n, flush=True)
+    nv, ni, pv, pt, pa = qs.compute_device(dp.ptr, dr.ptr, n, 1.0, 0)
+    got = (hipmem.download(pv, (nv, 3), np.float32), hipmem.download(pt, (ni // 3, 3), np.int32), hipmem.download(pa, (nv,), np.int32))
+    assert nv > 0 and _same(got, qs.compute_ses(pos, rad, 1.0, 0))
