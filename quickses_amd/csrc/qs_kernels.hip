@@ -200,33 +200,50 @@ __device__ __forceinline__ int seg_of_wave(const uint32_t *__restrict__ pre, con
     return seg_coarse<QS_COARSE_ITEMS>(pre, coarse, v);
 }
 
+/* inclusive scan over the wave's lanes (all active): six data-parallel-primitive adds, where a
+   shuffle through LDS per step made the scans bound by its latency */
+__device__ __forceinline__ uint32_t wave_incl_scan(uint32_t x)
+{
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x111, 0xf, 0xf, false); /* lane - 1, - 2, - 4, - 8 of the row of 16 */
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x112, 0xf, 0xf, false);
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x114, 0xf, 0xf, false);
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x118, 0xf, 0xf, false);
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x142, 0xa, 0xf, false); /* last lane of the row below, to rows 1 and 3 */
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x143, 0xc, 0xf, false); /* lane 31, to rows 2 and 3 */
+    return x;
+}
+/* the largest of the wave's values */
+__device__ __forceinline__ uint32_t wave_max(uint32_t x)
+{
+    x = max(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x111, 0xf, 0xf, false));
+    x = max(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x112, 0xf, 0xf, false));
+    x = max(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x114, 0xf, 0xf, false));
+    x = max(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x118, 0xf, 0xf, false));
+    x = max(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x142, 0xa, 0xf, false));
+    x = max(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x143, 0xc, 0xf, false));
+    return (uint32_t)__builtin_amdgcn_readlane((int)x, 63);
+}
+/* lane 63's value */
+__device__ __forceinline__ uint32_t wave_last(uint32_t x) { return (uint32_t)__builtin_amdgcn_readlane((int)x, 63); }
+
 /* exclusive scan over the block; returns this thread's prefix, *total the block sum */
 template <int NT>
 __device__ __forceinline__ uint32_t block_excl_scan(uint32_t v, uint32_t *total, uint32_t *lds)
 {
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    uint32_t x = v;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        uint32_t y = __shfl_up(x, d, 64);
-        if (lane >= d) x += y;
-    }
+    const uint32_t x = wave_incl_scan(v);
     if (lane == 63) lds[wid] = x;
     __syncthreads();
-    if (threadIdx.x == 0) {
-        uint32_t s = 0;
-        for (int w = 0; w < NT / 64; w++) {
-            uint32_t t = lds[w];
-            lds[w] = s;
-            s += t;
-        }
-        lds[NT / 64] = s;
+    uint32_t below = 0, all = 0;
+#pragma unroll
+    for (int w = 0; w < NT / 64; w++) {
+        const uint32_t t = lds[w];
+        below += (w < wid) ? t : 0u;
+        all += t;
     }
+    *total = all;
     __syncthreads();
-    uint32_t res = x - v + lds[wid];
-    *total = lds[NT / 64];
-    __syncthreads();
-    return res;
+    return x - v + below;
 }
 
 template <int NT>
@@ -242,10 +259,7 @@ __device__ __forceinline__ uint32_t block_sum(uint32_t v, uint32_t *lds)
 __device__ __forceinline__ uint32_t wave_sum_below(const uint32_t *__restrict__ sums, uint32_t b)
 {
     const uint32_t lane = threadIdx.x & 63;
-    uint32_t x = (lane < b) ? sums[lane] : 0u;
-#pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) x += (uint32_t)__shfl_xor((int)x, d, 64);
-    return x;
+    return wave_last(wave_incl_scan((lane < b) ? sums[lane] : 0u));
 }
 
 /* bit position of the r-th set bit (from 0) of m, which has more than r */
@@ -428,23 +442,15 @@ __global__ void __launch_bounds__(SCAN_NT) k_mc_scan4(const uint32_t *__restrict
     for (int k = 0; k < SCAN_IPT; k++) {
         /* triangles and cubes of a group of 64 words are scanned in one register (at most 64 x 320
            and 64 x 64) */
-        uint32_t xv = word_verts(cw[k]), xt = word_tris(cw[k]) | word_cubes(cw[k]) << 16;
-        const uint32_t own = xt;
-#pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-            const uint32_t yv = __shfl_up(xv, d, 64), yt = __shfl_up(xt, d, 64);
-            if (lane >= d) {
-                xv += yv;
-                xt += yt;
-            }
-        }
+        const uint32_t own = word_tris(cw[k]) | word_cubes(cw[k]) << 16;
+        const uint32_t xv = wave_incl_scan(word_verts(cw[k])), xt = wave_incl_scan(own);
         const uint64_t am = __ballot(cw[k] != 0u);
         pv[k] = rv + xv - word_verts(cw[k]);
         pt[k] = rt + ((xt - own) & 0xFFFFu);
         pc[k] = rc + ((xt - own) >> 16);
         pa[k] = ra + (uint32_t)__popcll(am & below);
-        rv += __shfl(xv, 63, 64);
-        const uint32_t last = __shfl(xt, 63, 64);
+        rv += wave_last(xv);
+        const uint32_t last = wave_last(xt);
         rt += last & 0xFFFFu;
         rc += last >> 16;
         ra += (uint32_t)__popcll(am);
@@ -528,20 +534,14 @@ __device__ __forceinline__ void scan1_offsets(const uint32_t *wsum, int wid, uin
 }
 
 /* exclusive prefix of the wave's SCAN_IPT groups of 64 in place; returns the wave's total */
-__device__ __forceinline__ uint32_t wave_groups_scan(uint32_t (&v)[SCAN_IPT], int lane)
+__device__ __forceinline__ uint32_t wave_groups_scan(uint32_t (&v)[SCAN_IPT])
 {
     uint32_t run = 0;
 #pragma unroll
     for (int k = 0; k < SCAN_IPT; k++) {
-        uint32_t x = v[k];
-#pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-            const uint32_t y = __shfl_up(x, d, 64);
-            if (lane >= d) x += y;
-        }
-        const uint32_t tot = __shfl(x, 63, 64);
+        const uint32_t x = wave_incl_scan(v[k]);
         v[k] = run + x - v[k];
-        run += tot;
+        run += wave_last(x);
     }
     return run;
 }
@@ -557,7 +557,7 @@ __global__ void __launch_bounds__(SCAN1_NT) k_scan1(const uint32_t *in, uint32_t
         uint32_t v[SCAN_IPT];
 #pragma unroll
         for (int k = 0; k < SCAN_IPT; k++) v[k] = (base + 64 * k < n) ? in[base + 64 * k] : 0u;
-        const uint32_t run = wave_groups_scan(v, lane);
+        const uint32_t run = wave_groups_scan(v);
         if (lane == 0) wsum[wid] = run;
         __syncthreads();
         uint32_t below, all;
@@ -603,7 +603,7 @@ __global__ void __launch_bounds__(SCAN1_NT) k_mc_scan1(const uint32_t *__restric
             pa[k] = ra + (uint32_t)__popcll(am & lbelow);
             ra += (uint32_t)__popcll(am);
         }
-        const uint32_t rv = wave_groups_scan(v, lane), rt = wave_groups_scan(t, lane), rc = wave_groups_scan(q, lane);
+        const uint32_t rv = wave_groups_scan(v), rt = wave_groups_scan(t), rc = wave_groups_scan(q);
         if (lane == 0) {
             wsum[0][wid] = rv;
             wsum[1][wid] = rt;
@@ -1319,12 +1319,7 @@ __global__ void __launch_bounds__(256) k_pass1_slab(QsBatch B, const uint32_t *_
     }
     /* exclusive prefix of the column lengths (ncol <= 256) */
     {
-        uint32_t v = len;
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            const uint32_t t = __shfl_up(v, o, 64);
-            if (lane >= o) v += t;
-        }
+        const uint32_t v = wave_incl_scan(len);
         __shared__ uint32_t wsum[4];
         if (lane == 63) wsum[wid] = v;
         __syncthreads();
@@ -1374,16 +1369,9 @@ __global__ void __launch_bounds__(256) k_pass1_slab(QsBatch B, const uint32_t *_
             const int n = p ? nr[1] : nr[0], first = p ? r0[1] : r0[0];
             const float thr = p ? sD : sN;
             uint32_t *const mask = (uint32_t *)(p ? insw : nearw);
-            int pre = n, most = n;
-#pragma unroll
-            for (int d = 1; d < 64; d <<= 1) {
-                const int t = __shfl_up(pre, d, 64);
-                if (lane >= d) pre += t;
-            }
-            const int nitems = __shfl(pre, 63, 64);
+            int pre = (int)wave_incl_scan((uint32_t)n);
+            const int nitems = (int)wave_last((uint32_t)pre), most = (int)wave_max((uint32_t)n);
             pre -= n; /* exclusive */
-#pragma unroll
-            for (int d = 1; d < 64; d <<= 1) most = max(most, __shfl_xor(most, d, 64));
             const bool walk = P1_FLAT * ((nitems + 63) >> 6) >= most;
             const int rounds = walk ? most : (nitems + 63) >> 6;
 #pragma unroll 1
@@ -2131,12 +2119,7 @@ __global__ void __launch_bounds__(256) k_pass2_r(QsBatch B, const uint64_t *__re
             cmask[lx] = c;
         }
         const uint32_t cnt = (uint32_t)__builtin_popcount(c);
-        uint32_t inc = cnt;
-#pragma unroll
-        for (int k = 1; k < 64; k *= 2) {
-            const uint32_t t = (uint32_t)__shfl_up((int)inc, k);
-            if (lx >= k) inc += t;
-        }
+        const uint32_t inc = wave_incl_scan(cnt);
         if (lx < LX) cpre[lx] = inc - cnt;
         if (lx == LX - 1) cpre[LX] = inc;
     }
@@ -2325,13 +2308,8 @@ __global__ void __launch_bounds__(256) k_pass2_r(QsBatch B, const uint64_t *__re
         /* lane l's rows are 2 l and 2 l + 1 */
         const uint32_t m0 = strace[2 * lane], m1 = strace[2 * lane + 1];
         const uint32_t n0 = (uint32_t)__popc(m0), nn = n0 + (uint32_t)__popc(m1);
-        uint32_t pre = nn;
-#pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-            const uint32_t t = (uint32_t)__shfl_up((int)pre, d, 64);
-            if (lane >= d) pre += t;
-        }
-        const uint32_t total = (uint32_t)__shfl((int)pre, 63, 64);
+        uint32_t pre = wave_incl_scan(nn);
+        const uint32_t total = wave_last(pre);
         pre -= nn; /* exclusive */
 #pragma unroll 1
         for (uint32_t base = 64u * (uint32_t)wid; base < total; base += 256u) {
