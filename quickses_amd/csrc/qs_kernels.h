@@ -20,6 +20,16 @@ size_t qs_bbox_part_floats(int nmol, int parts);
 /* off: per-molecule atom offsets (nmol + 1); or nullptr for one molecule of atoms [o0, o1) */
 void qs_launch_bbox(const float *pos, const float *rad, const uint32_t *off, uint32_t o0, uint32_t o1, int nmol, int parts,
                     float *part, float *out, hipStream_t s);
+/* the cells' steps below in one launch, a block per molecule, for molecules of at most CELLS_ATOMS
+   atoms and CELLS_MAX cells (lds: the largest qs_cells_lds_bytes, which is 0 for a molecule that is
+   too large); with gather, for molecules of at most CELLS_GATHER atoms, qs_launch_gather_aux's
+   included.  one (may be NULL): the run's only molecule, put into mols on the way */
+#define CELLS_GATHER 4096u
+#define CELLS_ATOMS 24576u
+#define CELLS_MAX 49152u
+size_t qs_cells_lds_bytes(const QsMol &m);
+void qs_launch_cells(const QsMol *mols, int nmol, const QsMol *one, size_t lds, bool gather, const float *pos, const float *rad, uint32_t *start,
+                     int *perm, int2 *cse, float4 *sx, float4 *aux, hipStream_t s);
 /* key: (cell, rank within the cell) per atom; count: atoms per cell (cleared before) */
 void qs_launch_hash_count(QsBatch B, uint32_t nblocks, const float *pos, int2 *key, uint32_t *count, hipStream_t s);
 void qs_launch_scatter(const int2 *key, int n, const uint32_t *start, int *perm, hipStream_t s);

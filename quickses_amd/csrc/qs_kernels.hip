@@ -861,10 +861,10 @@ __device__ __forceinline__ float sqrt_threshold(float T)
 {
     if (!(T > 0.0f)) return -1.0f;
     float s = T * T;
-    for (int i = 0; i < 8 && sqrtf(s) < T; i++) s = __uint_as_float(__float_as_uint(s) + 1u);
+    for (int i = 0; i < 8 && sqrt_rn(s) < T; i++) s = __uint_as_float(__float_as_uint(s) + 1u);
     for (int i = 0; i < 8 && s > 0.0f; i++) {
         float q = __uint_as_float(__float_as_uint(s) - 1u);
-        if (sqrtf(q) >= T) s = q;
+        if (sqrt_rn(q) >= T) s = q;
         else break;
     }
     return s;
@@ -930,6 +930,13 @@ __device__ __forceinline__ bool fast_interval(float h2, float zc, float inv_dx, 
     return d > eps && h2 > 0.015625f;
 }
 
+/* an atom's float thresholds of its near (r + probe) and inside (r - dx) tests, and its
+   neighbour-cell y and z (packed) */
+__device__ __forceinline__ float4 atom_aux(const float4 &a, const QsGrid &G, int acy, int acz)
+{
+    return make_float4(sqrt_threshold(QS_PROBE + a.w), sqrt_threshold(a.w - G.dx), __int_as_float((acy << 16) | acz), 0.0f);
+}
+
 /* per atom in cell order, once: the atom (perm gives its input index) as float4 x, y, z, r, the
    exact float thresholds of its near (r + probe) and inside (r - dx) tests, and its neighbour-cell
    y and z (packed) */
@@ -946,9 +953,113 @@ __global__ void __launch_bounds__(256) k_gather_aux(QsBatch B, const int *__rest
     const int id = perm[k];
     const float4 a = make_float4(pos[3 * (size_t)id], pos[3 * (size_t)id + 1], pos[3 * (size_t)id + 2], rad[id]);
     sx[k] = a;
-    const int acy = iclamp(cell_of(a.y, G.oy, G.dxn), 0, G.gn - 1);
-    const int acz = iclamp(cell_of(a.z, G.oz, G.dxn), 0, G.gn - 1);
-    aux[k] = make_float4(sqrt_threshold(QS_PROBE + a.w), sqrt_threshold(a.w - G.dx), __int_as_float((acy << 16) | acz), 0.0f);
+    aux[k] = atom_aux(a, G, iclamp(cell_of(a.y, G.oy, G.dxn), 0, G.gn - 1), iclamp(cell_of(a.z, G.oz, G.dxn), 0, G.gn - 1));
+}
+
+/* Cells of a molecule of at most PER * 1,024 atoms and CELLS_MAX cells in one block: hashing, counts,
+   their scan and the order (cell, index) in LDS, and with GATHER the gathered atoms, with the results
+   of k_hash_count, the scan, k_scatter, k_cell_finalize and k_gather_aux.  Bound by the latency of its
+   few dependent steps, where those launches (and a clear) each had that of a launch; an atom's place
+   within its cell is the number of the cell's atoms of lower index, so nothing is sorted.  The cells
+   of 300 atoms took 24 us and take 9, of 2,000 atoms 26 and 14.
+   With put, the run's one molecule comes in the arguments and goes to *put for the later launches. */
+constexpr uint32_t CELLS_NT = 1024;
+template <int PER, bool GATHER>
+__global__ void __launch_bounds__(CELLS_NT) k_cells(const QsMol *__restrict__ mols, QsMol one, QsMol *__restrict__ put,
+                                                    const float *__restrict__ pos, const float *__restrict__ rad,
+                                                    uint32_t *__restrict__ start, int *__restrict__ perm, int2 *__restrict__ cse,
+                                                    float4 *__restrict__ sx, float4 *__restrict__ aux)
+{
+    static_assert(PER % 4 == 0 && PER * CELLS_NT < 65536, "atoms four at a time, 16-bit places");
+    extern __shared__ uint32_t cells_lds[];
+    __shared__ uint32_t wsum[CELLS_NT / 64];
+    if (put && threadIdx.x == 0) *put = one;
+    const QsMol &M = put ? one : mols[blockIdx.x];
+    const QsGrid G = M.G;
+    const int gn = G.gn;
+    const uint32_t n = M.n_atoms, a0 = M.atom_off, ncell = (uint32_t)(gn * gn * gn), c0 = M.cell_off;
+    uint16_t *const cnt = (uint16_t *)cells_lds; /* atoms per cell, then the cells' first places */
+    uint16_t *const slot = (uint16_t *)(cells_lds + ncell / 2 + 1); /* atoms by cell, in the order they were counted */
+    for (uint32_t c = threadIdx.x; c <= ncell / 2; c += CELLS_NT) cells_lds[c] = 0u;
+    __syncthreads();
+    uint32_t hr[PER]; /* cell << 16 | rank in the cell */
+#pragma unroll
+    for (uint32_t k0 = 0; k0 < PER; k0 += 4) {
+        if (k0 * CELLS_NT >= n) break;
+        float p[4][3];
+#pragma unroll
+        for (uint32_t k = 0; k < 4; k++) {
+            const float *__restrict__ q = pos + 3 * (size_t)(a0 + min((k0 + k) * CELLS_NT + threadIdx.x, n - 1u));
+            p[k][0] = q[0];
+            p[k][1] = q[1];
+            p[k][2] = q[2];
+        }
+#pragma unroll
+        for (uint32_t k = 0; k < 4; k++) {
+            const int cx = iclamp(cell_of(p[k][0], G.ox, G.dxn), 0, gn - 1), cy = iclamp(cell_of(p[k][1], G.oy, G.dxn), 0, gn - 1),
+                      cz = iclamp(cell_of(p[k][2], G.oz, G.dxn), 0, gn - 1);
+            const uint32_t h = (uint32_t)((gn * gn * cx) + (gn * cy) + cz);
+            const uint32_t half = 16u * (h & 1u); /* (counts of two cells in a word) */
+            uint32_t r = 0;
+            if ((k0 + k) * CELLS_NT + threadIdx.x < n) r = (atomicAdd(&cells_lds[h >> 1], 1u << half) >> half) & 0xFFFFu;
+            hr[k0 + k] = h << 16 | r;
+        }
+    }
+    __syncthreads();
+    /* exclusive scan of the counts: a wave takes consecutive groups of 64 */
+    const uint32_t lane = threadIdx.x & 63, wid = threadIdx.x >> 6, ng = (ncell + CELLS_NT - 1) / CELLS_NT;
+    uint32_t run = 0;
+    for (uint32_t k = 0; k < ng; k++) {
+        const uint32_t c = (wid * ng + k) * 64u + lane;
+        const uint32_t v = c < ncell ? cnt[c] : 0u, x = wave_incl_scan(v);
+        if (c < ncell) cnt[c] = (uint16_t)(run + x - v);
+        run += wave_last(x);
+    }
+    if (lane == 0) wsum[wid] = run;
+    if (threadIdx.x == 0) cnt[ncell] = (uint16_t)n;
+    __syncthreads();
+    uint32_t before = 0;
+    for (uint32_t w = 0; w < wid; w++) before += wsum[w];
+    for (uint32_t k = 0; k < ng; k++) {
+        const uint32_t c = (wid * ng + k) * 64u + lane;
+        if (c < ncell) {
+            const uint32_t v = cnt[c] + before;
+            cnt[c] = (uint16_t)v;
+            start[c0 + c] = a0 + v;
+        }
+    }
+    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) start[c0 + ncell] = a0 + n;
+    __syncthreads();
+#pragma unroll
+    for (uint32_t k = 0; k < PER; k++) {
+        const uint32_t i = k * CELLS_NT + threadIdx.x;
+        if (i < n) slot[cnt[hr[k] >> 16] + (hr[k] & 0xFFFFu)] = (uint16_t)i;
+    }
+    for (uint32_t c = threadIdx.x; c < ncell; c += CELLS_NT) {
+        const uint32_t b = cnt[c], e = cnt[c + 1];
+        cse[c0 + c] = b == e ? make_int2(QS_EMPTY, QS_EMPTY) : make_int2((int)(a0 + b), (int)(a0 + e));
+    }
+    __syncthreads();
+    const float inv_gn = 1.0f / (float)gn;
+#pragma unroll
+    for (uint32_t k = 0; k < PER; k++) {
+        const uint32_t i = k * CELLS_NT + threadIdx.x;
+        if (i < n) {
+            const uint32_t h = hr[k] >> 16, b = cnt[h], e = cnt[h + 1];
+            uint32_t at = a0 + b;
+            for (uint32_t q = b; q < e; q++) at += slot[q] < i ? 1u : 0u;
+            perm[at] = (int)(a0 + i);
+            if constexpr (GATHER) {
+                const float *__restrict__ p = pos + 3 * (size_t)(a0 + i);
+                const float4 a = make_float4(p[0], p[1], p[2], rad[a0 + i]);
+                /* the cell's z and y: h < 2^16, so the quotients are exact */
+                const int xy = (int)(((float)h + 0.5f) * inv_gn), cz = (int)h - gn * xy;
+                const int cy = xy - gn * (int)(((float)xy + 0.5f) * inv_gn);
+                sx[at] = a;
+                aux[at] = atom_aux(a, G, cy, cz);
+            }
+        }
+    }
 }
 
 /* rows per wavefront: R consecutive y rows (R * dx <= neighbour-cell size, so they span at most
@@ -4000,6 +4111,26 @@ void qs_launch_closest_atom(const QsMol *mols, const uint32_t *vpre, const uint3
     if (!nv) return;
     hipLaunchKernelGGL(k_closest_atom, dim3(pgrid(nblk(std::min(nv, expect), 256))), dim3(256), 0, s, mols, vpre, vcoarse, vert, nv,
                        d_nv, A);
+}
+
+size_t qs_cells_lds_bytes(const QsMol &m)
+{
+    const uint64_t ncell = (uint64_t)m.G.gn * m.G.gn * m.G.gn;
+    if (m.n_atoms > CELLS_ATOMS || ncell > CELLS_MAX) return 0;
+    return ((size_t)ncell / 2 + 1) * 4 + ((size_t)m.n_atoms * 2 + 3) / 4 * 4;
+}
+
+void qs_launch_cells(const QsMol *mols, int nmol, const QsMol *one, size_t lds, bool gather, const float *pos, const float *rad, uint32_t *start,
+                     int *perm, int2 *cse, float4 *sx, float4 *aux, hipStream_t s)
+{
+    QsMol *const put = one ? (QsMol *)mols : nullptr;
+    const QsMol m = one ? *one : QsMol{};
+    if (gather)
+        hipLaunchKernelGGL((k_cells<CELLS_GATHER / CELLS_NT, true>), dim3(nmol), dim3(CELLS_NT), lds, s, mols, m, put, pos, rad,
+                           start, perm, cse, sx, aux);
+    else
+        hipLaunchKernelGGL((k_cells<CELLS_ATOMS / CELLS_NT, false>), dim3(nmol), dim3(CELLS_NT), lds, s, mols, m, put, pos, rad,
+                           start, perm, cse, sx, aux);
 }
 
 void qs_launch_put_mol(const QsMol &m, QsMol *dst, hipStream_t s) { hipLaunchKernelGGL(k_put_mol, dim3(1), dim3(64), 0, s, m, dst); }

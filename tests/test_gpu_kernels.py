@@ -134,3 +134,49 @@ def test_bounding_box_on_the_device(qs, n):
     nv, ni, pv, pt, pa = qs.compute_device(dp.ptr, dr.ptr, n, 1.0, 0)
     got = (hipmem.download(pv, (nv, 3), np.float32), hipmem.download(pt, (ni // 3, 3), np.int32), hipmem.download(pa, (nv,), np.int32))
     assert nv > 0 and _same(got, qs.compute_ses(pos, rad, 1.0, 0))
+
+
+def _cells_fetch(qs, what, n, dtype):
+    import ctypes
+
+    out = np.empty(n, dtype)
+    got = qs.lib().qs_fetch(what, ctypes.c_void_p(out.ctypes.data), ctypes.c_int64(out.nbytes))
+    assert got == out.nbytes
+    return out
+
+
+@pytest.mark.parametrize("sizes,box", [
+    ([2], 0), ([1023], 0), ([1025], 0), ([4096], 0), ([4097], 0), ([12288], 0), ([12289], 0),
+    ([1, 700, 0, 4096, 64, 2, 1024, 3000], 0), ([24576, 1, 5000, 0, 64, 2, 1024, 3000], 0), ([24577, 1, 5000, 0, 64, 2, 1024, 3000], 0),
+    ([200], 104.0), ([200], 110.0)])
+def test_cells_in_one_block_or_several_launches(qs, sizes, box):
+    """The cell order (cell, then index) and the cells' ranges at the sizes where one block takes over:
+    atoms gathered in the same launch up to 4,096, one molecule up to 12,288 atoms, a batch up to
+    24,576, and 49,152 cells (a box of 104 A has 36^3 cells, of 110 A 38^3)."""
+    rng = np.random.default_rng(len(sizes) + sum(sizes))
+    mols = []
+    for k, n in enumerate(sizes):
+        if box:
+            pos = (rng.random((n, 3)) * box).astype(np.float32)
+            pos[0], pos[1] = 0.0, box
+            mols.append((pos, np.full(n, 1.8, np.float32)))
+        else:
+            mols.append(qs.synth_ball(30 + k, n) if n else (np.zeros((0, 3), np.float32), np.zeros(0, np.float32)))
+    print("case cells: %s box=%g" % (sizes, box), flush=True)
+    qs.compute_batch(mols, 2.0, 0)
+    perm, cells, at = [], [], 0
+    for k, (pos, rad) in enumerate(mols):
+        G = qs.batch_grid(k)
+        gn, c = G["gn"], np.zeros(len(rad), np.int64)
+        for a in range(3):
+            e = ((pos[:, a] - np.float32(G["origin"][a])) / np.float32(G["dxn"])).astype(np.int64)
+            c = c * gn + np.clip(e, 0, gn - 1)
+        perm.append(at + np.argsort(c, kind="stable"))
+        lo = np.searchsorted(np.sort(c), np.arange(gn ** 3 + 1))
+        ranges = np.stack([at + lo[:-1], at + lo[1:]], -1)
+        ranges[lo[:-1] == lo[1:]] = 2 ** 31 - 2  # the marker of an empty cell
+        cells.append(ranges)
+        at += len(rad)
+    perm, cells = np.concatenate(perm), np.concatenate(cells)
+    assert np.array_equal(_cells_fetch(qs, b"perm", at, np.int32), perm)
+    assert np.array_equal(_cells_fetch(qs, b"cells", cells.size, np.int32).reshape(-1, 2), cells)
