@@ -749,7 +749,8 @@ static uint64_t plane_bytes(const QsMol &M)
 /* Planes each slab owns (CudaSurf.cu:626-636 sizes its slices from the SLICE setting instead),
    0 when the whole grid runs at once: that is when it fits the memory budget and its grid points
    fit 32-bit indexes (the grid-walk smoothing keys them so).  Option slab_planes forces slabs of
-   that many planes; option slab_mb sets the budget (default: half the device's free memory). */
+   that many planes; option slab_mb sets the budget (default: half the device's free memory, which
+   takes 13 us to ask for and is not asked for a grid that the engine's arrays already hold). */
 int Engine::slab_plan(const QsMol &M, int &planes)
 {
     planes = 0;
@@ -761,6 +762,11 @@ int Engine::slab_plan(const QsMol &M, int &planes)
     const uint64_t pb = plane_bytes(M);
     uint64_t budget = (uint64_t)g_opt.slab_mb << 20;
     if (!budget) {
+        const uint64_t vox = (uint64_t)g * g * g, nw = (uint64_t)g * g * M.W;
+        bool held = vox < (1ull << 32) && field.cap >= vox * 4 && s4.cap >= nw * 32 && ntb.cap >= nw * 24;
+        for (const DevBuf *b : {&outm, &shellm, &negm, &zerom}) held = held && b->cap >= nw * 8;
+        for (const DevBuf *b : {&wcnt, &vbw, &tbw, &alist, &avb, &acb}) held = held && b->cap >= nw * 4;
+        if (held) return 0;
         size_t free_b = 0, total_b = 0;
         QS_HIP(hipMemGetInfo(&free_b, &total_b));
         budget = free_b / 2;
