@@ -220,7 +220,8 @@ struct Engine {
     DevBuf colors_in;      /* per-atom colour table of qs_vertex_colors */
     DevBuf vert, vert2, vert3, vkey, tri, tri_out, atom;
     DevBuf deg_blk, keeppos, tri_loc;
-    DevBuf scan_tmp;
+    DevBuf scan_tmp, wsums /* tile sums of the marching-cubes word scans */;
+    bool wsums_clear = false; /* this run's field pass 1 cleared them */
     DevBuf inc_cnt, inc_start, inc_ent; /* per-vertex triangle incidences (smoothing of slab meshes) */
     DevBuf tpre_d;                      /* per-molecule first triangle (u64, nmol + 1), on the device */
     DevBuf tflag;                       /* field-pass-2 tiles holding a shell voxel (u8 per tile) */
@@ -337,7 +338,7 @@ struct Engine {
         for (DevBuf *b : {&in_pos, &in_rad, &d_off, &bb_part, &bb_out, &d_mols, &d_meta, &key, &count, &start,
                           &perm, &cse, &sx, &aux, &labels, &outm, &shellm, &field, &negm, &zerom, &s4, &wcnt,
                           &vbw, &tbw, &alist, &ntb, &avb, &acb, &vstart, &tstart, &normals, &colors_in, &totals, &bounds, &rback, &vert, &vert2, &vert3, &vkey,
-                          &tri, &tri_out, &atom, &deg_blk, &keeppos, &tri_loc, &scan_tmp, &inc_cnt, &inc_start, &inc_ent,
+                          &tri, &tri_out, &atom, &deg_blk, &keeppos, &tri_loc, &scan_tmp, &wsums, &inc_cnt, &inc_start, &inc_ent,
                           &tpre_d, &tflag, &field_dense})
             *b = DevBuf{};
         for (P2Tables *t : tables) delete t;
@@ -352,7 +353,7 @@ struct Engine {
         for (DevBuf *b : {&in_pos, &in_rad, &d_off, &bb_part, &bb_out, &d_mols, &d_meta, &key, &count, &start,
                           &perm, &cse, &sx, &aux, &labels, &outm, &shellm, &field, &negm, &zerom, &s4, &wcnt,
                           &vbw, &tbw, &alist, &ntb, &avb, &acb, &vstart, &tstart, &normals, &colors_in, &totals, &bounds, &rback, &vert, &vert2, &vert3, &vkey,
-                          &tri, &tri_out, &atom, &deg_blk, &keeppos, &tri_loc, &scan_tmp, &inc_cnt, &inc_start, &inc_ent,
+                          &tri, &tri_out, &atom, &deg_blk, &keeppos, &tri_loc, &scan_tmp, &wsums, &inc_cnt, &inc_start, &inc_ent,
                           &tpre_d, &tflag, &field_dense})
             release(*b);
         for (P2Tables *t : tables) {
@@ -457,6 +458,7 @@ struct Engine {
     int setup(const std::vector<MolIn> &in, const std::vector<BBox> &bb);
     int upload_mols();
     int fork_side();
+    int clear_wsums();
     int build_meta(size_t &at_atoms, size_t &at_p1, size_t &at_mc, size_t &at_wpre,
                    uint32_t &nb_atoms, uint32_t &nb_p1, uint32_t &nb_mc);
     /* allocate the workspace for batches up to these totals in one go */

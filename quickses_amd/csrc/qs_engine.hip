@@ -520,6 +520,10 @@ int Engine::field_stage(uint32_t nb_p1, size_t at_p1, StageTimer &tm)
     }
     /* this run's tile mark (the flags are not cleared: see qs_launch_pass1) */
     tmark = (uint8_t)(tmark == 255 ? 1 : tmark + 1);
+    /* the slab kernel clears the word scans' tile sums too */
+    const uint32_t nclear = p1mode == 0 ? (uint32_t)(4 * qs_scan_tiles(scan_nw)) : 0u;
+    QS_TRY(ensure(wsums, std::max<size_t>(nclear, 4) * 4));
+    wsums_clear = nb_p1 && p1mode == 0;
     if (nb_p1) {
         if (p1mode == 2)
             qs_launch_pass1_direct(batch(at_p1, 0, nmol), nb_p1, as<int2>(cse), as<float4>(sx), as<uint64_t>(outm),
@@ -528,7 +532,7 @@ int Engine::field_stage(uint32_t nb_p1, size_t at_p1, StageTimer &tm)
             qs_launch_pass1(batch(at_p1, 0, nmol), nb_p1, p1mode, p1_lds, as<uint32_t>(start), as<float4>(sx),
                             as<float4>(aux), as<uint64_t>(outm), as<uint64_t>(shellm),
                             p1mode == 0 ? as<uint64_t>(negm) : nullptr, p1mode == 0 ? as<uint64_t>(zerom) : nullptr, tf,
-                            tmark, stream);
+                            tmark, as<uint32_t>(wsums), nclear, stream);
         QS_HIP(hipGetLastError());
     }
     tm.mark("pass1");
@@ -591,6 +595,16 @@ int Engine::fork_side()
     return 0;
 }
 
+/* the word scans' tile sums start at zero: field pass 1 cleared them, or this does */
+int Engine::clear_wsums()
+{
+    const size_t bytes = 4 * qs_scan_tiles(std::max<uint64_t>(scan_nw, 1)) * sizeof(uint32_t);
+    QS_TRY(ensure(wsums, bytes));
+    if (!wsums_clear) QS_HIP(hipMemsetAsync(wsums.p, 0, bytes, stream));
+    wsums_clear = false;
+    return 0;
+}
+
 /* marching cubes over every molecule (sign masks must be ready) */
 int Engine::mesh_stage(size_t at_mc, uint32_t nb_mc, size_t at_wpre, StageTimer &tm, bool with_atoms)
 {
@@ -617,11 +631,11 @@ int Engine::mesh_stage(size_t at_mc, uint32_t nb_mc, size_t at_wpre, StageTimer 
     /* degenerate triangles per 256-triangle block and in total (totals[3]), counted by the
        triangle kernel (the block counts zeroed by the word scans, totals[3] by the scans) */
     QS_TRY(ensure(deg_blk, ((size_t)pool_t / 256 + 1) * 4));
+    QS_TRY(clear_wsums());
     if (nb_mc)
         qs_launch_mc_count(batch(at_mc, 0, nmol), nb_mc, as<uint64_t>(negm), as<uint64_t>(zerom), as<uint64_t>(s4),
-                           as<uint32_t>(wcnt), as<uint64_t>(ntb), stream);
+                           as<uint32_t>(wcnt), as<uint64_t>(ntb), as<uint32_t>(wsums), scan_w0, stream);
     if (scan_nw) {
-        QS_TRY(ensure(scan_tmp, 4 * qs_scan_tiles(scan_nw) * sizeof(uint32_t)));
         QsBlockStarts bs;
         bs.vstart = as<uint32_t>(vstart);
         bs.nv = pool_v / 256 + 1;
@@ -629,7 +643,7 @@ int Engine::mesh_stage(size_t at_mc, uint32_t nb_mc, size_t at_wpre, StageTimer 
         bs.nt = pool_t / 256 + 1;
         bs.zero = as<uint32_t>(deg_blk);
         bs.nzero = pool_t / 256 + 1;
-        qs_launch_mc_scans(as<uint32_t>(wcnt) + scan_w0, scan_nw, as<uint32_t>(scan_tmp),
+        qs_launch_mc_scans(as<uint32_t>(wcnt) + scan_w0, scan_nw, as<uint32_t>(wsums),
                            as<uint32_t>(vbw) + scan_w0, as<uint32_t>(tbw) + scan_w0, as<uint32_t>(alist), as<uint32_t>(avb),
                            as<uint32_t>(acb), as<uint32_t>(totals), (uint32_t)scan_w0, stream, bs);
         QS_HIP(hipGetLastError());
@@ -792,11 +806,11 @@ int Engine::slab_mesh(size_t at_mc, uint32_t nb_mc, size_t at_wpre, uint64_t own
     for (DevBuf *b : {&wcnt, &vbw, &tbw, &alist, &avb, &acb}) QS_TRY(ensure(*b, nw * 4));
     QS_TRY(ensure(ntb, nw * 24));
     QS_TRY(ensure(totals, 20));
+    QS_TRY(clear_wsums());
     if (nb_mc)
         qs_launch_mc_count(batch(at_mc, 0, 1), nb_mc, as<uint64_t>(negm), as<uint64_t>(zerom), as<uint64_t>(s4),
-                           as<uint32_t>(wcnt), as<uint64_t>(ntb), stream);
-    QS_TRY(ensure(scan_tmp, 4 * qs_scan_tiles(std::max<uint64_t>(scan_nw, 1)) * sizeof(uint32_t)));
-    qs_launch_mc_scans(as<uint32_t>(wcnt) + scan_w0, scan_nw, as<uint32_t>(scan_tmp),
+                           as<uint32_t>(wcnt), as<uint64_t>(ntb), as<uint32_t>(wsums), scan_w0, stream);
+    qs_launch_mc_scans(as<uint32_t>(wcnt) + scan_w0, scan_nw, as<uint32_t>(wsums),
                        as<uint32_t>(vbw) + scan_w0, as<uint32_t>(tbw) + scan_w0, as<uint32_t>(alist), as<uint32_t>(avb),
                        as<uint32_t>(acb), as<uint32_t>(totals), (uint32_t)scan_w0, stream);
     QS_HIP(hipGetLastError());
@@ -2055,6 +2069,7 @@ int qs_stage_mesh(const float *fp, const int *ip, const float *field, unsigned i
     qs_launch_field_signs(as<float>(E.field), G.g, W, as<uint32_t>(E.negm), as<uint32_t>(E.zerom), E.stream);
     StageTimer tm;
     for (int attempt = 0;; attempt++) {
+        E.wsums_clear = false;
         QS_TRY(E.mesh_stage(at_mc, nb_mc, at_wpre, tm, false));
         uint32_t hb[4];
         QS_HIP(hipMemcpyAsync(hb, E.totals.p, 16, hipMemcpyDeviceToHost, E.stream));

@@ -53,10 +53,10 @@ size_t qs_pass1_lds_bytes(const QsMol &M, int mode);
    tile holds no shell voxel (negm, zerom), and marks the tiles that do (tflag, at each molecule's
    tile_off, set to tmark); both may be NULL.  The flags are not cleared between runs: a run uses a
    mark of its own, and a stale flag that equals it only makes pass 2 rewrite the same sign words
-   for a tile without shell voxels. */
+   for a tile without shell voxels.  It clears nclear counters at clear on the way. */
 void qs_launch_pass1(QsBatch B, uint32_t nblocks, int mode, size_t lds_bytes, const uint32_t *cstart, const float4 *sx,
                      const float4 *aux, uint64_t *outm, uint64_t *shellm, uint64_t *negm, uint64_t *zerom, uint8_t *tflag,
-                     uint8_t tmark, hipStream_t s);
+                     uint8_t tmark, uint32_t *clear, uint32_t nclear, hipStream_t s);
 void qs_launch_pass1_direct(QsBatch B, uint32_t nblocks, const int2 *cse, const float4 *sx, uint64_t *outm, uint64_t *shellm,
                             hipStream_t s);
 
@@ -92,9 +92,11 @@ void qs_launch_labels_to_masks(const uint8_t *labels, int g, int W, uint64_t *ou
 uint32_t qs_mc_count_blocks(const QsMol &M);
 /* per row word: slot masks (words with vertices only), vertex and triangle counts, triangle-count
    bit planes (words with triangles only) */
-/* cnt: per row word its vertex, triangle and cube counts, packed */
+/* cnt: per row word its vertex, triangle and cube counts, packed; sums (cleared before): the counts'
+   sums {triangles, vertices, active words, cubes} per tile of the scans, which run over the words from
+   scan_w0 on that the launch counts */
 void qs_launch_mc_count(QsBatch B, uint32_t nblocks, const uint64_t *N, const uint64_t *Zm, uint64_t *S4, uint32_t *cnt,
-                        uint64_t *NT, hipStream_t s);
+                        uint64_t *NT, uint32_t *sums, uint64_t scan_w0, hipStream_t s);
 /* one thread per vertex / per polygonised cube over the active words (list, with their first
    vertex ids avb and first cubes acb), after one launch that gives vstart / tstart each 256-item
    block's first active word (nv / 256 + 1 and ncube / 256 + 1 entries) and clears deg_blk (ntri /
@@ -186,9 +188,8 @@ uint32_t qs_persistent_blocks(void);
 
 /* device-wide exclusive scan pieces */
 uint64_t qs_scan_tiles(uint64_t n);
-/* inputs of at most this many entries are scanned by one block in one launch (the generic scan,
-   and the marching-cubes word scans; one block's memory throughput makes more entries slower than
-   several blocks); inputs of at most QS_SCAN_SELF_TILES tiles of 2,048 are
+/* inputs of at most this many entries are scanned by one block in one launch (one block's memory
+   throughput makes more entries slower than several blocks); inputs of at most QS_SCAN_SELF_TILES tiles of 2,048 are
    scanned in two launches, each tile adding up the sums of the tiles before it itself */
 #define QS_SCAN1_MAX 8192u
 #define QS_SCAN_SELF_TILES 64u
@@ -213,8 +214,8 @@ struct QsBlockStarts {
 
 /* marching-cubes word scans over the packed counts of qs_launch_mc_count: vbw, tbw, the
    active-word list with its words' first vertices and cubes (avb, acb), and totals {triangles,
-   vertices, active words, 0, cubes}; sums holds 4 * qs_scan_tiles(nw) entries; list entries are list_base + the word's index in cnt; and the
-   block starts of bs */
+   vertices, active words, 0, cubes}; sums: its tile sums; list entries are list_base + the word's
+   index in cnt; and the block starts of bs */
 void qs_launch_mc_scans(const uint32_t *cnt, uint64_t nw, uint32_t *sums, uint32_t *vbw,
                         uint32_t *tbw, uint32_t *list, uint32_t *avb, uint32_t *acb, uint32_t *totals, uint32_t list_base,
                         hipStream_t s, QsBlockStarts bs = QsBlockStarts{});

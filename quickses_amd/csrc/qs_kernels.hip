@@ -212,6 +212,19 @@ __device__ __forceinline__ uint32_t wave_incl_scan(uint32_t x)
     x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x143, 0xc, 0xf, false); /* lane 31, to rows 2 and 3 */
     return x;
 }
+/* the next (previous) lane's v; lane 63 (0) gets edge */
+__device__ __forceinline__ uint64_t lane_above(uint64_t v, uint64_t edge)
+{
+    const int lo = __builtin_amdgcn_update_dpp((int)(uint32_t)edge, (int)(uint32_t)v, 0x130, 0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp((int)(uint32_t)(edge >> 32), (int)(uint32_t)(v >> 32), 0x130, 0xf, 0xf, false);
+    return (uint64_t)(uint32_t)hi << 32 | (uint32_t)lo;
+}
+__device__ __forceinline__ uint64_t lane_below(uint64_t v, uint64_t edge)
+{
+    const int lo = __builtin_amdgcn_update_dpp((int)(uint32_t)edge, (int)(uint32_t)v, 0x138, 0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp((int)(uint32_t)(edge >> 32), (int)(uint32_t)(v >> 32), 0x138, 0xf, 0xf, false);
+    return (uint64_t)(uint32_t)hi << 32 | (uint32_t)lo;
+}
 /* the largest of the wave's values */
 __device__ __forceinline__ uint32_t wave_max(uint32_t x)
 {
@@ -256,10 +269,11 @@ __device__ __forceinline__ uint32_t block_sum(uint32_t v, uint32_t *lds)
 
 /* sum of sums[0 .. b) for b <= 64, in every lane of the wave (a scan whose tile count is small
    takes its tiles' offsets this way instead of from a launch that scans the tile sums) */
+template <int STRIDE = 1>
 __device__ __forceinline__ uint32_t wave_sum_below(const uint32_t *__restrict__ sums, uint32_t b)
 {
     const uint32_t lane = threadIdx.x & 63;
-    return wave_last(wave_incl_scan((lane < b) ? sums[lane] : 0u));
+    return wave_last(wave_incl_scan((lane < b) ? sums[STRIDE * lane] : 0u));
 }
 
 /* bit position of the r-th set bit (from 0) of m, which has more than r */
@@ -344,57 +358,28 @@ __device__ __forceinline__ uint32_t word_cubes(uint32_t c) { return c >> 18; }
 
 /* Marching-cubes word scans in one pass: per row word its vertex, triangle and cube counts and
    "active" flag (any nonzero) are scanned together.  Plane 0 = triangles, 1 = vertices, 2 = active
-   words, 3 = cubes; tile sums are stored plane-major (4 x ntiles). */
-__global__ void __launch_bounds__(SCAN_NT) k_mc_reduce4(const uint32_t *__restrict__ cnt, uint64_t n, uint32_t *__restrict__ sums,
-                                                        uint64_t ntiles)
-{
-    __shared__ uint32_t lds[SCAN_NT / 64 + 1];
-    const uint64_t base = (uint64_t)blockIdx.x * SCAN_TILE;
-    uint32_t sv = 0, st = 0, sa = 0, sc = 0;
-#pragma unroll
-    for (int k = 0; k < SCAN_IPT; k++) {
-        const uint64_t i = base + (uint64_t)k * SCAN_NT + threadIdx.x;
-        if (i < n) {
-            const uint32_t c = cnt[i];
-            sv += word_verts(c);
-            st += word_tris(c);
-            sc += word_cubes(c);
-            sa += c ? 1u : 0u;
-        }
-    }
-    const uint32_t tt = block_sum<SCAN_NT>(st, lds);
-    const uint32_t tv = block_sum<SCAN_NT>(sv, lds);
-    const uint32_t ta = block_sum<SCAN_NT>(sa, lds);
-    const uint32_t tc = block_sum<SCAN_NT>(sc, lds);
-    if (threadIdx.x == 0) {
-        sums[blockIdx.x] = tt;
-        sums[ntiles + blockIdx.x] = tv;
-        sums[2 * ntiles + blockIdx.x] = ta;
-        sums[3 * ntiles + blockIdx.x] = tc;
-    }
-}
-
+   words, 3 = cubes; the count kernel adds up each tile's four sums, which lie together. */
 /* block p: exclusive scan of plane p of the tile sums in place, total to totals[p], plane 3's to
    totals[4]: totals[3] (the degenerate-triangle count, accumulated later) starts at zero */
 __global__ void __launch_bounds__(SCAN_NT) k_scan_planes(uint32_t *__restrict__ sums, uint64_t ntiles,
                                                          uint32_t *__restrict__ totals)
 {
     __shared__ uint32_t lds[SCAN_NT / 64 + 1];
-    uint32_t *plane = sums + (uint64_t)blockIdx.x * ntiles;
+    uint32_t *plane = sums + blockIdx.x; /* every fourth entry */
     uint32_t carry = 0;
     for (uint64_t b0 = 0; b0 < ntiles; b0 += SCAN_TILE) {
         const uint64_t base = b0 + (uint64_t)threadIdx.x * SCAN_IPT;
         uint32_t v[SCAN_IPT], s = 0;
 #pragma unroll
         for (int k = 0; k < SCAN_IPT; k++) {
-            v[k] = (base + k < ntiles) ? plane[base + k] : 0u;
+            v[k] = (base + k < ntiles) ? plane[4 * (base + k)] : 0u;
             s += v[k];
         }
         uint32_t tot;
         uint32_t run = carry + block_excl_scan<SCAN_NT>(s, &tot, lds);
 #pragma unroll
         for (int k = 0; k < SCAN_IPT; k++) {
-            if (base + k < ntiles) plane[base + k] = run;
+            if (base + k < ntiles) plane[4 * (base + k)] = run;
             run += v[k];
         }
         carry += tot;
@@ -415,7 +400,7 @@ __device__ __forceinline__ void mark_block_starts(uint32_t *__restrict__ start, 
 /* per word: first vertex (vbw) and first triangle (tbw); active words listed in order; with
    bs.vstart, the first active word of every 256-vertex and 256-cube block, and the triangle
    blocks' counters cleared */
-__global__ void __launch_bounds__(SCAN_NT) k_mc_scan4(const uint32_t *__restrict__ cnt, uint64_t n, const uint32_t *__restrict__ sums, uint64_t ntiles,
+__global__ void __launch_bounds__(SCAN_NT) k_mc_scan4(const uint32_t *__restrict__ cnt, uint64_t n, const uint32_t *__restrict__ sums,
                                                       uint32_t *__restrict__ vbw, uint32_t *__restrict__ tbw,
                                                       uint32_t *__restrict__ list, uint32_t *__restrict__ avb,
                                                       uint32_t *__restrict__ acb, uint32_t list_base, int self,
@@ -464,10 +449,10 @@ __global__ void __launch_bounds__(SCAN_NT) k_mc_scan4(const uint32_t *__restrict
     __syncthreads();
     uint32_t ov, ot, oa, oc;
     if (self) {
-        ot = wave_sum_below(sums, blockIdx.x);
-        ov = wave_sum_below(sums + ntiles, blockIdx.x);
-        oa = wave_sum_below(sums + 2 * ntiles, blockIdx.x);
-        oc = wave_sum_below(sums + 3 * ntiles, blockIdx.x);
+        ot = wave_sum_below<4>(sums, blockIdx.x);
+        ov = wave_sum_below<4>(sums + 1, blockIdx.x);
+        oa = wave_sum_below<4>(sums + 2, blockIdx.x);
+        oc = wave_sum_below<4>(sums + 3, blockIdx.x);
         if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) {
             uint32_t tv = ov, tt = ot, ta = oa, tc = oc;
             for (int w = 0; w < SCAN_NT / 64; w++) {
@@ -483,10 +468,10 @@ __global__ void __launch_bounds__(SCAN_NT) k_mc_scan4(const uint32_t *__restrict
             totals[4] = tc;
         }
     } else {
-        ov = sums[ntiles + blockIdx.x];
-        ot = sums[blockIdx.x];
-        oa = sums[2 * ntiles + blockIdx.x];
-        oc = sums[3 * ntiles + blockIdx.x];
+        ot = sums[4 * (size_t)blockIdx.x];
+        ov = sums[4 * (size_t)blockIdx.x + 1];
+        oa = sums[4 * (size_t)blockIdx.x + 2];
+        oc = sums[4 * (size_t)blockIdx.x + 3];
     }
     for (int w = 0; w < wid; w++) {
         ov += wsum[0][w];
@@ -514,8 +499,8 @@ __global__ void __launch_bounds__(SCAN_NT) k_mc_scan4(const uint32_t *__restrict
     }
 }
 
-/* The same scans in one block of SCAN1_NT threads for at most QS_SCAN1_MAX entries: one launch
-   instead of three for a small grid.  The block runs over chunks of SCAN1_NT * SCAN_IPT entries in
+/* The generic scan in one block of SCAN1_NT threads for at most QS_SCAN1_MAX entries: one launch
+   instead of three.  The block runs over chunks of SCAN1_NT * SCAN_IPT entries in
    order, each wave 64 consecutive entries per load as above, carrying the running totals. */
 #define SCAN1_NT 1024
 #define SCAN1_W (SCAN1_NT / 64)
@@ -569,85 +554,6 @@ __global__ void __launch_bounds__(SCAN1_NT) k_scan1(const uint32_t *in, uint32_t
         __syncthreads(); /* wsum is written again for the next chunk */
     }
     if (total && threadIdx.x == 0) *total = carry;
-}
-
-/* marching-cubes word scans (as k_mc_reduce4, k_scan_planes, k_mc_scan4): totals = {triangles,
-   vertices, active words, 0, cubes} */
-__global__ void __launch_bounds__(SCAN1_NT) k_mc_scan1(const uint32_t *__restrict__ cnt, uint64_t n, uint32_t *__restrict__ vbw, uint32_t *__restrict__ tbw,
-                                                       uint32_t *__restrict__ list, uint32_t *__restrict__ avb,
-                                                       uint32_t *__restrict__ acb, uint32_t list_base,
-                                                       uint32_t *__restrict__ totals, QsBlockStarts bs)
-{
-    __shared__ uint32_t wsum[4][SCAN1_W];
-    if (bs.zero)
-        for (uint32_t i = threadIdx.x; i < bs.nzero; i += SCAN1_NT) bs.zero[i] = 0u;
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    const uint64_t lbelow = (1ull << lane) - 1ull;
-    uint32_t cv = 0, ct = 0, ca = 0, cc = 0;
-    for (uint64_t c0 = 0; c0 < n; c0 += SCAN1_NT * SCAN_IPT) {
-        const uint64_t base = c0 + (uint64_t)wid * (64 * SCAN_IPT) + lane;
-        uint32_t v[SCAN_IPT], t[SCAN_IPT], q[SCAN_IPT], pa[SCAN_IPT], raw[SCAN_IPT];
-        uint32_t ra = 0;
-#pragma unroll
-        for (int k = 0; k < SCAN_IPT; k++) {
-            const uint64_t i = base + 64 * k;
-            const uint32_t c = (i < n) ? cnt[i] : 0u;
-            v[k] = word_verts(c);
-            t[k] = word_tris(c);
-            q[k] = word_cubes(c);
-            raw[k] = c;
-        }
-#pragma unroll
-        for (int k = 0; k < SCAN_IPT; k++) {
-            const uint64_t am = __ballot(raw[k] != 0u);
-            pa[k] = ra + (uint32_t)__popcll(am & lbelow);
-            ra += (uint32_t)__popcll(am);
-        }
-        const uint32_t rv = wave_groups_scan(v), rt = wave_groups_scan(t), rc = wave_groups_scan(q);
-        if (lane == 0) {
-            wsum[0][wid] = rv;
-            wsum[1][wid] = rt;
-            wsum[2][wid] = ra;
-            wsum[3][wid] = rc;
-        }
-        __syncthreads();
-        uint32_t bv, av, bt, at, ba, aa, bc, ac;
-        scan1_offsets(wsum[0], wid, bv, av);
-        scan1_offsets(wsum[1], wid, bt, at);
-        scan1_offsets(wsum[2], wid, ba, aa);
-        scan1_offsets(wsum[3], wid, bc, ac);
-#pragma unroll
-        for (int k = 0; k < SCAN_IPT; k++) {
-            const uint64_t i = base + 64 * k;
-            if (i < n) {
-                const uint32_t fv = cv + bv + v[k], ft = ct + bt + t[k];
-                vbw[i] = fv;
-                tbw[i] = ft;
-                if (raw[k]) {
-                    const uint32_t r = ca + ba + pa[k], fc = cc + bc + q[k];
-                    avb[r] = fv;
-                    acb[r] = fc;
-                    list[r] = list_base + (uint32_t)i;
-                    if (bs.vstart) {
-                        mark_block_starts(bs.vstart, bs.nv, fv, word_verts(raw[k]), r);
-                        mark_block_starts(bs.tstart, bs.nt, fc, word_cubes(raw[k]), r);
-                    }
-                }
-            }
-        }
-        cv += av;
-        ct += at;
-        ca += aa;
-        cc += ac;
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) {
-        totals[0] = ct;
-        totals[1] = cv;
-        totals[2] = ca;
-        totals[3] = 0u;
-        totals[4] = cc;
-    }
 }
 
 /* ------------------------------------------------------------------------------------------ */
@@ -1358,8 +1264,11 @@ __global__ void __launch_bounds__(256) k_pass1_slab(QsBatch B, const uint32_t *_
                                                     const float4 *__restrict__ sx, const float4 *__restrict__ aux,
                                                     uint64_t *__restrict__ outm_all, uint64_t *__restrict__ shellm_all,
                                                     uint64_t *__restrict__ negm_all, uint64_t *__restrict__ zerom_all,
-                                                    uint8_t *__restrict__ tflag, uint8_t tmark)
+                                                    uint8_t *__restrict__ tflag, uint8_t tmark,
+                                                    uint32_t *__restrict__ clear, uint32_t nclear)
 {
+    /* counters that a later launch adds to */
+    for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < nclear; i += gridDim.x * 256u) clear[i] = 0u;
     extern __shared__ __align__(16) uint64_t p1s_dyn[];
     __shared__ uint32_t colpre[P1S_MAXCOL + 1], colst[P1S_MAXCOL];
     __shared__ int q_id[4][P1_QCAP], q_rows[4][P1_QCAP], q_z[4][P1_QCAP];
@@ -2608,7 +2517,8 @@ struct MCView {
 /* countVertexPerCell MarchingCubes.cu:571-658 in word form: slot masks and per-word counts */
 __global__ void __launch_bounds__(256) k_mc_count(QsBatch B, const uint64_t *__restrict__ N_all,
                                                   const uint64_t *__restrict__ Zm_all, uint64_t *__restrict__ S4_all,
-                                                  uint32_t *__restrict__ cnt_all, uint64_t *__restrict__ NT_all)
+                                                  uint32_t *__restrict__ cnt_all, uint64_t *__restrict__ NT_all,
+                                                  uint32_t *__restrict__ sums, uint64_t scan_w0)
 {
     uint32_t lb;
     const QsMol &M = B.mols[batch_mol(B, xcd_block(blockIdx.x, gridDim.x), lb)];
@@ -2621,7 +2531,9 @@ __global__ void __launch_bounds__(256) k_mc_count(QsBatch B, const uint64_t *__r
     const uint32_t nbx = ((uint32_t)g * W + 255) / 256;
     const int idx = (int)(lb % nbx) * 256 + threadIdx.x;
     const int x = M.mc_lo + (int)(lb / nbx);
-    if (idx >= g * W || x >= M.mc_hi) return;
+    if (x >= M.mc_hi) return; /* whole block */
+    uint32_t counts = 0;
+    if (idx < g * W) {
     const int y = idx / W, w = idx - y * W;
     const int z0 = w * 64;
     const size_t wi = ((size_t)x * g + y) * W + w;
@@ -2632,20 +2544,33 @@ __global__ void __launch_bounds__(256) k_mc_count(QsBatch B, const uint64_t *__r
 
     /* the word and its neighbours one step along x, y and w, loaded together without branches: a
        neighbour outside the grid reads the word itself and is masked to zero (the point itself
-       is inside the grid) */
+       is inside the grid).  Bound by the address unit, which takes 16 cycles for a wave's load: the
+       neighbours along w come from the neighbour lanes (count and scans of 1M atoms at 0.5 A 144 us
+       with thirteen loads, 139 with seven; of 100 frames of 10,000 atoms 176 and 169) */
     const size_t sx = (size_t)g * W;
     const uint64_t *__restrict__ np = N + wi;
     const uint64_t *__restrict__ zp = Zm + wi;
     const bool hx = x + 1 < g, hy = y + 1 < g, hw = w + 1 < W;
     const size_t ox = hx ? sx : 0, oy = hy ? (size_t)W : 0, ow = hw ? 1 : 0;
     const uint64_t mx = hx ? ~0ull : 0ull, my = hy ? ~0ull : 0ull, mw = hw ? ~0ull : 0ull;
-    const uint64_t n00 = np[0], n00p = np[ow] & mw, n00m = np[w > 0 ? -1 : 0] & (w > 0 ? ~0ull : 0ull);
-    const uint64_t z00 = zp[0], z00p = zp[ow] & mw;
+    const uint64_t n00 = np[0], z00 = zp[0];
     const uint64_t n10 = np[ox] & mx, z10 = zp[ox] & mx;
     const uint64_t n01 = np[oy] & my, z01 = zp[oy] & my;
-    /* the cube's far x, y corners and the next words of its top corners */
+    /* the cube's far x, y corner, and the next words of its top corners: the next lane's words, but
+       for lane 63 */
     const uint64_t n11 = np[ox + oy] & mx & my;
-    const uint64_t n10p = np[ox + ow] & mx & mw, n11p = np[ox + oy + ow] & mx & my & mw, n01p = np[oy + ow] & my & mw;
+    uint64_t e00 = 0, ez00 = 0, e10 = 0, e01 = 0, e11 = 0, d00 = 0;
+    if ((threadIdx.x & 63) == 63) {
+        e00 = np[ow];
+        ez00 = zp[ow];
+        e10 = np[ox + ow] & mx;
+        e01 = np[oy + ow] & my;
+        e11 = np[ox + oy + ow] & mx & my;
+    }
+    if ((threadIdx.x & 63) == 0) d00 = np[w > 0 ? -1 : 0];
+    const uint64_t n00p = lane_above(n00, e00) & mw, z00p = lane_above(z00, ez00) & mw, n10p = lane_above(n10, e10) & mw;
+    const uint64_t n01p = lane_above(n01, e01) & mw, n11p = lane_above(n11, e11) & mw;
+    const uint64_t n00m = lane_below(n00, d00) & (w > 0 ? ~0ull : 0ull);
     const uint64_t n00_up = (n00 >> 1) | (n00p << 63); /* bit z = N[z+1] */
     const uint64_t n00_dn = (n00 << 1) | (n00m >> 63); /* bit z = N[z-1] */
     const uint64_t z00_up = (z00 >> 1) | (z00p << 63);
@@ -2724,7 +2649,36 @@ __global__ void __launch_bounds__(256) k_mc_count(QsBatch B, const uint64_t *__r
             NT[2] = p2;
         }
     }
-    cnt[wi] = word_counts(nv, nt, nc);
+    counts = word_counts(nv, nt, nc);
+    cnt[wi] = counts;
+    }
+    /* The block's counts go to the sums of their scan tiles: one tile, or two where the block crosses a
+       boundary (then wave by wave).  A launch that reads all counts again for that took 21 us on the
+       50,000-atom 0.2 A mesh and 30 on 256 molecules at 0.5 A; four adds per wave took 10 and 27 more
+       than it. */
+    __shared__ unsigned long long part[4][2];
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    const uint64_t s0 = M.word_off + (uint64_t)x * g * W - scan_w0;
+    const uint32_t b0 = (lb % nbx) * 256u, tile = (uint32_t)((s0 + (uint32_t)idx) / SCAN_TILE);
+    const uint32_t t0 = (uint32_t)((s0 + b0) / SCAN_TILE), t1 = (uint32_t)((s0 + min(b0 + 255u, (uint32_t)(g * W) - 1u)) / SCAN_TILE);
+    for (uint32_t t = t0; t <= t1; t++) {
+        const uint32_t c = tile == t ? counts : 0u;
+        const uint32_t na = (uint32_t)__popcll(__ballot(c != 0u));
+        unsigned long long p0 = 0ull, p1 = 0ull;
+        if (na) {
+            /* (at most 64 x 256 vertices, 64 x 320 triangles, 64 x 64 cubes) */
+            const uint32_t vt = wave_last(wave_incl_scan(word_verts(c) | word_tris(c) << 16));
+            p0 = (unsigned long long)(vt >> 16) | (unsigned long long)(vt & 0xFFFFu) << 32;
+            p1 = (unsigned long long)na | (unsigned long long)wave_last(wave_incl_scan(word_cubes(c))) << 32;
+        }
+        if (lane < 2) part[wid][lane] = lane ? p1 : p0;
+        __syncthreads();
+        if (threadIdx.x < 2) {
+            const unsigned long long p = part[0][lane] + part[1][lane] + part[2][lane] + part[3][lane];
+            if (p) atomicAdd((unsigned long long *)sums + 2 * (size_t)t + lane, p);
+        }
+        __syncthreads(); /* part is written again for the next tile */
+    }
 }
 
 /* row word wi of a grid -> (x, y, word) */
@@ -3962,13 +3916,13 @@ size_t qs_pass1_lds_bytes(const QsMol &M, int mode)
 
 void qs_launch_pass1(QsBatch B, uint32_t nblocks, int mode, size_t lds_bytes, const uint32_t *cstart, const float4 *sx,
                      const float4 *aux, uint64_t *outm, uint64_t *shellm, uint64_t *negm, uint64_t *zerom, uint8_t *tflag,
-                     uint8_t tmark, hipStream_t s)
+                     uint8_t tmark, uint32_t *clear, uint32_t nclear, hipStream_t s)
 {
     if (mode == 1)
         hipLaunchKernelGGL(k_pass1_rows, dim3(nblocks), dim3(256), 0, s, B, cstart, sx, aux, outm, shellm);
     else
         hipLaunchKernelGGL(k_pass1_slab, dim3(nblocks), dim3(256), lds_bytes, s, B, cstart, sx, aux, outm, shellm, negm, zerom,
-                           tflag, tmark);
+                           tflag, tmark, clear, nclear);
 }
 
 void qs_launch_pass1_direct(QsBatch B, uint32_t nblocks, const int2 *cse, const float4 *sx, uint64_t *outm, uint64_t *shellm,
@@ -4042,9 +3996,9 @@ uint32_t qs_mc_count_blocks(const QsMol &M)
 }
 
 void qs_launch_mc_count(QsBatch B, uint32_t nblocks, const uint64_t *N, const uint64_t *Zm, uint64_t *S4, uint32_t *cnt,
-                        uint64_t *NT, hipStream_t s)
+                        uint64_t *NT, uint32_t *sums, uint64_t scan_w0, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_mc_count, dim3(nblocks), dim3(256), 0, s, B, N, Zm, S4, cnt, NT);
+    hipLaunchKernelGGL(k_mc_count, dim3(nblocks), dim3(256), 0, s, B, N, Zm, S4, cnt, NT, sums, scan_w0);
 }
 
 void qs_launch_mc_emit(const QsMol *mols, const uint64_t *wpre, const uint32_t *wcoarse, const uint32_t *list, uint32_t nact,
@@ -4178,16 +4132,10 @@ void qs_launch_mc_scans(const uint32_t *cnt, uint64_t nw, uint32_t *sums, uint32
                         hipStream_t s, QsBlockStarts bs)
 {
     if (!nw) return;
-    if (nw <= QS_SCAN1_MAX) {
-        hipLaunchKernelGGL(k_mc_scan1, dim3(1), dim3(SCAN1_NT), 0, s, cnt, nw, vbw, tbw, list, avb, acb, list_base,
-                           totals, bs);
-        return;
-    }
     const uint64_t ntiles = qs_scan_tiles(nw);
     const int self = ntiles <= QS_SCAN_SELF_TILES;
-    hipLaunchKernelGGL(k_mc_reduce4, dim3((unsigned)ntiles), dim3(SCAN_NT), 0, s, cnt, nw, sums, ntiles);
     if (!self) hipLaunchKernelGGL(k_scan_planes, dim3(4), dim3(SCAN_NT), 0, s, sums, ntiles, totals);
-    hipLaunchKernelGGL(k_mc_scan4, dim3((unsigned)ntiles), dim3(SCAN_NT), 0, s, cnt, nw, sums, ntiles, vbw, tbw, list,
+    hipLaunchKernelGGL(k_mc_scan4, dim3((unsigned)ntiles), dim3(SCAN_NT), 0, s, cnt, nw, sums, vbw, tbw, list,
                        avb, acb, list_base, self, totals, bs);
 }
 
