@@ -2771,17 +2771,18 @@ __device__ __forceinline__ void item_word(const ItemWords &S, const uint32_t *__
                                           const uint32_t *__restrict__ list, uint32_t i, uint32_t &k, uint32_t &wi,
                                           uint32_t &first)
 {
-    if (S.nk <= 257u) {
-        uint32_t lo = 0, hi = S.nk - 1u;
-        while (lo < hi) {
-            const uint32_t mid = (lo + hi + 1) >> 1;
-            if (S.base[mid] <= i) lo = mid;
-            else hi = mid - 1;
-        }
-        k = S.k0 + lo;
-        wi = S.word[lo];
-        first = S.base[lo];
-    } else {
+    uint32_t lo = 0, hi = min(S.nk, 257u) - 1u;
+    while (lo < hi) {
+        const uint32_t mid = (lo + hi + 1) >> 1;
+        if (S.base[mid] <= i) lo = mid;
+        else hi = mid - 1;
+    }
+    k = S.k0 + lo;
+    wi = S.word[lo];
+    first = S.base[lo];
+    /* (opaque, so that these stay LDS reads: merged with the loads below they become flat loads) */
+    asm volatile("" : "+v"(wi), "+v"(first));
+    if (S.nk > 257u) { /* not staged */
         k = last_le(base, S.k0, S.k0 + S.nk - 1u, i);
         wi = list[k];
         first = base[k];
@@ -2997,7 +2998,7 @@ __global__ void __launch_bounds__(256) k_closest_atom(const QsMol *__restrict__ 
 {
     if (d_nv) nv = min(*d_nv, nv); /* the device count within the launch's pool */
     const uint32_t nb = (nv + 255u) >> 8;
-    /* persistent blocks over the 256-vertex blocks (grid a multiple of 8: see k_mc_vertices) */
+    /* persistent blocks over the 256-vertex blocks (grid a multiple of 8: see k_mc_emit) */
     for (uint32_t vb = blockIdx.x; vb < nb; vb += gridDim.x) {
         const uint32_t v = xcd_group<64>(vb, nb) * 256u + threadIdx.x;
         if (v >= nv) continue;
@@ -3012,16 +3013,36 @@ __global__ void __launch_bounds__(256) k_closest_atom(const QsMol *__restrict__ 
    vertex: its word from the active words' first vertex ids, its point and slot from the word's
    four slot masks (vertex ids run over the word's points in z order, slots x, y, z, point).
    ATOMS: the vertex's closest atom in the same pass (A). */
-template <bool ATOMS>
-__global__ void __launch_bounds__(256) k_mc_vertices(const QsMol *__restrict__ mols, const uint64_t *__restrict__ wpre,
-                                                     const uint32_t *__restrict__ wcoarse, const uint32_t *__restrict__ list,
-                                                     const uint32_t *__restrict__ avb, const uint32_t *__restrict__ vstart,
-                                                     uint32_t nact, uint32_t nv, const uint64_t *__restrict__ S4_all,
-                                                     const float *__restrict__ F_all, const uint64_t *__restrict__ outm_all,
-                                                     const uint64_t *__restrict__ shellm_all, float *__restrict__ vert,
-                                                     uint64_t *__restrict__ vkey, const uint32_t *__restrict__ d_counts, QsClosest A)
+/* triangles (generateTriangleVerticesSMEM MarchingCubes.cu:736-851 order), one thread per
+   polygonised cube (two triangles on average): its word from the active words' first cubes, its
+   place from the word's triangle-count planes.  Bound by the dependent memory trips of a block
+   (block start, word list, planes, corner masks) and by VALU issue, so both are paid once per cube:
+   the thread loads the sign words, slot masks and vertex counts of the cube's four (x, y) columns
+   together, and every corner's vertex id comes from them.  One thread per triangle, three corners'
+   masks each, took 0.20 ms on the 50,000-atom 0.2 A mesh and 0.92 ms on 256 molecules at 0.5 A
+   (47 M triangles); this takes 0.15 and 0.62 ms.  (64 registers for eight waves per SIMD, with
+   spills, were slower than 66 with seven: emission 1.11 against 1.06 ms.) */
+/* The two are launches of their own (VERT or TRI) or, for a small mesh, whose time is that of the
+   launches in turn, one launch whose first nbv blocks are the vertices': 7 us of 25 less on 2,000
+   atoms at 0.5 A. */
+template <bool VERT, bool TRI, bool ATOMS>
+__global__ void __launch_bounds__(256) k_mc_emit(const QsMol *__restrict__ mols, const uint64_t *__restrict__ wpre,
+                                                 const uint32_t *__restrict__ wcoarse, const uint32_t *__restrict__ list,
+                                                 const uint32_t *__restrict__ avb, const uint32_t *__restrict__ vstart,
+                                                 uint32_t nact, uint32_t nv, const uint64_t *__restrict__ S4_all,
+                                                 const float *__restrict__ F_all, const uint64_t *__restrict__ outm_all,
+                                                 const uint64_t *__restrict__ shellm_all, float *__restrict__ vert,
+                                                 uint64_t *__restrict__ vkey, const uint32_t *__restrict__ d_counts,
+                                                 const uint32_t *__restrict__ acb, const uint32_t *__restrict__ tstart,
+                                                 uint32_t ncube, uint32_t ntri, const uint64_t *__restrict__ N,
+                                                 const uint32_t *__restrict__ cnt, const uint32_t *__restrict__ vbw,
+                                                 const uint32_t *__restrict__ tbw, const uint64_t *__restrict__ NT,
+                                                 int *__restrict__ tri, uint32_t vbase, uint32_t *__restrict__ deg_blk,
+                                                 uint32_t *__restrict__ deg_total, QsClosest A, uint32_t nbv)
 {
     __shared__ ItemWords S;
+    if constexpr (VERT) {
+    if (!TRI || blockIdx.x < nbv) {
     /* with d_counts (triangles, vertices, active words) the counts come from the device, the
        launch covering the pool of nv vertices: blocks past the count leave at once */
     if (d_counts) {
@@ -3031,7 +3052,7 @@ __global__ void __launch_bounds__(256) k_mc_vertices(const QsMol *__restrict__ m
     const uint32_t nb = (nv + 255u) >> 8;
     /* persistent blocks over the 256-vertex blocks; the grid is a multiple of 8, so block vb runs
        on XCD vb % 8 and the renumbering keeps neighbouring rows' words on one L2 */
-    for (uint32_t vb = blockIdx.x; vb < nb; vb += gridDim.x) {
+    for (uint32_t vb = blockIdx.x; vb < nb; vb += VERT && TRI ? nbv : gridDim.x) {
     const uint32_t blk = xcd_group<64>(vb, nb);
     stage_item_words(S, avb, list, vstart, nact, nb, blk, wpre, wcoarse);
     const uint32_t v = blk * 256u + threadIdx.x;
@@ -3097,37 +3118,19 @@ __global__ void __launch_bounds__(256) k_mc_vertices(const QsMol *__restrict__ m
     }
     __syncthreads(); /* S is staged again for the next block */
     }
-}
-
-/* triangles (generateTriangleVerticesSMEM MarchingCubes.cu:736-851 order), one thread per
-   polygonised cube (two triangles on average): its word from the active words' first cubes, its
-   place from the word's triangle-count planes.  Bound by the dependent memory trips of a block
-   (block start, word list, planes, corner masks) and by VALU issue, so both are paid once per cube:
-   the thread loads the sign words, slot masks and vertex counts of the cube's four (x, y) columns
-   together, and every corner's vertex id comes from them.  One thread per triangle, three corners'
-   masks each, took 0.20 ms on the 50,000-atom 0.2 A mesh and 0.92 ms on 256 molecules at 0.5 A
-   (47 M triangles); this takes 0.15 and 0.62 ms.  (64 registers for eight waves per SIMD, with
-   spills, were slower than 66 with seven: emission 1.11 against 1.06 ms.) */
-__global__ void __launch_bounds__(256) k_mc_triangles(const QsMol *__restrict__ mols, const uint64_t *__restrict__ wpre,
-                                                      const uint32_t *__restrict__ wcoarse, const uint32_t *__restrict__ list,
-                                                      const uint32_t *__restrict__ acb, const uint32_t *__restrict__ tstart,
-                                                      uint32_t nact, uint32_t ncube, uint32_t ntri, const uint64_t *__restrict__ N,
-                                                      const uint64_t *__restrict__ S4, const uint32_t *__restrict__ cnt,
-                                                      const uint32_t *__restrict__ vbw, const uint32_t *__restrict__ tbw,
-                                                      const uint64_t *__restrict__ NT, int *__restrict__ tri, uint32_t vbase,
-                                                      uint32_t *__restrict__ deg_blk, uint32_t *__restrict__ deg_total,
-                                                      const uint32_t *__restrict__ d_counts)
-{
-    __shared__ ItemWords S;
+    return;
+    }
+    }
+    if constexpr (TRI) {
     __shared__ uint32_t S_before[4][256]; /* per cube: vertices before its four columns' lower points */
-    /* counts from the device as in k_mc_vertices; triangles past the pool are not written */
+    /* counts from the device as for the vertices; triangles past the pool are not written */
     if (d_counts) {
         nact = d_counts[2];
         ncube = min(d_counts[4], ncube);
     }
     const uint32_t nb = (ncube + 255u) >> 8;
-    /* persistent blocks over the 256-cube blocks, as in k_mc_vertices */
-    for (uint32_t vb = blockIdx.x; vb < nb; vb += gridDim.x) {
+    /* persistent blocks over the 256-cube blocks, as for the vertices */
+    for (uint32_t vb = blockIdx.x - (VERT ? nbv : 0u); vb < nb; vb += gridDim.x - (VERT ? nbv : 0u)) {
     const uint32_t blk = xcd_group<64>(vb, nb);
     stage_item_words(S, acb, list, tstart, nact, nb, blk, wpre, wcoarse);
     const uint32_t cube = blk * 256u + threadIdx.x;
@@ -3155,7 +3158,7 @@ __global__ void __launch_bounds__(256) k_mc_triangles(const QsMol *__restrict__ 
             nv4[q] = word_verts(cnt[cw]);
             vb4[q] = vbw[cw];
 #pragma unroll
-            for (int a = 0; a < 4; a++) s[q][a] = S4[4 * cw + a];
+            for (int a = 0; a < 4; a++) s[q][a] = S4_all[4 * cw + a];
         }
         uint32_t sg = 0; /* sign bits, bit 2 q + z */
 #pragma unroll
@@ -3178,7 +3181,7 @@ __global__ void __launch_bounds__(256) k_mc_triangles(const QsMol *__restrict__ 
                 sg |= (uint32_t)(N[cw] & 1ull) << (2 * q + 1);
                 uint32_t m = 0;
 #pragma unroll
-                for (int a = 0; a < 4; a++) m |= (uint32_t)(S4[4 * cw + a] & 1ull) << (2 * a + 1);
+                for (int a = 0; a < 4; a++) m |= (uint32_t)(S4_all[4 * cw + a] & 1ull) << (2 * a + 1);
                 if (word_verts(cnt[cw])) {
                     /* (a word without vertices below has none of its own slots set) */
                     sl = (has >> q) & 1u ? sl : sl & ~(255u << (8 * q));
@@ -3242,6 +3245,7 @@ __global__ void __launch_bounds__(256) k_mc_triangles(const QsMol *__restrict__ 
         }
     }
     __syncthreads(); /* S is staged again for the next block */
+    }
     }
 }
 
@@ -3442,7 +3446,7 @@ __global__ void __launch_bounds__(256) k_smooth(const QsMol *__restrict__ mols, 
     if (d_nv && *d_nv > nv) return;
     if (d_nv) nv = *d_nv;
     const uint32_t nb = (nv + 255u) >> 8;
-    /* persistent blocks over the 256-vertex blocks (grid a multiple of 8: see k_mc_vertices) */
+    /* persistent blocks over the 256-vertex blocks (grid a multiple of 8: see k_mc_emit) */
     for (uint32_t vb = blockIdx.x; vb < nb; vb += gridDim.x) {
         const uint32_t v = xcd_group<64>(vb, nb) * 256u + threadIdx.x;
         if (v >= nv) continue;
@@ -4018,18 +4022,34 @@ void qs_launch_mc_emit(const QsMol *mols, const uint64_t *wpre, const uint32_t *
     if (!starts_ready)
         hipLaunchKernelGGL(k_block_starts, dim3(pgrid(nblk(std::max<uint32_t>(nact, nzero), 256)), 2), dim3(256), 0, s, sv, st,
                            nact, d_counts ? d_counts + 2 : nullptr);
-    if (nv) {
-        const dim3 grid(pgrid(nblk(std::min(nv, expect), 256)));
-        if (atoms)
-            hipLaunchKernelGGL(k_mc_vertices<true>, grid, dim3(256), 0, s, mols, wpre, wcoarse, list, avb, vstart, nact, nv, S4, F,
-                               outm, shellm, vert, vkey, d_counts, *atoms);
-        else
-            hipLaunchKernelGGL(k_mc_vertices<false>, grid, dim3(256), 0, s, mols, wpre, wcoarse, list, avb, vstart, nact, nv, S4, F,
-                               outm, shellm, vert, vkey, d_counts, QsClosest{});
+    const unsigned gv = nv ? pgrid(nblk(std::min(nv, expect), 256)) : 0u, gt = ntri ? pgrid(nblk(std::min(ncube, expect), 256)) : 0u;
+    if (atoms && gv && gt) {
+        hipLaunchKernelGGL((k_mc_emit<true, true, true>), dim3(gv + gt), dim3(256), 0, s, mols, wpre, wcoarse, list, avb,
+                                                                                          vstart, nact, nv, S4, F, outm, shellm,
+                                                                                          vert, vkey, d_counts, acb, tstart,
+                                                                                          ncube, ntri, N, cnt, vbw, tbw, NT,
+                                                                                          tri, vbase, deg_blk, deg_total,
+                                                                                          *atoms, gv);
+        return;
     }
-    if (ntri)
-        hipLaunchKernelGGL(k_mc_triangles, dim3(pgrid(nblk(std::min(ncube, expect), 256))), dim3(256), 0, s, mols, wpre, wcoarse, list, acb, tstart,
-                           nact, ncube, ntri, N, S4, cnt, vbw, tbw, NT, tri, vbase, deg_blk, deg_total, d_counts);
+    if (gv && atoms)
+        hipLaunchKernelGGL((k_mc_emit<true, false, true>), dim3(gv), dim3(256), 0, s, mols, wpre, wcoarse, list, avb, vstart,
+                                                                                      nact, nv, S4, F, outm, shellm, vert, vkey,
+                                                                                      d_counts, acb, tstart, ncube, ntri, N,
+                                                                                      cnt, vbw, tbw, NT, tri, vbase, deg_blk,
+                                                                                      deg_total, *atoms, 0u);
+    else if (gv)
+        hipLaunchKernelGGL((k_mc_emit<true, false, false>), dim3(gv), dim3(256), 0, s, mols, wpre, wcoarse, list, avb, vstart,
+                                                                                       nact, nv, S4, F, outm, shellm, vert,
+                                                                                       vkey, d_counts, acb, tstart, ncube, ntri,
+                                                                                       N, cnt, vbw, tbw, NT, tri, vbase,
+                                                                                       deg_blk, deg_total, QsClosest{}, 0u);
+    if (gt)
+        hipLaunchKernelGGL((k_mc_emit<false, true, false>), dim3(gt), dim3(256), 0, s, mols, wpre, wcoarse, list, avb, vstart,
+                                                                                       nact, nv, S4, F, outm, shellm, vert,
+                                                                                       vkey, d_counts, acb, tstart, ncube, ntri,
+                                                                                       N, cnt, vbw, tbw, NT, tri, vbase,
+                                                                                       deg_blk, deg_total, QsClosest{}, 0u);
 }
 
 void qs_launch_smooth(const QsMol *mols, const uint32_t *vpre, const uint32_t *vcoarse, const uint64_t *N, const uint64_t *Zm,
