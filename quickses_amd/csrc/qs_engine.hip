@@ -1083,10 +1083,13 @@ int Engine::run_batch(const float *d_pos, const float *d_rad, const std::vector<
         if (smooth > 1) QS_TRY(ensure(vert3, (size_t)pool_v * 12));
         const float *src = as<float>(vert);
         float *dst = as<float>(vert2);
+        const uint64_t *wpre = (const uint64_t *)(as<uint32_t>(d_meta) + at_wpre);
+        const uint32_t *wcoarse = nmol > 1 ? as<uint32_t>(d_meta) + at_wpre + 2 * ((size_t)nmol + 1) : nullptr;
         for (int it = 0; it < smooth; it++) {
-            qs_launch_smooth(as<QsMol>(d_mols), d_vpre, nmol > 1 ? d_vpre + nmol + 1 : nullptr, as<uint64_t>(negm), as<uint64_t>(zerom), as<uint64_t>(s4),
-                             as<uint32_t>(vbw), as<uint64_t>(vkey), pool_v, as<uint64_t>(ntb), as<uint32_t>(tbw), as<int>(tri),
-                             src, dst, as<uint32_t>(totals) + 1, expect_v, stream);
+            qs_launch_smooth(as<QsMol>(d_mols), d_vpre, nmol > 1 ? d_vpre + nmol + 1 : nullptr, wpre, wcoarse, as<uint32_t>(alist),
+                             as<uint32_t>(vstart), as<uint64_t>(negm), as<uint64_t>(zerom), as<uint64_t>(s4), as<uint32_t>(vbw),
+                             as<uint64_t>(vkey), pool_v, pool_t, as<uint64_t>(ntb), as<uint32_t>(tbw), as<int>(tri), src, dst,
+                             as<uint32_t>(totals), expect_v, stream);
             src = dst;
             dst = (dst == as<float>(vert2)) ? as<float>(vert3) : as<float>(vert2);
         }

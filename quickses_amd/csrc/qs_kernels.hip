@@ -3310,26 +3310,34 @@ __device__ __forceinline__ SmoothView smooth_view(const QsMol &M, const uint64_t
 /* The incident cubes of an edge vertex: the 4 cubes around the edge in cube order (offsets -1 / 0
    of the two other axes, major first); every one inside the grid contains the sign change, so it
    is polygonised and its word's triangle records exist.  Their first triangles and counts (0 for
-   a cube outside the grid) are loaded here, all four before any is used. */
-__device__ __forceinline__ void smooth_edge_cubes(const SmoothView &S, int x, int y, int z, int sl, int (&nt4)[4],
-                                                  uint32_t (&tb4)[4])
+   a cube outside the grid, and for a point slot) are loaded here, all four before any is used. */
+__device__ __forceinline__ void smooth_edge_cubes(const uint64_t *__restrict__ NT, const uint32_t *__restrict__ tbw, int g, int W,
+                                                  int lim, int x, int y, int z, int sl, int (&nt4)[4], uint32_t (&tb4)[4])
 {
-    const int g = S.V.g, W = S.V.W, lim = S.V.lim;
+    /* the cube at the point, and the one below it, lie in the grid on each axis */
+    const bool xo = x < lim, yo = y < lim, zo = z < lim;
+    const bool xl = x > 0 && x <= lim, yl = y > 0 && y <= lim, zl = z > 0 && z <= lim;
+    const uint32_t row = (uint32_t)x * (uint32_t)g + (uint32_t)y;
 #pragma unroll
     for (int k = 0; k < 4; k++) {
-        const int hi = k >> 1, lo = k & 1;
-        const int cx = x - (sl != 0 ? 1 - hi : 0);
-        const int cy = y - (sl == 0 ? 1 - hi : (sl == 2 ? 1 - lo : 0));
-        const int cz = z - (sl != 2 ? 1 - lo : 0);
-        nt4[k] = 0;
-        tb4[k] = 0;
-        if (cx < 0 || cy < 0 || cz < 0 || cx >= lim || cy >= lim || cz >= lim) continue;
-        const size_t wi = ((size_t)cx * g + cy) * W + (cz >> 6);
-        const int b = cz & 63;
-        const uint64_t *np = S.NT + 3 * wi;
-        const uint64_t p0 = np[0], p1 = np[1], p2 = np[2], below = (1ull << b) - 1ull;
-        tb4[k] = S.tbw[wi] + (uint32_t)(__popcll(p0 & below) + 2 * __popcll(p1 & below) + 4 * __popcll(p2 & below));
-        nt4[k] = (int)((p0 >> b) & 1ull) + 2 * (int)((p1 >> b) & 1ull) + 4 * (int)((p2 >> b) & 1ull);
+        /* below the point on which axes (bit 1 of k: not on the first of the two others, bit 0: not
+           on the second) */
+        const bool hi = k >> 1, lo = k & 1;
+        const bool dx = sl != 0 && !hi, dy = sl == 0 ? !hi : (sl == 2 && !lo), dz = sl != 2 && !lo;
+        const bool ok = sl < 3 && (dx ? xl : xo) && (dy ? yl : yo) && (dz ? zl : zo);
+        const int cz = z - (dz ? 1 : 0);
+        const uint32_t wi = ok ? (row - (dx ? (uint32_t)g : 0u) - (dy ? 1u : 0u)) * (uint32_t)W + (uint32_t)(cz >> 6) : 0u;
+        const uint64_t *__restrict__ np = NT + 3 * (size_t)wi;
+        const uint64_t p0 = np[0], p1 = np[1], p2 = np[2];
+        const uint32_t b = (uint32_t)cz & 63u, h = b & 31u, bit = 1u << h, below = bit - 1u;
+        const bool top = b >= 32u;
+        const uint32_t ml = top ? ~0u : below, mh = top ? below : 0u;
+        tb4[k] = tbw[wi] + (uint32_t)(__popc((uint32_t)p0 & ml) + __popc((uint32_t)(p0 >> 32) & mh)) +
+                 2u * (uint32_t)(__popc((uint32_t)p1 & ml) + __popc((uint32_t)(p1 >> 32) & mh)) +
+                 4u * (uint32_t)(__popc((uint32_t)p2 & ml) + __popc((uint32_t)(p2 >> 32) & mh));
+        const uint32_t q0 = top ? (uint32_t)(p0 >> 32) : (uint32_t)p0, q1 = top ? (uint32_t)(p1 >> 32) : (uint32_t)p1,
+                       q2 = top ? (uint32_t)(p2 >> 32) : (uint32_t)p2;
+        nt4[k] = ok ? (int)(((q0 >> h) & 1u) | ((q1 >> h) & 1u) << 1 | ((q2 >> h) & 1u) << 2) : 0;
     }
 }
 
@@ -3340,72 +3348,81 @@ __device__ __forceinline__ void smooth_edge_cubes(const SmoothView &S, int x, in
    0.195 and 0.854, three 0.191 and 0.815, six 0.196 and 0.845 (registers). */
 constexpr int SM_U = 4;
 
-/* vertex v's Jacobi sum over the neighbour list walked from its cubes (edge vertex: the cubes of
-   smooth_edge_cubes; zero point: the 8 cubes around it), written to dst */
-__device__ __forceinline__ void smooth_sum(const SmoothView &S, uint32_t v, int x, int y, int z, int sl, const int (&nt4)[4],
-                                           const uint32_t (&tb4)[4], const int *__restrict__ tri,
-                                           const float *__restrict__ src, float *__restrict__ dst)
+/* vertex v's Jacobi sum over the neighbour list walked from its cubes, written to dst: an edge
+   vertex's, from the cubes of smooth_edge_cubes, U triangles per round */
+template <int U>
+__device__ __forceinline__ void smooth_edge(uint32_t v, const int (&nt4)[4], const uint32_t (&tb4)[4], const int *__restrict__ tri,
+                                            const float *__restrict__ src, float *__restrict__ dst)
+{
+    float sx = 0.0f, sy = 0.0f, sz = 0.0f;
+    uint32_t cnt = 0;
+    /* the four cubes' triangles as one sequence, U at a time: their corners are loaded
+       together, then the other corners' positions together, then added in order */
+    const int s1 = nt4[0], s2 = s1 + nt4[1], s3 = s2 + nt4[2], total = s3 + nt4[3];
+    const uint32_t d0 = tb4[0], d1 = tb4[1] - (uint32_t)s1, d2 = tb4[2] - (uint32_t)s2, d3 = tb4[3] - (uint32_t)s3;
+    for (int j = 0; j < total; j += U) {
+        uint32_t a[U], b[U], c[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int i = min(j + u, total - 1);
+            const uint32_t t = (uint32_t)i + (i < s1 ? d0 : (i < s2 ? d1 : (i < s3 ? d2 : d3)));
+            const int *tt = tri + 3 * (size_t)t;
+            a[u] = (uint32_t)tt[0];
+            b[u] = (uint32_t)tt[1];
+            c[u] = (uint32_t)tt[2];
+        }
+        bool hit[U];
+        float q[U][6];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            hit[u] = j + u < total && (a[u] == v || b[u] == v || c[u] == v);
+            const float *q0 = src + 3 * (size_t)(hit[u] ? (a[u] == v ? b[u] : a[u]) : v);
+            const float *q1 = src + 3 * (size_t)(hit[u] ? (c[u] == v ? b[u] : c[u]) : v);
+#pragma unroll
+            for (int e = 0; e < 3; e++) {
+                q[u][e] = q0[e];
+                q[u][3 + e] = q1[e];
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            if (!hit[u]) continue;
+            sx = sx + q[u][0];
+            sy = sy + q[u][1];
+            sz = sz + q[u][2];
+            sx = sx + q[u][3];
+            sy = sy + q[u][4];
+            sz = sz + q[u][5];
+            cnt += 2;
+        }
+    }
+    const float fc = (float)cnt;
+    dst[3 * (size_t)v + 0] = sx / fc;
+    dst[3 * (size_t)v + 1] = sy / fc;
+    dst[3 * (size_t)v + 2] = sz / fc;
+}
+
+/* a point vertex's, from the 8 cubes around it */
+__device__ __forceinline__ void smooth_point(const SmoothView &S, uint32_t v, int x, int y, int z, const int *__restrict__ tri,
+                                             const float *__restrict__ src, float *__restrict__ dst)
 {
     const int g = S.V.g, W = S.V.W, lim = S.V.lim;
     float sx = 0.0f, sy = 0.0f, sz = 0.0f;
     uint32_t cnt = 0;
-    if (sl < 3) {
-        /* the four cubes' triangles as one sequence, SM_U at a time: their corners are loaded
-           together, then the other corners' positions together, then added in order */
-        const int s1 = nt4[0], s2 = s1 + nt4[1], s3 = s2 + nt4[2], total = s3 + nt4[3];
-        const uint32_t d0 = tb4[0], d1 = tb4[1] - (uint32_t)s1, d2 = tb4[2] - (uint32_t)s2, d3 = tb4[3] - (uint32_t)s3;
-        for (int j = 0; j < total; j += SM_U) {
-            uint32_t a[SM_U], b[SM_U], c[SM_U];
-#pragma unroll
-            for (int u = 0; u < SM_U; u++) {
-                const int i = min(j + u, total - 1);
-                const uint32_t t = (uint32_t)i + (i < s1 ? d0 : (i < s2 ? d1 : (i < s3 ? d2 : d3)));
-                const int *tt = tri + 3 * (size_t)t;
-                a[u] = (uint32_t)tt[0];
-                b[u] = (uint32_t)tt[1];
-                c[u] = (uint32_t)tt[2];
-            }
-            bool hit[SM_U];
-            float q[SM_U][6];
-#pragma unroll
-            for (int u = 0; u < SM_U; u++) {
-                hit[u] = j + u < total && (a[u] == v || b[u] == v || c[u] == v);
-                const float *q0 = src + 3 * (size_t)(hit[u] ? (a[u] == v ? b[u] : a[u]) : v);
-                const float *q1 = src + 3 * (size_t)(hit[u] ? (c[u] == v ? b[u] : c[u]) : v);
-#pragma unroll
-                for (int e = 0; e < 3; e++) {
-                    q[u][e] = q0[e];
-                    q[u][3 + e] = q1[e];
-                }
-            }
-#pragma unroll
-            for (int u = 0; u < SM_U; u++) {
-                if (!hit[u]) continue;
-                sx = sx + q[u][0];
-                sy = sy + q[u][1];
-                sz = sz + q[u][2];
-                sx = sx + q[u][3];
-                sy = sy + q[u][4];
-                sz = sz + q[u][5];
-                cnt += 2;
-            }
-        }
-    } else {
-        /* a zero grid point: the 8 cubes around it, every corner that is this vertex */
-        for (int k = 0; k < 8; k++) {
-            const int cx = x - 1 + (k >> 2), cy = y - 1 + ((k >> 1) & 1), cz = z - 1 + (k & 1);
-            if (cx < 0 || cy < 0 || cz < 0 || cx >= lim || cy >= lim || cz >= lim) continue;
-            const int ci = S.V.cube_index(cx, cy, cz);
-            const int nt = tri_count(ci);
-            if (!nt) continue;
-            const uint32_t tb = cube_first_tri(S.NT, S.tbw, ((size_t)cx * g + cy) * W + (cz >> 6), cz & 63);
-            for (int t = 0; t < nt; t++) {
-                const int *tt = tri + 3 * (size_t)(tb + t);
-                const uint32_t a = (uint32_t)tt[0], b = (uint32_t)tt[1], c = (uint32_t)tt[2];
-                if (a == v) { push_pair(src, b, c, sx, sy, sz); cnt += 2; }
-                if (b == v) { push_pair(src, a, c, sx, sy, sz); cnt += 2; }
-                if (c == v) { push_pair(src, a, b, sx, sy, sz); cnt += 2; }
-            }
+    /* a zero grid point: the 8 cubes around it, every corner that is this vertex */
+    for (int k = 0; k < 8; k++) {
+        const int cx = x - 1 + (k >> 2), cy = y - 1 + ((k >> 1) & 1), cz = z - 1 + (k & 1);
+        if (cx < 0 || cy < 0 || cz < 0 || cx >= lim || cy >= lim || cz >= lim) continue;
+        const int ci = S.V.cube_index(cx, cy, cz);
+        const int nt = tri_count(ci);
+        if (!nt) continue;
+        const uint32_t tb = cube_first_tri(S.NT, S.tbw, ((size_t)cx * g + cy) * W + (cz >> 6), cz & 63);
+        for (int t = 0; t < nt; t++) {
+            const int *tt = tri + 3 * (size_t)(tb + t);
+            const uint32_t a = (uint32_t)tt[0], b = (uint32_t)tt[1], c = (uint32_t)tt[2];
+            if (a == v) { push_pair(src, b, c, sx, sy, sz); cnt += 2; }
+            if (b == v) { push_pair(src, a, c, sx, sy, sz); cnt += 2; }
+            if (c == v) { push_pair(src, a, b, sx, sy, sz); cnt += 2; }
         }
     }
     const float fc = (float)cnt;
@@ -3426,38 +3443,166 @@ __device__ __forceinline__ void vertex_point(uint64_t key, int g, int &x, int &y
     y = (int)(xy - (uint32_t)x * ug);
 }
 
+/* triangles and vertices that a smoothing block stages in LDS at most (10 bits per corner) */
+constexpr uint32_t SM_TRI = 1408, SM_VERT = 1024;
+/* expected vertices above which blocks stage: a smaller mesh is bound by a block's chain of loads, which
+   staging makes longer (2,000 atoms at 0.5 A: 9 us without, 12 with) */
+constexpr uint32_t SM_STAGED_MIN = 1u << 19;
+
 /* one Jacobi pass, one thread per vertex.  A polygonised cube's triangles are consecutive from
    its first triangle id (its word's triangle base plus the triangle-count planes below it), and
    its count is its bit of those planes, so each incident triangle's other corners are read from
    the triangle array.  An edge vertex is a corner of exactly the triangles whose case-table entry
-   is its cube edge (no other edge of the cube shares its id), so it finds them by id. */
-__global__ void __launch_bounds__(256) k_smooth(const QsMol *__restrict__ mols, const uint32_t *__restrict__ vpre,
-                                                const uint32_t *__restrict__ vcoarse,
-                                                const uint64_t *__restrict__ N_all, const uint64_t *__restrict__ Zm_all,
-                                                const uint64_t *__restrict__ S4_all, const uint32_t *__restrict__ vbw_all,
-                                                const uint64_t *__restrict__ vkey, uint32_t nv,
-                                                const uint64_t *__restrict__ NT_all,
-                                                const uint32_t *__restrict__ tbw_all, const int *__restrict__ tri,
-                                                const float *__restrict__ src,
-                                                float *__restrict__ dst, const uint32_t *__restrict__ d_nv)
+   is its cube edge (no other edge of the cube shares its id), so it finds them by id.
+   Bound by the address unit when every vertex gathers them from memory: eight triangles and the
+   other corners' positions are about 50 gathers, though neighbouring vertices share them.  With
+   STAGED a block loads them once, in order, into LDS: its 256 vertices lie in consecutive grid rows
+   [ra, rb] (row = x g + y), so their triangles lie in two ranges of the triangle array, the rows
+   [ra - 1, rb] of their own plane and of the plane below, and those triangles' corners in three
+   ranges of the vertices, the rows [ra - 1, rb + 1] of the planes below, own and above: about 1,150
+   triangles and 900 vertices.  A triangle is kept as its corners' places among the staged vertices.
+   A block whose ranges are larger (1 to 3 % of them) or whose vertices belong to two molecules
+   gathers from memory.  Then bound by VALU issue, and by waves in flight: 64 registers, so the
+   triangles' loads end before the positions' begin.  On 256 molecules at 0.5 A gathers took 0.793 ms
+   and this takes 0.566, on the 50,000-atom 0.2 A mesh 0.188 and 0.156, on 1M atoms at 0.5 A (two passes)
+   0.660 and 0.537. */
+template <bool STAGED>
+__global__ void __launch_bounds__(256, STAGED ? 8 : 1) k_smooth(const QsMol *__restrict__ mols, const uint32_t *__restrict__ vpre,
+                                                   const uint32_t *__restrict__ vcoarse, const uint64_t *__restrict__ wpre,
+                                                   const uint32_t *__restrict__ wcoarse, const uint32_t *__restrict__ list,
+                                                   const uint32_t *__restrict__ vstart, const uint64_t *__restrict__ N_all,
+                                                   const uint64_t *__restrict__ Zm_all, const uint64_t *__restrict__ S4_all,
+                                                   const uint32_t *__restrict__ vbw_all, const uint64_t *__restrict__ vkey,
+                                                   uint32_t nv, uint32_t ntri, const uint64_t *__restrict__ NT_all,
+                                                   const uint32_t *__restrict__ tbw_all, const int *__restrict__ tri,
+                                                   const float *__restrict__ src, float *__restrict__ dst,
+                                                   const uint32_t *__restrict__ d_counts)
 {
-    /* a mesh larger than the pool (the run is repeated with a larger one) has corner ids past
-       the pool: nothing to smooth then */
-    if (d_nv && *d_nv > nv) return;
-    if (d_nv) nv = *d_nv;
+    __shared__ uint32_t s_tri[STAGED ? SM_TRI : 1];           /* corners' places, in bits 2, 12 and 22 on */
+    __shared__ float s_pos[3][STAGED ? SM_VERT : 1];
+    /* a mesh larger than the pools (the run is repeated with larger ones) has ids past them: nothing
+       to smooth then */
+    if (d_counts[1] > nv || d_counts[0] > ntri) return;
+    nv = d_counts[1];
+    const uint32_t nact = d_counts[2];
     const uint32_t nb = (nv + 255u) >> 8;
     /* persistent blocks over the 256-vertex blocks (grid a multiple of 8: see k_mc_emit) */
     for (uint32_t vb = blockIdx.x; vb < nb; vb += gridDim.x) {
-        const uint32_t v = xcd_group<64>(vb, nb) * 256u + threadIdx.x;
-        if (v >= nv) continue;
-        const QsMol &M = mols[seg_of_wave(vpre, vcoarse, v)];
-        const SmoothView S = smooth_view(M, N_all, Zm_all, S4_all, vbw_all, NT_all, tbw_all);
-        int x, y, z, sl;
-        vertex_point(vkey[v], S.V.g, x, y, z, sl);
-        int nt4[4] = {0, 0, 0, 0};
-        uint32_t tb4[4] = {0u, 0u, 0u, 0u};
-        if (sl < 3) smooth_edge_cubes(S, x, y, z, sl, nt4, tb4);
-        smooth_sum(S, v, x, y, z, sl, nt4, tb4, tri, src, dst);
+        const uint32_t blk = xcd_group<64>(vb, nb), v = blk * 256u + threadIdx.x;
+        bool staged = false;
+        if constexpr (STAGED) {
+            const uint32_t w0 = list[vstart[blk]], w1 = list[blk + 1 < nb ? vstart[blk + 1] : nact - 1u];
+            const int m0 = wcoarse ? __builtin_amdgcn_readfirstlane(seg_coarse<QS_COARSE_ITEMS>(wpre, wcoarse, (uint64_t)w0)) : 0;
+            const int m1 = wcoarse ? __builtin_amdgcn_readfirstlane(seg_coarse<QS_COARSE_ITEMS>(wpre, wcoarse, (uint64_t)w1)) : 0;
+            if (m0 == m1) {
+                const QsMol &M = mols[m0];
+                const int g = M.G.g, W = (int)M.W, last = g * g - 1; /* (the last row holds nothing) */
+                const int ra = (int)((w0 - (uint32_t)M.word_off) / (uint32_t)W), rb = (int)((w1 - (uint32_t)M.word_off) / (uint32_t)W);
+                const uint32_t *__restrict__ vbw = vbw_all + M.word_off, *__restrict__ tbw = tbw_all + M.word_off;
+                /* the ranges of triangles (t, own plane and below) and vertices (u, own, below,
+                   above), and how many entries come before each in LDS */
+                const auto at = [&](int r) { return (size_t)iclamp(r, 0, last) * W; };
+                const uint32_t t0 = tbw[at(ra - 1)], t1 = tbw[at(ra - g - 1)];
+                const uint32_t na = tbw[at(rb + 1)] - t0, nt = na + tbw[at(rb - g + 1)] - t1;
+                const uint32_t u0 = vbw[at(ra - 1)], u1 = vbw[at(ra - g - 1)], u2 = vbw[at(ra + g - 1)];
+                const uint32_t nu0 = vbw[at(rb + 2)] - u0, nu1 = nu0 + vbw[at(rb - g + 2)] - u1, nu = nu1 + vbw[at(rb + g + 2)] - u2;
+                /* (and the rows' points, as offsets from the block's first, are exact in float) */
+                staged = nt - 1u < SM_TRI && nu - 1u < SM_VERT && (uint64_t)(rb - ra + 1) * (uint32_t)g < (1u << 20);
+                if (staged) {
+                    /* all of a thread's triangles, then all of its positions, are loaded before any is
+                       used (past the end the last one again) */
+                    constexpr uint32_t KT = (SM_TRI + 255u) / 256u, KV = SM_VERT / 256u;
+                    int tt[KT][3];
+#pragma unroll
+                    for (uint32_t k = 0; k < KT; k++) {
+                        const uint32_t i = min(k * 256u + threadIdx.x, nt - 1u);
+                        const int *__restrict__ q = tri + 3 * (size_t)(i + (i < na ? t0 : t1 - na));
+#pragma unroll
+                        for (int c = 0; c < 3; c++) tt[k][c] = q[c];
+                    }
+                    const uint64_t key = vkey[min(v, nv - 1u)];
+                    /* (the ranges' ids ascend from the plane below to the one above; where the rows are so
+                       empty that two ranges overlap, the later one's place is every use's) */
+                    const auto place = [&](int id) { return (uint32_t)id - ((uint32_t)id >= u2 ? u2 - nu1 : ((uint32_t)id >= u0 ? u0 : u1 - nu0)); };
+#pragma unroll
+                    for (uint32_t k = 0; k < KT; k++)
+                        if (k * 256u + threadIdx.x < nt)
+                            s_tri[k * 256u + threadIdx.x] = place(tt[k][0]) << 2 | place(tt[k][1]) << 12 | place(tt[k][2]) << 22;
+                    float pp[KV][3];
+#pragma unroll
+                    for (uint32_t k = 0; k < KV; k++) {
+                        const uint32_t i = min(k * 256u + threadIdx.x, nu - 1u);
+                        const float *__restrict__ q = src + 3 * (size_t)(i + (i < nu0 ? u0 : (i < nu1 ? u1 - nu0 : u2 - nu1)));
+#pragma unroll
+                        for (int c = 0; c < 3; c++) pp[k][c] = q[c];
+                    }
+                    /* the vertex's point: key >> 2 = row g + z */
+                    const float inv_g = 1.0f / (float)g;
+                    const int xa = ra / g, o = (int)((uint32_t)(key >> 2) - (uint32_t)ra * (uint32_t)g);
+                    const int dr = (int)(((float)o + 0.5f) * inv_g), z = o - dr * g, r = ra + dr - xa * g;
+                    const int dx_ = (int)(((float)r + 0.5f) * inv_g), x = xa + dx_, y = r - dx_ * g, sl = (int)(key & 3ull);
+                    /* its four cubes' first triangles (as places in LDS) and counts */
+                    int nt4[4];
+                    uint32_t tb4[4];
+                    smooth_edge_cubes(NT_all + 3 * M.word_off, tbw, g, W, M.G.lim, x, y, z, sl, nt4, tb4);
+#pragma unroll
+                    for (uint32_t k = 0; k < KV; k++)
+                        if (k * 256u + threadIdx.x < nu)
+#pragma unroll
+                            for (int c = 0; c < 3; c++) s_pos[c][k * 256u + threadIdx.x] = pp[k][c];
+                    __syncthreads();
+                    if (v < nv) {
+                        if (sl < 3) {
+                            /* cubes 2 and 3, and all of an x edge's, lie in the own plane */
+                            const uint32_t lo = sl == 0 ? 0u - t0 : na - t1;
+                            const int s1 = nt4[0], s2 = s1 + nt4[1], s3 = s2 + nt4[2], total = s3 + nt4[3];
+                            const uint32_t d0 = tb4[0] + lo, d1 = tb4[1] + lo - (uint32_t)s1, d2 = tb4[2] - t0 - (uint32_t)s2,
+                                           d3 = tb4[3] - t0 - (uint32_t)s3, me = place((int)v) << 2;
+                            const auto pos = [&](int c, uint32_t b) { return *(const float *)((const char *)s_pos[c] + b); };
+                            float sx = 0.0f, sy = 0.0f, sz = 0.0f;
+                            uint32_t cnt = 0;
+#pragma unroll 2
+                            for (int i = 0; i < total; i++) {
+                                const uint32_t p = s_tri[(uint32_t)i + (i < s1 ? d0 : (i < s2 ? d1 : (i < s3 ? d2 : d3)))];
+                                const uint32_t a = p & 0xFFCu, b = (p >> 10) & 0xFFCu, c = (p >> 20) & 0xFFCu;
+                                if (a == me || b == me || c == me) {
+                                    const uint32_t q0 = a == me ? b : a, q1 = c == me ? b : c;
+                                    sx = sx + pos(0, q0);
+                                    sy = sy + pos(1, q0);
+                                    sz = sz + pos(2, q0);
+                                    sx = sx + pos(0, q1);
+                                    sy = sy + pos(1, q1);
+                                    sz = sz + pos(2, q1);
+                                    cnt += 2;
+                                }
+                            }
+                            const float fc = (float)cnt;
+                            dst[3 * (size_t)v + 0] = sx / fc;
+                            dst[3 * (size_t)v + 1] = sy / fc;
+                            dst[3 * (size_t)v + 2] = sz / fc;
+                        } else {
+                            const SmoothView S = smooth_view(M, N_all, Zm_all, S4_all, vbw_all, NT_all, tbw_all);
+                            smooth_point(S, v, x, y, z, tri, src, dst);
+                        }
+                    }
+                    __syncthreads(); /* the next block is staged */
+                }
+            }
+        }
+        if (!staged && v < nv) {
+            const QsMol &M = mols[seg_of_wave(vpre, vcoarse, v)];
+            const SmoothView S = smooth_view(M, N_all, Zm_all, S4_all, vbw_all, NT_all, tbw_all);
+            int x, y, z, sl;
+            vertex_point(vkey[v], S.V.g, x, y, z, sl);
+            if (sl < 3) {
+                int nt4[4];
+                uint32_t tb4[4];
+                smooth_edge_cubes(S.NT, S.tbw, S.V.g, S.V.W, S.V.lim, x, y, z, sl, nt4, tb4);
+                smooth_edge<STAGED ? 1 : SM_U>(v, nt4, tb4, tri, src, dst);
+            } else {
+                smooth_point(S, v, x, y, z, tri, src, dst);
+            }
+        }
     }
 }
 
@@ -4052,14 +4197,20 @@ void qs_launch_mc_emit(const QsMol *mols, const uint64_t *wpre, const uint32_t *
                                                                                        deg_blk, deg_total, QsClosest{}, 0u);
 }
 
-void qs_launch_smooth(const QsMol *mols, const uint32_t *vpre, const uint32_t *vcoarse, const uint64_t *N, const uint64_t *Zm,
-                      const uint64_t *S4, const uint32_t *vbw, const uint64_t *vkey, uint32_t nv,
-                      const uint64_t *NT, const uint32_t *tbw, const int *tri, const float *src, float *dst,
-                      const uint32_t *d_nv, uint32_t expect, hipStream_t s)
+void qs_launch_smooth(const QsMol *mols, const uint32_t *vpre, const uint32_t *vcoarse, const uint64_t *wpre, const uint32_t *wcoarse,
+                      const uint32_t *list, const uint32_t *vstart, const uint64_t *N, const uint64_t *Zm, const uint64_t *S4,
+                      const uint32_t *vbw, const uint64_t *vkey, uint32_t nv, uint32_t ntri, const uint64_t *NT,
+                      const uint32_t *tbw, const int *tri, const float *src, float *dst, const uint32_t *d_counts, uint32_t expect,
+                      hipStream_t s)
 {
     if (!nv) return;
-    hipLaunchKernelGGL(k_smooth, dim3(pgrid(nblk(std::min(nv, expect), 256))), dim3(256), 0, s, mols, vpre, vcoarse, N, Zm, S4, vbw, vkey, nv,
-                       NT, tbw, tri, src, dst, d_nv);
+    const dim3 grid(pgrid(nblk(std::min(nv, expect), 256)));
+    if (std::min(nv, expect) > SM_STAGED_MIN)
+        hipLaunchKernelGGL(k_smooth<true>, grid, dim3(256), 0, s, mols, vpre, vcoarse, wpre, wcoarse, list, vstart, N, Zm, S4, vbw,
+                           vkey, nv, ntri, NT, tbw, tri, src, dst, d_counts);
+    else
+        hipLaunchKernelGGL(k_smooth<false>, grid, dim3(256), 0, s, mols, vpre, vcoarse, wpre, wcoarse, list, vstart, N, Zm, S4, vbw,
+                           vkey, nv, ntri, NT, tbw, tri, src, dst, d_counts);
 }
 
 void qs_launch_vertex_normals(const QsMol *mols, const uint32_t *vpre, const uint32_t *vcoarse, const uint64_t *vkey, uint32_t nv,

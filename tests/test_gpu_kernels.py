@@ -180,3 +180,12 @@ def test_cells_in_one_block_or_several_launches(qs, sizes, box):
     perm, cells = np.concatenate(perm), np.concatenate(cells)
     assert np.array_equal(_cells_fetch(qs, b"perm", at, np.int32), perm)
     assert np.array_equal(_cells_fetch(qs, b"cells", cells.size, np.int32).reshape(-1, 2), cells)
+
+
+@pytest.mark.parametrize("reso", [0.216, 0.22])
+def test_smoothing_staged_and_gathered(qs, orc, reso):
+    """Above and below the expected size from which a block stages its triangles and vertices; two
+    passes, so the second reads what the first wrote."""
+    pos, rad = qs.synth_ball(23, 4000)
+    print("case smoothing staged: reso=%.3f" % reso, flush=True)
+    assert _same(qs.compute_ses(pos, rad, reso, 2), orc.compute_ses(pos, rad, reso, 2))
