@@ -203,6 +203,9 @@ struct P2Group {
     P2Tables *tab = nullptr;
 };
 
+/* field pass 2 reads up to one 32-bit word past the last row of the outside masks */
+constexpr size_t OUTM_PAD = 16;
+
 struct Engine {
     int device = -1;
     hipStream_t stream = nullptr, side = nullptr;

@@ -247,7 +247,8 @@ int Engine::reserve(uint64_t vox, uint64_t atoms, uint64_t cells, uint64_t verts
     atoms += 1;
     cells += 1;
     verts += 1;
-    for (DevBuf *b : {&outm, &shellm, &negm, &zerom}) QS_TRY(ensure(*b, nw * 8));
+    QS_TRY(ensure(outm, nw * 8 + OUTM_PAD));
+    for (DevBuf *b : {&shellm, &negm, &zerom}) QS_TRY(ensure(*b, nw * 8));
     for (DevBuf *b : {&wcnt, &vbw, &tbw, &alist, &avb, &acb}) QS_TRY(ensure(*b, nw * 4));
     QS_TRY(ensure(s4, nw * 32));
     QS_TRY(ensure(ntb, nw * 24));
@@ -505,7 +506,7 @@ int Engine::group_tables(P2Group &grp)
 int Engine::field_stage(uint32_t nb_p1, size_t at_p1, StageTimer &tm)
 {
     const int nmol = (int)mols.size();
-    QS_TRY(ensure(outm, std::max<uint64_t>(nw_total, 1) * 8));
+    QS_TRY(ensure(outm, std::max<uint64_t>(nw_total, 1) * 8 + OUTM_PAD));
     QS_TRY(ensure(shellm, std::max<uint64_t>(nw_total, 1) * 8));
     QS_TRY(ensure(field, std::max<uint64_t>(vox_total, 1) * 4));
     QS_TRY(ensure(negm, std::max<uint64_t>(nw_total, 1) * 8));
@@ -778,7 +779,8 @@ int Engine::slab_plan(const QsMol &M, int &planes)
     if (!budget) {
         const uint64_t vox = (uint64_t)g * g * g, nw = (uint64_t)g * g * M.W;
         bool held = vox < (1ull << 32) && field.cap >= vox * 4 && s4.cap >= nw * 32 && ntb.cap >= nw * 24;
-        for (const DevBuf *b : {&outm, &shellm, &negm, &zerom}) held = held && b->cap >= nw * 8;
+        held = held && outm.cap >= nw * 8 + OUTM_PAD;
+        for (const DevBuf *b : {&shellm, &negm, &zerom}) held = held && b->cap >= nw * 8;
         for (const DevBuf *b : {&wcnt, &vbw, &tbw, &alist, &avb, &acb}) held = held && b->cap >= nw * 4;
         if (held) return 0;
         size_t free_b = 0, total_b = 0;
@@ -2031,7 +2033,7 @@ int qs_stage_pass2(const float *fp, const int *ip, const uint8_t *labels, float 
     const uint64_t V = E.vox_total;
     const int W = (int)E.mols[0].W;
     QS_TRY(ensure(E.labels, V));
-    QS_TRY(ensure(E.outm, E.nw_total * 8));
+    QS_TRY(ensure(E.outm, E.nw_total * 8 + OUTM_PAD));
     QS_TRY(ensure(E.shellm, E.nw_total * 8));
     QS_HIP(hipMemcpyAsync(E.labels.p, labels, V, hipMemcpyHostToDevice, E.stream));
     qs_launch_labels_to_masks(as<uint8_t>(E.labels), G.g, W, as<uint64_t>(E.outm), as<uint64_t>(E.shellm), E.stream);

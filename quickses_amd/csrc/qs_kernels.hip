@@ -1936,26 +1936,48 @@ __global__ void __launch_bounds__(256) k_pass2_r(QsBatch B, const uint64_t *__re
     const bool vyz = gy < g && gz < g;
     const float dx = G.dx;
 
-    /* the outside rows of the tile and its R halo into LDS; fl: some row has an outside voxel */
+    /* the outside rows of the tile and its R halo into LDS; fl: some row has an outside voxel.  A row's
+       R + 32 + R bits lie in the 32-bit words before, at and after the tile's, which are one load; a
+       row outside the planes [p1_lo, p1_hi), which are all that is stored, reads another one and is
+       cleared (no output voxel reads it).  All loads are in flight before the first is used.  (Two
+       64-bit words under branches, one row after the other, took 0.440 instead of 0.425 ms on the
+       50,000-atom 0.2 A mesh and 0.393 instead of 0.382 on 200,000 atoms at 0.3 A.) */
     int fl = 0;
     auto load_rows = [&]() {
+        struct __attribute__((packed, aligned(4))) U3 {
+            uint32_t x, y, z;
+        };
+        constexpr int NL = (LX * LY + 255) / 256;
+        const int zw = tz0 >> 5;
+        const bool first = zw == 0;
+        const uint32_t kc = zw + 1 < 2 * W ? ~0u : 0u;
+        const uint32_t *__restrict__ o32 = (const uint32_t *)outm + (first ? 0 : zw - 1);
+        U3 w[NL];
+        bool ok[NL];
 #pragma unroll
-        for (int row = threadIdx.x; row < LX * LY; row += 256) {
-            int lx = row / LY, ly = row - lx * LY;
-            int gx = tx0 - R + lx, gy_ = ty0 - R + ly;
-            uint64_t m = 0ull;
-            /* planes outside [p1_lo, p1_hi) are not stored (and are read by no output voxel) */
-            if (gx >= M.p1_lo && gx < M.p1_hi && gy_ >= 0 && gy_ < g)
-                m = row_bits(outm + ((size_t)gx * g + gy_) * W, W, tz0 - R, LZ);
-            rows[row] = m;
-            fl |= (m != 0ull);
-            /* bit z of d: an outside voxel within c of z (bit z + R of m is z) */
-            uint32_t d = __builtin_amdgcn_alignbit((uint32_t)(m >> 32), (uint32_t)m, R);
+        for (int k = 0; k < NL; k++) {
+            const int row = min((int)threadIdx.x + 256 * k, LX * LY - 1);
+            const int lx = row / LY, ly = row - lx * LY;
+            const int gx = tx0 - R + lx, gy_ = ty0 - R + ly;
+            ok[k] = gx >= M.p1_lo && gx < M.p1_hi && gy_ >= 0 && gy_ < g;
+            w[k] = *(const U3 *)(o32 + (size_t)(ok[k] ? gx * g + gy_ : M.p1_lo * g) * (2 * (size_t)W));
+        }
+#pragma unroll
+        for (int k = 0; k < NL; k++) {
+            const int row = (int)threadIdx.x + 256 * k;
+            if (row >= LX * LY) break;
+            const uint32_t wa = first ? 0u : w[k].x, wb = first ? w[k].x : w[k].y, wc = (first ? w[k].y : w[k].z) & kc;
+            const uint32_t kk = ok[k] ? ~0u : 0u;
+            const uint32_t lo = __builtin_amdgcn_alignbit(wb, wa, 32 - R) & kk;
+            const uint32_t hi = __builtin_amdgcn_alignbit(wc, wb, 32 - R) & kk & ((1u << (LZ - 32)) - 1u);
+            rows[row] = (uint64_t)hi << 32 | lo;
+            fl |= (lo | hi) != 0u;
+            /* bit z of d: an outside voxel within c of z (bit z + R of the row is z) */
+            uint32_t d = __builtin_amdgcn_alignbit(hi, lo, R);
             dil[row] = d;
 #pragma unroll
             for (int c = 1; c <= R; c++) {
-                d |= __builtin_amdgcn_alignbit((uint32_t)(m >> 32), (uint32_t)m, R - c) |
-                     __builtin_amdgcn_alignbit((uint32_t)(m >> 32), (uint32_t)m, R + c);
+                d |= __builtin_amdgcn_alignbit(hi, lo, R - c) | __builtin_amdgcn_alignbit(hi, lo, R + c);
                 dil[c * NR + row] = d;
             }
         }
