@@ -189,3 +189,21 @@ def test_smoothing_staged_and_gathered(qs, orc, reso):
     pos, rad = qs.synth_ball(23, 4000)
     print("case smoothing staged: reso=%.3f" % reso, flush=True)
     assert _same(qs.compute_ses(pos, rad, reso, 2), orc.compute_ses(pos, rad, reso, 2))
+
+
+@pytest.mark.parametrize("shift", [0, 4, 8])
+def test_mesh_copied_to_any_alignment(qs, shift):
+    """The caller's arrays at 16-byte boundaries and off them; nothing past their ends is written."""
+    from quickses_amd import hipmem
+
+    pos, rad = qs.synth_ball(31, 900)
+    want = qs.compute_ses(pos, rad, 0.5, 1)
+    nv, nt = len(want[0]), len(want[1])
+    dp, dr = hipmem.DeviceArray(pos), hipmem.DeviceArray(rad)
+    outs = [hipmem.DeviceArray(np.full(n + 8, -7, np.int32)) for n in (3 * nv, 3 * nt, nv)]
+    print("case mesh copy: shift=%d" % shift, flush=True)
+    qs.compute_device_noalloc(dp.ptr, dr.ptr, len(rad), 0.5, 1, outs[0].ptr + shift, nv, outs[1].ptr + shift, nt, outs[2].ptr + shift)
+    for buf, ref in zip(outs, (want[0].view(np.int32), want[1], want[2])):
+        got, k = hipmem.download(buf.ptr, (ref.size + 8,), np.int32), shift // 4
+        assert np.array_equal(got[k:k + ref.size], ref.ravel())
+        assert (got[:k] == -7).all() and (got[k + ref.size:] == -7).all()
