@@ -690,13 +690,9 @@ int Engine::mesh_stage(size_t at_mc, uint32_t nb_mc, size_t at_wpre, StageTimer 
     QS_HIP(hipGetLastError());
     tm.mark("mc_emit");
     if (with_atoms && !fused) {
-        /* (beside the smoothing passes, which read the same vertices, unless stages are timed: 4.79
-           instead of 4.85 ms for the 256 molecules) */
-        if (!tm.on) QS_TRY(fork_side());
         qs_launch_closest_atom(as<QsMol>(d_mols), d_vpre, nmol > 1 ? d_vpre + nmol + 1 : nullptr, near, as<float>(vert), pool_v,
-                               counts + 1, expect_v, side_pending ? side : stream);
+                               counts + 1, expect_v, stream);
         QS_HIP(hipGetLastError());
-        if (side_pending) QS_HIP(hipEventRecord(ev_side, side));
         tm.mark("closest_atom");
     }
     return 0;
