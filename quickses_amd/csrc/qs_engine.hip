@@ -1540,7 +1540,7 @@ void API_computeSES(float resoSES, qs_float3 *atomPos, float *atomRad, unsigned 
     const size_t bytes = (size_t)E.nv * 16 + (size_t)E.nt * 12;
     const bool copied = bytes <= COPY_KERNEL_MAX && g_cur[0].pinned && g_cur[1].pinned && g_cur[2].pinned;
     if (copied) {
-        qs_launch_copy_mesh(E.res_vert, E.res_atom, E.res_tri, E.nv, E.nt, g_vertices, g_atom_ids, g_triangles, E.stream);
+        qs_launch_copy_mesh(E.res_vert, E.res_atom, E.res_tri, E.nv, E.nt, 0u, g_vertices, g_atom_ids, g_triangles, E.stream);
         ok = hipGetLastError() == hipSuccess;
     } else if (E.nv) {
         ok = hipMemcpyAsync(g_vertices, E.res_vert, (size_t)E.nv * 12, hipMemcpyDeviceToHost, E.stream) == hipSuccess &&
@@ -1634,7 +1634,7 @@ int qs_compute_device_noalloc(const float *d_pos, const float *d_rad, unsigned i
         return set_error(5, "output capacity too small: %u vertices and %u triangles (capacity %u and %u)", E.nv, E.nt,
                          vert_cap, tri_cap);
     if ((E.nv && (!d_vert || !d_atom_id)) || (E.nt && !d_tri)) return set_error(3, "output pointer is NULL");
-    qs_launch_copy_mesh(E.res_vert, E.res_atom, E.res_tri, E.nv, E.nt, d_vert, d_atom_id, d_tri, E.stream);
+    qs_launch_copy_mesh(E.res_vert, E.res_atom, E.res_tri, E.nv, E.nt, 0u, d_vert, d_atom_id, d_tri, E.stream);
     QS_HIP(hipGetLastError());
     QS_HIP(hipStreamSynchronize(E.stream));
     if (nvert) *nvert = E.nv;

@@ -182,9 +182,10 @@ void qs_launch_tri_compact_one(const int *tri, uint32_t nt, const uint32_t *dpre
    out[0..n)} */
 void qs_launch_tri_kept_before(const int *tri, const uint32_t *dpre, const uint64_t *idx, int n, uint32_t tcap, uint32_t *out,
                                const uint32_t *totals, const uint32_t *vpre, uint32_t *rb, hipStream_t s);
-/* a mesh's vertices, atom ids and triangles into other arrays (device or pinned host memory) */
-void qs_launch_copy_mesh(const float *v, const int *a, const int *t, uint32_t nv, uint32_t nt, float *dv, int *da, int *dt,
-                         hipStream_t s);
+/* a mesh's vertices, atom ids and triangles, their corners less v0, into other arrays (device or pinned
+   host memory) */
+void qs_launch_copy_mesh(const float *v, const int *a, const int *t, uint32_t nv, uint32_t nt, uint32_t v0, float *dv, int *da,
+                         int *dt, hipStream_t s);
 void qs_launch_tri_localize(const int *tri, uint32_t nt, const uint32_t *tpre, const uint32_t *vpre, int nmol, int *out,
                             hipStream_t s);
 

@@ -3940,22 +3940,26 @@ __global__ void __launch_bounds__(256) k_copy(const uint4 *__restrict__ src, uin
     for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < n16; i += (uint64_t)gridDim.x * 256) dst[i] = src[i];
 }
 
-/* a mesh's three arrays (4-byte items) to the caller's, in one launch: small ones are bound by the
-   start of each copy, not by its bytes */
-__device__ __forceinline__ void copy_items(const uint32_t *__restrict__ src, uint32_t *__restrict__ dst, size_t n)
+/* a mesh's three arrays (4-byte items) to the caller's, in one launch, its corner ids less v0: small
+   ones are bound by the start of each copy, not by its bytes */
+__device__ __forceinline__ void copy_items(const uint32_t *__restrict__ src, uint32_t *__restrict__ dst, size_t n, uint32_t v0)
 {
     const size_t i0 = (size_t)blockIdx.x * 256 + threadIdx.x, step = (size_t)gridDim.x * 256;
     const size_t n4 = (((uintptr_t)src | (uintptr_t)dst) & 15u) ? 0 : n / 4;
-    for (size_t i = i0; i < n4; i += step) ((uint4 *)dst)[i] = ((const uint4 *)src)[i];
-    for (size_t i = 4 * n4 + i0; i < n; i += step) dst[i] = src[i];
+    for (size_t i = i0; i < n4; i += step) {
+        const uint4 q = ((const uint4 *)src)[i];
+        ((uint4 *)dst)[i] = make_uint4(q.x - v0, q.y - v0, q.z - v0, q.w - v0);
+    }
+    for (size_t i = 4 * n4 + i0; i < n; i += step) dst[i] = src[i] - v0;
 }
 __global__ void __launch_bounds__(256) k_copy_mesh(const uint32_t *__restrict__ v, const uint32_t *__restrict__ a,
-                                                   const uint32_t *__restrict__ t, uint32_t nv, uint32_t nt, uint32_t *__restrict__ dv,
-                                                   uint32_t *__restrict__ da, uint32_t *__restrict__ dt)
+                                                   const uint32_t *__restrict__ t, uint32_t nv, uint32_t nt, uint32_t v0,
+                                                   uint32_t *__restrict__ dv, uint32_t *__restrict__ da,
+                                                   uint32_t *__restrict__ dt)
 {
-    copy_items(v, dv, 3 * (size_t)nv);
-    copy_items(a, da, nv);
-    copy_items(t, dt, 3 * (size_t)nt);
+    copy_items(v, dv, 3 * (size_t)nv, 0u);
+    copy_items(a, da, nv, 0u);
+    copy_items(t, dt, 3 * (size_t)nt, v0);
 }
 
 /* triangles of a batch with vertex indices local to their molecule */
@@ -4308,13 +4312,13 @@ void qs_launch_copy(const void *src, void *dst, uint64_t bytes, hipStream_t s)
     hipLaunchKernelGGL(k_copy, dim3((unsigned)blocks), dim3(256), 0, s, (const uint4 *)src, (uint4 *)dst, n16);
 }
 
-void qs_launch_copy_mesh(const float *v, const int *a, const int *t, uint32_t nv, uint32_t nt, float *dv, int *da, int *dt,
-                         hipStream_t s)
+void qs_launch_copy_mesh(const float *v, const int *a, const int *t, uint32_t nv, uint32_t nt, uint32_t v0, float *dv, int *da,
+                         int *dt, hipStream_t s)
 {
     const size_t items = 4 * (size_t)nv + 3 * (size_t)nt;
     if (!items) return;
     hipLaunchKernelGGL(k_copy_mesh, dim3((unsigned)std::min<size_t>((items / 4 + 255) / 256 + 1, 2048)), dim3(256), 0, s,
-                       (const uint32_t *)v, (const uint32_t *)a, (const uint32_t *)t, nv, nt, (uint32_t *)dv, (uint32_t *)da,
+                       (const uint32_t *)v, (const uint32_t *)a, (const uint32_t *)t, nv, nt, v0, (uint32_t *)dv, (uint32_t *)da,
                        (uint32_t *)dt);
 }
 

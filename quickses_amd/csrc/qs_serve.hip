@@ -174,12 +174,6 @@ int run_batch_requests(Server *S, Engine &E, std::vector<Request *> &batch)
         QS_TRY(E.upload_input(as<float>(E.in_rad) + in[i].atom_off, batch[i]->rad.data(), k * 4));
     }
     QS_TRY(E.run_batch(as<float>(E.in_pos), as<float>(E.in_rad), in, batch[0]->smooth, &bbs));
-    if (E.nt) {
-        QS_TRY(ensure(E.tri_loc, (size_t)E.nt * 12));
-        qs_launch_tri_localize(E.res_tri, E.nt, as<uint32_t>(E.bounds), as<uint32_t>(E.d_off) + (nb + 1), nb,
-                               as<int>(E.tri_loc), E.stream);
-        QS_HIP(hipGetLastError());
-    }
     {
         std::lock_guard<std::mutex> lk(S->mu);
         for (int i = 0; i < nb; i++) {
@@ -203,16 +197,12 @@ int run_batch_requests(Server *S, Engine &E, std::vector<Request *> &batch)
         if (r->state == FAILED) continue;
         const uint64_t vb = ((uint64_t)r->nv * 12 + 255) & ~255ull, tb = ((uint64_t)r->nt * 12 + 255) & ~255ull;
         uint8_t *dst = base + r->arena_off;
-        if (r->nv) {
-            QS_HIP(hipMemcpyAsync(dst, E.res_vert + 3 * (size_t)E.vert_off[i], (size_t)r->nv * 12, hipMemcpyDeviceToDevice,
-                                  E.stream));
-            QS_HIP(hipMemcpyAsync(dst + vb + tb, E.res_atom + E.vert_off[i], (size_t)r->nv * 4, hipMemcpyDeviceToDevice,
-                                  E.stream));
-        }
-        if (r->nt)
-            QS_HIP(hipMemcpyAsync(dst + vb, as<int>(E.tri_loc) + 3 * (size_t)E.tri_off[i], (size_t)r->nt * 12,
-                                  hipMemcpyDeviceToDevice, E.stream));
+        /* one launch per request, which takes its corner ids down to its own vertices: with three copies
+           per request and a pass over all triangles 16 requests took 2.15 instead of 2.04 ms */
+        qs_launch_copy_mesh(E.res_vert + 3 * (size_t)E.vert_off[i], E.res_atom + E.vert_off[i], E.res_tri + 3 * (size_t)E.tri_off[i],
+                            r->nv, r->nt, E.vert_off[i], (float *)dst, (int *)(dst + vb + tb), (int *)(dst + vb), E.stream);
     }
+    QS_HIP(hipGetLastError());
     QS_HIP(hipStreamSynchronize(E.stream));
     return 0;
 }
