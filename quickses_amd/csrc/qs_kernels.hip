@@ -1250,7 +1250,8 @@ __device__ __forceinline__ void lds_or_range(uint32_t *row, int L, int R)
    the inside intervals, which one pair in seven has at 0.5 A, are taken apart from the near ones,
    so that the lanes without one do not wait; and an interval of 32 voxels is ORed with one 64-bit
    shift.  50,000 atoms at 0.2 A 0.313 -> 0.185 ms, 256 molecules at 0.5 A 1.05 -> 0.60 ms, a million
-   atoms at 0.5 A 0.87 -> 0.49 ms. */
+   atoms at 0.5 A 0.87 -> 0.49 ms; with the row prefixes by data-parallel primitives instead of
+   shuffles through LDS 0.170, 0.56 and 0.45. */
 #define P1S_MAXROWS 256   /* rows per slab block at most (row indexes in the queue are 8-bit) */
 #define P1S_DEFROWS 64    /* rows per slab block when no tuned count is set */
 #define P1S_MAXCOL 256
@@ -1850,7 +1851,7 @@ __device__ __forceinline__ uint32_t zdist2(uint64_t m, int z)
    Bound by VALU issue and, at R = 7, by LDS reads of the dilated rows.  Evaluating every shell
    voxel with an outside voxel in reach (28 to 38 % of the shell; 8 to 15 % are read) by x minima and
    trace took 0.592 ms on the 50,000-atom 0.2 A mesh (R 7), 0.610 on 200,000 atoms at 0.3 A (R 5) and
-   0.923 on 100 frames of 10,000 atoms at 0.5 A (R 3); this takes 0.468, 0.431 and 0.614. */
+   0.923 on 100 frames of 10,000 atoms at 0.5 A (R 3); this takes 0.425, 0.382 and 0.555. */
 
 /* entry it of a per-plane bit list: the plane lx with cpre[lx] <= it < cpre[lx + 1] (binary
    search) and the z of the (it - cpre[lx])-th set bit of cmask[lx] */
@@ -3042,7 +3043,7 @@ __global__ void __launch_bounds__(256) k_closest_atom(const QsMol *__restrict__ 
    the thread loads the sign words, slot masks and vertex counts of the cube's four (x, y) columns
    together, and every corner's vertex id comes from them.  One thread per triangle, three corners'
    masks each, took 0.20 ms on the 50,000-atom 0.2 A mesh and 0.92 ms on 256 molecules at 0.5 A
-   (47 M triangles); this takes 0.15 and 0.62 ms.  (64 registers for eight waves per SIMD, with
+   (47 M triangles); this takes 0.14 and 0.56 ms.  (64 registers for eight waves per SIMD, with
    spills, were slower than 66 with seven: emission 1.11 against 1.06 ms.) */
 /* The two are launches of their own (VERT or TRI) or, for a small mesh, whose time is that of the
    launches in turn, one launch whose first nbv blocks are the vertices': 7 us of 25 less on 2,000
