@@ -213,6 +213,7 @@ struct Engine {
     bool side_pending = false; /* closest-atom work on `side` not yet joined into `stream` */
 
     DevBuf in_pos, in_rad, d_off, bb_part, bb_out, d_mols, d_meta;
+    DevBuf slot /* atoms by cell, in any order within one */;
     DevBuf key /* cell and rank within the cell per atom */, count, start, perm, cse, sx, aux;
     DevBuf labels, outm, shellm, field, negm, zerom;
     DevBuf s4, wcnt /* per row word: vertex, triangle and cube counts */, vbw, tbw, alist, totals, bounds;
@@ -339,7 +340,7 @@ struct Engine {
     void forget_buffers()
     {
         for (DevBuf *b : {&in_pos, &in_rad, &d_off, &bb_part, &bb_out, &d_mols, &d_meta, &key, &count, &start,
-                          &perm, &cse, &sx, &aux, &labels, &outm, &shellm, &field, &negm, &zerom, &s4, &wcnt,
+                          &perm, &slot, &cse, &sx, &aux, &labels, &outm, &shellm, &field, &negm, &zerom, &s4, &wcnt,
                           &vbw, &tbw, &alist, &ntb, &avb, &acb, &vstart, &tstart, &normals, &colors_in, &totals, &bounds, &rback, &vert, &vert2, &vert3, &vkey,
                           &tri, &tri_out, &atom, &deg_blk, &keeppos, &tri_loc, &scan_tmp, &wsums, &inc_cnt, &inc_start, &inc_ent,
                           &tpre_d, &tflag, &field_dense})
@@ -354,7 +355,7 @@ struct Engine {
     void release_all()
     {
         for (DevBuf *b : {&in_pos, &in_rad, &d_off, &bb_part, &bb_out, &d_mols, &d_meta, &key, &count, &start,
-                          &perm, &cse, &sx, &aux, &labels, &outm, &shellm, &field, &negm, &zerom, &s4, &wcnt,
+                          &perm, &slot, &cse, &sx, &aux, &labels, &outm, &shellm, &field, &negm, &zerom, &s4, &wcnt,
                           &vbw, &tbw, &alist, &ntb, &avb, &acb, &vstart, &tstart, &normals, &colors_in, &totals, &bounds, &rback, &vert, &vert2, &vert3, &vkey,
                           &tri, &tri_out, &atom, &deg_blk, &keeppos, &tri_loc, &scan_tmp, &wsums, &inc_cnt, &inc_start, &inc_ent,
                           &tpre_d, &tflag, &field_dense})
@@ -459,7 +460,7 @@ struct Engine {
     }
 
     int setup(const std::vector<MolIn> &in, const std::vector<BBox> &bb);
-    int upload_mols();
+    int upload_mols(uint32_t *clear = nullptr, uint32_t nclear = 0);
     int fork_side();
     int clear_wsums();
     int build_meta(size_t &at_atoms, size_t &at_p1, size_t &at_mc, size_t &at_wpre,

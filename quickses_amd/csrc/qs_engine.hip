@@ -256,6 +256,7 @@ int Engine::reserve(uint64_t vox, uint64_t atoms, uint64_t cells, uint64_t verts
     QS_TRY(ensure(in_pos, atoms * 12));
     for (DevBuf *b : {&in_rad, &perm}) QS_TRY(ensure(*b, atoms * 4));
     QS_TRY(ensure(key, atoms * 8));
+    QS_TRY(ensure(slot, atoms * 4));
     for (DevBuf *b : {&sx, &aux}) QS_TRY(ensure(*b, atoms * 16));
     QS_TRY(ensure(count, (cells + 1) * 4));
     QS_TRY(ensure(start, (cells + 1) * 4 + 16));
@@ -458,15 +459,16 @@ int Engine::build_meta(size_t &at_atoms, size_t &at_p1, size_t &at_mc, size_t &a
     return 0;
 }
 
-/* the molecules' records and the block prefixes to the device.  One molecule needs no prefixes (see
+/* the molecules' records and the block prefixes to the device, and a clear of nclear counters.  One molecule needs no prefixes (see
    batch), and its record goes in a launch's arguments: a copy takes two to three times as long */
-int Engine::upload_mols()
+int Engine::upload_mols(uint32_t *clear, uint32_t nclear)
 {
     if (mols.size() == 1) {
-        qs_launch_put_mol(mols[0], as<QsMol>(d_mols), stream);
+        qs_launch_put_mol(mols[0], as<QsMol>(d_mols), clear, nclear, stream);
         QS_HIP(hipGetLastError());
         return 0;
     }
+    if (nclear) QS_HIP(hipMemsetAsync(clear, 0, (size_t)nclear * 4, stream));
     QS_TRY(upload(d_mols.p, mols.data(), mols.size() * sizeof(QsMol)));
     return upload(d_meta.p, h_meta.data(), h_meta.size() * 4);
 }
@@ -1043,19 +1045,18 @@ int Engine::run_batch(const float *d_pos, const float *d_rad, const std::vector<
             qs_launch_gather_aux(batch(at_atoms, 0, nmol), nb_atoms, as<int>(perm), d_pos, d_rad, as<float4>(sx), as<float4>(aux),
                                  stream);
     } else {
-        QS_TRY(upload_mols());
-        /* per atom its cell and rank within the cell; per cell its atom count (cleared by a fill) */
+        /* per atom its cell and rank within the cell; per cell its atom count (cleared before) */
         QS_TRY(ensure(key, (size_t)std::max<uint32_t>(n, 1) * 8));
+        QS_TRY(ensure(slot, (size_t)std::max<uint32_t>(n, 1) * 4));
         QS_TRY(ensure(count, ncell * 4));
-        QS_HIP(hipMemsetAsync(count.p, 0, ncell * 4, stream));
+        QS_TRY(upload_mols(as<uint32_t>(count), (uint32_t)ncell));
         if (nb_atoms) qs_launch_hash_count(batch(at_atoms, 0, nmol), nb_atoms, d_pos, as<int2>(key), as<uint32_t>(count), stream);
         /* start[c] = atoms in cells < c (global); start[ncell] = n */
         QS_TRY(scan(as<uint32_t>(count), as<uint32_t>(start), ncell, as<uint32_t>(start) + ncell));
         if (n) {
-            qs_launch_scatter(as<int2>(key), (int)n, as<uint32_t>(start), as<int>(perm), stream);
-            qs_launch_cell_finalize(as<uint32_t>(start), as<uint32_t>(count), (int)ncell, as<int>(perm), as<int2>(cse), stream);
-            qs_launch_gather_aux(batch(at_atoms, 0, nmol), nb_atoms, as<int>(perm), d_pos, d_rad, as<float4>(sx), as<float4>(aux),
-                                 stream);
+            qs_launch_scatter(as<int2>(key), (int)n, as<uint32_t>(start), as<int>(slot), stream);
+            qs_launch_place(batch(at_atoms, 0, nmol), nb_atoms, as<uint32_t>(start), as<int>(slot), (uint32_t)ncell, d_pos,
+                            d_rad, as<int>(perm), as<int2>(cse), as<float4>(sx), as<float4>(aux), stream);
         }
     }
     QS_HIP(hipGetLastError());

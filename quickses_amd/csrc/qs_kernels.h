@@ -10,8 +10,8 @@
 #include "qs_common.h"
 
 /* atoms into cells */
-/* one molecule's record to the device, in the launch's arguments */
-void qs_launch_put_mol(const QsMol &m, QsMol *dst, hipStream_t s);
+/* one molecule's record to the device, in the launch's arguments, and a clear of n counters */
+void qs_launch_put_mol(const QsMol &m, QsMol *dst, uint32_t *clear, uint32_t n, hipStream_t s);
 
 /* bounding boxes: `parts` partial boxes per molecule (qs_bbox_parts of the largest atom count); out
    may be pinned host memory */
@@ -32,8 +32,12 @@ void qs_launch_cells(const QsMol *mols, int nmol, const QsMol *one, size_t lds, 
                      int *perm, int2 *cse, float4 *sx, float4 *aux, hipStream_t s);
 /* key: (cell, rank within the cell) per atom; count: atoms per cell (cleared before) */
 void qs_launch_hash_count(QsBatch B, uint32_t nblocks, const float *pos, int2 *key, uint32_t *count, hipStream_t s);
-void qs_launch_scatter(const int2 *key, int n, const uint32_t *start, int *perm, hipStream_t s);
-void qs_launch_cell_finalize(const uint32_t *start, const uint32_t *count, int ncell, int *perm, int2 *cse, hipStream_t s);
+/* slot: the atoms by cell, in any order within one */
+void qs_launch_scatter(const int2 *key, int n, const uint32_t *start, int *slot, hipStream_t s);
+/* the atoms in the order (cell, index): perm, and as qs_launch_gather_aux sx and aux; the cells' ranges
+   cse; start has the ncell cells' first places and the end */
+void qs_launch_place(QsBatch B, uint32_t nblocks, const uint32_t *start, const int *slot, uint32_t ncell, const float *pos,
+                     const float *rad, int *perm, int2 *cse, float4 *sx, float4 *aux, hipStream_t s);
 /* atoms in cell order (sx) with their exact thresholds and neighbour cells (aux) */
 void qs_launch_gather_aux(QsBatch B, uint32_t nblocks, const int *perm, const float *pos, const float *rad, float4 *sx,
                           float4 *aux, hipStream_t s);

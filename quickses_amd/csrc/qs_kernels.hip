@@ -656,7 +656,7 @@ __global__ void __launch_bounds__(64) k_bbox_final(const float *__restrict__ par
 
 /* hashAtoms Kernels.cu:185-216: cell id x-major (global over the batch); count atoms per cell.
    key[atom] = (cell, the atom's rank among its cell's atoms in the order the counts were taken):
-   the scatter places it with that rank, and the cell's atoms are put in index order afterwards. */
+   the scatter gives it a place in its cell with that rank, and k_place orders the cell's atoms. */
 __global__ void __launch_bounds__(256) k_hash_count(QsBatch B, const float *__restrict__ pos, int2 *__restrict__ key,
                                                     uint32_t *__restrict__ count)
 {
@@ -675,37 +675,12 @@ __global__ void __launch_bounds__(256) k_hash_count(QsBatch B, const float *__re
 }
 
 __global__ void __launch_bounds__(256) k_scatter(const int2 *__restrict__ key, int n, const uint32_t *__restrict__ start,
-                                                 int *__restrict__ perm)
+                                                 int *__restrict__ slot)
 {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     const int2 hr = key[i];
-    perm[start[hr.x] + (uint32_t)hr.y] = i;
-}
-
-/* Per cell: order its atoms by input index, so the whole order is (cell, index) -- the order a
-   stable sort by cell id gives (thrust::sort CudaSurf.cu:610-612) -- and write the cell range
-   (sortCell Kernels.cu:306-341). */
-__global__ void __launch_bounds__(256) k_cell_finalize(const uint32_t *__restrict__ start, const uint32_t *__restrict__ count,
-                                                       int ncell, int *__restrict__ perm, int2 *__restrict__ cse)
-{
-    int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= ncell) return;
-    uint32_t s = start[c], k = count[c];
-    if (k == 0) {
-        cse[c] = make_int2(QS_EMPTY, QS_EMPTY);
-        return;
-    }
-    for (uint32_t a = s + 1; a < s + k; a++) {
-        int v = perm[a];
-        uint32_t b = a;
-        while (b > s && perm[b - 1] > v) {
-            perm[b] = perm[b - 1];
-            b--;
-        }
-        perm[b] = v;
-    }
-    cse[c] = make_int2((int)s, (int)(s + k));
+    slot[start[hr.x] + (uint32_t)hr.y] = i;
 }
 
 /* ------------------------------------------------------------------------------------------ */
@@ -862,9 +837,43 @@ __global__ void __launch_bounds__(256) k_gather_aux(QsBatch B, const int *__rest
     aux[k] = atom_aux(a, G, iclamp(cell_of(a.y, G.oy, G.dxn), 0, G.gn - 1), iclamp(cell_of(a.z, G.oz, G.dxn), 0, G.gn - 1));
 }
 
+/* Every atom to its place in the order (cell, index), the order a stable sort by cell id gives
+   (thrust::sort CudaSurf.cu:610-612): its cell's first place plus the number of the cell's atoms (in
+   slot, in any order) of lower index; with the gathered atom as k_gather_aux writes it, and every cell's
+   range (sortCell Kernels.cu:306-341).  Bound by the gathers of the atoms.  With a thread per cell that
+   sorted its atoms in place, a gather after it and a clear before, all steps of the cells of 50,000
+   atoms took 33 us instead of 27, of 200,000 49 instead of 40, of a million 136 instead of 128 (and
+   159 with a thread per atom in input order, whose writes are then scattered). */
+__global__ void __launch_bounds__(256) k_place(QsBatch B, const uint32_t *__restrict__ start,
+                                               const int *__restrict__ slot, uint32_t ncell, const float *__restrict__ pos,
+                                               const float *__restrict__ rad, int *__restrict__ perm, int2 *__restrict__ cse,
+                                               float4 *__restrict__ sx, float4 *__restrict__ aux)
+{
+    for (uint32_t c = blockIdx.x * 256u + threadIdx.x; c < ncell; c += gridDim.x * 256u) {
+        const uint32_t b = start[c], e = start[c + 1];
+        cse[c] = b == e ? make_int2(QS_EMPTY, QS_EMPTY) : make_int2((int)b, (int)e);
+    }
+    uint32_t lb;
+    const QsMol &M = B.mols[batch_mol(B, blockIdx.x, lb)];
+    const uint32_t i = lb * 256 + threadIdx.x;
+    if (i >= M.n_atoms) return;
+    const QsGrid G = M.G;
+    /* (threads go by place, not by atom: gathers of atoms, but writes next to each other) */
+    const uint32_t id = (uint32_t)slot[M.atom_off + i];
+    const float4 a = make_float4(pos[3 * (size_t)id], pos[3 * (size_t)id + 1], pos[3 * (size_t)id + 2], rad[id]);
+    const int cx = iclamp(cell_of(a.x, G.ox, G.dxn), 0, G.gn - 1), cy = iclamp(cell_of(a.y, G.oy, G.dxn), 0, G.gn - 1),
+              cz = iclamp(cell_of(a.z, G.oz, G.dxn), 0, G.gn - 1);
+    const uint32_t h = M.cell_off + (uint32_t)((G.gn * G.gn * cx) + (G.gn * cy) + cz), b = start[h], e = start[h + 1];
+    uint32_t at = b;
+    for (uint32_t q = b; q < e; q++) at += slot[q] < (int)id ? 1u : 0u;
+    perm[at] = (int)id;
+    sx[at] = a;
+    aux[at] = atom_aux(a, G, cy, cz);
+}
+
 /* Cells of a molecule of at most PER * 1,024 atoms and CELLS_MAX cells in one block: hashing, counts,
    their scan and the order (cell, index) in LDS, and with GATHER the gathered atoms, with the results
-   of k_hash_count, the scan, k_scatter, k_cell_finalize and k_gather_aux.  Bound by the latency of its
+   of k_hash_count, the scan, k_scatter and k_place.  Bound by the latency of its
    few dependent steps, where those launches (and a clear) each had that of a launch; an atom's place
    within its cell is the number of the cell's atoms of lower index, so nothing is sorted.  The cells
    of 300 atoms took 24 us and take 9, of 2,000 atoms 26 and 14.
@@ -3929,10 +3938,11 @@ __global__ void __launch_bounds__(256) k_tri_kept_before(const int *__restrict__
     }
 }
 
-/* one molecule's record, from the launch's arguments */
-__global__ void __launch_bounds__(64) k_put_mol(QsMol m, QsMol *__restrict__ dst)
+/* one molecule's record, from the launch's arguments, and a clear of n counters */
+__global__ void __launch_bounds__(256) k_put_mol(QsMol m, QsMol *__restrict__ dst, uint32_t *__restrict__ clear, uint32_t n)
 {
-    if (threadIdx.x == 0) *dst = m;
+    if (blockIdx.x == 0 && threadIdx.x == 0) *dst = m;
+    for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < n; i += gridDim.x * 256u) clear[i] = 0u;
 }
 
 /* plain device copy (16-byte vectors, grid-stride): the reference point for traffic counters */
@@ -4027,14 +4037,15 @@ void qs_launch_hash_count(QsBatch B, uint32_t nblocks, const float *pos, int2 *k
     hipLaunchKernelGGL(k_hash_count, dim3(nblocks), dim3(256), 0, s, B, pos, key, count);
 }
 
-void qs_launch_scatter(const int2 *key, int n, const uint32_t *start, int *perm, hipStream_t s)
+void qs_launch_scatter(const int2 *key, int n, const uint32_t *start, int *slot, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_scatter, dim3(nblk(n, 256)), dim3(256), 0, s, key, n, start, perm);
+    hipLaunchKernelGGL(k_scatter, dim3(nblk(n, 256)), dim3(256), 0, s, key, n, start, slot);
 }
 
-void qs_launch_cell_finalize(const uint32_t *start, const uint32_t *count, int ncell, int *perm, int2 *cse, hipStream_t s)
+void qs_launch_place(QsBatch B, uint32_t nblocks, const uint32_t *start, const int *slot, uint32_t ncell, const float *pos,
+                     const float *rad, int *perm, int2 *cse, float4 *sx, float4 *aux, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_cell_finalize, dim3(nblk(ncell, 256)), dim3(256), 0, s, start, count, ncell, perm, cse);
+    hipLaunchKernelGGL(k_place, dim3(nblocks), dim3(256), 0, s, B, start, slot, ncell, pos, rad, perm, cse, sx, aux);
 }
 
 void qs_launch_gather_aux(QsBatch B, uint32_t nblocks, const int *perm, const float *pos, const float *rad, float4 *sx,
@@ -4303,7 +4314,10 @@ void qs_launch_cells(const QsMol *mols, int nmol, const QsMol *one, size_t lds, 
                            start, perm, cse, sx, aux);
 }
 
-void qs_launch_put_mol(const QsMol &m, QsMol *dst, hipStream_t s) { hipLaunchKernelGGL(k_put_mol, dim3(1), dim3(64), 0, s, m, dst); }
+void qs_launch_put_mol(const QsMol &m, QsMol *dst, uint32_t *clear, uint32_t n, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_put_mol, dim3(std::min(std::max(nblk(n, 1024), 1u), 512u)), dim3(256), 0, s, m, dst, clear, n);
+}
 
 void qs_launch_copy(const void *src, void *dst, uint64_t bytes, hipStream_t s)
 {
