@@ -1067,6 +1067,14 @@ int Engine::run_batch(const float *d_pos, const float *d_rad, const std::vector<
     if (nmol == 1 && mols[0].G.g && !g_arena) QS_TRY(slab_plan(mols[0], slab_planes));
     if (g_arena && nmol == 1 && (uint64_t)mols[0].G.g * mols[0].G.g * mols[0].G.g >= (1ull << 32))
         return set_error(6, "grid of %d^3 points: too large for the fixed scratch region", mols[0].G.g);
+    /* the run's one read-back, gathered by the triangle filter's kernel (straight into the pinned
+       staging): totals, per-molecule first vertices and kept-triangle offsets */
+    std::vector<uint32_t> hb(4 + 2 * ((size_t)nmol + 1));
+    QS_TRY(ensure(rback, hb.size() * 4));
+    QS_TRY(ensure(bounds, ((size_t)nmol + 1) * 8));
+    uint32_t *fs = (uint32_t *)stage(hb.size() * 4);
+    uint32_t *rb = fs ? fs : as<uint32_t>(rback);
+    bool filtered = false; /* the triangles, by the first smoothing pass's launch */
     if (slab_planes) {
         QS_TRY(run_slabs(slab_planes, smooth, tm));
     } else {
@@ -1084,11 +1092,21 @@ int Engine::run_batch(const float *d_pos, const float *d_rad, const std::vector<
         float *dst = as<float>(vert2);
         const uint64_t *wpre = (const uint64_t *)(as<uint32_t>(d_meta) + at_wpre);
         const uint32_t *wcoarse = nmol > 1 ? as<uint32_t>(d_meta) + at_wpre + 2 * ((size_t)nmol + 1) : nullptr;
+        /* One molecule whose triangle pool the compaction needs no scan for (TRI_SELF_BLOCKS) has it run
+           by blocks of the first pass's launch: a launch less on a mesh that is a chain of short ones
+           (2,000 atoms at 0.5 A: 129 -> 118 us in all, 300 at 1.0 A: 115 -> 103).  Above that the
+           scan is a launch of its own before it, and a launch's share of the run is below 1 %. */
+        QsCompact compact{};
+        filtered = nmol == 1 && pool_v && pool_t && pool_t / 256 + 1 <= TRI_SELF_BLOCKS;
+        if (filtered) {
+            QS_TRY(ensure(tri_out, (size_t)pool_t * 12));
+            compact = QsCompact{as<uint32_t>(deg_blk), as<int>(tri_out), as<uint32_t>(d_off) + 2, as<uint32_t>(bounds), rb};
+        }
         for (int it = 0; it < smooth; it++) {
             qs_launch_smooth(as<QsMol>(d_mols), d_vpre, nmol > 1 ? d_vpre + nmol + 1 : nullptr, wpre, wcoarse, as<uint32_t>(alist),
                              as<uint32_t>(vstart), as<uint64_t>(negm), as<uint64_t>(zerom), as<uint64_t>(s4), as<uint32_t>(vbw),
                              as<uint64_t>(vkey), pool_v, pool_t, as<uint64_t>(ntb), as<uint32_t>(tbw), as<int>(tri), src, dst,
-                             as<uint32_t>(totals), expect_v, stream);
+                             as<uint32_t>(totals), expect_v, filtered && it == 0 ? &compact : nullptr, stream);
             src = dst;
             dst = (dst == as<float>(vert2)) ? as<float>(vert3) : as<float>(vert2);
         }
@@ -1120,27 +1138,22 @@ int Engine::run_batch(const float *d_pos, const float *d_rad, const std::vector<
         qs_launch_deg_count(as<int>(tri), nt_all, as<uint32_t>(deg_blk), as<uint32_t>(totals) + 3, stream);
         QS_HIP(hipGetLastError());
     }
-    QS_TRY(ensure(keeppos, (nblk_t + 1) * 4));
-    QS_TRY(ensure(tri_out, (size_t)std::max<uint32_t>(tcap, 1) * 12));
-    QS_TRY(ensure(bounds, ((size_t)nmol + 1) * 8));
-    /* the run's one read-back, gathered by the last kernel (straight into the pinned staging): totals,
-       per-molecule first vertices and kept-triangle offsets */
-    std::vector<uint32_t> hb(4 + 2 * ((size_t)nmol + 1));
-    QS_TRY(ensure(rback, hb.size() * 4));
-    uint32_t *fs = (uint32_t *)stage(hb.size() * 4);
-    uint32_t *rb = fs ? fs : as<uint32_t>(rback);
-    uint32_t *vpre = as<uint32_t>(d_off) + (nmol + 1);
-    /* a block of the compaction adds up the counts of up to TRI_SELF_BLOCKS blocks itself */
-    const bool self = nmol == 1 && nblk_t <= TRI_SELF_BLOCKS;
-    if (!self) QS_TRY(scan(as<uint32_t>(deg_blk), as<uint32_t>(keeppos), nblk_t, as<uint32_t>(keeppos) + nblk_t));
-    const uint32_t *dpre = self ? as<uint32_t>(deg_blk) : as<uint32_t>(keeppos);
-    if (nmol == 1) {
-        qs_launch_tri_compact_one(as<int>(tri), tcap, dpre, self, as<uint32_t>(totals), as<int>(tri_out),
-                                  multi_slab ? nullptr : as<uint32_t>(totals), nv, vpre, as<uint32_t>(bounds), rb, stream);
-    } else {
-        qs_launch_tri_compact(as<int>(tri), tcap, dpre, as<uint32_t>(totals), as<int>(tri_out), as<uint32_t>(totals), stream);
-        qs_launch_tri_kept_before(as<int>(tri), dpre, as<uint64_t>(tpre_d), nmol + 1, tcap, as<uint32_t>(bounds),
-                                  as<uint32_t>(totals), vpre, rb, stream);
+    if (!filtered) {
+        QS_TRY(ensure(keeppos, (nblk_t + 1) * 4));
+        QS_TRY(ensure(tri_out, (size_t)std::max<uint32_t>(tcap, 1) * 12));
+        uint32_t *vpre = as<uint32_t>(d_off) + (nmol + 1);
+        /* a block of the compaction adds up the counts of up to TRI_SELF_BLOCKS blocks itself */
+        const bool self = nmol == 1 && nblk_t <= TRI_SELF_BLOCKS;
+        if (!self) QS_TRY(scan(as<uint32_t>(deg_blk), as<uint32_t>(keeppos), nblk_t, as<uint32_t>(keeppos) + nblk_t));
+        const uint32_t *dpre = self ? as<uint32_t>(deg_blk) : as<uint32_t>(keeppos);
+        if (nmol == 1) {
+            qs_launch_tri_compact_one(as<int>(tri), tcap, dpre, self, as<uint32_t>(totals), as<int>(tri_out),
+                                      multi_slab ? nullptr : as<uint32_t>(totals), nv, vpre, as<uint32_t>(bounds), rb, stream);
+        } else {
+            qs_launch_tri_compact(as<int>(tri), tcap, dpre, as<uint32_t>(totals), as<int>(tri_out), as<uint32_t>(totals), stream);
+            qs_launch_tri_kept_before(as<int>(tri), dpre, as<uint64_t>(tpre_d), nmol + 1, tcap, as<uint32_t>(bounds),
+                                      as<uint32_t>(totals), vpre, rb, stream);
+        }
     }
     QS_HIP(hipGetLastError());
     if (!fs) QS_HIP(hipMemcpyAsync(hb.data(), rb, hb.size() * 4, hipMemcpyDeviceToHost, stream));

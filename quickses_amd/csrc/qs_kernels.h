@@ -141,12 +141,18 @@ void qs_launch_mesh_bases(const uint32_t *vbw, const uint32_t *tbw, const uint64
 void qs_launch_closest_atom(const QsMol *mols, const uint32_t *vpre, const uint32_t *vcoarse, const QsClosest &A,
                             const float *vert, uint32_t nv, const uint32_t *d_nv, uint32_t expect, hipStream_t s);
 /* one Laplacian pass over the pools of nv vertices and ntri triangles (list, vstart: the active words
-   and each 256-vertex block's first one) */
+   and each 256-vertex block's first one).  compact (may be NULL; at most TRI_SELF_BLOCKS blocks of
+   triangles): qs_launch_tri_compact_one's work in the same launch, its counts from d_counts */
+struct QsCompact {
+    const uint32_t *deg_blk;
+    int *out;
+    uint32_t *vpre, *kept, *rb;
+};
 void qs_launch_smooth(const QsMol *mols, const uint32_t *vpre, const uint32_t *vcoarse, const uint64_t *wpre, const uint32_t *wcoarse,
                       const uint32_t *list, const uint32_t *vstart, const uint64_t *N, const uint64_t *Zm, const uint64_t *S4,
                       const uint32_t *vbw, const uint64_t *vkey, uint32_t nv, uint32_t ntri, const uint64_t *NT,
                       const uint32_t *tbw, const int *tri, const float *src, float *dst, const uint32_t *d_counts, uint32_t expect,
-                      hipStream_t s);
+                      const QsCompact *compact, hipStream_t s);
 
 /* Laplacian passes over a triangle array (meshes built in x-slabs): per-vertex incidence counts
    (cnt, nv entries, cleared by the caller) from the triangles, then, after an exclusive scan of

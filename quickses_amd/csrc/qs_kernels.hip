@@ -3475,6 +3475,75 @@ __device__ __forceinline__ void vertex_point(uint64_t key, int g, int &x, int &y
     y = (int)(xy - (uint32_t)x * ug);
 }
 
+/* ------------------------------------------------------------------------------------------ */
+/* degenerate-triangle filter (CudaSurf.cu:820-829), order preserving: block b of 256 triangles
+   writes its kept ones from position 256 b - dpre[b] on, dpre being the exclusive prefix of the
+   per-block degenerate counts */
+__device__ __forceinline__ bool tri_degenerate(const int *__restrict__ tri, uint32_t t)
+{
+    const int x = tri[3 * (size_t)t], y = tri[3 * (size_t)t + 1], z = tri[3 * (size_t)t + 2];
+    return !(x != y && y != z && x != z);
+}
+
+/* ONE: one molecule.  Its read-back {totals[0..3], first vertices (0, nv), kept triangles before its
+   first and last (0, nt - *ndeg)} and the last two pairs (vpre, kept) are written here too.
+   self: dpre holds the per-block counts themselves (at most TRI_SELF_BLOCKS of them) and each block
+   adds up those before it, which only happens when there is something to drop. */
+template <bool ONE>
+__device__ __forceinline__ void tri_compact(const int *__restrict__ tri, uint32_t nt, const uint32_t *__restrict__ dpre,
+                                            const uint32_t *__restrict__ totals, int *__restrict__ out,
+                                            const uint32_t *__restrict__ d_nt, int self, uint32_t nv, uint32_t *__restrict__ vpre,
+                                            uint32_t *__restrict__ kept, uint32_t *__restrict__ rb, uint32_t bid, uint32_t nblocks)
+{
+    __shared__ uint32_t wkeep[4], lds[256 / 64 + 1];
+    const uint32_t ndeg = totals[3];
+    if (ONE && bid == 0 && threadIdx.x < 8) {
+        const uint32_t t = threadIdx.x, all_t = d_nt ? *d_nt : nt, all_v = d_nt ? totals[1] : nv;
+        const uint32_t end = t == 5 ? all_v : (t == 7 ? all_t - ndeg : 0u);
+        rb[t] = t < 4 ? totals[t] : end;
+        if (t >= 6) kept[t - 6] = end;
+        else if (t >= 4) vpre[t - 4] = end;
+    }
+    if (ndeg == 0) return; /* nothing to drop: the caller keeps the input array */
+    if (d_nt) nt = min(*d_nt, nt); /* the device count within the launch's pool */
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    /* persistent blocks over the 256-triangle blocks */
+    for (uint32_t b = bid; b * 256u < nt; b += nblocks) {
+        const uint32_t t = b * 256u + threadIdx.x;
+        const bool keep = t < nt && !tri_degenerate(tri, t);
+        const uint64_t km = __ballot(keep);
+        if (lane == 0) wkeep[wid] = (uint32_t)__popcll(km);
+        __syncthreads();
+        uint32_t before;
+        if (ONE && self) {
+            uint32_t x = 0;
+            for (uint32_t k = threadIdx.x; k < b; k += 256u) x += dpre[k];
+            before = block_sum<256>(x, lds);
+        } else {
+            before = dpre[b];
+        }
+        uint32_t o = b * 256u - before + (uint32_t)__popcll(km & ((1ull << lane) - 1ull));
+        for (int k = 0; k < wid; k++) o += wkeep[k];
+        if (keep) {
+            out[3 * (size_t)o] = tri[3 * (size_t)t];
+            out[3 * (size_t)o + 1] = tri[3 * (size_t)t + 1];
+            out[3 * (size_t)o + 2] = tri[3 * (size_t)t + 2];
+        }
+        __syncthreads(); /* wkeep is written again for the next block */
+    }
+}
+
+template <bool ONE>
+__global__ void __launch_bounds__(256) k_tri_compact(const int *__restrict__ tri, uint32_t nt,
+                                                     const uint32_t *__restrict__ dpre, const uint32_t *__restrict__ totals,
+                                                     int *__restrict__ out, const uint32_t *__restrict__ d_nt, int self, uint32_t nv,
+                                                     uint32_t *__restrict__ vpre, uint32_t *__restrict__ kept,
+                                                     uint32_t *__restrict__ rb)
+{
+    tri_compact<ONE>(tri, nt, dpre, totals, out, d_nt, self, nv, vpre, kept, rb, blockIdx.x, gridDim.x);
+}
+
+/* ------------------------------------------------------------------------------------------ */
 /* triangles and vertices that a smoothing block stages in LDS at most (10 bits per corner) */
 constexpr uint32_t SM_TRI = 1408, SM_VERT = 1024;
 /* expected vertices above which blocks stage: a smaller mesh is bound by a block's chain of loads, which
@@ -3497,8 +3566,11 @@ constexpr uint32_t SM_STAGED_MIN = 1u << 19;
    gathers from memory.  Then bound by VALU issue, and by waves in flight: 64 registers, so the
    triangles' loads end before the positions' begin.  On 256 molecules at 0.5 A gathers took 0.793 ms
    and this takes 0.566, on the 50,000-atom 0.2 A mesh 0.188 and 0.156, on 1M atoms at 0.5 A (two passes)
-   0.660 and 0.537. */
-template <bool STAGED>
+   0.660 and 0.537.
+   COMPACT: blocks from nbs on filter the triangles, which the pass only reads too (one molecule, the
+   work of k_tri_compact<true>): on a small mesh, a chain of short launches, one launch less (2,000
+   atoms at 0.5 A: 129 -> 118 us in all). */
+template <bool STAGED, bool COMPACT>
 __global__ void __launch_bounds__(256, STAGED ? 8 : 1) k_smooth(const QsMol *__restrict__ mols, const uint32_t *__restrict__ vpre,
                                                    const uint32_t *__restrict__ vcoarse, const uint64_t *__restrict__ wpre,
                                                    const uint32_t *__restrict__ wcoarse, const uint32_t *__restrict__ list,
@@ -3508,8 +3580,16 @@ __global__ void __launch_bounds__(256, STAGED ? 8 : 1) k_smooth(const QsMol *__r
                                                    uint32_t nv, uint32_t ntri, const uint64_t *__restrict__ NT_all,
                                                    const uint32_t *__restrict__ tbw_all, const int *__restrict__ tri,
                                                    const float *__restrict__ src, float *__restrict__ dst,
-                                                   const uint32_t *__restrict__ d_counts)
+                                                   const uint32_t *__restrict__ d_counts, QsCompact K, uint32_t nbs)
 {
+    const uint32_t nblocks = COMPACT ? nbs : gridDim.x;
+    if constexpr (COMPACT) {
+        if (blockIdx.x >= nbs) {
+            tri_compact<true>(tri, ntri, K.deg_blk, d_counts, K.out, d_counts, 1, 0u, K.vpre, K.kept, K.rb, blockIdx.x - nbs,
+                              gridDim.x - nbs);
+            return;
+        }
+    }
     __shared__ uint32_t s_tri[STAGED ? SM_TRI : 1];           /* corners' places, in bits 2, 12 and 22 on */
     __shared__ float s_pos[3][STAGED ? SM_VERT : 1];
     /* a mesh larger than the pools (the run is repeated with larger ones) has ids past them: nothing
@@ -3519,7 +3599,7 @@ __global__ void __launch_bounds__(256, STAGED ? 8 : 1) k_smooth(const QsMol *__r
     const uint32_t nact = d_counts[2];
     const uint32_t nb = (nv + 255u) >> 8;
     /* persistent blocks over the 256-vertex blocks (grid a multiple of 8: see k_mc_emit) */
-    for (uint32_t vb = blockIdx.x; vb < nb; vb += gridDim.x) {
+    for (uint32_t vb = blockIdx.x; vb < nb; vb += nblocks) {
         const uint32_t blk = xcd_group<64>(vb, nb), v = blk * 256u + threadIdx.x;
         bool staged = false;
         if constexpr (STAGED) {
@@ -3798,15 +3878,6 @@ __global__ void __launch_bounds__(256) k_vertex_colors(const QsMol *__restrict__
 }
 
 /* ------------------------------------------------------------------------------------------ */
-/* degenerate-triangle filter (CudaSurf.cu:820-829), order preserving: block b of 256 triangles
-   writes its kept ones from position 256 b - dpre[b] on, dpre being the exclusive prefix of the
-   per-block degenerate counts */
-__device__ __forceinline__ bool tri_degenerate(const int *__restrict__ tri, uint32_t t)
-{
-    const int x = tri[3 * (size_t)t], y = tri[3 * (size_t)t + 1], z = tri[3 * (size_t)t + 2];
-    return !(x != y && y != z && x != z);
-}
-
 /* Per-molecule first vertex and first triangle of a batch, from the word scans: molecule m's are
    the exclusive scans at its first row word (wpre[m]; at or past the scanned words nw for a
    molecule without words, whose mesh is empty and starts at the totals).  vpre / tpre get nmol + 1 entries, the last one the
@@ -3858,55 +3929,6 @@ __global__ void __launch_bounds__(256) k_deg_count(const int *__restrict__ tri, 
     if (threadIdx.x == 0) {
         deg_blk[blockIdx.x] = sum;
         if (sum) atomicAdd(deg_total, sum);
-    }
-}
-
-/* ONE: one molecule.  Its read-back {totals[0..3], first vertices (0, nv), kept triangles before its
-   first and last (0, nt - *ndeg)} and the last two pairs (vpre, kept) are written here too.
-   self: dpre holds the per-block counts themselves (at most TRI_SELF_BLOCKS of them) and each block
-   adds up those before it, which only happens when there is something to drop. */
-template <bool ONE>
-__global__ void __launch_bounds__(256) k_tri_compact(const int *__restrict__ tri, uint32_t nt,
-                                                     const uint32_t *__restrict__ dpre, const uint32_t *__restrict__ totals,
-                                                     int *__restrict__ out, const uint32_t *__restrict__ d_nt, int self, uint32_t nv,
-                                                     uint32_t *__restrict__ vpre, uint32_t *__restrict__ kept,
-                                                     uint32_t *__restrict__ rb)
-{
-    __shared__ uint32_t wkeep[4], lds[256 / 64 + 1];
-    const uint32_t ndeg = totals[3];
-    if (ONE && blockIdx.x == 0 && threadIdx.x < 8) {
-        const uint32_t t = threadIdx.x, all_t = d_nt ? *d_nt : nt, all_v = d_nt ? totals[1] : nv;
-        const uint32_t end = t == 5 ? all_v : (t == 7 ? all_t - ndeg : 0u);
-        rb[t] = t < 4 ? totals[t] : end;
-        if (t >= 6) kept[t - 6] = end;
-        else if (t >= 4) vpre[t - 4] = end;
-    }
-    if (ndeg == 0) return; /* nothing to drop: the caller keeps the input array */
-    if (d_nt) nt = min(*d_nt, nt); /* the device count within the launch's pool */
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    /* persistent blocks over the 256-triangle blocks */
-    for (uint32_t b = blockIdx.x; b * 256u < nt; b += gridDim.x) {
-        const uint32_t t = b * 256u + threadIdx.x;
-        const bool keep = t < nt && !tri_degenerate(tri, t);
-        const uint64_t km = __ballot(keep);
-        if (lane == 0) wkeep[wid] = (uint32_t)__popcll(km);
-        __syncthreads();
-        uint32_t before;
-        if (ONE && self) {
-            uint32_t x = 0;
-            for (uint32_t k = threadIdx.x; k < b; k += 256u) x += dpre[k];
-            before = block_sum<256>(x, lds);
-        } else {
-            before = dpre[b];
-        }
-        uint32_t o = b * 256u - before + (uint32_t)__popcll(km & ((1ull << lane) - 1ull));
-        for (int k = 0; k < wid; k++) o += wkeep[k];
-        if (keep) {
-            out[3 * (size_t)o] = tri[3 * (size_t)t];
-            out[3 * (size_t)o + 1] = tri[3 * (size_t)t + 1];
-            out[3 * (size_t)o + 2] = tri[3 * (size_t)t + 2];
-        }
-        __syncthreads(); /* wkeep is written again for the next block */
     }
 }
 
@@ -4257,16 +4279,21 @@ void qs_launch_smooth(const QsMol *mols, const uint32_t *vpre, const uint32_t *v
                       const uint32_t *list, const uint32_t *vstart, const uint64_t *N, const uint64_t *Zm, const uint64_t *S4,
                       const uint32_t *vbw, const uint64_t *vkey, uint32_t nv, uint32_t ntri, const uint64_t *NT,
                       const uint32_t *tbw, const int *tri, const float *src, float *dst, const uint32_t *d_counts, uint32_t expect,
-                      hipStream_t s)
+                      const QsCompact *compact, hipStream_t s)
 {
     if (!nv) return;
     const dim3 grid(pgrid(nblk(std::min(nv, expect), 256)));
-    if (std::min(nv, expect) > SM_STAGED_MIN)
-        hipLaunchKernelGGL(k_smooth<true>, grid, dim3(256), 0, s, mols, vpre, vcoarse, wpre, wcoarse, list, vstart, N, Zm, S4, vbw,
-                           vkey, nv, ntri, NT, tbw, tri, src, dst, d_counts);
-    else
-        hipLaunchKernelGGL(k_smooth<false>, grid, dim3(256), 0, s, mols, vpre, vcoarse, wpre, wcoarse, list, vstart, N, Zm, S4, vbw,
-                           vkey, nv, ntri, NT, tbw, tri, src, dst, d_counts);
+    if (compact) {
+        const unsigned nbs = grid.x, nbc = std::max(1u, std::min(nblk(ntri, 256), COMPACT_BLOCKS));
+        hipLaunchKernelGGL((k_smooth<false, true>), dim3(nbs + nbc), dim3(256), 0, s, mols, vpre, vcoarse, wpre, wcoarse, list, vstart,
+                           N, Zm, S4, vbw, vkey, nv, ntri, NT, tbw, tri, src, dst, d_counts, *compact, nbs);
+    } else if (std::min(nv, expect) > SM_STAGED_MIN) {
+        hipLaunchKernelGGL((k_smooth<true, false>), grid, dim3(256), 0, s, mols, vpre, vcoarse, wpre, wcoarse, list, vstart, N, Zm, S4,
+                           vbw, vkey, nv, ntri, NT, tbw, tri, src, dst, d_counts, QsCompact{}, 0u);
+    } else {
+        hipLaunchKernelGGL((k_smooth<false, false>), grid, dim3(256), 0, s, mols, vpre, vcoarse, wpre, wcoarse, list, vstart, N, Zm,
+                           S4, vbw, vkey, nv, ntri, NT, tbw, tri, src, dst, d_counts, QsCompact{}, 0u);
+    }
 }
 
 void qs_launch_vertex_normals(const QsMol *mols, const uint32_t *vpre, const uint32_t *vcoarse, const uint64_t *vkey, uint32_t nv,

@@ -207,3 +207,18 @@ def test_mesh_copied_to_any_alignment(qs, shift):
         got, k = hipmem.download(buf.ptr, (ref.size + 8,), np.int32), shift // 4
         assert np.array_equal(got[k:k + ref.size], ref.ravel())
         assert (got[:k] == -7).all() and (got[k + ref.size:] == -7).all()
+
+
+@pytest.mark.parametrize("n,smooth", [(2, 1), (5, 1), (5, 2), (7, 1)])
+def test_triangles_filtered_beside_smoothing(qs, orc, n, smooth):
+    """A lattice whose mesh has triangles to drop: below the pool size up to which the
+    first of the passes filters them, and above it (n = 7); the next run reads what this one left."""
+    ax = np.arange(n, dtype=np.float32) * np.float32(2.5) - np.float32(2.5 * (n // 2))
+    pos, rad = np.stack(np.meshgrid(ax, ax, ax, indexing="ij"), -1).reshape(-1, 3), np.full(n ** 3, 1.6, np.float32)
+    G, _, _, _, _, _, fld = orc.field(pos, rad, 0.1)
+    tri = orc.edge_weld(G, G.g - 1, fld)[1]
+    want = orc.compute_ses(pos, rad, 0.1, smooth)
+    assert len(tri) > len(want[1])
+    for run in range(2):
+        print("case filter beside smoothing: n=%d smooth=%d run=%d" % (n, smooth, run), flush=True)
+        assert _same(qs.compute_ses(pos, rad, 0.1, smooth), want)
