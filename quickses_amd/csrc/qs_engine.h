@@ -309,6 +309,9 @@ struct Engine {
     uint32_t nv = 0, nt_all = 0, nt = 0, n_active = 0;
     size_t p1_lds = 0; /* dynamic LDS of the field pass 1 launch (largest molecule of the batch) */
     bool batch_valid = false; /* result arrays, vert_off / tri_off and their device copies belong to run_batch */
+    /* the grid arrays and the counts are those of mols: the last run or stage finished (qs_fetch reads
+       nothing otherwise, as a call that stopped early leaves new grids beside older arrays) */
+    bool grid_valid = false;
     /* field holds shell voxels' values only (field pass 2), the others come from outm / shellm; else
        it holds every voxel.  In grid order either way. */
     bool field_sparse = false;
@@ -335,6 +338,15 @@ struct Engine {
     float *res_vert = nullptr;
     int *res_tri = nullptr, *res_atom = nullptr;
 
+    /* at the start of a run or stage: nothing of the last one's grid may be read through new records */
+    void forget_grid()
+    {
+        grid_valid = batch_valid = false;
+        field_sparse = field_band = false;
+        run_flags = nullptr;
+        groups.clear();
+    }
+
     /* drops every device buffer record without freeing it (buffers carved from a fixed region,
        which the next run reuses from its start), and the cached pass-2 tables with them */
     void forget_buffers()
@@ -347,8 +359,7 @@ struct Engine {
             *b = DevBuf{};
         for (P2Tables *t : tables) delete t;
         tables.clear();
-        groups.clear();
-        batch_valid = false;
+        forget_grid();
     }
 
     /* frees every device buffer and the stream (the engine can be initialised again) */
@@ -365,7 +376,7 @@ struct Engine {
             delete t;
         }
         tables.clear();
-        groups.clear();
+        forget_grid();
         if (stream) (void)hipStreamSynchronize(stream);
         if (up) (void)hipHostFree(up);
         up = nullptr;
@@ -378,7 +389,6 @@ struct Engine {
         if (ev_side) (void)hipEventDestroy(ev_side);
         ev_emit = ev_side = nullptr;
         device = -1;
-        batch_valid = false;
     }
 
     int init()

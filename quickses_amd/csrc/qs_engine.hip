@@ -955,7 +955,7 @@ int Engine::run_batch(const float *d_pos, const float *d_rad, const std::vector<
         QS_HIP(hipStreamSynchronize(side));
         side_pending = false;
     }
-    batch_valid = false;
+    forget_grid();
     nv = nt = nt_all = n_active = 0;
     res_vert = nullptr;
     res_tri = nullptr;
@@ -1188,7 +1188,7 @@ int Engine::run_batch(const float *d_pos, const float *d_rad, const std::vector<
     nt = tri_off[nmol];
     res_tri = ndeg ? as<int>(tri_out) : as<int>(tri);
     res_atom = as<int>(atom);
-    batch_valid = true; /* device copies: vertex offsets after the molecule prefixes in d_off, triangle offsets in bounds */
+    grid_valid = batch_valid = true; /* device copies: vertex offsets after the molecule prefixes in d_off, triangle offsets in bounds */
     tm.report(mols[0].G, n);
     return 0;
 }
@@ -1347,6 +1347,7 @@ void *batch_host_array(int k, size_t bytes)
 /* one-molecule batch with a given grid (stage-wise entry points) */
 int single_grid(Engine &E, const QsGrid &G, size_t &at_mc, uint32_t &nb_mc, size_t &at_wpre)
 {
+    E.forget_grid();
     E.mols.assign(1, QsMol{});
     QsMol &M = E.mols[0];
     M.G = G;
@@ -1361,7 +1362,6 @@ int single_grid(Engine &E, const QsGrid &G, size_t &at_mc, uint32_t &nb_mc, size
     E.scan_w0 = 0;
     E.scan_nw = E.nw_total;
     E.multi_slab = false;
-    E.batch_valid = false;
     E.vert_off.assign(2, 0);
     E.tri_off.assign(2, 0);
     size_t at_atoms, at_p1;
@@ -1981,7 +1981,7 @@ int64_t qs_fetch(const char *what, void *host, int64_t bytes)
 {
     Engine &E = g_eng;
     std::string w = what ? what : "";
-    if (E.mols.empty()) return -1;
+    if (E.mols.empty() || !E.grid_valid) return -1;
     const QsGrid &G = E.mols[0].G;
     const uint64_t V = E.vox_total;
     const void *src = nullptr;
@@ -2007,9 +2007,9 @@ int64_t qs_fetch(const char *what, void *host, int64_t bytes)
         return (int64_t)V0;
     }
     else if (w == "field") {
-        if (E.fill_field(&src) != 0) return -1;
-        if (hipStreamSynchronize(E.stream) != hipSuccess) return -1;
         need = (int64_t)V * 4;
+        if (bytes < need || E.fill_field(&src) != 0) return -1;
+        if (hipStreamSynchronize(E.stream) != hipSuccess) return -1;
     }
     else if (w == "shellm") { src = E.shellm.p; need = (int64_t)E.nw_total * 8; }
     else if (w == "perm") { src = E.perm.p; need = (int64_t)E.n_atoms_total * 4; }
@@ -2064,6 +2064,7 @@ int qs_stage_pass2(const float *fp, const int *ip, const uint8_t *labels, float 
     const void *dense = nullptr;
     QS_TRY(E.fill_field(&dense));
     QS_HIP(hipStreamSynchronize(E.stream));
+    E.grid_valid = true;
     QS_HIP(hipMemcpy(field, dense, V * 4, hipMemcpyDeviceToHost));
     return 0;
 }
@@ -2100,6 +2101,7 @@ int qs_stage_mesh(const float *fp, const int *ip, const float *field, unsigned i
         if (!E.pools_overflowed(E.nv, E.nt_all)) break;
         if (attempt) return set_error(4, "mesh pools overflowed again");
     }
+    E.grid_valid = true;
     if (nvert) *nvert = E.nv;
     if (ntri) *ntri = E.nt_all;
     if ((int64_t)E.nv * 3 > vert_cap || (int64_t)E.nt_all * 3 > tri_cap) return set_error(5, "output capacity too small");

@@ -1,0 +1,52 @@
+"""What one call leaves for the next: results of calls that stopped early, of other molecules and of
+optional passes asked for afterwards."""
+import ctypes
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+FETCHES = ("labels", "field", "shellm", "perm", "cells", "vert_unsmoothed", "tri_all")
+
+
+def _fetch(qs, what, nbytes):
+    out = np.zeros(nbytes, np.uint8)
+    return qs.lib().qs_fetch(what.encode(), ctypes.c_void_p(out.ctypes.data), ctypes.c_int64(nbytes))
+
+
+def _refused(qs, kind):
+    """A call of `kind` that the library refuses after a run of another shape."""
+    pos, rad = qs.synth_ball(91, 900)
+    if kind == "second molecule's voxel size":
+        with pytest.raises(qs.QuickSESError):
+            qs.compute_batch([(pos, rad), (pos[:50], rad[:50])], [0.5, 0.0], 1)
+    elif kind == "first molecule's coordinates":
+        with pytest.raises(qs.QuickSESError):
+            qs.compute_batch([(pos + np.float32(2e5), rad), (pos, rad)], 0.5, 1)
+    elif kind == "voxel size":
+        with pytest.raises(qs.QuickSESError):
+            qs.compute_ses(pos, rad, -1.0, 1)
+    else:  # a larger grid that no x-slab of 1 MiB holds
+        qs.set_option("slab_mb", 1)
+        try:
+            with pytest.raises(qs.QuickSESError, match="x-slab"):
+                qs.compute_ses(pos, rad, 0.2, 1)
+        finally:
+            qs.set_option("slab_mb", 0)
+
+
+@pytest.mark.parametrize("kind", ["second molecule's voxel size", "first molecule's coordinates", "voxel size", "slab memory"])
+def test_fetch_after_a_refused_call(qs, orc, kind):
+    """Nothing is read (and no field pass is run) through the records of a call that did not finish."""
+    pos, rad = qs.synth_ball(90, 300)
+    print("case refused call: %s" % kind, flush=True)
+    qs.compute_ses(pos, rad, 0.5, 1)
+    _refused(qs, kind)
+    for what in FETCHES:
+        assert _fetch(qs, what, 64 << 20) == -1, what
+    assert qs.last_slab_count() == 0
+    qs.compute_ses(pos, rad, 0.5, 1)
+    g = qs.last_grid()["g"]
+    assert _fetch(qs, "field", 4 * g ** 3 - 1) == -1
+    assert np.array_equal(qs.fetch("field", np.float32, g ** 3).view(np.uint32), orc.field(pos, rad, 0.5)[6].view(np.uint32))
