@@ -330,7 +330,7 @@ struct Engine {
     int n_slabs = 1;
     /* vertex and triangle pools of the current run, and the least pools later runs start from
        (grown when a run needed more) */
-    uint32_t pool_v = 0, pool_t = 0, expect_v = 0;
+    uint32_t pool_v = 0, pool_t = 0, expect_v = 0, block_v = 0;
     uint64_t ntflags = 0; /* tile flags of the run's fixed-R pass-2 molecules */
     uint8_t tmark = 0;    /* the field passes' tile mark, 1-255, changed every run */
     uint64_t cap_v = 0, cap_t = 0;

@@ -688,12 +688,12 @@ int Engine::mesh_stage(size_t at_mc, uint32_t nb_mc, size_t at_wpre, StageTimer 
                       field_sparse ? as<uint64_t>(shellm) : nullptr, as<float>(vert), as<uint64_t>(vkey), as<uint32_t>(acb),
                       as<uint32_t>(tstart), pool_t, pool_t, as<uint64_t>(negm), as<uint32_t>(wcnt), as<uint32_t>(vbw),
                       as<uint32_t>(tbw), as<uint64_t>(ntb), as<int>(tri), 0u, as<uint32_t>(deg_blk), as<uint32_t>(totals) + 3, counts,
-                      stream, with_atoms && fused ? &near : nullptr, scan_nw != 0, expect_v);
+                      stream, with_atoms && fused ? &near : nullptr, scan_nw != 0, block_v);
     QS_HIP(hipGetLastError());
     tm.mark("mc_emit");
     if (with_atoms && !fused) {
         qs_launch_closest_atom(as<QsMol>(d_mols), d_vpre, nmol > 1 ? d_vpre + nmol + 1 : nullptr, near, as<float>(vert), pool_v,
-                               counts + 1, expect_v, stream);
+                               counts + 1, block_v, stream);
         QS_HIP(hipGetLastError());
         tm.mark("closest_atom");
     }
@@ -702,10 +702,17 @@ int Engine::mesh_stage(size_t at_mc, uint32_t nb_mc, size_t at_wpre, StageTimer 
 
 /* Vertex and triangle pools of a run: about 8 A^2 of surface per atom (measured 2-6 A^2 on the
    benchmark molecules, cavities included), at least what earlier runs needed (cap_v, cap_t).
-   expect_v: the vertices (and about the cubes) that launches over the pools have blocks for, 15 %
-   above the area of a packed ball of the molecule's atoms; blocks past the pool's contents leave at
-   once, but 240,000 of them took 60 us on 256 molecules at 0.5 A (4.91 -> 4.77 ms of stages with the
-   compaction's), and blocks loop where a mesh has more. */
+   expect_v: the vertices (and about the cubes) to expect, 15 % above the area of a ball of that many
+   atoms packed as the benchmark molecules are (0.05 atoms / A^3, radii about 1.6 A).  Launches over the
+   pools have blocks for block_v of them, as 240,000 blocks past the pool's contents, which leave at
+   once, took 60 us on 256 molecules at 0.5 A (4.91 -> 4.77 ms of stages with the compaction's), and a
+   block loops where a mesh has more.  A launch that leaves units idle waits for its blocks' turns: 60
+   separate atoms of 6 A at 0.5 A have 16 times the surface of a packed ball, and with blocks for that
+   ball their emission took 123 us and smoothing 75, with the pool's 23 and 14.  So a launch has blocks
+   for BLOCK_ITEMS items (four blocks per unit) where the pool has room for them: that mesh 292 -> 106 us
+   in all, 600 such atoms 499 -> 200.  With eight blocks per unit those took 108 and 194, but sheets of
+   50,000 atoms at 0.7 A, 870 and 450 us either way before, 892 and 461; with two 106 and 214. */
+constexpr uint32_t BLOCK_ITEMS = 1u << 18;
 void Engine::plan_pools()
 {
     uint64_t ev = 4096;
@@ -722,6 +729,7 @@ void Engine::plan_pools()
     pool_v = (uint32_t)std::min<uint64_t>(ev, (1ull << 31) - 1);
     pool_t = (uint32_t)std::min<uint64_t>(et, (1ull << 31) / 3 - 1);
     expect_v = mols.empty() || !n_atoms_total ? pool_v : (uint32_t)std::min(expect, (double)pool_v);
+    block_v = std::min(pool_v, std::max(expect_v, BLOCK_ITEMS));
 }
 
 /* after a run's results are read: did its pools hold the mesh?  If not, they grow to fit */
@@ -1106,7 +1114,7 @@ int Engine::run_batch(const float *d_pos, const float *d_rad, const std::vector<
             qs_launch_smooth(as<QsMol>(d_mols), d_vpre, nmol > 1 ? d_vpre + nmol + 1 : nullptr, wpre, wcoarse, as<uint32_t>(alist),
                              as<uint32_t>(vstart), as<uint64_t>(negm), as<uint64_t>(zerom), as<uint64_t>(s4), as<uint32_t>(vbw),
                              as<uint64_t>(vkey), pool_v, pool_t, as<uint64_t>(ntb), as<uint32_t>(tbw), as<int>(tri), src, dst,
-                             as<uint32_t>(totals), expect_v, filtered && it == 0 ? &compact : nullptr, stream);
+                             as<uint32_t>(totals), expect_v, block_v, filtered && it == 0 ? &compact : nullptr, stream);
             src = dst;
             dst = (dst == as<float>(vert2)) ? as<float>(vert3) : as<float>(vert2);
         }

@@ -124,12 +124,12 @@ void qs_launch_mc_emit(const QsMol *mols, const uint64_t *wpre, const uint32_t *
                        const uint32_t *acb, uint32_t *tstart, uint32_t ncube, uint32_t ntri, const uint64_t *N, const uint32_t *cnt,
                        const uint32_t *vbw, const uint32_t *tbw, const uint64_t *NT, int *tri, uint32_t vbase, uint32_t *deg_blk,
                        uint32_t *deg_total, const uint32_t *d_counts, hipStream_t s, const QsClosest *atoms = nullptr,
-                       bool starts_ready = false, uint32_t expect = ~0u);
+                       bool starts_ready = false, uint32_t block_items = ~0u);
 
 /* Launches whose item counts live on the device take them from the d_* pointers (when given),
    the host counts being the pools the launch covers: marching-cubes totals are counts[0]
-   triangles, counts[1] vertices, counts[2] active words, counts[4] cubes.  expect: items to launch
-   blocks for (at most the host count's); if there are more, the blocks loop. */
+   triangles, counts[1] vertices, counts[2] active words, counts[4] cubes.  block_items: items to
+   launch blocks for (at most the host count's); if there are more, the blocks loop. */
 
 /* per-molecule first vertex (vpre, u32) and first triangle (tpre, u64) from the word scans at each
    molecule's first word (wpre[m]; at or past the nw scanned words for none), nmol + 1 entries
@@ -139,9 +139,10 @@ void qs_launch_mesh_bases(const uint32_t *vbw, const uint32_t *tbw, const uint64
 
 /* per-vertex stages */
 void qs_launch_closest_atom(const QsMol *mols, const uint32_t *vpre, const uint32_t *vcoarse, const QsClosest &A,
-                            const float *vert, uint32_t nv, const uint32_t *d_nv, uint32_t expect, hipStream_t s);
+                            const float *vert, uint32_t nv, const uint32_t *d_nv, uint32_t block_items, hipStream_t s);
 /* one Laplacian pass over the pools of nv vertices and ntri triangles (list, vstart: the active words
-   and each 256-vertex block's first one).  compact (may be NULL; at most TRI_SELF_BLOCKS blocks of
+   and each 256-vertex block's first one).  expect: the vertices to expect, which choose the kernel.
+   compact (may be NULL; at most TRI_SELF_BLOCKS blocks of
    triangles): qs_launch_tri_compact_one's work in the same launch, its counts from d_counts */
 struct QsCompact {
     const uint32_t *deg_blk;
@@ -152,7 +153,7 @@ void qs_launch_smooth(const QsMol *mols, const uint32_t *vpre, const uint32_t *v
                       const uint32_t *list, const uint32_t *vstart, const uint64_t *N, const uint64_t *Zm, const uint64_t *S4,
                       const uint32_t *vbw, const uint64_t *vkey, uint32_t nv, uint32_t ntri, const uint64_t *NT,
                       const uint32_t *tbw, const int *tri, const float *src, float *dst, const uint32_t *d_counts, uint32_t expect,
-                      const QsCompact *compact, hipStream_t s);
+                      uint32_t block_items, const QsCompact *compact, hipStream_t s);
 
 /* Laplacian passes over a triangle array (meshes built in x-slabs): per-vertex incidence counts
    (cnt, nv entries, cleared by the caller) from the triangles, then, after an exclusive scan of

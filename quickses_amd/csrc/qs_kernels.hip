@@ -4234,7 +4234,7 @@ void qs_launch_mc_emit(const QsMol *mols, const uint64_t *wpre, const uint32_t *
                        const uint32_t *acb, uint32_t *tstart, uint32_t ncube, uint32_t ntri, const uint64_t *N, const uint32_t *cnt,
                        const uint32_t *vbw, const uint32_t *tbw, const uint64_t *NT, int *tri, uint32_t vbase, uint32_t *deg_blk,
                        uint32_t *deg_total, const uint32_t *d_counts, hipStream_t s, const QsClosest *atoms, bool starts_ready,
-                       uint32_t expect)
+                       uint32_t block_items)
 {
     if (!nact || (!nv && !ntri)) return;
     /* the per-block degenerate counts start at zero (the triangle kernel adds to them), over the
@@ -4245,7 +4245,8 @@ void qs_launch_mc_emit(const QsMol *mols, const uint64_t *wpre, const uint32_t *
     if (!starts_ready)
         hipLaunchKernelGGL(k_block_starts, dim3(pgrid(nblk(std::max<uint32_t>(nact, nzero), 256)), 2), dim3(256), 0, s, sv, st,
                            nact, d_counts ? d_counts + 2 : nullptr);
-    const unsigned gv = nv ? pgrid(nblk(std::min(nv, expect), 256)) : 0u, gt = ntri ? pgrid(nblk(std::min(ncube, expect), 256)) : 0u;
+    const unsigned gv = nv ? pgrid(nblk(std::min(nv, block_items), 256)) : 0u,
+                   gt = ntri ? pgrid(nblk(std::min(ncube, block_items), 256)) : 0u;
     if (atoms && gv && gt) {
         hipLaunchKernelGGL((k_mc_emit<true, true, true>), dim3(gv + gt), dim3(256), 0, s, mols, wpre, wcoarse, list, avb,
                                                                                           vstart, nact, nv, S4, F, outm, shellm,
@@ -4279,10 +4280,10 @@ void qs_launch_smooth(const QsMol *mols, const uint32_t *vpre, const uint32_t *v
                       const uint32_t *list, const uint32_t *vstart, const uint64_t *N, const uint64_t *Zm, const uint64_t *S4,
                       const uint32_t *vbw, const uint64_t *vkey, uint32_t nv, uint32_t ntri, const uint64_t *NT,
                       const uint32_t *tbw, const int *tri, const float *src, float *dst, const uint32_t *d_counts, uint32_t expect,
-                      const QsCompact *compact, hipStream_t s)
+                      uint32_t block_items, const QsCompact *compact, hipStream_t s)
 {
     if (!nv) return;
-    const dim3 grid(pgrid(nblk(std::min(nv, expect), 256)));
+    const dim3 grid(pgrid(nblk(std::min(nv, block_items), 256)));
     if (compact) {
         const unsigned nbs = grid.x, nbc = std::max(1u, std::min(nblk(ntri, 256), COMPACT_BLOCKS));
         hipLaunchKernelGGL((k_smooth<false, true>), dim3(nbs + nbc), dim3(256), 0, s, mols, vpre, vcoarse, wpre, wcoarse, list, vstart,
@@ -4314,10 +4315,10 @@ void qs_launch_vertex_colors(const QsMol *mols, const uint32_t *vpre, const uint
 }
 
 void qs_launch_closest_atom(const QsMol *mols, const uint32_t *vpre, const uint32_t *vcoarse, const QsClosest &A,
-                            const float *vert, uint32_t nv, const uint32_t *d_nv, uint32_t expect, hipStream_t s)
+                            const float *vert, uint32_t nv, const uint32_t *d_nv, uint32_t block_items, hipStream_t s)
 {
     if (!nv) return;
-    hipLaunchKernelGGL(k_closest_atom, dim3(pgrid(nblk(std::min(nv, expect), 256))), dim3(256), 0, s, mols, vpre, vcoarse, vert, nv,
+    hipLaunchKernelGGL(k_closest_atom, dim3(pgrid(nblk(std::min(nv, block_items), 256))), dim3(256), 0, s, mols, vpre, vcoarse, vert, nv,
                        d_nv, A);
 }
 

@@ -50,3 +50,25 @@ def test_fetch_after_a_refused_call(qs, orc, kind):
     g = qs.last_grid()["g"]
     assert _fetch(qs, "field", 4 * g ** 3 - 1) == -1
     assert np.array_equal(qs.fetch("field", np.float32, g ** 3).view(np.uint32), orc.field(pos, rad, 0.5)[6].view(np.uint32))
+
+
+def test_emission_of_more_surface_than_a_packed_ball(qs):
+    """Sixty separate atoms of 6 A have as many vertices as 3,000 packed ones: a launch must have blocks
+    for them, not for sixty packed atoms (blocks that looped took six times the packed mesh's time)."""
+    rng = np.random.default_rng(1)
+    apart = ((rng.random((60, 3)) * 40).astype(np.float32), np.full(60, 6.0, np.float32))
+    packed = qs.synth_ball(92, 3000)
+    times = {}
+    qs.set_option("timing", 1)
+    try:
+        for name, (pos, rad) in (("apart", apart), ("packed", packed)):
+            print("case emission time: %s" % name, flush=True)
+            rows = []
+            for _ in range(12):
+                V = qs.compute_ses(pos, rad, 0.5, 1)[0]
+                t = qs.stage_times()
+                rows.append(t["mc_emit"] + t.get("closest_atom", 0.0) + t["smooth"])
+            times[name] = float(np.median(rows[2:])) / len(V)
+    finally:
+        qs.set_option("timing", 0)
+    assert times["apart"] < 2.5 * times["packed"], times
