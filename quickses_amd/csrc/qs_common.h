@@ -39,7 +39,10 @@ struct QsNormFlags {
    offsets within it: a negative voxel next to a voxel whose nearest outside voxel lies r steps along
    an axis may see it no longer.  That takes a non-negative value at norm r^2, so a probe of r whole
    voxels (`edge`): then far voxels (n >= hi, or none in reach) with an outside voxel r + 1 steps away
-   along an axis are stored too.  `all`: every shell voxel is stored. */
+   along an axis are stored too.  `all`: every shell voxel with n > lo is stored.  With lo = -1 that is
+   the whole field.  Normals read the neighbours of those two ends too, so with lo a step further from
+   the probe radius (a voxel that near to the outside has only positive ones within two steps) they
+   have what they read; above it there is no bound within the window that leaves much out. */
 struct QsBand {
     int lo, hi;
     int edge, all;

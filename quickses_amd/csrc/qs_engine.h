@@ -105,11 +105,14 @@ void load_default_tuning();
 /* pass-2 candidate tables: window offsets sorted by squared norm, and for each minimal norm the
    end of the range of norms whose float distance can still be the minimum                      */
 
+/* the shell values that field pass 2 stores: those the mesh reads, those its normals read too, all */
+enum FieldKeep { KEEP_MESH = 0, KEEP_NORMALS = 1, KEEP_ALL = 2 };
+
 struct OffsetTables {
     int r = -1;
     float dx = 0, cmax = 0, bound = 0;
     std::vector<int> offs, norm_start, enum_end;
-    QsBand band = {0, 255, 0, 1};
+    QsBand band[3] = {{-1, 255, 0, 1}, {-1, 255, 0, 1}, {-1, 255, 0, 1}}; /* by FieldKeep */
 };
 
 void build_offset_tables(int r, float dx, float coord_max, OffsetTables &T);
@@ -186,7 +189,7 @@ struct P2Tables {
     DevBuf dev; /* offs, then norm_start, then enum_end; none when every norm is decided by flags */
     size_t norm_at, end_at;
     QsNormFlags flags;
-    QsBand band;
+    QsBand band[3];
     const int *offs() const { return (const int *)dev.p; }
     const int *norm() const { return dev.p ? (const int *)dev.p + norm_at : nullptr; }
     const int *end() const { return dev.p ? (const int *)dev.p + end_at : nullptr; }
@@ -315,10 +318,11 @@ struct Engine {
     /* field holds shell voxels' values only (field pass 2), the others come from outm / shellm; else
        it holds every voxel.  In grid order either way. */
     bool field_sparse = false;
-    /* the stored shell values are those the mesh reads only (QsBand); complete_field evaluates the
-       rest.  normals_used: the last result's normals were asked for, so the next run stores every
-       value at once, as its normals would need them (the mesh is the same either way) */
-    bool field_band = false, normals_used = false;
+    /* the shell values that are stored (complete_field evaluates more).  normals_used: the last result's
+       normals were asked for, so the next run stores what its normals would read at once (the mesh is
+       the same either way) */
+    FieldKeep field_kept = KEEP_ALL;
+    bool normals_used = false;
     const uint8_t *run_flags = nullptr; /* the run's tile marks, null when field pass 1 set none */
     /* the last run's atom ids are cell-sorted positions (option atom_ids_sorted at run time) */
     bool ids_sorted = false;
@@ -342,7 +346,8 @@ struct Engine {
     void forget_grid()
     {
         grid_valid = batch_valid = false;
-        field_sparse = field_band = false;
+        field_sparse = false;
+        field_kept = KEEP_ALL;
         run_flags = nullptr;
         groups.clear();
     }
@@ -480,8 +485,8 @@ struct Engine {
     int run_batch(const float *d_pos, const float *d_rad, const std::vector<MolIn> &in, int smooth,
                   const std::vector<BBox> *host_bbox);
     int field_stage(uint32_t nb_p1, size_t at_p1, StageTimer &tm);
-    int run_pass2(bool all);
-    int complete_field();
+    int run_pass2(FieldKeep keep);
+    int complete_field(FieldKeep keep);
     int fill_field(const void **dense);
     int mesh_stage(size_t at_mc, uint32_t nb_mc, size_t at_wpre, StageTimer &tm, bool with_atoms);
     int group_tables(P2Group &grp);

@@ -230,12 +230,17 @@ void build_offset_tables(int r, float dx, float coord_max, OffsetTables &T)
         if (d + delta < probe) klo = n;
         if (d - delta <= probe) khi = n;
     }
-    T.band = QsBand{0, 255, 0, 1};
+    for (QsBand &b : T.band) b = QsBand{-1, 255, 0, 1};
     if (klo >= 0 && khi <= r * r && nmax < 255) {
-        int lo = -1;
-        while (std::sqrt((double)(lo + 1)) + 1.0 <= std::sqrt((double)klo) + 1e-9) lo++;
+        /* the largest norm that a number of steps leaves at klo or below */
+        auto below = [&](double steps) {
+            int lo = -1;
+            while (std::sqrt((double)(lo + 1)) + steps <= std::sqrt((double)klo) + 1e-9) lo++;
+            return lo;
+        };
         const double far = std::sqrt((double)khi) + 1.0;
-        T.band = QsBand{lo, std::min((int)std::floor(far * far + 1e-9) + 1, 255), khi == r * r ? 1 : 0, 0};
+        T.band[KEEP_MESH] = QsBand{below(1.0), std::min((int)std::floor(far * far + 1e-9) + 1, 255), khi == r * r ? 1 : 0, 0};
+        T.band[KEEP_NORMALS].lo = below(2.0);
     }
 }
 
@@ -484,7 +489,7 @@ int Engine::group_tables(P2Group &grp)
     OffsetTables T;
     build_offset_tables(grp.r, grp.dx, grp.cmax, T);
     P2Tables *t = new P2Tables{grp.r, grp.dx, grp.cmax, DevBuf{}, T.offs.size(), T.offs.size() + T.norm_start.size(),
-                               QsNormFlags{{0, 0, 0, 0}}, T.band};
+                               QsNormFlags{{0, 0, 0, 0}}, {T.band[0], T.band[1], T.band[2]}};
     bool decided = grp.path == 0;
     for (int n = 0; n < 256 && n + 1 < (int)T.norm_start.size(); n++) {
         if (T.enum_end[n] == T.norm_start[n + 1]) t->flags.w[n >> 6] |= 1ull << (n & 63);
@@ -540,22 +545,21 @@ int Engine::field_stage(uint32_t nb_p1, size_t at_p1, StageTimer &tm)
     }
     tm.mark("pass1");
     run_flags = tf;
-    QS_TRY(run_pass2(normals_used));
+    QS_TRY(run_pass2(normals_used ? KEEP_NORMALS : KEEP_MESH));
     normals_used = false;
     field_sparse = true;
     tm.mark("pass2");
     return 0;
 }
 
-/* field pass 2 over every molecule: the values a mesh reads, or all */
-int Engine::run_pass2(bool all)
+/* field pass 2 over every molecule */
+int Engine::run_pass2(FieldKeep keep)
 {
-    field_band = false;
+    field_kept = KEEP_ALL;
     for (auto &grp : groups) {
         QS_TRY(group_tables(grp));
-        QsBand band = grp.tab->band;
-        if (all) band = QsBand{0, 255, 0, 1};
-        if (grp.path == 0 && !band.all) field_band = true;
+        const QsBand band = grp.tab->band[keep];
+        if (grp.path == 0 && !(band.all && band.lo < 0)) field_kept = keep;
         qs_launch_pass2(batch(grp.bpre_at, grp.mid_at, (int)grp.mols.size()), grp.nblocks, grp.r, grp.path, as<uint64_t>(outm),
                         as<uint64_t>(shellm), as<float>(field), as<uint32_t>(negm), as<uint32_t>(zerom),
                         grp.tab->offs(), grp.tab->norm(), grp.tab->end(), grp.tab->flags, band,
@@ -566,10 +570,14 @@ int Engine::run_pass2(bool all)
 }
 
 /* the shell values that the last run left out (its masks and tile marks are still there; the
-   sign words are written again with the same bits) */
-int Engine::complete_field()
+   sign words are written again with the same bits).  Normals asked for once, after a run that stored
+   what the mesh reads, take this pass and their own kernel: on 50,000 atoms at 0.2 A 0.45 + 0.29 ms
+   after a mesh of 1.30 (with every shell value in both runs 0.29 after 1.86), on 2,000 at 0.5 A 41 us
+   after 98.  A run that stores what normals read at once takes 1.37 ms and 105 us, 5 to 11 % more than
+   one that does not, so only a program that asks for normals every time gets it. */
+int Engine::complete_field(FieldKeep keep)
 {
-    return field_sparse && field_band ? run_pass2(true) : 0;
+    return field_sparse && field_kept < keep ? run_pass2(keep) : 0;
 }
 
 /* every voxel of every molecule's field (pass 2 stores the shell voxels only):
@@ -578,7 +586,7 @@ int Engine::fill_field(const void **dense)
 {
     *dense = field.p;
     if (!field_sparse) return 0;
-    QS_TRY(complete_field());
+    QS_TRY(complete_field(KEEP_ALL));
     QS_TRY(ensure(field_dense, std::max<uint64_t>(vox_total, 1) * 4));
     for (const QsMol &M : mols)
         qs_launch_field_expand(as<float>(field) + M.vox_off, as<uint64_t>(outm) + M.word_off, as<uint64_t>(shellm) + M.word_off,
@@ -1852,7 +1860,7 @@ static int launch_normals(Engine &E, float *d_out)
 {
     if (!E.batch_valid) return set_error(3, "no mesh to take normals of");
     if (E.multi_slab) return set_error(3, "normals: the last mesh was built in x-slabs; its field is not kept");
-    QS_TRY(E.complete_field());
+    QS_TRY(E.complete_field(KEEP_NORMALS));
     E.normals_used = true;
     const int nmol = (int)E.mols.size();
     const uint32_t *d_vpre = as<uint32_t>(E.d_off) + (nmol + 1);
@@ -2067,7 +2075,7 @@ int qs_stage_pass2(const float *fp, const int *ip, const uint8_t *labels, float 
     QS_TRY(ensure(E.negm, E.nw_total * 8));
     QS_TRY(ensure(E.zerom, E.nw_total * 8));
     E.run_flags = nullptr;
-    QS_TRY(E.run_pass2(true));
+    QS_TRY(E.run_pass2(KEEP_ALL));
     E.field_sparse = true;
     const void *dense = nullptr;
     QS_TRY(E.fill_field(&dense));

@@ -2011,7 +2011,7 @@ __global__ void __launch_bounds__(256) k_pass2_r(QsBatch B, const uint64_t *__re
         const int a = ab / (R + 1), b = ab - a * (R + 1);
         const int rem = (set ? band.lo : band.hi - 1) - a * a - b * b; /* c^2 <= rem */
         int c = rem < 0 ? 255 : min((int)__builtin_amdgcn_sqrtf((float)rem + 0.5f), R);
-        if (band.all) c = set ? 255 : R; /* the whole window, and nothing */
+        if (band.all && !set) c = R; /* the whole window */
         zlen[set][a][b] = (uint8_t)c;
     }
     int has_shell;

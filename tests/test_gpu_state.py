@@ -72,3 +72,37 @@ def test_emission_of_more_surface_than_a_packed_ball(qs):
     finally:
         qs.set_option("timing", 0)
     assert times["apart"] < 2.5 * times["packed"], times
+
+
+def _overwrite_field(qs, orc, g):
+    """Every value of a field of up to g^3 points replaced by 7 (a caller's field without a surface)."""
+    s = orc._Grid()
+    s.g, s.gn, s.r, s.reso, s.dx_n = g, 1, 3, 0.5, 3.2
+    V, T = qs.stage_mesh(orc.Grid(s).params(g - 1), np.full(g ** 3, 7.0, np.float32))
+    assert len(V) == 0 and len(T) == 0
+
+
+@pytest.mark.parametrize("reso,n", [(0.16, 60), (0.2, 300), (0.28, 300), (0.3, 300), (0.35, 400), (0.4, 400), (0.5, 800), (0.7, 800),
+                                    (1.0, 1500), (1.4, 1500), (1.6, 1500)])
+@pytest.mark.parametrize("offset", [0.0, 30000.0])
+def test_normals_read_stored_values_only(qs, orc, reso, n, offset):
+    """The mesh, its normals and the field read no value that their own field pass did not store: in
+    between, the field is another's.  Normals after the mesh, and from the run after (which stores what
+    they read at once), are those of the whole field."""
+    pos, rad = qs.synth_ball(93, n)
+    pos = pos + np.float32(offset)
+    print("case stored values: reso=%.2f offset=%g" % (reso, offset), flush=True)
+    want = orc.compute_ses(pos, rad, reso, 1)
+    qs.compute_ses(pos, rad, reso, 1)
+    g = qs.last_grid()["g"]
+    field = orc.field(pos, rad, reso)[6].view(np.uint32)
+    assert np.array_equal(qs.fetch("field", np.float32, g ** 3).view(np.uint32), field)
+    whole = qs.vertex_normals(len(want[0])).view(np.uint32)
+    qs.compute_ses(pos, rad, reso, 1)  # (the last run whose field pass is that of a run with normals)
+    for _ in range(2):  # after an ordinary run, then after a run with normals
+        _overwrite_field(qs, orc, g)
+        V, T, A = qs.compute_ses(pos, rad, reso, 1)
+        assert np.array_equal(T, want[1]) and np.array_equal(A, want[2])
+        assert np.array_equal(V.view(np.uint32), want[0].view(np.uint32))
+        assert np.array_equal(qs.vertex_normals(len(V)).view(np.uint32), whole)
+    assert np.array_equal(qs.fetch("field", np.float32, g ** 3).view(np.uint32), field)
