@@ -1049,10 +1049,14 @@ int Engine::run_batch(const float *d_pos, const float *d_rad, const std::vector<
         cells_lds = std::max(cells_lds, l);
         most_atoms = std::max(most_atoms, M.n_atoms);
     }
-    /* A block per molecule leaves the other units idle, which a few large molecules would have to
-       wait for: one of 10,007 atoms takes 28 us instead of 29 in six launches (and 2 us more for every
-       thousand), 100 of 10,000 take 79 instead of 147 and 256 of up to 20,000 111 instead of 188. */
-    if (one_block && (most_atoms <= 12288u || nmol >= 8)) {
+    /* A block per molecule waits for the largest one's: about 16 us and 1.74 more for every thousand of
+       its atoms, and 0.025 for every thousand of the run's.  The launches over the device take 28 us and
+       0.09 for every thousand of the run's (both for a batch; one molecule takes 6 us less either way).
+       The line between them, measured: one molecule of 7,000 atoms 103.5 us in one block and 106.0 over
+       the device (the whole call), 8,000 107.9 and 108.1, 12,288 121.5 and 111.9; 8 x 12,288 atoms (the
+       cells) 41.2 and 38.5, 12 x 12,288 41.0 and 41.5; one of 24,000 and 7 of 1,000 55.8 and 29.9;
+       16 x 24,000 66.0 and 63.8, 24 x 24,000 71.7 and 82.2; 128 x 8,000 58 and 121. */
+    if (one_block && 27ull * most_atoms <= (uint64_t)n + 200000ull) {
         const bool gather = most_atoms <= CELLS_GATHER;
         if (nmol > 1) QS_TRY(upload_mols());
         qs_launch_cells(as<QsMol>(d_mols), nmol, nmol == 1 ? &mols[0] : nullptr, cells_lds, gather, d_pos, d_rad,

@@ -222,3 +222,29 @@ def test_triangles_filtered_beside_smoothing(qs, orc, n, smooth):
     for run in range(2):
         print("case filter beside smoothing: n=%d smooth=%d run=%d" % (n, smooth, run), flush=True)
         assert _same(qs.compute_ses(pos, rad, 0.1, smooth), want)
+
+
+@pytest.mark.parametrize("sizes", [[7692], [7693], [24000] + [1000] * 7, [12000] * 10, [12000] * 11, [10000, 9000, 500, 30000], [2] * 300])
+def test_cells_on_both_sides_of_the_block_rule(qs, sizes):
+    """A block per molecule or launches over the device, by the largest molecule's atoms and the run's."""
+    test_cells_in_one_block_or_several_launches(qs, sizes, 0)
+
+
+def test_cells_of_one_large_molecule_in_a_batch(qs):
+    """A batch does not wait for one block that sorts its largest molecule (55 us, where the molecule
+    alone takes 24 over the device)."""
+    small = [qs.synth_ball(95 + k, 1000) for k in range(7)]
+    large = qs.synth_ball(94, 24000)
+    times = {}
+    qs.set_option("timing", 1)
+    try:
+        for name, mols in (("alone", [large]), ("with small ones", [large] + small)):
+            print("case cells: one large molecule %s" % name, flush=True)
+            rows = []
+            for _ in range(12):
+                qs.compute_batch(mols, 2.0, 0)
+                rows.append(qs.stage_times()["cells"])
+            times[name] = float(np.median(rows[2:]))
+    finally:
+        qs.set_option("timing", 0)
+    assert times["with small ones"] < 1.8 * times["alone"], times
