@@ -493,7 +493,7 @@ struct Engine {
     void plan_pools();
     bool pools_overflowed(uint32_t nv_, uint32_t nt_);
     /* x-slab form of one molecule's field and mesh stages: owned planes per slab (0: one pass) */
-    int slab_plan(const QsMol &M, int &planes);
+    int slab_plan(const QsMol &M, int smooth, int &planes);
     int run_slabs(int planes, int smooth, StageTimer &tm);
     int slab_mesh(size_t at_mc, uint32_t nb_mc, size_t at_wpre, uint64_t owned_word, uint32_t vbase, uint32_t tbase,
                   uint32_t &n_owned, uint32_t &n_tri);

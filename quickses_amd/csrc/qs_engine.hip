@@ -779,8 +779,9 @@ static uint64_t plane_bytes(const QsMol &M)
    0 when the whole grid runs at once: that is when it fits the memory budget and its grid points
    fit 32-bit indexes (the grid-walk smoothing keys them so).  Option slab_planes forces slabs of
    that many planes; option slab_mb sets the budget (default: half the device's free memory, which
-   takes 13 us to ask for and is not asked for a grid that the engine's arrays already hold). */
-int Engine::slab_plan(const QsMol &M, int &planes)
+   takes 13 us to ask for and is not asked where the engine's arrays already hold the grid and the mesh
+   pools, so that a whole-grid run allocates next to nothing). */
+int Engine::slab_plan(const QsMol &M, int smooth, int &planes)
 {
     planes = 0;
     const int g = M.G.g, R = M.G.r;
@@ -796,6 +797,10 @@ int Engine::slab_plan(const QsMol &M, int &planes)
         held = held && outm.cap >= nw * 8 + OUTM_PAD;
         for (const DevBuf *b : {&shellm, &negm, &zerom}) held = held && b->cap >= nw * 8;
         for (const DevBuf *b : {&wcnt, &vbw, &tbw, &alist, &avb, &acb}) held = held && b->cap >= nw * 4;
+        plan_pools();
+        held = held && vkey.cap >= (size_t)pool_v * 8 && atom.cap >= (size_t)pool_v * 4 && vert.cap >= (size_t)pool_v * 12;
+        held = held && (smooth < 1 || vert2.cap >= (size_t)pool_v * 12) && (smooth < 2 || vert3.cap >= (size_t)pool_v * 12);
+        held = held && tri.cap >= (size_t)pool_t * 12 && tri_out.cap >= (size_t)pool_t * 12;
         if (held) return 0;
         size_t free_b = 0, total_b = 0;
         QS_HIP(hipMemGetInfo(&free_b, &total_b));
@@ -1084,7 +1089,7 @@ int Engine::run_batch(const float *d_pos, const float *d_rad, const std::vector<
 
     /* ---- field, mesh: the whole grid at once, or one molecule in x-slabs ---- */
     int slab_planes = 0;
-    if (nmol == 1 && mols[0].G.g && !g_arena) QS_TRY(slab_plan(mols[0], slab_planes));
+    if (nmol == 1 && mols[0].G.g && !g_arena) QS_TRY(slab_plan(mols[0], smooth, slab_planes));
     if (g_arena && nmol == 1 && (uint64_t)mols[0].G.g * mols[0].G.g * mols[0].G.g >= (1ull << 32))
         return set_error(6, "grid of %d^3 points: too large for the fixed scratch region", mols[0].G.g);
     /* the run's one read-back, gathered by the triangle filter's kernel (straight into the pinned
