@@ -30,8 +30,10 @@ int set_error(int code, const char *fmt, ...);
 #define QS_HIP(call)                                                                                     \
     do {                                                                                                 \
         hipError_t e_ = (call);                                                                          \
-        if (e_ != hipSuccess)                                                                            \
+        if (e_ != hipSuccess) {                                                                          \
+            (void)hipGetLastError(); /* (it would be taken for the next call's) */                       \
             return set_error(2, "%s failed: %s (%s:%d)", #call, hipGetErrorString(e_), __FILE__, __LINE__); \
+        }                                                                                                \
     } while (0)
 
 #define QS_TRY(expr)          \

@@ -108,30 +108,52 @@ def test_normals_read_stored_values_only(qs, orc, reso, n, offset):
     assert np.array_equal(qs.fetch("field", np.float32, g ** 3).view(np.uint32), field)
 
 
+class _SmallMemory:
+    """All of the device's free memory taken but for the given MiB."""
+
+    def __init__(self, mib):
+        from quickses_amd import hipmem
+
+        self.free, free, total = hipmem.free, ctypes.c_size_t(), ctypes.c_size_t()
+        self.taken = []
+        while True:
+            assert hipmem.hip().hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+            left = free.value - (mib << 20)
+            if left < (8 << 20):
+                break
+            self.taken.append(hipmem.alloc(min(left, 32 << 30)))
+
+    def __enter__(self):
+        return self
+
+    def __exit__(self, *exc):
+        for p in self.taken:
+            self.free(p)
+
+
 def test_slabs_where_the_grid_is_held_but_the_mesh_is_not(qs):
     """A grid whose arrays an earlier run left, and pools that the free memory does not hold: the
     molecule is meshed in x-slabs, as it is when nothing is held."""
-    from quickses_amd import hipmem
-
     rng = np.random.default_rng(4)
     pos = (rng.random((60000, 3)) * 60).astype(np.float32)
     pos[0], pos[1] = 0.0, 60.0
     rad = np.full(len(pos), 1.7, np.float32)
     print("case held grid, small memory", flush=True)
     qs.compute_ses(pos[:8], rad[:8], 0.2, 1)  # the same grid (41 M points), a small mesh
-    free, total = ctypes.c_size_t(), ctypes.c_size_t()
-    taken = []
-    try:
-        while True:
-            assert hipmem.hip().hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
-            left = free.value - (380 << 20)  # (the grid takes 245 MB, the pools 1 GB)
-            if left < (8 << 20):
-                break
-            taken.append(hipmem.alloc(min(left, 32 << 30)))
+    with _SmallMemory(380):  # (the grid takes 245 MB, the pools 1 GB)
         tight = qs.compute_ses(pos, rad, 0.2, 1)
-    finally:
-        for p in taken:
-            hipmem.free(p)
     whole = qs.compute_ses(pos, rad, 0.2, 1)
     assert len(whole[1]) > 0 and np.array_equal(tight[1], whole[1]) and np.array_equal(tight[2], whole[2])
     assert np.array_equal(tight[0].view(np.uint32), whole[0].view(np.uint32))
+
+
+def test_call_after_one_that_ran_out_of_memory(qs, orc):
+    """The failed call's error is not reported by the next one."""
+    n = 8 << 20  # (100 MB of positions)
+    print("case out of memory, then an ordinary call", flush=True)
+    with _SmallMemory(64):
+        with pytest.raises(qs.QuickSESError, match="memory"):
+            qs.compute_ses(np.zeros((n, 3), np.float32), np.full(n, 1.7, np.float32), 0.5, 1)
+    small = qs.synth_ball(96, 300)
+    got, want = qs.compute_ses(*small, 0.5, 1), orc.compute_ses(*small, 0.5, 1)
+    assert np.array_equal(got[1], want[1]) and np.array_equal(got[0].view(np.uint32), want[0].view(np.uint32))
