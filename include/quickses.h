@@ -102,8 +102,8 @@ int qs_compute_device(const float *d_pos, const float *d_rad, unsigned int N, fl
  * a file-scope device array that each device the library runs on holds until the process ends;
  * a molecule whose buffers do not fit (about 20 M grid points, a 20,000-atom molecule at 0.5 A
  * takes about 100 MiB) is rejected with error 6 and a message.  The mesh is written to the
- * caller's device buffers: d_vert (3 * vert_cap floats), d_atom_id (vert_cap ints), d_tri
- * (3 * tri_cap ints); when it has more vertices or triangles than that, error 5 and nothing is
+ * caller's buffers: d_vert (3 * vert_cap floats), d_atom_id (vert_cap ints), d_tri (3 * tri_cap
+ * ints), by one kernel if all are in this device's memory, else by copies; when it has more vertices or triangles than that, error 5 and nothing is
  * written.  *nvert, *nidx as for qs_compute_device (nidx = 3 * triangles).  The same mesh as
  * qs_compute_device, bit for bit; the call is synchronous.  Calls share the device's region
  * (it keeps the last call's contents, and every run clears what it needs), so calls that

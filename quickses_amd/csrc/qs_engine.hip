@@ -1447,6 +1447,17 @@ constexpr int QS_MAX_DEV = 16;
 Engine g_eng_na[QS_MAX_DEV];        /* the no-allocation entry point's engine per device */
 void *g_scratch_ptr[QS_MAX_DEV];    /* device address of `scratch` on each device */
 
+/* is p device memory of device dev, at an address of 4-byte items? */
+bool on_device(const void *p, int dev)
+{
+    hipPointerAttribute_t a{};
+    if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return a.type == hipMemoryTypeDevice && a.device == dev && ((uintptr_t)p & 3u) == 0;
+}
+
 }  // namespace
 
 /* ========================================================================================== */
@@ -1673,8 +1684,18 @@ int qs_compute_device_noalloc(const float *d_pos, const float *d_rad, unsigned i
         return set_error(5, "output capacity too small: %u vertices and %u triangles (capacity %u and %u)", E.nv, E.nt,
                          vert_cap, tri_cap);
     if ((E.nv && (!d_vert || !d_atom_id)) || (E.nt && !d_tri)) return set_error(3, "output pointer is NULL");
-    qs_launch_copy_mesh(E.res_vert, E.res_atom, E.res_tri, E.nv, E.nt, 0u, d_vert, d_atom_id, d_tri, E.stream);
-    QS_HIP(hipGetLastError());
+    /* one kernel where it can write the caller's arrays, three copies where they are on another device
+       or in host memory, which the copies reach and a kernel may not */
+    if ((!E.nv || (on_device(d_vert, dev) && on_device(d_atom_id, dev))) && (!E.nt || on_device(d_tri, dev))) {
+        qs_launch_copy_mesh(E.res_vert, E.res_atom, E.res_tri, E.nv, E.nt, 0u, d_vert, d_atom_id, d_tri, E.stream);
+        QS_HIP(hipGetLastError());
+    } else {
+        if (E.nv) {
+            QS_HIP(hipMemcpyAsync(d_vert, E.res_vert, (size_t)E.nv * 12, hipMemcpyDeviceToDevice, E.stream));
+            QS_HIP(hipMemcpyAsync(d_atom_id, E.res_atom, (size_t)E.nv * 4, hipMemcpyDeviceToDevice, E.stream));
+        }
+        if (E.nt) QS_HIP(hipMemcpyAsync(d_tri, E.res_tri, (size_t)E.nt * 12, hipMemcpyDeviceToDevice, E.stream));
+    }
     QS_HIP(hipStreamSynchronize(E.stream));
     if (nvert) *nvert = E.nv;
     if (nidx) *nidx = 3 * E.nt;

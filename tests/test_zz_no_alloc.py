@@ -85,3 +85,38 @@ def test_noalloc_errors(qs):
     finally:
         dp.free()
         dr.free()
+
+
+@pytest.mark.parametrize("kind", ["pageable", "pinned", "mixed"])
+def test_noalloc_outputs_in_host_memory(qs, kind):
+    """Output arrays that no kernel of the device may write are reached by copies."""
+    import ctypes
+
+    from quickses_amd import hipmem
+
+    pos, rad = qs.synth_ball(406, 700)
+    dp, dr = hipmem.DeviceArray(pos), hipmem.DeviceArray(rad)
+    ref = _reference(qs, hipmem, dp, dr, len(rad), 0.5, 1)
+    outs = [np.full(a.size, -7, a.dtype) for a in ref]
+    pinned, pv = [], ctypes.c_void_p()
+    ptrs = [o.ctypes.data for o in outs]
+    if kind == "pinned":
+        for o in outs:
+            assert hipmem.hip().hipHostMalloc(ctypes.byref(pv), o.nbytes, 0) == 0
+            pinned.append(pv.value)
+        ptrs = pinned
+    dev = hipmem.DeviceArray(outs[0]) if kind == "mixed" else None
+    if dev:
+        ptrs[0] = dev.ptr
+    print("case noalloc into host memory: %s" % kind, flush=True)
+    try:
+        nv, ni = qs.compute_device_noalloc(dp.ptr, dr.ptr, len(rad), 0.5, 1, ptrs[0], len(ref[0]), ptrs[1], len(ref[1]), ptrs[2])
+        assert (nv, ni) == (len(ref[0]), 3 * len(ref[1]))
+        for k, p in enumerate(pinned):
+            ctypes.memmove(outs[k].ctypes.data, p, outs[k].nbytes)
+        if dev:
+            outs[0] = hipmem.download(dev.ptr, outs[0].shape, outs[0].dtype)
+    finally:
+        for p in pinned:
+            hipmem.hip().hipHostFree(ctypes.c_void_p(p))
+    _same([o.reshape(a.shape) for o, a in zip(outs, ref)], ref)
