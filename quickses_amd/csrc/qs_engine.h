@@ -219,7 +219,7 @@ struct Engine {
 
     DevBuf in_pos, in_rad, d_off, bb_part, bb_out, d_mols, d_meta;
     DevBuf slot /* atoms by cell, in any order within one */;
-    DevBuf key /* cell and rank within the cell per atom */, count, start, perm, cse, sx, aux;
+    DevBuf count, start, perm, cse, sx, aux;
     DevBuf labels, outm, shellm, field, negm, zerom;
     DevBuf s4, wcnt /* per row word: vertex, triangle and cube counts */, vbw, tbw, alist, totals, bounds;
     DevBuf rback; /* the run's read-back: totals, vertex and kept-triangle offsets */
@@ -358,7 +358,7 @@ struct Engine {
        which the next run reuses from its start), and the cached pass-2 tables with them */
     void forget_buffers()
     {
-        for (DevBuf *b : {&in_pos, &in_rad, &d_off, &bb_part, &bb_out, &d_mols, &d_meta, &key, &count, &start,
+        for (DevBuf *b : {&in_pos, &in_rad, &d_off, &bb_part, &bb_out, &d_mols, &d_meta, &count, &start,
                           &perm, &slot, &cse, &sx, &aux, &labels, &outm, &shellm, &field, &negm, &zerom, &s4, &wcnt,
                           &vbw, &tbw, &alist, &ntb, &avb, &acb, &vstart, &tstart, &normals, &colors_in, &totals, &bounds, &rback, &vert, &vert2, &vert3, &vkey,
                           &tri, &tri_out, &atom, &deg_blk, &keeppos, &tri_loc, &scan_tmp, &wsums, &inc_cnt, &inc_start, &inc_ent,
@@ -372,7 +372,7 @@ struct Engine {
     /* frees every device buffer and the stream (the engine can be initialised again) */
     void release_all()
     {
-        for (DevBuf *b : {&in_pos, &in_rad, &d_off, &bb_part, &bb_out, &d_mols, &d_meta, &key, &count, &start,
+        for (DevBuf *b : {&in_pos, &in_rad, &d_off, &bb_part, &bb_out, &d_mols, &d_meta, &count, &start,
                           &perm, &slot, &cse, &sx, &aux, &labels, &outm, &shellm, &field, &negm, &zerom, &s4, &wcnt,
                           &vbw, &tbw, &alist, &ntb, &avb, &acb, &vstart, &tstart, &normals, &colors_in, &totals, &bounds, &rback, &vert, &vert2, &vert3, &vkey,
                           &tri, &tri_out, &atom, &deg_blk, &keeppos, &tri_loc, &scan_tmp, &wsums, &inc_cnt, &inc_start, &inc_ent,

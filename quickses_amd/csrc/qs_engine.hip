@@ -260,7 +260,6 @@ int Engine::reserve(uint64_t vox, uint64_t atoms, uint64_t cells, uint64_t verts
     QS_TRY(ensure(field, vox * 4));
     QS_TRY(ensure(in_pos, atoms * 12));
     for (DevBuf *b : {&in_rad, &perm}) QS_TRY(ensure(*b, atoms * 4));
-    QS_TRY(ensure(key, atoms * 8));
     QS_TRY(ensure(slot, atoms * 4));
     for (DevBuf *b : {&sx, &aux}) QS_TRY(ensure(*b, atoms * 16));
     QS_TRY(ensure(count, (cells + 1) * 4));
@@ -1070,16 +1069,17 @@ int Engine::run_batch(const float *d_pos, const float *d_rad, const std::vector<
             qs_launch_gather_aux(batch(at_atoms, 0, nmol), nb_atoms, as<int>(perm), d_pos, d_rad, as<float4>(sx), as<float4>(aux),
                                  stream);
     } else {
-        /* per atom its cell and rank within the cell; per cell its atom count (cleared before) */
-        QS_TRY(ensure(key, (size_t)std::max<uint32_t>(n, 1) * 8));
+        /* per atom its cell and rank within the cell, in the memory of sx, which is written after they are
+           read; per cell its atom count (cleared before) */
+        int2 *const key = as<int2>(sx);
         QS_TRY(ensure(slot, (size_t)std::max<uint32_t>(n, 1) * 4));
         QS_TRY(ensure(count, ncell * 4));
         QS_TRY(upload_mols(as<uint32_t>(count), (uint32_t)ncell));
-        if (nb_atoms) qs_launch_hash_count(batch(at_atoms, 0, nmol), nb_atoms, d_pos, as<int2>(key), as<uint32_t>(count), stream);
+        if (nb_atoms) qs_launch_hash_count(batch(at_atoms, 0, nmol), nb_atoms, d_pos, key, as<uint32_t>(count), stream);
         /* start[c] = atoms in cells < c (global); start[ncell] = n */
         QS_TRY(scan(as<uint32_t>(count), as<uint32_t>(start), ncell, as<uint32_t>(start) + ncell));
         if (n) {
-            qs_launch_scatter(as<int2>(key), (int)n, as<uint32_t>(start), as<int>(slot), stream);
+            qs_launch_scatter(key, (int)n, as<uint32_t>(start), as<int>(slot), stream);
             qs_launch_place(batch(at_atoms, 0, nmol), nb_atoms, as<uint32_t>(start), as<int>(slot), (uint32_t)ncell, d_pos,
                             d_rad, as<int>(perm), as<int2>(cse), as<float4>(sx), as<float4>(aux), stream);
         }

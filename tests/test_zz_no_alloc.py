@@ -120,3 +120,20 @@ def test_noalloc_outputs_in_host_memory(qs, kind):
         for p in pinned:
             hipmem.hip().hipHostFree(ctypes.c_void_p(p))
     _same([o.reshape(a.shape) for o, a in zip(outs, ref)], ref)
+
+
+@pytest.mark.parametrize("n,reso,smooth", [(1164000, 2.0, 1), (328600, 1.0, 1), (75300, 0.5, 1)])
+def test_noalloc_region_holds_what_it_held(qs, n, reso, smooth):
+    """Molecules that fill the region: their working buffers fit (the mesh then does not fit arrays of
+    no entries), so no buffer beside them is larger than it has to be."""
+    from quickses_amd import hipmem
+
+    pos = (np.random.default_rng(5).random((n, 3)) * (n / 0.08) ** (1 / 3)).astype(np.float32)
+    dp, dr = hipmem.DeviceArray(pos), hipmem.DeviceArray(np.full(n, 1.7, np.float32))
+    print("case noalloc full region: n=%d reso=%.1f" % (n, reso), flush=True)
+    try:
+        with pytest.raises(qs.QuickSESError, match="capacity"):
+            qs.compute_device_noalloc(dp.ptr, dr.ptr, n, reso, smooth, 0, 0, 0, 0, 0)
+    finally:
+        dp.free()
+        dr.free()
