@@ -200,7 +200,7 @@ void qs_launch_copy_mesh(const float *v, const int *a, const int *t, uint32_t nv
 void qs_launch_tri_localize(const int *tri, uint32_t nt, const uint32_t *tpre, const uint32_t *vpre, int nmol, int *out,
                             hipStream_t s);
 
-/* blocks of the persistent launches (rounded down to a multiple of 8, at least 8) */
+/* most blocks of the launches over pools (rounded down to a multiple of 8, at least 8) */
 void qs_set_persistent_blocks(uint32_t n);
 uint32_t qs_persistent_blocks(void);
 

@@ -3030,7 +3030,7 @@ __global__ void __launch_bounds__(256) k_closest_atom(const QsMol *__restrict__ 
 {
     if (d_nv) nv = min(*d_nv, nv); /* the device count within the launch's pool */
     const uint32_t nb = (nv + 255u) >> 8;
-    /* persistent blocks over the 256-vertex blocks (grid a multiple of 8: see k_mc_emit) */
+    /* persistent blocks over the 256-vertex blocks (on XCDs as in k_mc_emit) */
     for (uint32_t vb = blockIdx.x; vb < nb; vb += gridDim.x) {
         const uint32_t v = xcd_group<64>(vb, nb) * 256u + threadIdx.x;
         if (v >= nv) continue;
@@ -3082,8 +3082,10 @@ __global__ void __launch_bounds__(256) k_mc_emit(const QsMol *__restrict__ mols,
         nv = min(d_counts[1], nv);
     }
     const uint32_t nb = (nv + 255u) >> 8;
-    /* persistent blocks over the 256-vertex blocks; the grid is a multiple of 8, so block vb runs
-       on XCD vb % 8 and the renumbering keeps neighbouring rows' words on one L2 */
+    /* persistent blocks over the 256-vertex blocks: block vb runs on XCD vb % 8 and the renumbering keeps
+       neighbouring rows' words on one L2, but not in a block's later turns, whose XCD is the grid's
+       remainder by 8 away (nor the cubes' blocks behind nbv of vertices).  Grids rounded to a multiple of 8
+       took the same time: 2 M separate spheres' vertices at 1.0 A, in 8 turns, 322 and 325 us in all. */
     for (uint32_t vb = blockIdx.x; vb < nb; vb += VERT && TRI ? nbv : gridDim.x) {
     const uint32_t blk = xcd_group<64>(vb, nb);
     stage_item_words(S, avb, list, vstart, nact, nb, blk, wpre, wcoarse);
@@ -3598,7 +3600,7 @@ __global__ void __launch_bounds__(256, STAGED ? 8 : 1) k_smooth(const QsMol *__r
     nv = d_counts[1];
     const uint32_t nact = d_counts[2];
     const uint32_t nb = (nv + 255u) >> 8;
-    /* persistent blocks over the 256-vertex blocks (grid a multiple of 8: see k_mc_emit) */
+    /* persistent blocks over the 256-vertex blocks (on XCDs as in k_mc_emit) */
     for (uint32_t vb = blockIdx.x; vb < nb; vb += nblocks) {
         const uint32_t blk = xcd_group<64>(vb, nb), v = blk * 256u + threadIdx.x;
         bool staged = false;
@@ -4010,12 +4012,11 @@ __global__ void __launch_bounds__(256) k_tri_localize(const int *__restrict__ tr
 
 static inline unsigned nblk(uint64_t n, unsigned b) { return (unsigned)((n + b - 1) / b); }
 
-/* Launches over a pool of items whose count lives on the device cover the pool with blocks that
-   loop over 256-item blocks up to the count.  They use at most g_persist_blocks blocks, a multiple
-   of 8 so that a block keeps its XCD from one item block to the next.  The default is one block
-   per 256-item block of the pool (blocks past the count leave at once): fewer, longer-lived blocks
-   were slower on these gather-bound kernels (smoothing +15 % and closest atom +11 % with 2048
-   blocks, +19 % and +50 % with 1024, on the 50,000-atom 0.2 A mesh). */
+/* Launches over a pool of items whose count lives on the device have blocks that loop over 256-item
+   blocks up to the count (blocks past it leave at once), at most g_persist_blocks, by default without
+   limit.  With one block per item block of the mesh these gather-bound kernels were faster than with
+   fewer, longer-lived blocks (smoothing +15 % and closest atom +11 % with 2048 blocks, +19 % and +50 %
+   with 1024, on the 50,000-atom 0.2 A mesh). */
 static uint32_t g_persist_blocks = 1u << 30;
 
 void qs_set_persistent_blocks(uint32_t n) { g_persist_blocks = std::max<uint32_t>(8u, n & ~7u); }
