@@ -268,7 +268,7 @@ int Engine::reserve(uint64_t vox, uint64_t atoms, uint64_t cells, uint64_t verts
     for (DevBuf *b : {&vert, &vert2, &vert3}) QS_TRY(ensure(*b, verts * 12));
     QS_TRY(ensure(vkey, verts * 8));
     QS_TRY(ensure(atom, verts * 4));
-    for (DevBuf *b : {&tri, &tri_out, &tri_loc}) QS_TRY(ensure(*b, tris * 12));
+    for (DevBuf *b : {&tri, &tri_out}) QS_TRY(ensure(*b, tris * 12)); /* (results leave without tri_loc) */
     for (DevBuf *b : {&vstart, &deg_blk, &keeppos, &tstart}) QS_TRY(ensure(*b, (tris / 256 + 2) * 4));
     const size_t m = (size_t)nmol + 1;
     QS_TRY(ensure(d_off, m * 8 + 64));

@@ -157,3 +157,19 @@ def test_call_after_one_that_ran_out_of_memory(qs, orc):
     small = qs.synth_ball(96, 300)
     got, want = qs.compute_ses(*small, 0.5, 1), orc.compute_ses(*small, 0.5, 1)
     assert np.array_equal(got[1], want[1]) and np.array_equal(got[0].view(np.uint32), want[0].view(np.uint32))
+
+
+def test_server_reserves_what_its_batches_use(qs):
+    """A worker's workspace at its start: 25.2 bytes per grid point of a budget that counts 24 (every
+    buffer has as much headroom), with no buffer that nothing on the served path reads."""
+    from quickses_amd import hipmem
+
+    before, after, total = ctypes.c_size_t(), ctypes.c_size_t(), ctypes.c_size_t()
+    budget, result = 6 << 30, 64 << 20
+    print("case server workspace", flush=True)
+    qs.compute_ses(*qs.synth_ball(97, 100), 0.5, 1)  # (the library's code and its own buffers are loaded)
+    assert hipmem.hip().hipMemGetInfo(ctypes.byref(before), ctypes.byref(total)) == 0
+    with qs.Server(hbm_budget_bytes=budget, result_bytes=result, workers=1):
+        assert hipmem.hip().hipMemGetInfo(ctypes.byref(after), ctypes.byref(total)) == 0
+    used = before.value - after.value - result
+    assert 0.9 * budget < used < 1.08 * budget, used / budget
