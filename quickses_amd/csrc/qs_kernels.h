@@ -237,6 +237,5 @@ struct QsBlockStarts {
 void qs_launch_mc_scans(const uint32_t *cnt, uint64_t nw, uint32_t *sums, uint32_t *vbw,
                         uint32_t *tbw, uint32_t *list, uint32_t *avb, uint32_t *acb, uint32_t *totals, uint32_t list_base,
                         hipStream_t s, QsBlockStarts bs = QsBlockStarts{});
-void qs_launch_gather_u32(const uint32_t *src, const uint64_t *idx, int n, uint32_t *out, hipStream_t s);
 
 #endif

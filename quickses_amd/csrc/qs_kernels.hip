@@ -2531,7 +2531,6 @@ struct MCView {
 
     __device__ __forceinline__ size_t widx(int x, int y, int z) const { return ((size_t)x * g + y) * W + (z >> 6); }
     __device__ __forceinline__ bool nbit(int x, int y, int z) const { return (N[widx(x, y, z)] >> (z & 63)) & 1ull; }
-    __device__ __forceinline__ bool zbit(int x, int y, int z) const { return (Zm[widx(x, y, z)] >> (z & 63)) & 1ull; }
     __device__ __forceinline__ int cube_index(int x, int y, int z) const
     {
         int ci = (int)nbit(x, y, z);
@@ -4425,20 +4424,6 @@ void qs_launch_tile_scan(const uint32_t *in, uint32_t *out, uint64_t n, const ui
 {
     hipLaunchKernelGGL(k_tile_scan, dim3((unsigned)qs_scan_tiles(n)), dim3(SCAN_NT), 0, s, in, out, n, offsets, total,
                        self_sums);
-}
-
-/* value of a uint32 array at given indices (per-molecule boundaries of scans) */
-__global__ void k_gather_u32(const uint32_t *__restrict__ src, const uint64_t *__restrict__ idx, int n,
-                             uint32_t *__restrict__ out)
-{
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) out[i] = src[idx[i]];
-}
-
-void qs_launch_gather_u32(const uint32_t *src, const uint64_t *idx, int n, uint32_t *out, hipStream_t s)
-{
-    if (n <= 0) return;
-    hipLaunchKernelGGL(k_gather_u32, dim3(nblk(n, 256)), dim3(256), 0, s, src, idx, n, out);
 }
 
 void qs_launch_smooth_incid_build(const int *tri, uint32_t nt, uint32_t nv, uint32_t *cnt, uint32_t *start, uint32_t *ent,
