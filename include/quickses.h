@@ -205,6 +205,20 @@ int qs_stage_pass2(const float *fparams, const int *iparams, const uint8_t *labe
 int qs_stage_mesh(const float *fparams, const int *iparams, const float *field, unsigned int *nvert,
                   unsigned int *ntri, float *vert, int64_t vert_cap, int *tri, int64_t tri_cap);
 
+/* The bounds that the field passes rely on, evaluated on the host by the code they use (no GPU; for
+ * checks of them).  Return 0, or -1 for arguments out of range.
+ *   qs_rule_band      field pass 2's window half-width r, voxel size and largest coordinate: the range of
+ *                     squared window norms whose voxels are stored, band[4] = {lo, hi, edge, all}, for
+ *                     a mesh (keep 0), for its normals too (1), for the whole field (2)
+ *   qs_rule_interval  field pass 1's closed form of n z-intervals on a grid axis (origin o, g points): atom
+ *                     coordinate a, threshold ss and (x, y) sum S of the test S + (a - z)^2 < ss, root of
+ *                     ss - S: [lo, hi], and whether it decides the interval
+ *   qs_rule_rows      the rows an atom may reach along y, from its radius and its root */
+int qs_rule_band(int r, float dx, float coord_max, int keep, int *band);
+int qs_rule_interval(int n, float o, int g, float dx, const float *a, const float *ss, const float *S, const float *root, int *lo,
+                     int *hi, int *decided);
+int qs_rule_rows(int n, float o, int g, float dx, const float *a, const float *rad, const float *root, int *lo, int *hi);
+
 /* Request server (no reference counterpart; the reference meshes one molecule per synchronous
  * call).  Requests of any size and voxel size are submitted at any time; `workers` threads,
  * each with its own engine and HIP stream, take pending requests in arrival order while their

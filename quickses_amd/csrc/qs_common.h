@@ -2,6 +2,7 @@
 #ifndef QS_COMMON_H
 #define QS_COMMON_H
 
+#include <math.h>
 #include <stdint.h>
 
 #define QS_PROBE 1.4f         /* probe radius, Angstrom (Kernels.cu:26) */
@@ -84,5 +85,44 @@ struct QsBatch {
     const int *mid;
     int n;
 };
+
+/* Field pass 1: the bounds of its closed forms, for the kernel and for host checks of them. */
+#ifdef __HIPCC__
+#define QS_HD __host__ __device__ __forceinline__
+#else
+#define QS_HD inline
+#endif
+
+/* How far a float predicate's interval end may lie from its closed form along an axis of origin o
+   (|o| + g dx bounds the coordinates), in voxels: qs_interval_eps0 + qs_interval_eps1 * ss for a
+   threshold ss (see qs_closed_interval) */
+QS_HD float qs_interval_eps0(float o, int g, float dx, float inv_dx) { return 1.2e-7f * inv_dx * (fabsf(o) + 6.0f * (float)g * dx + 4.0f); }
+QS_HD float qs_interval_eps1(float inv_dx) { return 9.6e-7f * inv_dx; }
+
+/* margin of the rows an atom reaches, each of which is tested exactly: the bound above along y, and the
+   root of 4 u ss for a half-width near zero (sqrt(ss) = r + probe at most) */
+QS_HD float qs_row_margin(float o, int g, float dx, float inv_dx) { return qs_interval_eps0(o, g, dx, inv_dx) + 1.0e-3f; }
+QS_HD float qs_row_margin_r(float inv_dx) { return 6.0e-4f * inv_dx; }
+QS_HD int qs_row_lo(float yc, float h, float ym) { return (int)ceilf(yc - h - ym); }
+QS_HD int qs_row_hi(float yc, float h, float ym) { return (int)floorf(yc + h + ym); }
+
+/* The z-interval of an atom in a row (all z of [zlo, zhi] with fl(S + fl(e(z)^2)) < ss) from its closed
+   form, zc -+ h in voxel units (h2 = ss - S, h = root / dx, root within an ulp of sqrt(h2)), without
+   evaluating the predicate.  The predicate's roundings move a boundary by at most
+   u (A + g dx + 5/2 H + ss / 2H) / dx voxels and the closed form is off by at most u (4 g dx + 5 H) / dx
+   (u = 2^-24, A the largest |z| of the grid, H = sqrt(h2) <= (1 + ss) / 2), so an end that is farther
+   than eps = 2 u (A + 5 g dx + 4 + 8 ss) / dx from every grid point is decided by its side of it; the
+   bound takes H >= 1/8.  False: an end is nearer than that, or H is smaller (a few intervals in a
+   thousand). */
+QS_HD bool qs_closed_interval(float root, float h2, float zc, float inv_dx, float eps, int zlo, int zhi, int &L, int &R)
+{
+    const float h = root * inv_dx;
+    const float lo = zc - h, hi = zc + h;
+    const int l = (int)ceilf(lo), r = (int)floorf(hi);
+    L = l > zlo ? l : zlo;
+    R = r < zhi ? r : zhi;
+    const float d = fminf(fabsf(lo - rintf(lo)), fabsf(hi - rintf(hi)));
+    return d > eps && h2 > 0.015625f;
+}
 
 #endif

@@ -2115,6 +2115,39 @@ int qs_stage_pass2(const float *fp, const int *ip, const uint8_t *labels, float 
     return 0;
 }
 
+int qs_rule_band(int r, float dx, float coord_max, int keep, int *band)
+{
+    if (r < 1 || r > 64 || !(dx > 0.0f) || keep < KEEP_MESH || keep > KEEP_ALL || !band) return -1;
+    OffsetTables T;
+    build_offset_tables(r, dx, coord_max, T);
+    const QsBand &b = T.band[keep];
+    const int v[4] = {b.lo, b.hi, b.edge, b.all};
+    std::copy(v, v + 4, band);
+    return 0;
+}
+
+int qs_rule_interval(int n, float o, int g, float dx, const float *a, const float *ss, const float *S, const float *root, int *lo,
+                     int *hi, int *decided)
+{
+    if (n < 0 || g < 1 || !(dx > 0.0f) || !a || !ss || !S || !root || !lo || !hi || !decided) return -1;
+    const float inv_dx = 1.0f / dx, eps0 = qs_interval_eps0(o, g, dx, inv_dx), eps1 = qs_interval_eps1(inv_dx);
+    for (int i = 0; i < n; i++)
+        decided[i] = qs_closed_interval(root[i], ss[i] - S[i], (a[i] - o) * inv_dx, inv_dx, eps0 + eps1 * ss[i], 0, g - 1, lo[i], hi[i]);
+    return 0;
+}
+
+int qs_rule_rows(int n, float o, int g, float dx, const float *a, const float *rad, const float *root, int *lo, int *hi)
+{
+    if (n < 0 || g < 1 || !(dx > 0.0f) || !a || !rad || !root || !lo || !hi) return -1;
+    const float inv_dx = 1.0f / dx, ym0 = qs_row_margin(o, g, dx, inv_dx), ymr = qs_row_margin_r(inv_dx);
+    for (int i = 0; i < n; i++) {
+        const float h = root[i] * inv_dx, yc = (a[i] - o) * inv_dx, ym = ym0 + ymr * (rad[i] + QS_PROBE);
+        lo[i] = qs_row_lo(yc, h, ym);
+        hi[i] = qs_row_hi(yc, h, ym);
+    }
+    return 0;
+}
+
 int qs_stage_mesh(const float *fp, const int *ip, const float *field, unsigned int *nvert, unsigned int *ntri, float *vert,
                   int64_t vert_cap, int *tri, int64_t tri_cap)
 {

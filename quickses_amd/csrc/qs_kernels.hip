@@ -794,21 +794,10 @@ __device__ __forceinline__ void row_interval(const RowAtom &A, float ss, int zlo
     R = r;
 }
 
-/* The interval of row_interval from its closed form, zc -+ h in voxel units (h2 = ss - S, h = sqrt(h2)
-   / dx), without evaluating the predicate.  The predicate's roundings move a boundary by at most
-   u (A + g dx + 5/2 H + ss / 2H) / dx voxels and the closed form is off by at most u (4 g dx + 5 H) / dx
-   (u = 2^-24, A the largest |z| of the grid, H = sqrt(h2) <= (1 + ss) / 2), so an end that is farther
-   than eps = 2 u (A + 5 g dx + 4 + 8 ss) / dx from every grid point is decided by its side of it; the
-   bound takes H >= 1/8.  False: an end is nearer than that, or H is smaller (a few intervals in a
-   thousand). */
+/* the interval of row_interval from its closed form (qs_closed_interval), or false */
 __device__ __forceinline__ bool fast_interval(float h2, float zc, float inv_dx, float eps, int zlo, int zhi, int &L, int &R)
 {
-    const float h = __builtin_amdgcn_sqrtf(h2) * inv_dx;
-    const float lo = zc - h, hi = zc + h;
-    L = max((int)ceilf(lo), zlo);
-    R = min((int)floorf(hi), zhi);
-    const float d = fminf(fabsf(lo - rintf(lo)), fabsf(hi - rintf(hi)));
-    return d > eps && h2 > 0.015625f;
+    return qs_closed_interval(__builtin_amdgcn_sqrtf(h2), h2, zc, inv_dx, eps, zlo, zhi, L, R);
 }
 
 /* an atom's float thresholds of its near (r + probe) and inside (r - dx) tests, and its
@@ -1318,11 +1307,8 @@ __global__ void __launch_bounds__(256) k_pass1_slab(QsBatch B, const uint32_t *_
     for (int t = threadIdx.x; t < gn + 2; t += 256) yfirst[t] = zfirst[t] = g;
     __syncthreads();
     const float dx = G.dx, inv_dx = 1.0f / G.dx;
-    /* fast_interval's bound: eps0 + eps1 * ss (|oz| + g dx >= A) */
-    const float eps0 = 1.2e-7f * inv_dx * (fabsf(G.oz) + 6.0f * (float)g * dx + 4.0f), eps1 = 9.6e-7f * inv_dx;
-    /* margin of the rows an atom reaches, each of which is tested exactly: fast_interval's bound
-       along y, and the root of 4 u ss for a half-width near zero (sqrt(ss) = r + probe at most) */
-    const float ymargin = 1.2e-7f * inv_dx * (fabsf(G.oy) + 6.0f * (float)g * dx + 4.0f) + 1.0e-3f, ymargin_r = 6.0e-4f * inv_dx;
+    const float eps0 = qs_interval_eps0(G.oz, g, dx, inv_dx), eps1 = qs_interval_eps1(inv_dx);
+    const float ymargin = qs_row_margin(G.oy, g, dx, inv_dx), ymargin_r = qs_row_margin_r(inv_dx);
     for (int i = threadIdx.x; i < g; i += 256) {
         const int cy = min(cell_of(grid_pos(G.oy, i, dx), G.oy, G.dxn), gn + 1);
         const int cyp = i ? min(cell_of(grid_pos(G.oy, i - 1, dx), G.oy, G.dxn), gn + 1) : -1;
@@ -1390,8 +1376,8 @@ __global__ void __launch_bounds__(256) k_pass1_slab(QsBatch B, const uint32_t *_
             if (X < sD) {
                 const float h = __builtin_amdgcn_sqrtf(sD - X) * inv_dx, yc = (ay - G.oy) * inv_dx - (float)y0;
                 const float ym = ymargin + ymargin_r * (a.w + QS_PROBE);
-                r0[1] = max((int)ceilf(yc - h - ym), r0[0]);
-                nr[1] = max(min((int)floorf(yc + h + ym), rr >> 8) - r0[1] + 1, 0);
+                r0[1] = max(qs_row_lo(yc, h, ym), r0[0]);
+                nr[1] = max(min(qs_row_hi(yc, h, ym), rr >> 8) - r0[1] + 1, 0);
             }
         }
 #pragma unroll 1
@@ -1476,8 +1462,8 @@ __global__ void __launch_bounds__(256) k_pass1_slab(QsBatch B, const uint32_t *_
                     /* rows the atom can reach in y (a superset: the exact test is per row) */
                     const float h = __builtin_amdgcn_sqrtf(ax.x - X) * inv_dx, yc = (a.y - G.oy) * inv_dx;
                     const float ym = ymargin + ymargin_r * (a.w + QS_PROBE);
-                    ylo = max(ylo, (int)ceilf(yc - h - ym));
-                    yhi = min(yhi, (int)floorf(yc + h + ym));
+                    ylo = max(ylo, qs_row_lo(yc, h, ym));
+                    yhi = min(yhi, qs_row_hi(yc, h, ym));
                     const int r0 = max(ylo - y0, 0), r1 = min(yhi - y0, rows_hi);
                     /* voxels whose z cell admits the atom, labelled ones only (z <= g - 2) */
                     const int zlo = zfirst[max(acz - 1, 0)];
