@@ -159,7 +159,9 @@ int qs_batch_wait_host(int slot, const float **vert, const int **tri, const int 
  * faces); an edge vertex blends its edge's two end points with its edge parameter.
  * qs_vertex_normals copies 3 * nvert floats to host memory (nvert must equal the last mesh's
  * vertex count; after API_computeSES that is *NVert).  qs_vertex_normals_device writes them to
- * a device array and reports the kernel time in *ms (may be NULL).  Returns 0 or an error code. */
+ * a device array and reports the kernel time in *ms (may be NULL).  The first normals after meshes
+ * without any evaluate the field values that they read and the mesh did not; the next mesh then
+ * evaluates those at once.  Returns 0 or an error code. */
 int qs_vertex_normals(float *out, unsigned int nvert);
 int qs_vertex_normals_device(float *d_out, float *ms);
 
@@ -192,11 +194,12 @@ int qs_batch_grid(int m, float *fparams, int *iparams);
 /* Copies of the last computation's intermediate arrays to host memory (stage-wise checks; for
  * a batch, the concatenated arrays, and "labels" of its first molecule):
  *   "labels" uint8[g^3] (0 outside, 1 shell, 2 inside), "field" float[g^3] (every voxel: field
- *   pass 2 stores the shell voxels only, the others are filled in for the copy),
+ *   pass 2 stores the shell voxels that the mesh reads only; it runs again for the others, and the
+ *   rest is filled in for the copy),
  *   "shellm" uint64[g*g*ceil(g/64)] (shell mask, bit z%64 of word (x*g+y)*ceil(g/64)+z/64),
  *   "perm" int32[N] (cell-sorted order), "cells" int32[2*gn^3] (start,end pairs),
  *   "vert_unsmoothed" float[3*NVert], "tri_all" int32[3*T] (before the degenerate filter).
- * Returns the number of bytes copied, or -1. */
+ * Returns the number of bytes copied, or -1 (also after a computation that did not finish). */
 int64_t qs_fetch(const char *what, void *host, int64_t bytes);
 
 /* Stage entry points on caller-given inputs (host memory):

@@ -579,7 +579,7 @@ int Engine::complete_field(FieldKeep keep)
     return field_sparse && field_kept < keep ? run_pass2(keep) : 0;
 }
 
-/* every voxel of every molecule's field (pass 2 stores the shell voxels only):
+/* every voxel of every molecule's field (pass 2 stores shell voxels only):
    *dense receives the device array, molecule m at its voxel offset */
 int Engine::fill_field(const void **dense)
 {

@@ -30,7 +30,8 @@ void qs_launch_bbox(const float *pos, const float *rad, const uint32_t *off, uin
 size_t qs_cells_lds_bytes(const QsMol &m);
 void qs_launch_cells(const QsMol *mols, int nmol, const QsMol *one, size_t lds, bool gather, const float *pos, const float *rad, uint32_t *start,
                      int *perm, int2 *cse, float4 *sx, float4 *aux, hipStream_t s);
-/* key: (cell, rank within the cell) per atom; count: atoms per cell (cleared before) */
+/* key: (cell, rank within the cell) per atom (it may lie where qs_launch_place writes sx: it is read before);
+   count: atoms per cell (cleared before) */
 void qs_launch_hash_count(QsBatch B, uint32_t nblocks, const float *pos, int2 *key, uint32_t *count, hipStream_t s);
 /* slot: the atoms by cell, in any order within one */
 void qs_launch_scatter(const int2 *key, int n, const uint32_t *start, int *slot, hipStream_t s);

@@ -2806,8 +2806,8 @@ __device__ __forceinline__ void item_word(const ItemWords &S, const uint32_t *__
     }
 }
 
-/* Field value of voxel z of grid row `row` (= x * g + y).  Field pass 2 stores shell voxels only, at
-   their grid places; every other voxel is the probe radius outside and -dx inside, read from the
+/* Field value of voxel z of grid row `row` (= x * g + y).  Field pass 2 stores shell voxels only (of
+   them those that its QsBand keeps: callers read no others), at their grid places; every other voxel is the probe radius outside and -dx inside, read from the
    outside and shell masks (W words per row), which are loaded together with the place.  shellm ==
    nullptr: F holds every voxel. */
 __device__ __forceinline__ float field_at(const float *__restrict__ F, const uint64_t *__restrict__ outm,

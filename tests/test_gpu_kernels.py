@@ -224,7 +224,7 @@ def test_triangles_filtered_beside_smoothing(qs, orc, n, smooth):
         assert _same(qs.compute_ses(pos, rad, 0.1, smooth), want)
 
 
-@pytest.mark.parametrize("sizes", [[7692], [7693], [24000] + [1000] * 7, [12000] * 10, [12000] * 11, [10000, 9000, 500, 30000], [2] * 300])
+@pytest.mark.parametrize("sizes", [[7692], [7693], [24000] + [1000] * 7, [12000] * 10, [12000] * 11, [10000, 9000, 500, 30000], [2] * 300, [24576] * 18, [24576] * 19])
 def test_cells_on_both_sides_of_the_block_rule(qs, sizes):
     """A block per molecule or launches over the device, by the largest molecule's atoms and the run's."""
     test_cells_in_one_block_or_several_launches(qs, sizes, 0)
