@@ -2034,6 +2034,8 @@ int64_t qs_fetch(const char *what, void *host, int64_t bytes)
     int64_t need = 0;
     const bool grid_kept = !E.multi_slab; /* a slab run keeps only its last slab's grid arrays */
     if (!grid_kept && (w == "labels" || w == "field" || w == "shellm")) return -1;
+    /* (a mesh of a caller's field has no masks: an earlier run's may be smaller) */
+    if (!E.field_sparse && (w == "labels" || w == "shellm")) return -1;
     if (w == "labels") {
         /* molecule 0 of the last run, reconstructed from the outside / shell masks */
         const uint64_t V0 = (uint64_t)G.g * G.g * G.g;

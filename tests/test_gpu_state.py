@@ -82,6 +82,16 @@ def _overwrite_field(qs, orc, g):
     assert len(V) == 0 and len(T) == 0
 
 
+def test_fetch_after_a_mesh_of_a_callers_field(qs, orc):
+    """A caller's field comes without masks: an earlier run's, of another grid, are not read as its."""
+    qs.compute_ses(*qs.synth_ball(98, 50), 1.0, 0)
+    print("case fetch after a stage call", flush=True)
+    _overwrite_field(qs, orc, 200)
+    for what in ("labels", "shellm"):
+        assert _fetch(qs, what, 64 << 20) == -1, what
+    assert _fetch(qs, "field", 4 * 200 ** 3) == 4 * 200 ** 3
+
+
 @pytest.mark.parametrize("reso,n", [(0.16, 60), (0.2, 300), (0.28, 300), (0.3, 300), (0.35, 400), (0.4, 400), (0.5, 800), (0.7, 800),
                                     (1.0, 1500), (1.4, 1500), (1.6, 1500)])
 @pytest.mark.parametrize("offset", [0.0, 30000.0])
