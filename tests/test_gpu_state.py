@@ -122,19 +122,22 @@ class _SmallMemory:
     """All of the device's free memory taken but for the given MiB."""
 
     def __init__(self, mib):
+        self.mib, self.taken = mib, []
+
+    def __enter__(self):
         from quickses_amd import hipmem
 
         self.free, free, total = hipmem.free, ctypes.c_size_t(), ctypes.c_size_t()
-        self.taken = []
         while True:
             assert hipmem.hip().hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
-            left = free.value - (mib << 20)
+            left = free.value - (self.mib << 20)
             if left < (8 << 20):
-                break
-            self.taken.append(hipmem.alloc(min(left, 32 << 30)))
-
-    def __enter__(self):
-        return self
+                return self
+            try:
+                self.taken.append(hipmem.alloc(min(left, 32 << 30)))
+            except RuntimeError:  # (the rest is in smaller pieces)
+                hipmem.hip().hipGetLastError()
+                return self
 
     def __exit__(self, *exc):
         for p in self.taken:
